@@ -1,8 +1,11 @@
 // hip_convert / hip_fp4_blockscale_to_bf16 / hip_float_to_fp4_blockscale for gfx950.
 //
-// The dequantisation pairs (FP8/FP4 -> BF16/FP32/FP16) are HBM-bound streams: each lane moves
-// 16 source bytes per step with one 128-bit load and writes its results with 128-bit stores,
-// and the grid is a fixed multiple of the CU count walking the buffer with a grid stride.
+// Every pair is an HBM-bound stream.  A lane handles as many elements as fill 16 bytes on the wider side of the pair, so
+// that both the loads and the stores of a wave are contiguous spans (a lane that stores two or four 16-byte pieces side by
+// side touches every line twice or four times), four such pieces are requested before the first is used, and the grid is a
+// fixed multiple of the CU count walking the buffer with a grid stride.  Scalar kernels take what is left: the last few
+// elements, misaligned pointers, odd block lengths.  Measured on a 4096 x 12288 weight, BF16 -> float -> FP4 with block scales
+// -> BF16 (659 MB moved): 380 -> 123 us, 5.4 TB/s, what a plain device copy reaches; float -> FP8 and back likewise (462 -> 142).
 // Numerics follow the reference kernels element for element (decode, one FP32 multiply by the
 // scale, integer round-to-nearest-even to BF16): cccc-cuda/cuda_functions.cu:2566-2596 (E4M3),
 // :2735-2785 (E5M2), :2834-2884 (FP4), :2896-2960 (FP4 block scale), :3066-3090 (dispatch).
@@ -39,50 +42,69 @@ __device__ __forceinline__ void store_one(void* dst, size_t i, float v)
     else { ((uint16_t*)dst)[i] = (uint16_t)f32_to_bf16_bits(v); }
 }
 
-// 16 consecutive results starting at element i0 (i0 % 16 == 0, dst suitably aligned)
+// A 16-byte piece of results, PIECE elements from element i0 on (dst 16-byte aligned, i0 a multiple of PIECE)
 template <int DST>
-__device__ __forceinline__ void store_sixteen(void* dst, size_t i0, const float (&v)[16])
+constexpr int kPiece = DST == DT_FLOAT ? 4 : 8;
+
+template <int DST>
+__device__ __forceinline__ void store_piece(void* dst, size_t i0, const float (&v)[kPiece<DST>])
 {
-    if (DST == DT_FLOAT)
-    {
-        f32x4* out = (f32x4*)((float*)dst + i0);
+    u32x4 p;
 #pragma unroll
-        for (int q = 0; q < 4; q++) { out[q] = f32x4{ v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3] }; }
-    }
-    else
+    for (int j = 0; j < 4; j++)
     {
-        uint32_t p[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
+        if constexpr (DST == DT_FLOAT) { p[j] = f32_to_bits(v[j]); }
+        else
         {
             const uint32_t lo = DST == DT_HALF ? f32_to_half_bits(v[2 * j]) : f32_to_bf16_bits(v[2 * j]);
             const uint32_t hi = DST == DT_HALF ? f32_to_half_bits(v[2 * j + 1]) : f32_to_bf16_bits(v[2 * j + 1]);
             p[j] = lo | (hi << 16);
         }
-        u32x4* out = (u32x4*)((uint16_t*)dst + i0);
-        out[0] = u32x4{ p[0], p[1], p[2], p[3] };
-        out[1] = u32x4{ p[4], p[5], p[6], p[7] };
     }
+    *(u32x4*)((char*)dst + i0 * (DST == DT_FLOAT ? 4 : 2)) = p;
+}
+
+constexpr int kInFlight = 4;            // pieces a lane requests before it uses the first
+
+// Walks n_pieces pieces with every lane of the grid: load(piece) -> value for up to kInFlight pieces, then use(piece, value).
+template <typename Load, typename Use>
+__device__ __forceinline__ void stream_pieces(size_t n_pieces, Load load, Use use)
+{
+    const size_t stride = (size_t)gridDim.x * kThreads;
+    size_t v = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    for (; v + (kInFlight - 1) * stride < n_pieces; v += kInFlight * stride)
+    {
+        decltype(load(v)) x[kInFlight];
+#pragma unroll
+        for (int u = 0; u < kInFlight; u++) { x[u] = load(v + u * stride); }
+#pragma unroll
+        for (int u = 0; u < kInFlight; u++) { use(v + u * stride, x[u]); }
+    }
+    for (; v < n_pieces; v += stride) { use(v, load(v)); }
 }
 
 // ---- FP8 (1 byte / element) -> FP32 / FP16 / BF16
 
 template <int SRC, int DST>
-__global__ __launch_bounds__(kThreads) void dequant8_vec_kernel(const uint8_t* __restrict__ src, void* __restrict__ dst, size_t n_vec, float scale)
+__global__ __launch_bounds__(kThreads) void dequant8_vec_kernel(const uint8_t* __restrict__ src, void* __restrict__ dst, size_t n_pieces, float scale)
 {
-    const size_t stride = (size_t)gridDim.x * kThreads;
-    for (size_t v = (size_t)blockIdx.x * kThreads + threadIdx.x; v < n_vec; v += stride)
-    {
-        const u32x4 w = __builtin_nontemporal_load((const u32x4*)src + v);
-        float out[16];
+    constexpr int P = kPiece<DST>, D = P / 4;
+    stream_pieces(n_pieces,
+        [&](size_t v) {
+            if constexpr (D == 2) { return __builtin_nontemporal_load((const u32x2*)src + v); }
+            else { return __builtin_nontemporal_load((const uint32_t*)src + v); }
+        },
+        [&](size_t v, auto w) {
+            float out[P];
 #pragma unroll
-        for (int d = 0; d < 4; d++)
-        {
-#pragma unroll
-            for (int b = 0; b < 4; b++) { out[4 * d + b] = decode8<SRC>((w[d] >> (8 * b)) & 0xFFu) * scale; }
-        }
-        store_sixteen<DST>(dst, v * 16, out);
-    }
+            for (int i = 0; i < P; i++)
+            {
+                uint32_t d;
+                if constexpr (D == 2) { d = w[i / 4]; } else { d = w; }
+                out[i] = decode8<SRC>((d >> (8 * (i & 3))) & 0xFFu) * scale;
+            }
+            store_piece<DST>(dst, v * P, out);
+        });
 }
 
 template <int SRC, int DST>
@@ -100,35 +122,51 @@ int launch_dequant8(const void* src, void* dst, unsigned n, float scale, const c
 {
     if (n == 0) { return 0; }
     const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15u) == 0;
-    const size_t n_vec = aligned ? (size_t)n / 16 : 0;
-    if (n_vec) { dequant8_vec_kernel<SRC, DST><<<grid_for(n_vec), kThreads, 0, stream()>>>((const uint8_t*)src, dst, n_vec, scale); }
-    const size_t done = n_vec * 16;
+    const size_t n_pieces = aligned ? (size_t)n / kPiece<DST> : 0;
+    if (n_pieces) { dequant8_vec_kernel<SRC, DST><<<grid_for(n_pieces), kThreads, 0, stream()>>>((const uint8_t*)src, dst, n_pieces, scale); }
+    const size_t done = n_pieces * kPiece<DST>;
     if (done < n) { dequant8_scalar_kernel<SRC, DST><<<grid_for(n - done), kThreads, 0, stream()>>>((const uint8_t*)src, dst, done, n, scale); }
     return finish(what);
 }
 
 // ---- FP4 (two elements / byte) -> FP32 / BF16, per-tensor scale or per-block E4M3 scale
 
-// One lane handles 8 packed bytes = 16 elements.  BLOCKSCALE: elements [16 v, 16 v + 16) share one
-// scale byte when block_size % 16 == 0 (checked by the launcher).
+// A piece shares one scale byte when block_size is a multiple of its length (checked by the launcher); the shift replaces the
+// division of the piece index, the launcher passes log2(block_size / piece) and falls back to the scalar kernel otherwise.
+// The nibbles are decoded by the hardware conversion, two at a time, after code 8 (+0.0 in the reference's table, not -0.0)
+// has been cleared: 50 M elements of a 4096 x 12288 weight with the software decoder took 35.5 us, 3.6 TB/s.
 template <int DST, bool BLOCKSCALE>
 __global__ __launch_bounds__(kThreads) void dequant4_vec_kernel(const uint8_t* __restrict__ src, const uint8_t* __restrict__ scales,
-                                                               void* __restrict__ dst, size_t n_vec, unsigned block_size, float scale)
+                                                               void* __restrict__ dst, size_t n_pieces, int block_shift, float scale)
 {
-    const size_t stride = (size_t)gridDim.x * kThreads;
-    for (size_t v = (size_t)blockIdx.x * kThreads + threadIdx.x; v < n_vec; v += stride)
-    {
-        const u32x2 w = __builtin_nontemporal_load((const u32x2*)src + v);
-        const float s = BLOCKSCALE ? e4m3_to_f32(scales[(v * 16) / block_size]) : scale;
-        float out[16];
-#pragma unroll
-        for (int d = 0; d < 2; d++)
-        {
-#pragma unroll
-            for (int q = 0; q < 8; q++) { out[8 * d + q] = fp4_to_f32((w[d] >> (4 * q)) & 0xFu) * s; }
-        }
-        store_sixteen<DST>(dst, v * 16, out);
-    }
+    constexpr int P = kPiece<DST>;
+    struct Piece { uint32_t w, s; };
+    stream_pieces(n_pieces,
+        [&](size_t v) {
+            Piece p;
+            p.w = P == 8 ? __builtin_nontemporal_load((const uint32_t*)src + v) : (uint32_t)__builtin_nontemporal_load((const uint16_t*)src + v);
+            p.s = BLOCKSCALE ? scales[v >> block_shift] : 0u;
+            return p;
+        },
+        [&](size_t v, const Piece& p) {
+            const float s = BLOCKSCALE ? e4m3_to_f32(p.s) : scale;
+            const uint32_t mag = p.w & 0x77777777u;
+            const uint32_t w = mag | (p.w & (mag + 0x77777777u) & 0x88888888u);       // sign bits of the non-zero magnitudes only
+            float out[P];
+#define CCQ_PAIR(i)                                                                                  \
+            if constexpr (2 * (i) < P)                                                               \
+            {                                                                                        \
+                const f32x2 f = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, i);                \
+                out[2 * (i)] = f[0] * s;                                                             \
+                out[2 * (i) + 1] = f[1] * s;                                                         \
+            }
+            CCQ_PAIR(0)
+            CCQ_PAIR(1)
+            CCQ_PAIR(2)
+            CCQ_PAIR(3)
+#undef CCQ_PAIR
+            store_piece<DST>(dst, v * P, out);
+        });
 }
 
 template <int DST, bool BLOCKSCALE>
@@ -149,14 +187,17 @@ template <int DST, bool BLOCKSCALE>
 int launch_dequant4(const void* src, const void* scales, void* dst, unsigned n, unsigned block_size, float scale, const char* what)
 {
     if (n == 0) { return 0; }
-    const bool aligned = (((uintptr_t)src & 7u) | ((uintptr_t)dst & 15u)) == 0;
-    const bool vec_ok = aligned && (!BLOCKSCALE || block_size % 16 == 0);
-    const size_t n_vec = vec_ok ? (size_t)n / 16 : 0;
-    if (n_vec)
+    constexpr unsigned P = kPiece<DST>;
+    const bool aligned = (((uintptr_t)src & 3u) | ((uintptr_t)dst & 15u)) == 0;
+    int block_shift = 0;
+    while ((P << block_shift) < block_size && block_shift < 26) { block_shift++; }
+    const bool vec_ok = aligned && (!BLOCKSCALE || (P << block_shift) == block_size);
+    const size_t n_pieces = vec_ok ? (size_t)n / P : 0;
+    if (n_pieces)
     {
-        dequant4_vec_kernel<DST, BLOCKSCALE><<<grid_for(n_vec), kThreads, 0, stream()>>>((const uint8_t*)src, (const uint8_t*)scales, dst, n_vec, block_size, scale);
+        dequant4_vec_kernel<DST, BLOCKSCALE><<<grid_for(n_pieces), kThreads, 0, stream()>>>((const uint8_t*)src, (const uint8_t*)scales, dst, n_pieces, block_shift, scale);
     }
-    const size_t done = n_vec * 16;
+    const size_t done = n_pieces * P;
     if (done < n)
     {
         dequant4_scalar_kernel<DST, BLOCKSCALE><<<grid_for(n - done), kThreads, 0, stream()>>>((const uint8_t*)src, (const uint8_t*)scales, dst, done, n, block_size, scale);
@@ -164,7 +205,7 @@ int launch_dequant4(const void* src, const void* scales, void* dst, unsigned n, 
     return finish(what);
 }
 
-// ---- the remaining pairs of the table: one element per lane, not on the hot path
+// ---- casts and encoders
 
 // Truncating encoders of the reference (cccc-cuda/cuda_functions.cu:2382-2412, :2694-2724, :2796-2832)
 __device__ __forceinline__ uint32_t f32_to_e5m2_trunc(float f)
@@ -222,33 +263,108 @@ __device__ __forceinline__ float load_plain(const void* src, int type, size_t i)
     return bf16_bits_to_f32(((const uint16_t*)src)[i]);
 }
 
+__device__ __forceinline__ uint32_t cast_bits(float v, int dst_type)
+{
+    if (dst_type == DT_HALF) { return f32_to_half_bits(v); }
+    return (v != v) ? ((f32_to_bits(v) >> 16) | 0x40u) : f32_to_bf16_bits(v);
+}
+
 // Plain casts (no scale): float->bf16, half->float, half->bf16, bf16->float, bf16->half.
 // BF16 results round to nearest even; NaN inputs stay NaN (quiet bit forced).
-__global__ __launch_bounds__(kThreads) void cast_kernel(const void* __restrict__ src, int src_type, void* __restrict__ dst, int dst_type, size_t n)
+__global__ __launch_bounds__(kThreads) void cast_kernel(const void* __restrict__ src, int src_type, void* __restrict__ dst, int dst_type, size_t begin, size_t n)
 {
     const size_t stride = (size_t)gridDim.x * kThreads;
-    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
+    for (size_t i = begin + (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
     {
         const float v = load_plain(src, src_type, i);
         if (dst_type == DT_FLOAT) { ((float*)dst)[i] = v; }
-        else if (dst_type == DT_HALF) { ((uint16_t*)dst)[i] = (uint16_t)f32_to_half_bits(v); }
-        else
-        {
-            const uint32_t bits = (v != v) ? ((f32_to_bits(v) >> 16) | 0x40u) : f32_to_bf16_bits(v);
-            ((uint16_t*)dst)[i] = (uint16_t)bits;
-        }
+        else { ((uint16_t*)dst)[i] = (uint16_t)cast_bits(v, dst_type); }
     }
 }
 
+// Four consecutive values of a plain type as floats: one 16-byte or 8-byte load
+template <int SRC>
+struct Quad
+{
+    typedef u32x2 raw;
+    __device__ static float at(const raw& r, int i)
+    {
+        const uint32_t h = (r[i >> 1] >> (16 * (i & 1))) & 0xFFFFu;
+        return SRC == DT_HALF ? half_bits_to_f32(h) : bf16_bits_to_f32(h);
+    }
+};
+template <>
+struct Quad<DT_FLOAT>
+{
+    typedef u32x4 raw;
+    __device__ static float at(const raw& r, int i) { return bits_to_f32(r[i]); }
+};
+
+// The same casts, four elements per lane and step (4096 x 12288 BF16 -> float: 95 us one element at a time).
+template <int SRC, int DST>
+__global__ __launch_bounds__(kThreads) void cast_vec_kernel(const void* __restrict__ src, void* __restrict__ dst, size_t n_quads)
+{
+    stream_pieces(n_quads,
+        [&](size_t v) { return __builtin_nontemporal_load((const typename Quad<SRC>::raw*)src + v); },
+        [&](size_t v, const typename Quad<SRC>::raw& r) {
+            if constexpr (DST == DT_FLOAT)
+            {
+                ((f32x4*)dst)[v] = f32x4{ Quad<SRC>::at(r, 0), Quad<SRC>::at(r, 1), Quad<SRC>::at(r, 2), Quad<SRC>::at(r, 3) };
+            }
+            else
+            {
+                uint32_t b[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) { b[i] = cast_bits(Quad<SRC>::at(r, i), DST); }
+                ((u32x2*)dst)[v] = u32x2{ b[0] | (b[1] << 16), b[2] | (b[3] << 16) };
+            }
+        });
+}
+
+template <int SRC, int DST>
+int launch_cast(const void* src, void* dst, unsigned n)
+{
+    const bool aligned = (((uintptr_t)src | (uintptr_t)dst) & 15u) == 0;
+    const size_t n_quads = aligned ? (size_t)n / 4 : 0;
+    if (n_quads) { cast_vec_kernel<SRC, DST><<<grid_for(n_quads), kThreads, 0, stream()>>>(src, dst, n_quads); }
+    const size_t done = n_quads * 4;
+    if (done < n) { cast_kernel<<<grid_for(n - done), kThreads, 0, stream()>>>(src, SRC, dst, DST, done, n); }
+    return finish("convert_cast");
+}
+
 // Quantising casts: float|bf16 -> e4m3, float -> e5m2 (value * scale, truncating encoders).
-__global__ __launch_bounds__(kThreads) void encode8_kernel(const void* __restrict__ src, int src_type, uint8_t* __restrict__ dst, int dst_type, size_t n, float scale)
+template <int DST>
+__device__ __forceinline__ uint32_t encode8(float v) { return DST == DT_E5M2 ? f32_to_e5m2_trunc(v) : f32_to_e4m3_trunc(v); }
+
+template <int SRC, int DST>
+__global__ __launch_bounds__(kThreads) void encode8_kernel(const void* __restrict__ src, uint8_t* __restrict__ dst, size_t begin, size_t n, float scale)
 {
     const size_t stride = (size_t)gridDim.x * kThreads;
-    for (size_t i = (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
-    {
-        const float v = load_plain(src, src_type, i) * scale;
-        dst[i] = (uint8_t)(dst_type == DT_E5M2 ? f32_to_e5m2_trunc(v) : f32_to_e4m3_trunc(v));
-    }
+    for (size_t i = begin + (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) { dst[i] = (uint8_t)encode8<DST>(load_plain(src, SRC, i) * scale); }
+}
+
+template <int SRC, int DST>
+__global__ __launch_bounds__(kThreads) void encode8_vec_kernel(const void* __restrict__ src, uint8_t* __restrict__ dst, size_t n_quads, float scale)
+{
+    stream_pieces(n_quads,
+        [&](size_t v) { return __builtin_nontemporal_load((const typename Quad<SRC>::raw*)src + v); },
+        [&](size_t v, const typename Quad<SRC>::raw& r) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) { w |= encode8<DST>(Quad<SRC>::at(r, i) * scale) << (8 * i); }
+            ((uint32_t*)dst)[v] = w;
+        });
+}
+
+template <int SRC, int DST>
+int launch_encode8(const void* src, void* dst, unsigned n, float scale)
+{
+    const bool aligned = (((uintptr_t)src & 15u) | ((uintptr_t)dst & 3u)) == 0;
+    const size_t n_quads = aligned ? (size_t)n / 4 : 0;
+    if (n_quads) { encode8_vec_kernel<SRC, DST><<<grid_for(n_quads), kThreads, 0, stream()>>>(src, (uint8_t*)dst, n_quads, scale); }
+    const size_t done = n_quads * 4;
+    if (done < n) { encode8_kernel<SRC, DST><<<grid_for(n - done), kThreads, 0, stream()>>>(src, (uint8_t*)dst, done, n, scale); }
+    return finish("convert_to_fp8");
 }
 
 // float -> packed FP4 with a per-tensor scale; one lane per output byte.
@@ -265,13 +381,13 @@ __global__ __launch_bounds__(kThreads) void encode4_kernel(const float* __restri
     }
 }
 
-// float -> FP4 nibbles + truncating E4M3 dequant scale per block; one lane per block.
+// float -> FP4 nibbles + truncating E4M3 dequant scale per block; one lane per block, blocks first_block and up.
 __global__ __launch_bounds__(kThreads) void encode4_blockscale_kernel(const float* __restrict__ src, uint8_t* __restrict__ nibbles, uint8_t* __restrict__ scales,
-                                                                     size_t n, unsigned block_size)
+                                                                     size_t first_block, size_t n, unsigned block_size)
 {
     const size_t n_blocks = (n + block_size - 1) / block_size;
     const size_t stride = (size_t)gridDim.x * kThreads;
-    for (size_t b = (size_t)blockIdx.x * kThreads + threadIdx.x; b < n_blocks; b += stride)
+    for (size_t b = first_block + (size_t)blockIdx.x * kThreads + threadIdx.x; b < n_blocks; b += stride)
     {
         const size_t lo = b * block_size;
         const size_t hi = (lo + block_size < n) ? lo + block_size : n;
@@ -287,6 +403,29 @@ __global__ __launch_bounds__(kThreads) void encode4_blockscale_kernel(const floa
             nibbles[i >> 1] = (uint8_t)(l | (h << 4));
         }
     }
+}
+
+// Whole blocks of 16 or 32 elements: BLOCK / 4 neighbouring lanes share a block, each with one 16-byte load, and find its
+// largest magnitude through lane exchanges inside their row of 16.  One lane per block read 64 bytes at a stride of 64, twice:
+// 254 us for a 4096 x 12288 weight (234 MB, 0.9 TB/s).
+template <int BLOCK>
+__global__ __launch_bounds__(kThreads) void encode4_blockscale_vec_kernel(const float* __restrict__ src, uint8_t* __restrict__ nibbles, uint8_t* __restrict__ scales,
+                                                                         size_t n_quads)
+{
+    constexpr int LANES = BLOCK / 4;
+    // a group of lanes is complete in every step: n_quads is a multiple of LANES, and so are the stride and a group's first lane
+    stream_pieces(n_quads,
+        [&](size_t v) { return __builtin_nontemporal_load((const f32x4*)src + v); },
+        [&](size_t v, const f32x4& x) {
+            float amax = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+            amax = fmaxf(amax, dpp_f32<0xB1>(amax));                                  // quad_perm [1,0,3,2]
+            amax = fmaxf(amax, dpp_f32<0x4E>(amax));                                  // quad_perm [2,3,0,1]
+            if (LANES == 8) { amax = fmaxf(amax, dpp_f32<0x141>(amax)); }             // row_half_mirror
+            const float fwd = (amax > 1e-10f) ? (6.0f / amax) : 1.0f;
+            const uint32_t w = f32_to_fp4(x[0] * fwd) | (f32_to_fp4(x[1] * fwd) << 4) | (f32_to_fp4(x[2] * fwd) << 8) | (f32_to_fp4(x[3] * fwd) << 12);
+            ((uint16_t*)nibbles)[v] = (uint16_t)w;
+            if (v % LANES == 0) { scales[v / LANES] = (uint8_t)f32_to_e4m3_trunc((amax > 1e-10f) ? (amax / 6.0f) : 1.0f); }
+        });
 }
 
 // Largest magnitude.  16-byte loads over the aligned body (scalar loads for a misaligned pointer and the tail), wave
@@ -367,18 +506,14 @@ int hip_convert(const void* src, int src_type, void* dst, int dst_type, unsigned
     case DT_E4M3 * 8 + DT_HALF: return launch_dequant8<DT_E4M3, DT_HALF>(src, dst, n, scale, "fp8e4m3_to_half");
     case DT_FP4 * 8 + DT_BF16: return launch_dequant4<DT_BF16, false>(src, nullptr, dst, n, 1, scale, "fp4_to_bf16");
     case DT_FP4 * 8 + DT_FLOAT: return launch_dequant4<DT_FLOAT, false>(src, nullptr, dst, n, 1, scale, "fp4_to_float");
-    case DT_FLOAT * 8 + DT_BF16:
-    case DT_HALF * 8 + DT_FLOAT:
-    case DT_HALF * 8 + DT_BF16:
-    case DT_BF16 * 8 + DT_FLOAT:
-    case DT_BF16 * 8 + DT_HALF:
-        if (n) { cast_kernel<<<grid_for(n), kThreads, 0, stream()>>>(src, src_type, dst, dst_type, n); }
-        return finish("convert_cast");
-    case DT_FLOAT * 8 + DT_E4M3:
-    case DT_FLOAT * 8 + DT_E5M2:
-    case DT_BF16 * 8 + DT_E4M3:
-        if (n) { encode8_kernel<<<grid_for(n), kThreads, 0, stream()>>>(src, src_type, (uint8_t*)dst, dst_type, n, scale); }
-        return finish("convert_to_fp8");
+    case DT_FLOAT * 8 + DT_BF16: return launch_cast<DT_FLOAT, DT_BF16>(src, dst, n);
+    case DT_HALF * 8 + DT_FLOAT: return launch_cast<DT_HALF, DT_FLOAT>(src, dst, n);
+    case DT_HALF * 8 + DT_BF16: return launch_cast<DT_HALF, DT_BF16>(src, dst, n);
+    case DT_BF16 * 8 + DT_FLOAT: return launch_cast<DT_BF16, DT_FLOAT>(src, dst, n);
+    case DT_BF16 * 8 + DT_HALF: return launch_cast<DT_BF16, DT_HALF>(src, dst, n);
+    case DT_FLOAT * 8 + DT_E4M3: return launch_encode8<DT_FLOAT, DT_E4M3>(src, dst, n, scale);
+    case DT_FLOAT * 8 + DT_E5M2: return launch_encode8<DT_FLOAT, DT_E5M2>(src, dst, n, scale);
+    case DT_BF16 * 8 + DT_E4M3: return launch_encode8<DT_BF16, DT_E4M3>(src, dst, n, scale);
     case DT_FLOAT * 8 + DT_FP4:
         if (n) { encode4_kernel<<<grid_for((n + 1) / 2), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst, n, scale); }
         return finish("float_to_fp4");
@@ -397,6 +532,20 @@ int hip_float_to_fp4_blockscale(const void* src, void* dst_nibbles, void* dst_sc
     if (block_size == 0 || (block_size & 1u)) { return -1; }
     if (n_elems == 0) { return 0; }
     const size_t n_blocks = ((size_t)n_elems + block_size - 1) / block_size;
-    encode4_blockscale_kernel<<<grid_for(n_blocks), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst_nibbles, (uint8_t*)dst_scales, n_elems, block_size);
+    const bool vec_ok = (((uintptr_t)src & 15u) | ((uintptr_t)dst_nibbles & 1u)) == 0 && (block_size == 16 || block_size == 32);
+    const size_t whole = vec_ok ? (size_t)n_elems / block_size : 0;                 // complete blocks
+    const size_t n_quads = whole * block_size / 4;
+    if (whole && block_size == 16)
+    {
+        encode4_blockscale_vec_kernel<16><<<grid_for(n_quads), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst_nibbles, (uint8_t*)dst_scales, n_quads);
+    }
+    else if (whole)
+    {
+        encode4_blockscale_vec_kernel<32><<<grid_for(n_quads), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst_nibbles, (uint8_t*)dst_scales, n_quads);
+    }
+    if (whole < n_blocks)
+    {
+        encode4_blockscale_kernel<<<grid_for(n_blocks - whole), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst_nibbles, (uint8_t*)dst_scales, whole, n_elems, block_size);
+    }
     return finish("float_to_fp4_blockscale");
 }

@@ -184,3 +184,42 @@ def test_absmax_of_a_tensor(gpu, oracle, src_type, n, offset):
     got = res.cpu().numpy()
     assert got[1] == 123.0
     assert got[0] == np.nanmax(np.abs(vals[offset:offset + n]))
+
+
+@pytest.mark.parametrize("n", [3, 4, 67, 1 << 12, (1 << 24) + 4096 * 4 + 7])
+def test_vector_casts_and_encoders_at_the_edges(gpu, oracle, n):
+    """Four-element kernels: fewer elements than a piece, a ragged tail, and more pieces than the grid keeps in flight at once
+    (256 CUs x 16 workgroups x 256 lanes x 4 pieces = 2^24 elements), with NaN, infinities and both zeros among the values."""
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal(n) * 2.0 ** rng.integers(-12, 12, n)).astype(np.float32)
+    x[:3] = [-0.0, np.inf, -np.inf]
+    if n > 8:
+        x[5] = np.nan
+    xb = oracle.f32_to_bf16(np.nan_to_num(x, nan=0.5))
+    for src, st, dt, npdt, scale in ((xb, oracle.BF16, oracle.FLOAT, np.uint32, 1.0), (xb, oracle.BF16, oracle.HALF, np.uint16, 1.0),
+                                     (x, oracle.FLOAT, oracle.BF16, np.uint16, 1.0), (x, oracle.FLOAT, oracle.E5M2, np.uint8, 0.9),
+                                     (x, oracle.FLOAT, oracle.E4M3, np.uint8, 3.7), (xb, oracle.BF16, oracle.E4M3, np.uint8, 1.0)):
+        rc, out = run_convert(gpu, src, st, dt, n, scale, npdt)
+        rc2, want = oracle.convert(src, st, dt, n, scale)
+        assert rc == 0 and rc2 == 0
+        assert np.array_equal(out, want.view(npdt)), (st, dt)
+
+
+@pytest.mark.parametrize("n,block", [(16, 16), (15, 16), (16 * 257, 16), (32 * 129 + 31, 32), (31, 32), ((1 << 24) + 16 * 1000 + 9, 16), ((1 << 24) + 64, 32), (4096, 8)])
+def test_fp4_blockscale_round_trip_at_the_edges(gpu, oracle, n, block):
+    """The lane-group encoder (whole blocks of 16 or 32) and the scalar rest behind it; the codes decoded again."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal(n) * 2.0 ** rng.integers(-9, 9, n)).astype(np.float32)
+    xd = to_dev(torch, dev, x)
+    nib = torch.zeros((n + 1) // 2 + 16, dtype=torch.uint8, device=dev)
+    sc = torch.zeros((n + block - 1) // block + 16, dtype=torch.uint8, device=dev)
+    assert lib.float_to_fp4_blockscale(xd.data_ptr(), nib.data_ptr(), sc.data_ptr(), n, block) == 0
+    wn, ws = oracle.quantize_fp4_blockscale_kernel(x, block)
+    gn, gs = nib.cpu().numpy(), sc.cpu().numpy()
+    assert np.array_equal(gn[:wn.size], wn) and np.array_equal(gs[:ws.size], ws)
+    assert not gn[wn.size:].any() and not gs[ws.size:].any()
+    back = torch.zeros(n + 16, dtype=torch.int16, device=dev)
+    assert lib.fp4_blockscale_to_bf16(nib.data_ptr(), sc.data_ptr(), back.data_ptr(), n, block) == 0
+    got = from_dev(back, np.uint16)
+    assert np.array_equal(got[:n], oracle.dequant_fp4_blockscale_to_bf16(wn, ws, n, block)) and not got[n:].any()
