@@ -2,6 +2,7 @@
 #include "../../include/cccc_hip_quant.h"
 #include "decode_kernels.h"
 #include "runtime.h"
+#include <algorithm>
 #include <cstdio>
 
 using namespace ccq;
@@ -351,7 +352,9 @@ int hip_attention_decode_fused_bf16(const void* q, const void* k, const void* v,
     if (!aligned16(k_cache) || !aligned16(v_cache) || !aligned16(workspace)) { return -1; }
     const AttentionWorkspace w = attention_workspace(n_q_heads, t_kv);
     if (workspace_bytes < w.total || w.n_blocks > ATT_MAX_BLOCKS) { return -1; }
-    const dim3 grid(w.n_blocks, n_kv_heads);
+    // Chunks per kv head: two workgroups per CU over all heads, and no fewer than the 64 the merge takes in one trip to memory.
+    const int chunks = std::min(w.n_blocks, std::max(64, 2 * cu_count() / n_kv_heads));
+    const dim3 grid(chunks, n_kv_heads);
     float2* stats = (float2*)((char*)workspace + w.stats);
     float* partial = (float*)((char*)workspace + w.partial);
     const float scale = 1.0f / sqrtf(128.0f);
@@ -359,8 +362,8 @@ int hip_attention_decode_fused_bf16(const void* q, const void* k, const void* v,
 #define CCQ_ATTN_FUSED(G)                                                                                                                    \
     attn_fused_kernel<G><<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_norm_w, \
                                                      (const uint16_t*)k_norm_w, (const uint16_t*)cos_tab, (const uint16_t*)sin_tab,        \
-                                                     (uint16_t*)k_cache, (uint16_t*)v_cache, stats, partial, t_kv, w.n_blocks, pos,        \
-                                                     n_q_heads, epsilon, scale)
+                                                     (uint16_t*)k_cache, (uint16_t*)v_cache, stats, partial, t_kv, pos, n_q_heads,        \
+                                                     epsilon, scale)
     switch (n_q_heads / n_kv_heads)
     {
     case 1: CCQ_ATTN_FUSED(1); break;
@@ -370,7 +373,7 @@ int hip_attention_decode_fused_bf16(const void* q, const void* k, const void* v,
     }
 #undef CCQ_ATTN_FUSED
     const int n_out = n_q_heads * 128;
-    attn_rescale_combine_kernel<<<n_out / 64, 256, 0, stream()>>>(partial, stats, (uint16_t*)y, n_out, t_kv, w.n_blocks, pos);
+    attn_rescale_combine_kernel<<<n_out / 64, 256, 0, stream()>>>(partial, stats, (uint16_t*)y, n_out, t_kv, chunks, pos);
     return finish("attention_decode_fused");
 }
 
@@ -392,10 +395,10 @@ int hip_attention_decode_exact_bf16(const void* q, const void* k, const void* v,
     const float scale = 1.0f / sqrtf(128.0f);
     const int* pos = (const int*)d_pos;
 #define CCQ_ATTN_EXACT(G)                                                                                                                            \
-    attn_fused_kernel<G, true><<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_norm_w,   \
-                                                           (const uint16_t*)k_norm_w, (const uint16_t*)cos_tab, (const uint16_t*)sin_tab,          \
-                                                           (uint16_t*)k_cache, (uint16_t*)v_cache, stats, partial, t_kv, w.n_blocks, pos,          \
-                                                           n_q_heads, epsilon, scale, scores);                                                      \
+    attn_fused_scores_kernel<G><<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_norm_w,  \
+                                                            (const uint16_t*)k_norm_w, (const uint16_t*)cos_tab, (const uint16_t*)sin_tab,         \
+                                                            (uint16_t*)k_cache, (uint16_t*)v_cache, stats, scores, t_kv, w.n_blocks, pos,          \
+                                                            epsilon, scale);                                                                        \
     attn_pv_kernel<G><<<grid, 256, 0, stream()>>>(scores, stats, (const uint16_t*)v_cache, partial, t_kv, w.n_blocks, pos, n_q_heads)
     switch (n_q_heads / n_kv_heads)
     {

@@ -1105,16 +1105,25 @@ static __global__ __launch_bounds__(256) void attn_combine_kernel(const float* _
 //   waves 0..G-1 normalise and rotate the G query heads of this KV head; the block holding row *d_pos
 //   also normalises / rotates k, appends k and v to the caches, and uses them from LDS;
 //   stats[qh][block] = (max, sum expf(s - max)), partial[block][qh][128] = sum expf(s_t - max) v_t.
+// (the fields are 32 bits wide and pass through `arrive` before the first use: as 16-bit values the compiler converts each
+// one in the block that loads it and so waits for it there, one trip to memory after the other)
 struct HeadLoads
 {
-    uint16_t xl, xr, c, sn, wl, wr;       // lane's two elements of the head, its cos / sin, the two norm weights
+    uint32_t xl, xr, c, sn, wl, wr;       // lane's two elements of the head, its cos / sin, the two norm weights
 };
 
+// without norm weights their places are loaded from the head itself, so that no load hangs on a branch
 __device__ __forceinline__ HeadLoads load_head(const uint16_t* __restrict__ src, const uint16_t* __restrict__ nw, const uint16_t* __restrict__ cos_row,
                                                const uint16_t* __restrict__ sin_row, int lane)
 {
-    return HeadLoads{ src[lane], src[lane + 64], cos_row[lane], sin_row[lane], nw ? nw[lane] : (uint16_t)0, nw ? nw[lane + 64] : (uint16_t)0 };
+    const uint16_t* w = nw ? nw : src;
+    return HeadLoads{ src[lane], src[lane + 64], cos_row[lane], sin_row[lane], w[lane], w[lane + 64] };
 }
+
+__device__ __forceinline__ void arrive(HeadLoads& h) { asm volatile("" : "+v"(h.xl), "+v"(h.xr), "+v"(h.c), "+v"(h.sn), "+v"(h.wl), "+v"(h.wr)); }
+
+// loads above stay above (no instruction: a load that only one branch uses would otherwise move into it)
+__device__ __forceinline__ void loads_end() { asm volatile("" ::: "memory"); }
 
 // normed == false (no per-head norm weights, Llama-style): the head is rotated as the projection left it
 __device__ __forceinline__ void norm_rope_finish(const HeadLoads& h, bool normed, float eps, float& out_l, float& out_r)
@@ -1139,24 +1148,224 @@ __device__ __forceinline__ void norm_rope_head(const uint16_t* __restrict__ src,
     norm_rope_finish(load_head(src, nw, cos_row, sin_row, lane), nw != nullptr, eps, out_l, out_r);
 }
 
-// SCORES_ONLY: the front half alone -- norm, rotation, append, the block's BF16 scores written to scores[qh][t] and their
-// (max, sum expf(s - max)) to stats -- for the route that rounds the probabilities of the whole row to BF16 before they
-// meet V (attn_pv_kernel and attn_combine_kernel follow); no value row is read here.
-template <int G, bool SCORES_ONLY = false>
+// Launch 1 walks its rows as a stream: grid (chunks, kv heads), chunk c owns `span` consecutive blocks of 64 rows with
+// span = ceil(live blocks / chunks), and each of its four waves takes every fourth 16-row tile of them with a softmax of its
+// own (running maximum and sum per head, sums rescaled where the maximum grows), the next tile's rows requested before the
+// current one is used.  Nothing is exchanged between the waves until the end, so the loop has no barrier, and the launch
+// behind merges at most `chunks` partial results however long the cache is: with one workgroup per 64 rows, 32000 rows of 8
+// heads left 500 partial results per head: 31.5 us here and 47 us for their merge, now 25.2 and 4.8 (bound: the 131 MB of
+// rows, 19 us); up to 64 blocks it is level (4096 rows 7.1 us, 640 rows 5.4).
+// Scores of a tile: K[16 keys x 128] . q^T[128 x heads] as four v_mfma_f32_16x16x32_bf16 (products of BF16 values are exact
+// in FP32), key lane i = lane % 16, dims 32 c + 8 g + 0..7 (g = lane / 16), the heads repeated over the 16 columns; the result
+// lane holds head i % G, keys 4 g + 0..3.  Values: lane (i, g) holds dims 8 i + 0..7 of keys 4 g + it, so the probabilities
+// it needs are those of the lanes of its own quad.
+// Cache rows are read once per token: streaming (non-temporal) loads, like the weights, are worth 2.6 us per launch here.
+__device__ __forceinline__ void att_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }      // leaves the rows in flight alone
+
+__host__ __device__ inline int attention_chunk_span(int live_blocks, int chunks) { return live_blocks <= chunks ? 1 : (live_blocks + chunks - 1) / chunks; }
+
+// the value of lane h of the quad (h a constant after unrolling)
+__device__ __forceinline__ float quad_lane(float v, int h) { return h == 0 ? dpp_f32<0x00>(v) : h == 1 ? dpp_f32<0x55>(v) : h == 2 ? dpp_f32<0xAA>(v) : dpp_f32<0xFF>(v); }
+
+template <int G>
 __global__ __launch_bounds__(256) void attn_fused_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                         const uint16_t* __restrict__ q_norm_w, const uint16_t* __restrict__ k_norm_w,
                                                         const uint16_t* __restrict__ cos_tab, const uint16_t* __restrict__ sin_tab,
                                                         uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
                                                         float2* __restrict__ stats, float* __restrict__ partial,
-                                                        int t_kv, int n_blocks, const int* __restrict__ d_pos, int n_q, float eps, float scale,
-                                                        uint16_t* __restrict__ scores = nullptr)
+                                                        int t_kv, const int* __restrict__ d_pos, int n_q, float eps, float scale)
 {
     __shared__ float acc_lds[16][G][128];   // [key slot in workgroup][head][dim]
-    __shared__ float s_lds[G][ATT_KEYS];    // scores, then expf(s - block max)
+    __shared__ float2 wave_stat[4][G];      // (max, sum) of a wave's rows
+    __shared__ __attribute__((aligned(16))) uint16_t q_lds[G][128];     // normalised, rotated query heads (BF16 values)
+    __shared__ __attribute__((aligned(16))) uint16_t k_new[128];
+    __shared__ __attribute__((aligned(16))) uint16_t v_new[128];
+    const int kvh = blockIdx.y, chunk = blockIdx.x, n_chunks = gridDim.x;
+    const int pos = *d_pos;
+    if (pos < 0 || pos >= t_kv) { return; }         // a position outside the cache: nothing to append, nothing to attend
+    const int span = attention_chunk_span(pos / ATT_KEYS + 1, n_chunks);
+    const int t0 = chunk * span * ATT_KEYS;
+    if (t0 > pos) { return; }
+    const int t1 = min(t0 + span * ATT_KEYS, pos + 1);
+    const bool has_new = t1 > pos;                  // this chunk holds the row being appended
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane & 15, g = lane >> 4;
+    const uint16_t* cos_row = cos_tab + (size_t)pos * 64;
+    const uint16_t* sin_row = sin_tab + (size_t)pos * 64;
+    const uint16_t* kbase = k_cache + (size_t)kvh * t_kv * 128 + g * 8;
+    const uint16_t* vbase = v_cache + (size_t)kvh * t_kv * 128 + sub * 8;
+    // The new token's few bytes are requested before the cache rows, and the key rows before the value rows: loads return in
+    // the order they were issued.  Every wave requests a query head and the new row's key (wave 2: value), also where it has
+    // no use for them: a load in a branch would be waited for at the branch's end.
+    HeadLoads hq = load_head(q + (size_t)(kvh * G + min(wave, G - 1)) * 128, q_norm_w, cos_row, sin_row, lane);
+    HeadLoads hn = load_head((wave == 2 ? v : k) + (size_t)kvh * 128, k_norm_w, cos_row, sin_row, lane);
+    loads_end();
+    u32x4 kraw[4], vraw[4];
+    auto load_keys = [&](int t) {                   // rows past the end, and row pos itself, are replaced or discarded at their use
+        const uint16_t* row = kbase + (size_t)min(t + sub, pos) * 128;
+#pragma unroll
+        for (int c = 0; c < 4; c++) { kraw[c] = __builtin_nontemporal_load((const u32x4*)(row + c * 32)); }
+    };
+    auto load_values = [&](int t) {
+#pragma unroll
+        for (int it = 0; it < 4; it++) { vraw[it] = __builtin_nontemporal_load((const u32x4*)(vbase + (size_t)min(t + 4 * g + it, pos) * 128)); }
+    };
+    int t = t0 + wave * 16;
+    load_keys(t);
+    load_values(t);
+    loads_end();
+    arrive(hq);
+    arrive(hn);
+    if (wave < G)
+    {
+        float l, r;
+        norm_rope_finish(hq, q_norm_w != nullptr, eps, l, r);
+        q_lds[wave][lane] = (uint16_t)f32_to_bf16_bits(l);
+        q_lds[wave][lane + 64] = (uint16_t)f32_to_bf16_bits(r);
+    }
+    if (has_new && wave == 3)
+    {
+        float l, r;
+        norm_rope_finish(hn, k_norm_w != nullptr, eps, l, r);
+        k_new[lane] = (uint16_t)f32_to_bf16_bits(l);
+        k_new[lane + 64] = (uint16_t)f32_to_bf16_bits(r);
+        uint16_t* dst = k_cache + ((size_t)kvh * t_kv + pos) * 128;
+        dst[lane] = (uint16_t)f32_to_bf16_bits(l);
+        dst[lane + 64] = (uint16_t)f32_to_bf16_bits(r);
+    }
+    if (has_new && wave == 2)
+    {
+        const uint16_t a = (uint16_t)hn.xl, b = (uint16_t)hn.xr;
+        v_new[lane] = a;
+        v_new[lane + 64] = b;
+        uint16_t* dst = v_cache + ((size_t)kvh * t_kv + pos) * 128;
+        dst[lane] = a;
+        dst[lane + 64] = b;
+    }
+    att_lds_barrier();
+    u32x4 qf[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) { qf[c] = *(const u32x4*)&q_lds[sub % G][c * 32 + g * 8]; }
+    float m = -INFINITY, l = 0.0f;          // head `sub % G`: maximum over the wave's rows, sum over the lane's
+    float acc[G][8];
+#pragma unroll
+    for (int gq = 0; gq < G; gq++)
+#pragma unroll
+        for (int d = 0; d < 8; d++) { acc[gq][d] = 0.0f; }
+    for (; t < t1; t += ATT_KEYS)
+    {
+        const bool edge = t + 16 > pos;     // the tile holds row pos or rows past it
+        f32x4 sc = { 0.0f, 0.0f, 0.0f, 0.0f };
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+        {
+            u32x4 kc = kraw[c];
+            if (edge && t + sub == pos) { kc = *(const u32x4*)&k_new[c * 32 + g * 8]; }
+            sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kc), __builtin_bit_cast(bf16x8, qf[c]), sc, 0, 0, 0);
+        }
+        const bool more = t + ATT_KEYS < t1;
+        if (more) { load_keys(t + ATT_KEYS); }
+        float s[4], tile_max = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+        {
+            s[j] = bf16_round(scale * sc[j]);
+            if (edge && t + 4 * g + j > pos) { s[j] = -INFINITY; }
+            tile_max = fmaxf(tile_max, s[j]);
+        }
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16));
+        tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
+        const float nm = fmaxf(m, tile_max);
+        const float off = nm > -INFINITY ? nm : 0.0f;       // (nothing above -inf so far: every term is 0)
+        const float alpha = expf(m - off);
+        const bool grows = __any(nm > m);
+        f32x4 p;
+#pragma unroll
+        for (int j = 0; j < 4; j++) { p[j] = expf(s[j] - off); }
+        l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+        m = nm;
+        if (grows)
+        {
+#pragma unroll
+            for (int gq = 0; gq < G; gq++)
+            {
+                const float a = quad_lane(alpha, gq);
+#pragma unroll
+                for (int d = 0; d < 8; d++) { acc[gq][d] *= a; }
+            }
+        }
+#pragma unroll
+        for (int it = 0; it < 4; it++)
+        {
+            u32x4 raw = vraw[it];
+            if (edge)
+            {
+                const int row = t + 4 * g + it;
+                if (row == pos) { raw = *(const u32x4*)&v_new[sub * 8]; }
+                if (row > pos) { raw = u32x4{ 0u, 0u, 0u, 0u }; }       // read from the row being appended, which may still hold anything (0 * NaN is NaN)
+            }
+            float vf[8];
+            unpack8_bf16(raw, vf);
+#pragma unroll
+            for (int gq = 0; gq < G; gq++)
+            {
+                const float pg = quad_lane(p[it], gq);
+#pragma unroll
+                for (int d = 0; d < 8; d++) { acc[gq][d] = fmaf(pg, vf[d], acc[gq][d]); }
+            }
+        }
+        if (more) { load_values(t + ATT_KEYS); }
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (sub < G && g == 0) { wave_stat[wave][sub] = make_float2(m, l); }
+    const int slot = wave * 4 + g;
+#pragma unroll
+    for (int gq = 0; gq < G; gq++)
+#pragma unroll
+        for (int d = 0; d < 8; d++) { acc_lds[slot][gq][sub * 8 + d] = acc[gq][d]; }
+    __syncthreads();
+    for (int o = threadIdx.x; o < G * 128; o += 256)
+    {
+        const int gq = o >> 7, d = o & 127;
+        float2 st[4];
+        float top = -INFINITY, total = 0.0f, sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; w++)
+        {
+            st[w] = wave_stat[w][gq];
+            top = fmaxf(top, st[w].x);
+        }
+#pragma unroll
+        for (int w = 0; w < 4; w++)
+        {
+            const float weight = st[w].x > -INFINITY ? expf(st[w].x - top) : 0.0f;      // 0: a wave without rows
+            float part = 0.0f;
+#pragma unroll
+            for (int sl = 0; sl < 4; sl++) { part += acc_lds[4 * w + sl][gq][d]; }
+            total = fmaf(part, weight, total);
+            sum = fmaf(st[w].y, weight, sum);
+        }
+        __builtin_nontemporal_store(total, &partial[((size_t)chunk * n_q + kvh * G + gq) * 128 + d]);      // read once, by the merge kernel
+        if (d == 0) { stats[(size_t)(kvh * G + gq) * n_chunks + chunk] = make_float2(top, sum); }
+    }
+}
+
+// The front half alone, one workgroup per block of 64 rows -- norm, rotation, append, the block's BF16 scores written to
+// scores[qh][t] and their (max, sum expf(s - max)) to stats -- for the route that rounds the probabilities of the whole row
+// to BF16 before they meet V (attn_pv_kernel and attn_combine_kernel follow); no value row is read here.
+template <int G>
+__global__ __launch_bounds__(256) void attn_fused_scores_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                                        const uint16_t* __restrict__ q_norm_w, const uint16_t* __restrict__ k_norm_w,
+                                                        const uint16_t* __restrict__ cos_tab, const uint16_t* __restrict__ sin_tab,
+                                                        uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
+                                                        float2* __restrict__ stats, uint16_t* __restrict__ scores,
+                                                        int t_kv, int n_blocks, const int* __restrict__ d_pos, float eps, float scale)
+{
+    __shared__ float s_lds[G][ATT_KEYS];
     static_assert(ATT_KEYS == 64, "the score stage gives each of the four waves one 16-key matrix-core tile");
     __shared__ __attribute__((aligned(16))) uint16_t q_lds[G][128];     // normalised, rotated query heads (BF16 values)
     __shared__ __attribute__((aligned(16))) uint16_t k_new[128];
-    __shared__ float v_new[128];
     const int kvh = blockIdx.y, blk = blockIdx.x;
     const int pos = *d_pos;
     if (pos < 0 || pos >= t_kv) { return; }         // a position outside the cache: nothing to append, nothing to attend
@@ -1168,30 +1377,24 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(const uint16_t* __restr
     const int sub = lane & 15, key_in_wave = lane >> 4;
     const uint16_t* cos_row = cos_tab + (size_t)pos * 64;
     const uint16_t* sin_row = sin_tab + (size_t)pos * 64;
-    // the query head's few bytes are requested before the cache rows, and the key rows before the value rows:
-    // loads return in the order they were issued
-    HeadLoads hq{};
-    if (wave < G) { hq = load_head(q + (size_t)(kvh * G + wave) * 128, q_norm_w, cos_row, sin_row, lane); }
-    // Cache rows are read once per token: streaming (non-temporal) loads, like the weights, are worth 2.6 us per launch here.
+    // The new token's few bytes are requested before the cache rows, and the key rows before the value rows: loads return in
+    // the order they were issued.  Every wave requests a query head and the new row's key (wave 2: value), also where it has
+    // no use for them: a load in a branch would be waited for at the branch's end.
+    HeadLoads hq = load_head(q + (size_t)(kvh * G + min(wave, G - 1)) * 128, q_norm_w, cos_row, sin_row, lane);
+    HeadLoads hn = load_head((wave == 2 ? v : k) + (size_t)kvh * 128, k_norm_w, cos_row, sin_row, lane);
+    loads_end();
     // Keys in the layout of the matrix-core row operand: wave w owns keys 16 w .. 16 w + 15 of the block, lane
-    // (i = lane % 16, g = lane / 16) holds dims 32 c + 8 g .. + 7 of key i for c = 0..3.  Values as before: lane
-    // (sub, key_in_wave) holds dims 8 sub .. + 7 of key it * 16 + wave * 4 + key_in_wave.
-    u32x4 kraw[4], vraw[ATT_ITS];
+    // (i = lane % 16, g = lane / 16) holds dims 32 c + 8 g .. + 7 of key i for c = 0..3.
+    u32x4 kraw[4];
     const int key_row = wave * 16 + sub;                                         // this lane's key within the block
     {
         const int t = min(t0 + key_row, n_keys - 1);                             // rows past the end, and row pos itself, are replaced or discarded below
 #pragma unroll
         for (int c = 0; c < 4; c++) { kraw[c] = __builtin_nontemporal_load((const u32x4*)(k_cache + ((size_t)kvh * t_kv + t) * 128 + c * 32 + key_in_wave * 8)); }
     }
-    if constexpr (!SCORES_ONLY)
-    {
-#pragma unroll
-        for (int it = 0; it < ATT_ITS; it++)
-        {
-            const int t = min(t0 + it * 16 + wave * 4 + key_in_wave, n_keys - 1);
-            vraw[it] = __builtin_nontemporal_load((const u32x4*)(v_cache + ((size_t)kvh * t_kv + t) * 128 + sub * 8));
-        }
-    }
+    loads_end();
+    arrive(hq);
+    arrive(hn);
     if (wave < G)
     {
         float l, r;
@@ -1202,7 +1405,7 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(const uint16_t* __restr
     if (has_new && wave == 3)
     {
         float l, r;
-        norm_rope_head(k + (size_t)kvh * 128, k_norm_w, cos_row, sin_row, eps, lane, l, r);
+        norm_rope_finish(hn, k_norm_w != nullptr, eps, l, r);
         k_new[lane] = (uint16_t)f32_to_bf16_bits(l);
         k_new[lane + 64] = (uint16_t)f32_to_bf16_bits(r);
         uint16_t* dst = k_cache + ((size_t)kvh * t_kv + pos) * 128;
@@ -1211,9 +1414,7 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(const uint16_t* __restr
     }
     if (has_new && wave == 2)
     {
-        const uint16_t a = v[(size_t)kvh * 128 + lane], b = v[(size_t)kvh * 128 + lane + 64];
-        v_new[lane] = bf16_bits_to_f32(a);
-        v_new[lane + 64] = bf16_bits_to_f32(b);
+        const uint16_t a = (uint16_t)hn.xl, b = (uint16_t)hn.xr;
         uint16_t* dst = v_cache + ((size_t)kvh * t_kv + pos) * 128;
         dst[lane] = a;
         dst[lane + 64] = b;
@@ -1240,10 +1441,7 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(const uint16_t* __restr
                 const int kl = wave * 16 + key_in_wave * 4 + v;
                 const float sv = bf16_round(scale * sc[v]);
                 s_lds[sub][kl] = t0 + kl < n_keys ? sv : -INFINITY;
-                if constexpr (SCORES_ONLY)
-                {
-                    if (t0 + kl < n_keys) { scores[(size_t)(kvh * G + sub) * t_kv + t0 + kl] = (uint16_t)(__builtin_bit_cast(uint32_t, sv) >> 16); }
-                }
+                if (t0 + kl < n_keys) { scores[(size_t)(kvh * G + sub) * t_kv + t0 + kl] = (uint16_t)(__builtin_bit_cast(uint32_t, sv) >> 16); }
             }
         }
     }
@@ -1256,64 +1454,14 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(const uint16_t* __restr
         for (int j = 0; j < PER_LANE; j++) { m = fmaxf(m, v[j] = (lane + 64 * j < ATT_KEYS) ? s_lds[wave][lane + 64 * j] : -INFINITY); }
         m = wave_max(m);                                    // finite: the block holds at least one valid key
 #pragma unroll
-        for (int j = 0; j < PER_LANE; j++)
-        {
-            const float e = expf(v[j] - m);
-            if (lane + 64 * j < ATT_KEYS) { s_lds[wave][lane + 64 * j] = e; }
-            l += e;
-        }
+        for (int j = 0; j < PER_LANE; j++) { l += expf(v[j] - m); }
         l = wave_sum(l);
         if (lane == 0) { stats[(size_t)(kvh * G + wave) * n_blocks + blk] = make_float2(m, l); }
-    }
-    if constexpr (SCORES_ONLY) { return; }
-    __syncthreads();
-    float acc[G][8];
-#pragma unroll
-    for (int gq = 0; gq < G; gq++)
-#pragma unroll
-        for (int d = 0; d < 8; d++) { acc[gq][d] = 0.0f; }
-#pragma unroll
-    for (int it = 0; it < ATT_ITS; it++)
-    {
-        const int kl = it * 16 + wave * 4 + key_in_wave;
-        float vf[8];
-        unpack8_bf16(vraw[it], vf);
-        if (t0 + kl == pos)
-        {
-#pragma unroll
-            for (int d = 0; d < 8; d++) { vf[d] = v_new[sub * 8 + d]; }
-        }
-        if (t0 + kl > pos)                                  // read from the row being appended, which may still hold anything (0 * NaN is NaN)
-        {
-#pragma unroll
-            for (int d = 0; d < 8; d++) { vf[d] = 0.0f; }
-        }
-#pragma unroll
-        for (int gq = 0; gq < G; gq++)
-        {
-            const float p = s_lds[gq][kl];                  // 0 for rows past the end
-#pragma unroll
-            for (int d = 0; d < 8; d++) { acc[gq][d] = fmaf(p, vf[d], acc[gq][d]); }
-        }
-    }
-    const int slot = wave * 4 + key_in_wave;
-#pragma unroll
-    for (int gq = 0; gq < G; gq++)
-#pragma unroll
-        for (int d = 0; d < 8; d++) { acc_lds[slot][gq][sub * 8 + d] = acc[gq][d]; }
-    __syncthreads();
-    for (int o = threadIdx.x; o < G * 128; o += 256)
-    {
-        const int gq = o >> 7, d = o & 127;
-        float total = 0.0f;
-#pragma unroll
-        for (int sl = 0; sl < 16; sl++) { total += acc_lds[sl][gq][d]; }
-        __builtin_nontemporal_store(total, &partial[((size_t)blk * n_q + kvh * G + gq) * 128 + d]);      // read once, by the merge kernel
     }
 }
 
 // Launch 2: y[qh][d] = bf16(sum_b w_b partial[b][qh][d]), w_b = expf(max_b - max) / sum_b' l_b' expf(max_b' - max),
-// in a fixed order.  64 outputs (half a head) per workgroup; n_blocks <= ATT_MAX_BLOCKS.
+// in a fixed order, over the chunks b launch 1 wrote.  64 outputs (half a head) per workgroup; n_blocks <= ATT_MAX_BLOCKS.
 constexpr int ATT_MAX_BLOCKS = 1024;
 
 // Every load of the common case is requested before anything is known -- the position, up to four (max, sum)
@@ -1342,17 +1490,18 @@ static __global__ __launch_bounds__(256) void attn_rescale_combine_kernel(const 
     for (int j = 0; j < PRE; j++) { pre[j] = __builtin_nontemporal_load(&partial[(size_t)min(wave + 4 * j, n_blocks - 1) * n_out + o]); }
 
     if (pos < 0 || pos >= t_kv) { return; }
-    const int n_active = pos / ATT_KEYS + 1;
+    const int live = pos / ATT_KEYS + 1, span = attention_chunk_span(live, n_blocks);
+    const int n_active = span == 1 ? live : (live + span - 1) / span;      // (the divisions would cost a short context 0.6 us)
     float total = 0.0f, inv;
     if (n_active <= 64)
     {
         // Up to 64 blocks: every wave holds one block's statistics per lane and works out the weights for
         // itself (the same reductions in the same order as below, whose other three wave sums are zero), so
         // nothing is exchanged before the final sum over the four waves.
-        const bool live = lane < n_active;
-        const float m = wave_max(live ? mine.x : -INFINITY);
-        const float e = live ? expf(mine.x - m) : 0.0f;
-        const float l = wave_sum(live ? mine.y * e : 0.0f);
+        const bool used = lane < n_active;
+        const float m = wave_max(used ? mine.x : -INFINITY);
+        const float e = used ? expf(mine.x - m) : 0.0f;
+        const float l = wave_sum(used ? mine.y * e : 0.0f);
         inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
         for (int j = 0; j < PRE; j++)

@@ -292,6 +292,40 @@ def test_fused_attention_appends_and_attends(gpu, oracle, dec, n_q, n_kv, t_kv):
             assert ulp_close(from_dev(y2, np.uint16).reshape(n_q, 128), want2, ulps=3.0, floor=4e-3 * np.abs(want2).max()).all()
 
 
+@pytest.mark.parametrize("n_q,n_kv,t_kv", [(8, 8, 4500), (16, 8, 8300), (32, 8, 12500), (4, 1, 33000)])
+def test_fused_attention_streams_long_caches(gpu, oracle, dec, n_q, n_kv, t_kv):
+    """More blocks of 64 rows than workgroups per kv head (64, or 512 for the single head): each walks several blocks, the last of
+    them partly or not at all filled.  The rows grow towards the end, so that the running maximum moves, and the rows from the
+    position on hold NaN patterns.  Same bounds as the test above (output against an unrounded softmax of BF16 scores)."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(9)
+    cfg = dec.DecodeConfig(n_q=n_q, n_kv=n_kv, t_kv=t_kv)
+    cos, sin = dec.rope_tables(cfg)
+    kc = oracle.f32_to_bf16(rng.standard_normal((n_kv, t_kv, 128), dtype=np.float32) * np.linspace(0.2, 1.2, t_kv, dtype=np.float32)[None, :, None])
+    vc = oracle.f32_to_bf16(rng.standard_normal((n_kv, t_kv, 128), dtype=np.float32))
+    ws_bytes = lib.c.hip_attention_decode_workspace_bytes(n_q, n_kv, t_kv)
+    ws = torch.full((ws_bytes,), 0xFF, dtype=torch.uint8, device=dev)
+    cd, sd = to_dev(torch, dev, cos), to_dev(torch, dev, sin)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    for pos in (p for p in (4095, 4096, 4159, 8191, 8192, 8258, 32768, t_kv - 1) if 4 * p >= t_kv and p < t_kv):
+        q, k, v = (oracle.f32_to_bf16(rng.standard_normal((n, 128)).astype(np.float32)) for n in (n_q, n_kv, n_kv))
+        kd, vd = to_dev(torch, dev, kc), to_dev(torch, dev, vc)
+        for d in (kd, vd):
+            d.view(n_kv, t_kv, 128)[:, pos:] = -1
+        qd, knd, vnd = (to_dev(torch, dev, a) for a in (q, k, v))
+        pd = torch.tensor([pos], dtype=torch.int32, device=dev)
+        y = torch.zeros(n_q * 128, dtype=torch.int16, device=dev)
+        assert lib.c.hip_attention_decode_fused_bf16(ptr(qd), ptr(knd), ptr(vnd), None, None, ptr(cd), ptr(sd), ptr(kd), ptr(vd), ptr(y), ptr(ws), ws_bytes,
+                                                     n_q, n_kv, 128, t_kv, ptr(pd), ctypes.c_float(1e-6)) == 0
+        qr = dec.rope(dec.f(q), dec.f(cos[pos]), dec.f(sin[pos]))
+        k_all, v_all = (from_dev(d, np.uint16).reshape(n_kv, t_kv, 128)[:, :pos + 1] for d in (kd, vd))
+        assert np.array_equal(v_all[:, pos], v) and np.array_equal(k_all[:, :pos], kc[:, :pos])
+        want = dec.attention(qr, dec.f(k_all), dec.f(v_all), pos, n_q, n_kv)
+        got = from_dev(y, np.uint16).reshape(n_q, 128)
+        assert ulp_close(got, want, ulps=3.0, floor=4e-3 * np.abs(want).max()).all(), pos
+        assert np.linalg.norm(dec.f(got) - want) <= 4e-3 * np.linalg.norm(want), pos
+
+
 def test_argmax_and_embed(gpu, oracle):
     torch, dev, lib = gpu
     rng = np.random.default_rng(3)
