@@ -18,6 +18,7 @@
 #include "linear_args.h"
 #include "quant_device.h"
 #include "runtime.h"
+#include <algorithm>
 #include <type_traits>
 
 namespace ccq
@@ -284,7 +285,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const LinearArgs a, cons
 // PD: how many k-tiles ahead the weights are requested (the activations PD + 1 when PD > 1).  One is enough where two
 // workgroups share a CU and each k-tile carries 64 matrix-core instructions per wave; the k-split launches of a short
 // prompt (one 64-token tile, about one workgroup per CU) are bound by their weight bytes and run a k-tile per memory
-// latency with PD = 1 -- they take PD = 3.
+// latency with PD = 1 -- they, and all tiles of plan_short, take PD = 3.
 template <int WT, bool SCALED, int MB, bool SPLIT, bool TILED, int AT = DT_BF16, int NB = 4, bool PAIR = false, bool SEG = false, int PD = 1, int WGS_PER_CU = 2>
 __global__ __launch_bounds__(256, WGS_PER_CU) void gemm_mfma_direct_kernel(const LinearArgs a_in, const int n_tiles, float* __restrict__ partial)
 {
@@ -1104,27 +1105,92 @@ void launch_gemm4_mfma_direct(const LinearArgs& a, const uint8_t* tiled_scales, 
     else { gemm4_mfma_direct_kernel<BLOCK, MB, false, NB><<<grid, 256, 0, stream()>>>(a, tiled_scales, n_tiles, nullptr); }
 }
 
-// splits > 1: `partial` holds splits * tokens * n_out floats
 template <int WT, int MB, bool TILED, int AT = DT_BF16, int NB = 4>
-void launch_gemm_mfma_direct(const LinearArgs& a, int splits = 1, float* partial = nullptr, const AddNormArgs* e = nullptr)
+void launch_gemm_mfma_direct(const LinearArgs& a)
 {
     const int n_tiles = (a.n_out + 64 * NB - 1) / (64 * NB);
     const int m_tiles = (a.tokens + MB * 16 - 1) / (MB * 16);
-    const dim3 grid(((n_tiles + 7) & ~7) * m_tiles, splits);
-    const bool scaled = a.w_scale != 1.0f;
-    if (splits > 1)
-    {
-        constexpr int PD = MB <= 4 ? 3 : 1;          // 64- and 32-token tiles split k only up to 64 tokens: bound by the weight bytes
-        if (scaled) { gemm_mfma_direct_kernel<WT, true, MB, true, TILED, AT, NB, false, false, PD><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-        else { gemm_mfma_direct_kernel<WT, false, MB, true, TILED, AT, NB, false, false, PD><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-        launch_splitk_combine<AT>(partial, splits, a, e);
-    }
-    else
-    {
-        if (scaled) { gemm_mfma_direct_kernel<WT, true, MB, false, TILED, AT, NB><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
-        else { gemm_mfma_direct_kernel<WT, false, MB, false, TILED, AT, NB><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
-    }
+    const dim3 grid(((n_tiles + 7) & ~7) * m_tiles);
+    if (a.w_scale != 1.0f) { gemm_mfma_direct_kernel<WT, true, MB, false, TILED, AT, NB><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
+    else { gemm_mfma_direct_kernel<WT, false, MB, false, TILED, AT, NB><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
 }
+
+// Tiles of the FP8 GEMM for launches that leave the chip with two workgroups per CU or fewer: prompts of up to a few hundred
+// tokens, narrow outputs.  Such a launch is not bound by the matrix cores but by what one workgroup takes per k-tile (latency,
+// LDS reads) and by a fixed part, so its time is estimated as
+//   3.5 us (launch, first loads, stores) + k-tiles of a workgroup x us per k-tile + 3 us + 0.5 us per MB of partial sums if split
+// with the us per k-tile measured for one and for two workgroups per CU and each tile shape, and the tile shape and k split
+// with the least estimate is taken.  Smaller tiles with weights requested three k-tiles ahead need fewer k ranges, so fewer
+// FP32 partial sums are written, read and added (E5M2 file layout, 100 tokens, this against the 128 x 256 tiles with up to
+// eight k ranges it replaces: 4096 x 4096 14.8 - 15.6 against 22.3 us, K 12288 28.8 against 31.8, the q, k, v launch 17.4
+// against 21.9, the gate / up pair 41.9 against 47; HALF, E4M3 with a scale, tiled copies, 301 tokens: 4096 x 4096 25.1
+// against 29.1, 1024 x 4096 13.2 against 22.5, 12288 x 4096 47.8 against 64.8).  Over a grid of 7 shapes x 8 token counts the
+// choice is within 10 % of the fastest combination, mostly within 4 %.
+struct ShortTile
+{
+    int mb, nb;
+    float one[3], two[3];            // us per k-tile with one / two workgroups per CU: tiled copy, file layout, with a scale
+};
+
+constexpr ShortTile kShortTiles[] = {
+    { 2, 1, { 0.115f, 0.135f, 0.15f }, { 0.21f, 0.25f, 0.28f } },       // 32 tokens x 64 features
+    { 2, 2, { 0.17f, 0.22f, 0.21f }, { 0.32f, 0.42f, 0.40f } },
+    { 4, 1, { 0.20f, 0.21f, 0.25f }, { 0.375f, 0.38f, 0.43f } },
+    { 4, 2, { 0.29f, 0.32f, 0.35f }, { 0.48f, 0.63f, 0.63f } },
+    { 4, 4, { 0.49f, 0.58f, 0.71f }, { 0.93f, 1.15f, 1.4f } },
+    { 8, 2, { 0.0f, 0.54f, 0.0f }, { 0.0f, 0.92f, 0.0f } },             // file layout only: a 16 x 64-byte load serves twice the products
+};
+
+struct ShortPlan
+{
+    int mb, nb, splits;
+    double us;               // estimate; 0: no shape fits
+};
+
+inline ShortPlan plan_short(const LinearArgs& a, bool row_major, bool scaled, bool pair, int max_splits)
+{
+    const int cus = cu_count(), kts = a.K / 64, col = scaled ? 2 : row_major ? 1 : 0;
+    ShortPlan best = { 0, 0, 1, 0.0 };
+    long long n_all = 0;
+    for (int s = 0; s < a.n_segments; s++) { n_all += a.seg_n_out[s]; }
+    if (a.n_segments == 0) { n_all = a.n_out; }
+    for (const ShortTile& t : kShortTiles)
+    {
+        if (t.one[col] == 0.0f || (t.mb == 2 && a.tokens > 64) || (t.mb == 8 && a.tokens <= 64) || (pair && t.nb == 1)) { continue; }
+        const int width = 64 * (pair ? t.nb / 2 : t.nb);
+        long long tiles = 0;
+        for (int s = 0; s < a.n_segments; s++) { tiles += (a.seg_n_out[s] + width - 1) / width; }
+        if (a.n_segments == 0) { tiles = (a.n_out + width - 1) / width; }
+        tiles *= (a.tokens + 16 * t.mb - 1) / (16 * t.mb);
+        for (int s = 1; s <= max_splits; s++)
+        {
+            if (tiles * s > 2LL * cus || (s > 1 && kts / s < 4)) { break; }
+            double us = 3.5 + (double)((kts + s - 1) / s) * (tiles * s <= cus ? t.one[col] : t.two[col]);
+            if (s > 1) { us += 3.0 + 0.5e-6 * (double)s * a.tokens * n_all * (pair ? 8 : 4); }
+            if (best.us == 0.0 || us < best.us) { best = ShortPlan{ t.mb, t.nb, s, us }; }
+        }
+    }
+    // (a shape in between -- too many tiles here, k ranges needed -- takes the widest tile)
+    if (best.us == 0.0 && max_splits > 1) { best = ShortPlan{ 4, 4, 1, 1.0 }; }
+    return best;
+}
+
+// the same estimate for an unsplit launch of the larger tiles (weights one k-tile ahead), to compare with
+inline double direct_us(const LinearArgs& a, int mb, int nb, long long tiles, bool row_major, bool scaled)
+{
+    const long long rounds = (tiles + cu_count() - 1) / cu_count();
+    double per = mb == 8 ? (nb == 4 ? 0.77 : 0.58) : (nb == 4 ? 0.46 : nb == 3 ? 0.36 : 0.26);
+    if (rounds == 1) { per *= mb == 8 ? 1.13 : 1.25; }
+    else if (rounds == 2) { per *= mb == 8 ? 0.95 : 1.0; }
+    if (scaled) { per *= mb == 8 ? 1.15 : 1.5; }
+    if (row_major) { per *= mb == 8 ? 1.05 : 1.3; }
+    return 3.5 + (double)(a.K / 64) * per * (double)rounds;
+}
+
+// Launches `plan` (gemm_short_*.hip); a.n_segments > 0: up to three linears, pair: gate / up with the SwiGLU product.  Split
+// plans need `partial` (splits * tokens * all features floats, twice that for a pair).  `e` as in gemm_mfma: behind a split
+// plan the combine launch does it, behind an unsplit one the row kernel, with `partial` holding the linear's output.
+void launch_gemm_short(const LinearArgs& a, int w_type, bool half, bool tiled, bool pair, const ShortPlan& plan, float* partial, const AddNormArgs* e);
 
 // FP4 (tiled copies, K % 128 == 0): 64-token x 256-feature tiles, two workgroups per CU
 template <int BLOCK>
@@ -1211,10 +1277,10 @@ void launch_gemm_mfma_direct_segments(LinearArgs a)
     for (int s = 0; s < a.n_segments; s++) { scaled = scaled || a.seg_w_scale[s] != 1.0f; }
     const long long tiles8 = (long long)n_tiles * ((a.tokens + 127) / 128);
     const int n_pad = (n_tiles + 7) & ~7;
-    // Few tiles (q, k, v of a 4096-wide model are 24 feature tiles; up to 512 tokens that is under one workgroup for every
-    // second CU): the k range is split over workgroups as in plan_direct, every segment's partial sums laid out as its own
-    // split GEMM one after the other, and one combine launch finishes all of them (36-layer model, 128 tokens: 8.0 -> 7.0 ms;
-    // 256 tokens 8.4 -> 7.6; 512 tokens 10.8 -> 10.5).
+    // on the file layout the 128-token tile is worth having from one workgroup per CU on, see plan_direct
+    const bool big = a.tokens > 64 && (tiles8 >= 2LL * cus || (!TILED && tiles8 >= cus));
+    // Few tiles (q, k, v of a 4096-wide model are 24 feature tiles of 256): smaller tiles, the k range split over workgroups if
+    // that pays, every segment's partial sums laid out as its own split GEMM one after the other and one combine launch for all.
     {
         int n_all = 0;
         bool by4 = true;
@@ -1226,35 +1292,18 @@ void launch_gemm_mfma_direct_segments(LinearArgs a)
         }
         const int mb = a.tokens > 64 ? 8 : (a.tokens > 32 ? 4 : 2);
         const long long base = (long long)n_tiles * ((a.tokens + mb * 16 - 1) / (mb * 16));
-        long long splits = cus / base;
-        if (splits > (mb == 8 ? 8 : 16)) { splits = mb == 8 ? 8 : 16; }
-        if (splits > a.K / 512) { splits = a.K / 512; }
-        float* partial = splits >= 2 && by4 ? (float*)workspace((size_t)splits * a.tokens * n_all * sizeof(float)) : nullptr;
-        if (partial)
+        const long long splits = std::min({ cus / base, mb == 8 ? 8LL : 16LL, (long long)a.K / 512 });
+        ShortPlan plan = plan_short(a, !TILED, scaled, false, by4 && splits >= 2 ? (int)splits : 1);
+        float* partial = plan.splits > 1 ? (float*)workspace((size_t)plan.splits * a.tokens * n_all * sizeof(float)) : nullptr;
+        if (plan.splits > 1 && !partial) { plan = plan_short(a, !TILED, scaled, false, 1); }
+        const int m_old = big ? 8 : 4;
+        if (plan.us > 0.0 && plan.us < direct_us(a, m_old, 4, (long long)n_tiles * ((a.tokens + 16 * m_old - 1) / (16 * m_old)), !TILED, scaled))
         {
-            const dim3 grid(n_pad * ((a.tokens + mb * 16 - 1) / (mb * 16)), (unsigned)splits);
-            if (mb == 8)
-            {
-                if (scaled) { gemm_mfma_direct_kernel<WT, true, 8, true, TILED, DT_BF16, 4, false, true><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-                else { gemm_mfma_direct_kernel<WT, false, 8, true, TILED, DT_BF16, 4, false, true><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-            }
-            else if (mb == 4)
-            {
-                if (scaled) { gemm_mfma_direct_kernel<WT, true, 4, true, TILED, DT_BF16, 4, false, true, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-                else { gemm_mfma_direct_kernel<WT, false, 4, true, TILED, DT_BF16, 4, false, true, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-            }
-            else
-            {
-                if (scaled) { gemm_mfma_direct_kernel<WT, true, 2, true, TILED, DT_BF16, 4, false, true, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-                else { gemm_mfma_direct_kernel<WT, false, 2, true, TILED, DT_BF16, 4, false, true, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-            }
-            const long long blocks = ((long long)a.tokens * (n_all / 4) + 255) / 256, cap = (long long)cus * 16;
-            gemm_splitk_combine_kernel<DT_BF16, true, false><<<(unsigned)(blocks < cap ? blocks : cap), 256, 0, stream()>>>(partial, (int)splits, a);
+            launch_gemm_short(a, WT, false, TILED, false, plan, partial, nullptr);
             return;
         }
     }
-    // (on the file layout the 128-token tile is worth having from one workgroup per CU on, see plan_direct)
-    if (a.tokens > 64 && (tiles8 >= 2LL * cus || (!TILED && tiles8 >= cus)))
+    if (big)
     {
         const dim3 grid(n_pad * ((a.tokens + 127) / 128));
         if (scaled) { gemm_mfma_direct_kernel<WT, true, 8, false, TILED, DT_BF16, 4, false, true><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
@@ -1275,36 +1324,27 @@ void launch_gemm_mfma_direct_pair(const LinearArgs& a)
     const int n_tiles = (a.n_out + 127) / 128;
     const int m_tiles = (a.tokens + 127) / 128;
     const bool scaled = a.w_scale != 1.0f || a.w_scale_pair != 1.0f;
-    // Up to 128 tokens of a 12288-wide pair are 96 workgroups: the k range is split in two or more and the combine launch
-    // adds the gate and the up sums and writes the SwiGLU product with the same roundings (36-layer model, 128 tokens:
-    // 8.0 -> 7.3 ms; from 129 tokens on, 192 workgroups or more, the split only costs).
+    // Few tiles (up to 128 tokens of a 12288-wide pair are 96): smaller ones, the k range split over workgroups if that pays;
+    // the combine launch then adds the gate and the up sums and writes the SwiGLU product with the same roundings.
     {
         const int mb = a.tokens > 64 ? 8 : (a.tokens > 32 ? 4 : 2);
-        const int m_split = (a.tokens + mb * 16 - 1) / (mb * 16);
-        long long splits = cu_count() / ((long long)n_tiles * m_split);
-        if (splits > 8) { splits = 8; }
-        if (splits > a.K / 512) { splits = a.K / 512; }
-        float* partial = splits >= 2 && a.n_out % 4 == 0 ? (float*)workspace((size_t)2 * splits * a.tokens * a.n_out * sizeof(float)) : nullptr;
-        if (partial)
+        const long long base = (long long)n_tiles * ((a.tokens + mb * 16 - 1) / (mb * 16));
+        const long long splits = std::min({ cu_count() / base, 8LL, (long long)a.K / 512 });
+        ShortPlan plan = plan_short(a, !TILED, scaled, true, a.n_out % 4 == 0 && splits >= 2 ? (int)splits : 1);
+        float* partial = plan.splits > 1 ? (float*)workspace((size_t)2 * plan.splits * a.tokens * a.n_out * sizeof(float)) : nullptr;
+        if (plan.splits > 1 && !partial) { plan = plan_short(a, !TILED, scaled, true, 1); }
+        const double big_us = direct_us(a, 8, 4, (long long)n_tiles * m_tiles, !TILED, scaled);
+        if (plan.us > 0.0 && plan.us < big_us)
         {
-            const dim3 grid(((n_tiles + 7) & ~7) * m_split, (unsigned)splits);
-            if (mb == 8)
-            {
-                if (scaled) { gemm_mfma_direct_kernel<WT, true, 8, true, TILED, DT_BF16, 4, true><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-                else { gemm_mfma_direct_kernel<WT, false, 8, true, TILED, DT_BF16, 4, true><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-            }
-            else if (mb == 4)
-            {
-                if (scaled) { gemm_mfma_direct_kernel<WT, true, 4, true, TILED, DT_BF16, 4, true, false, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-                else { gemm_mfma_direct_kernel<WT, false, 4, true, TILED, DT_BF16, 4, true, false, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-            }
-            else
-            {
-                if (scaled) { gemm_mfma_direct_kernel<WT, true, 2, true, TILED, DT_BF16, 4, true, false, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-                else { gemm_mfma_direct_kernel<WT, false, 2, true, TILED, DT_BF16, 4, true, false, 3><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-            }
-            const long long blocks = ((long long)a.tokens * (a.n_out / 4) + 255) / 256, cap = (long long)cu_count() * 16;
-            gemm_splitk_combine_kernel<DT_BF16, false, true><<<(unsigned)(blocks < cap ? blocks : cap), 256, 0, stream()>>>(partial, (int)splits, a);
+            launch_gemm_short(a, WT, false, TILED, true, plan, partial, nullptr);
+            return;
+        }
+        // 64-token tiles on the tiled copy where they spread over the CUs in fewer whole rounds (12288-wide, 512 tokens: three
+        // rounds of 768 workgroups, 88 us, against 384 larger ones in two, 97; 301 tokens 62 against 86)
+        const int m4 = (a.tokens + 63) / 64;
+        if (TILED && !scaled && direct_us(a, 4, 4, (long long)n_tiles * m4, false, false) < 0.97 * big_us)
+        {
+            gemm_mfma_direct_kernel<WT, false, 4, false, TILED, DT_BF16, 4, true><<<((n_tiles + 7) & ~7) * m4, 256, 0, stream()>>>(a, n_tiles, nullptr);
             return;
         }
     }
@@ -1328,7 +1368,8 @@ void launch_gemm_mfma(const LinearArgs& a)
 // evenly over the CUs (384 tiles on 256 CUs leave half of them with twice the work: 36 % of peak where 512 even tiles
 // reach 42 %), and 48-feature waves with 64-token tiles cost ~5 % against the larger tiles.  Too few tiles in every
 // shape: the k range is split over workgroups (256-feature tiles, about one workgroup per CU, 1024 elements of k or more
-// each; 512 or more up to 64 tokens) and a second kernel adds the partial sums.
+// each; 512 or more up to 64 tokens) and a second kernel adds the partial sums.  (FP8: plan_short then takes over, with at
+// most that many k ranges and so within the scratch asked for here.)
 struct DirectPlan
 {
     int nb, mb, splits;
@@ -1442,15 +1483,15 @@ inline DirectPlan plan_direct_fp4(const LinearArgs& a, SplitScratch* scratch)
 // kernel that keeps the weights out of LDS -- on the tiled copy of the weight when one is registered
 // (1.10-1.15x the row-major rate: a wave's load is then eight full cache lines instead of sixteen half
 // lines).  The tile shape comes from plan_direct (128- or 64-token tiles of 256, 192 or 128 features, whichever spreads
-// most evenly over the CUs); when none fills the machine the k range is split over workgroups (about one per CU, 16 k-tiles or more each) and a
-// second kernel adds the partial sums -- 2x on 512 tokens x 4096 features x K 12288.  Everything else (FP4,
+// most evenly over the CUs), or from plan_short where smaller tiles finish earlier (up to two workgroups per CU), which may
+// also split the k range over workgroups with a second kernel to add the partial sums.  Everything else (FP4,
 // ragged K) takes the two-operand kernel: 128 x 128 tiles with the XCD-aware order when they
 // give every CU at least two workgroups (k step 128 for long K, where it halves the barriers per FLOP),
 // otherwise 128 x 64 tiles to put more workgroups on the machine.
 // `scratch`: see SplitScratch; nullptr = the stream's grow-on-demand workspace.  Returns false (nothing launched)
 // only when a fixed scratch buffer is too small for the k-split this shape takes.
-// `e`: the caller wants the residual add and the norm behind the linear in the combine launch of a k split; false
-// (nothing launched) when this shape does not split.
+// `e`: the caller wants the residual add and the norm behind the linear in its second launch; false (nothing launched) when
+// plan_direct finds tiles enough without a k split.
 template <int WT, int BLOCK, int AT = DT_BF16>
 bool gemm_mfma(const LinearArgs& a, const uint8_t* tiled = nullptr, SplitScratch* scratch = nullptr, const AddNormArgs* e = nullptr)
 {
@@ -1483,20 +1524,24 @@ bool gemm_mfma(const LinearArgs& a, const uint8_t* tiled = nullptr, SplitScratch
             if (plan.refused || (e && plan.splits <= 1)) { return false; }
             const int nb = plan.nb, mb = plan.mb, splits = plan.splits;
             float* const partial = plan.partial;
-            if (nb == 2) { tiled ? launch_gemm_mfma_direct<WT, 4, true, AT, 2>(d) : launch_gemm_mfma_direct<WT, 4, false, AT, 2>(d); }
+            // few tiles: smaller ones, at most as many k ranges as plan_direct found room for
+            const bool scaled = a.w_scale != 1.0f;
+            const ShortPlan small = plan_short(d, tiled == nullptr, scaled, false, splits);
+            const long long tiles = (long long)((a.n_out + 64 * nb - 1) / (64 * nb)) * ((a.tokens + 16 * mb - 1) / (16 * mb));
+            if (small.us > 0.0 && (splits > 1 || small.us < direct_us(a, mb, nb, tiles, tiled == nullptr, scaled)))
+            {
+                launch_gemm_short(d, WT, AT == DT_HALF, tiled != nullptr, false, small, partial, e);
+            }
+            else if (nb == 2) { tiled ? launch_gemm_mfma_direct<WT, 4, true, AT, 2>(d) : launch_gemm_mfma_direct<WT, 4, false, AT, 2>(d); }
             else if (tiled)
             {
                 if (nb == 3) { mb == 8 ? launch_gemm_mfma_direct<WT, 8, true, AT, 3>(d) : launch_gemm_mfma_direct<WT, 4, true, AT, 3>(d); }
-                else if (mb == 8) { launch_gemm_mfma_direct<WT, 8, true, AT>(d, splits, partial, e); }
-                else if (mb == 2 && splits > 1) { launch_gemm_mfma_direct<WT, 2, true, AT>(d, splits, partial, e); }
-                else { launch_gemm_mfma_direct<WT, 4, true, AT>(d, splits, partial, e); }
+                else { mb == 8 ? launch_gemm_mfma_direct<WT, 8, true, AT>(d) : launch_gemm_mfma_direct<WT, 4, true, AT>(d); }
             }
             else
             {
                 if (nb == 3) { mb == 8 ? launch_gemm_mfma_direct<WT, 8, false, AT, 3>(d) : launch_gemm_mfma_direct<WT, 4, false, AT, 3>(d); }
-                else if (mb == 8) { launch_gemm_mfma_direct<WT, 8, false, AT>(d, splits, partial, e); }
-                else if (mb == 2 && splits > 1) { launch_gemm_mfma_direct<WT, 2, false, AT>(d, splits, partial, e); }
-                else { launch_gemm_mfma_direct<WT, 4, false, AT>(d, splits, partial, e); }
+                else { mb == 8 ? launch_gemm_mfma_direct<WT, 8, false, AT>(d) : launch_gemm_mfma_direct<WT, 4, false, AT>(d); }
             }
             return true;
         }

@@ -532,3 +532,64 @@ def test_prompt_and_steps_on_a_non_blocking_stream(gpu, pkg, oracle, dec):
     assert np.array_equal(got[1], want[1])
     for a, b in zip(got[2], want[2]):
         assert np.array_equal(a[:, :75], b[:, :75])
+
+
+@pytest.mark.parametrize("w_type,tiled", [("e5m2", False), ("e5m2", True), ("e4m3", False), ("e4m3", True)])
+@pytest.mark.parametrize("tokens,n_out,K", [(17, 1000, 256), (33, 64, 4096), (32, 16456, 128), (64, 72, 1088), (65, 1000, 2112), (129, 72, 4160), (100, 8328, 128),
+                                            (100, 16392, 128), (128, 16392, 192), (257, 4104, 64), (300, 1032, 2048)])
+def test_short_launches_at_the_edges_of_their_tiles(gpu, oracle, w_type, tiled, tokens, n_out, K):
+    """Launches of up to two workgroups per CU: every tile shape of 32 / 64 / 128 tokens x 64 / 128 / 256 features, unsplit and with a
+    k range split, widths and token counts one past a tile, one k-tile up to an odd number of them; the exact contraction, and
+    nothing written past the output."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(tokens + n_out + K)
+    wt, sc = (oracle.E5M2, 1.0) if w_type == "e5m2" else (oracle.E4M3, 0.013)
+    W = rng.integers(0, 256, size=(n_out, K), dtype=np.uint8)
+    if w_type == "e5m2": W[(W & 0x7C) == 0x7C] = 0x3C
+    else: W[(W & 0x7F) == 0x7F] = 0x38
+    X = oracle.f32_to_bf16((rng.standard_normal((tokens, K)) * (0.05 if w_type == "e5m2" else 1.0)).astype(np.float32))
+    wd, xd = to_dev(torch, dev, W), to_dev(torch, dev, X)
+    keep = None
+    if tiled:
+        keep = torch.zeros(lib.tiled_size(wt, n_out, K), dtype=torch.uint8, device=dev)
+        assert lib.weight_prepare(wd.data_ptr(), wt, n_out, K, K, keep.data_ptr()) == 0
+    try:
+        y = torch.zeros(tokens * n_out + 64, dtype=torch.int16, device=dev)
+        assert lib.linear(wd.data_ptr(), wt, xd.data_ptr(), y.data_ptr(), n_out, tokens, K, sc) == 0
+        got = from_dev(y, np.uint16)
+        assert not got[tokens * n_out:].any()
+        check_rows(oracle.bf16_to_f32(got[:tokens * n_out].reshape(tokens, n_out)).astype(np.float64),
+                   oracle.linear_exact(oracle.dequant_fp8_to_bf16(W, wt, sc), X), "short launch")
+    finally:
+        if tiled:
+            assert lib.weight_release(wd.data_ptr()) == 0
+
+
+@pytest.mark.parametrize("tiled", [False, True])
+def test_residual_add_and_norm_behind_an_unsplit_short_launch(gpu, oracle, tiled):
+    """200 tokens x 4096 features, K 2048: 256 tiles of 64 x 64 and no k split, so the add and the norm follow as the row kernel;
+    the bits of the separate calls."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(3)
+    tokens, n_out, K = 200, 4096, 2048
+    W = rng.integers(0, 256, size=(n_out, K), dtype=np.uint8)
+    W[(W & 0x7C) == 0x7C] = 0x3C
+    X = oracle.f32_to_bf16((rng.standard_normal((tokens, K)) * 0.05).astype(np.float32))
+    R = oracle.f32_to_bf16(rng.standard_normal((tokens, n_out)).astype(np.float32))
+    Wn = oracle.f32_to_bf16((1.0 + 0.1 * rng.standard_normal(n_out)).astype(np.float32))
+    wd, xd, rd, nd = (to_dev(torch, dev, a) for a in (W, X, R, Wn))
+    keep = None
+    if tiled:
+        keep = torch.zeros(lib.tiled_size(oracle.E5M2, n_out, K), dtype=torch.uint8, device=dev)
+        assert lib.weight_prepare(wd.data_ptr(), oracle.E5M2, n_out, K, K, keep.data_ptr()) == 0
+    try:
+        o, s3, y3, s1, y1 = (torch.zeros(tokens * n_out + 64, dtype=torch.int16, device=dev) for _ in range(5))
+        assert lib.linear(wd.data_ptr(), oracle.E5M2, xd.data_ptr(), o.data_ptr(), n_out, tokens, K, 1.0) == 0
+        assert lib.c.hip_add_bf16(ptr(rd), ptr(o), ptr(s3), tokens * n_out) == 0
+        assert lib.c.hip_rms_norm_fwd(oracle.BF16, ptr(s3), ptr(y3), ptr(nd), None, tokens, n_out, ctypes.c_float(1e-6)) == 0
+        assert lib.c.hip_quant_gemm_add_rms_norm(n_out, tokens, K, ptr(wd), oracle.E5M2, K, ctypes.c_float(1.0), ptr(xd), K,
+                                                 ptr(rd), ptr(s1), ptr(nd), ptr(y1), ctypes.c_float(1e-6)) == 0
+        assert np.array_equal(from_dev(s1, np.uint16), from_dev(s3, np.uint16)) and np.array_equal(from_dev(y1, np.uint16), from_dev(y3, np.uint16))
+    finally:
+        if tiled:
+            assert lib.weight_release(wd.data_ptr()) == 0
