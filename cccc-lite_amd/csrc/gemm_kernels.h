@@ -1192,6 +1192,88 @@ inline double direct_us(const LinearArgs& a, int mb, int nb, long long tiles, bo
 // plan the combine launch does it, behind an unsplit one the row kernel, with `partial` holding the linear's output.
 void launch_gemm_short(const LinearArgs& a, int w_type, bool half, bool tiled, bool pair, const ShortPlan& plan, float* partial, const AddNormArgs* e);
 
+// Tiles of the FP4 GEMM.  A workgroup converts its weights itself and a k-tile of it is bound by latency until four or more
+// share a CU, so small tiles that reside several to a CU finish earlier than 256-feature ones with more k ranges, and the 128 x 128
+// tile (half the registers of 128 x 256, so two per CU, and each converted weight used for 128 tokens) is ahead wherever
+// there are many tiles.  The time is estimated as for FP8,
+//   3.5 us + k-tiles of a workgroup x us per k-tile + 3 us + 0.5 us per MB of partial sums if split,
+// with the us per k-tile measured at one and two workgroups per CU and, `each`, per workgroup of a CU beyond (block 16, weights
+// of 33 MB each that rotate through more than the memory-side cache holds).  Against the 128 x 256, 64 x 256 and 128 x 192 tiles alone,
+// which it is compared with (n_out x K, tokens: before -> after): 4096 x 4096, 100: 26.8 -> 17.5 us; 301: 31.8 -> 26.2; 1024 x
+// 4096, 301: 27.7 -> 15.9; 2048: 55.9 -> 31.8; 14336 x 4096, 48: 27.7 -> 22.0; 301: 77.8 -> 56.3; 1024: 134.6 -> 126.1; 4096 x
+// 14336, 100: 38.3 -> 29.4; gate / up pair of 14336 x 4096, 100: 47.6 -> 41.4; 512: 142.7 -> 129.3; 2048: 506.9 -> 457.5.
+struct ShortTileFp4
+{
+    int mb, nb;
+    double one, two, each;
+};
+
+constexpr ShortTileFp4 kShortTilesFp4[] = {
+    { 2, 1, 0.333, 0.36, 0.12 },         // 32 tokens x 64 features
+    { 2, 2, 0.39, 0.465, 0.19 },
+    { 4, 1, 0.36, 0.42, 0.175 },
+    { 4, 2, 0.43, 0.63, 0.285 },
+    { 8, 2, 0.57, 0.95, 0.47 },
+};
+
+// the larger tiles: 128 x 256 takes a CU to itself, two of the others share one
+constexpr ShortTileFp4 kLargeTilesFp4[] = {
+    { 4, 3, 0.52, 0.85, 0.42 },
+    { 4, 4, 0.60, 1.06, 0.53 },
+    { 8, 3, 0.80, 1.38, 0.69 },
+    { 8, 4, 1.00, 2.00, 1.00 },
+};
+
+inline double estimate_fp4_us(const LinearArgs& a, const ShortTileFp4& t, int splits, bool pair)
+{
+    const int width = 64 * (pair ? t.nb / 2 : t.nb), cus = cu_count();
+    long long features = a.n_out, tiles = (a.n_out + width - 1) / width;
+    if (a.n_segments > 0)
+    {
+        features = tiles = 0;
+        for (int s = 0; s < a.n_segments; s++)
+        {
+            features += a.seg_n_out[s];
+            tiles += (a.seg_n_out[s] + width - 1) / width;
+        }
+    }
+    const long long per_cu = (tiles * ((a.tokens + 16 * t.mb - 1) / (16 * t.mb)) * splits + cus - 1) / cus;
+    const double k_tile = per_cu <= 1 ? t.one : std::max(t.two, t.each * (double)per_cu);
+    double us = 3.5 + (double)((a.K / 64 + splits - 1) / splits) * k_tile;
+    if (splits > 1) { us += 3.0 + 0.5e-6 * (double)splits * a.tokens * features * (pair ? 8 : 4); }
+    return us;
+}
+
+// The fastest of these tiles with up to max_splits k ranges (4 k-tiles or more each), if its estimate is 4 % or more below that of
+// the larger tile mb x nb with large_splits (nearer than that the two measure level, either way within 2 %); us == 0 otherwise.
+inline ShortPlan plan_short_fp4(const LinearArgs& a, int mb, int nb, int large_splits, int max_splits, bool pair)
+{
+    ShortPlan best = { 0, 0, 1, 0.0 };
+    double limit = 0.0;
+    for (const ShortTileFp4& t : kLargeTilesFp4)
+    {
+        if (t.mb == mb && t.nb == nb) { limit = 0.96 * estimate_fp4_us(a, t, large_splits, pair); }
+    }
+    for (const ShortTileFp4& t : kShortTilesFp4)
+    {
+        if ((t.mb == 2 && a.tokens > 64) || (t.mb == 8 && a.tokens <= 64) || (pair && t.nb == 1)) { continue; }
+        for (int s = 1; s <= max_splits && (s == 1 || a.K / 64 / s >= 4); s++)
+        {
+            const double us = estimate_fp4_us(a, t, s, pair);
+            if (us < limit)
+            {
+                limit = us;
+                best = ShortPlan{ t.mb, t.nb, s, us };
+            }
+        }
+    }
+    return best;
+}
+
+// Launches `plan` (gemm_short_fp4.hip); a.W = the tiled codes, or a.seg_W = the segments' tiled copies; pair, `partial` and
+// `e` as for launch_gemm_short.
+void launch_gemm4_short(const LinearArgs& a, const uint8_t* tiled_scales, int block, bool pair, const ShortPlan& plan, float* partial, const AddNormArgs* e);
+
 // FP4 (tiled copies, K % 128 == 0): 64-token x 256-feature tiles, two workgroups per CU
 template <int BLOCK>
 void launch_gemm4_mfma_direct_segments(LinearArgs a)
@@ -1220,7 +1302,15 @@ void launch_gemm4_mfma_direct_segments(LinearArgs a)
         long long splits = cus / ((long long)n_tiles * m_tiles);
         if (splits > (mb == 8 ? 8 : 16)) { splits = mb == 8 ? 8 : 16; }
         if (splits > a.K / 512) { splits = a.K / 512; }
-        float* partial = splits >= 2 && by4 ? (float*)workspace((size_t)splits * a.tokens * n_all * sizeof(float)) : nullptr;
+        if (splits < 2 || !by4) { splits = 1; }
+        float* partial = splits > 1 ? (float*)workspace((size_t)splits * a.tokens * n_all * sizeof(float)) : nullptr;
+        if (!partial) { splits = 1; }
+        const ShortPlan plan = plan_short_fp4(a, splits > 1 ? mb : 4, 4, (int)splits, (int)splits, false);
+        if (plan.us > 0.0)
+        {
+            launch_gemm4_short(a, nullptr, BLOCK, false, plan, partial, nullptr);
+            return;
+        }
         if (partial)
         {
             const dim3 grid(((n_tiles + 7) & ~7) * m_tiles, (unsigned)splits);
@@ -1247,6 +1337,13 @@ void launch_gemm4_mfma_direct_pair(const LinearArgs& a)
     if (splits > 8) { splits = 8; }
     if (splits > a.K / 512) { splits = a.K / 512; }
     float* partial = splits >= 2 && a.n_out % 4 == 0 ? (float*)workspace((size_t)2 * splits * a.tokens * a.n_out * sizeof(float)) : nullptr;
+    if (!partial) { splits = 1; }
+    const ShortPlan plan = plan_short_fp4(a, 4, 4, (int)splits, (int)splits, true);
+    if (plan.us > 0.0)
+    {
+        launch_gemm4_short(a, tiled_scales, BLOCK, true, plan, partial, nullptr);
+        return;
+    }
     if (partial)
     {
         const dim3 grid(((n_tiles + 7) & ~7) * m_tiles, (unsigned)splits);
@@ -1505,7 +1602,10 @@ bool gemm_mfma(const LinearArgs& a, const uint8_t* tiled = nullptr, SplitScratch
             const uint8_t* scales = tiled + (long long)((a.n_out + 15) / 16) * (a.K / 128) * 1024;
             const DirectPlan plan = plan_direct_fp4(a, scratch);
             if (plan.refused || (e && plan.splits <= 1)) { return false; }
-            if (plan.nb == 3) { plan.mb == 8 ? launch_gemm4_mfma_direct<BLOCK, 8, 3>(d, scales) : launch_gemm4_mfma_direct<BLOCK, 4, 3>(d, scales); }
+            // at most as many k ranges as plan_direct_fp4 found room for
+            const ShortPlan small = plan_short_fp4(a, plan.mb, plan.nb, plan.splits, plan.splits, false);
+            if (small.us > 0.0) { launch_gemm4_short(d, scales, BLOCK, false, small, plan.partial, e); }
+            else if (plan.nb == 3) { plan.mb == 8 ? launch_gemm4_mfma_direct<BLOCK, 8, 3>(d, scales) : launch_gemm4_mfma_direct<BLOCK, 4, 3>(d, scales); }
             else if (plan.mb == 8) { launch_gemm4_mfma_direct<BLOCK, 8>(d, scales, plan.splits, plan.partial, e); }
             else { launch_gemm4_mfma_direct<BLOCK, 4>(d, scales, plan.splits, plan.partial, e); }
             return true;

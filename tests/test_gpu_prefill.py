@@ -593,3 +593,29 @@ def test_residual_add_and_norm_behind_an_unsplit_short_launch(gpu, oracle, tiled
     finally:
         if tiled:
             assert lib.weight_release(wd.data_ptr()) == 0
+
+
+@pytest.mark.parametrize("block", [16, 32])
+@pytest.mark.parametrize("tokens,n_out,K", [(17, 1000, 256), (33, 72, 4096), (32, 16456, 128), (64, 1032, 1152), (65, 1000, 2176), (129, 72, 4096),
+                                            (100, 8328, 128), (128, 16392, 256), (257, 4104, 128), (300, 1032, 2048), (48, 14344, 4096)])
+def test_fp4_small_tiles_at_their_edges(gpu, oracle, block, tokens, n_out, K):
+    """Every FP4 GEMM tile of 32 / 64 / 128 tokens x 64 / 128 features, unsplit and with a k range split, widths and token counts one
+    past a tile, one chunk of k up to an odd number of them; the exact contraction, and nothing written past the output."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(tokens + n_out + K + block)
+    W = rng.integers(0, 256, size=(n_out, K // 2), dtype=np.uint8)
+    S = rng.integers(0x20, 0x40, size=(n_out, K // block), dtype=np.uint8)
+    X = oracle.f32_to_bf16(rng.standard_normal((tokens, K)).astype(np.float32))
+    wd, sd, xd = (to_dev(torch, dev, v) for v in (W, S, X))
+    keep = torch.zeros(lib.tiled_size(oracle.FP4, n_out, K), dtype=torch.uint8, device=dev)
+    assert lib.weight_prepare_fp4(wd.data_ptr(), sd.data_ptr(), block, n_out, K, keep.data_ptr()) == 0
+    try:
+        y = torch.zeros(tokens * n_out + 64, dtype=torch.int16, device=dev)
+        assert lib.linear(wd.data_ptr(), oracle.FP4, xd.data_ptr(), y.data_ptr(), n_out, tokens, K, 1.0, sd.data_ptr(), block) == 0
+        assert lib.last_kernel() == "gemm_mfma_tiled"
+        got = from_dev(y, np.uint16)
+        assert not got[tokens * n_out:].any()
+        want = oracle.linear_exact(oracle.dequant_weight(W.reshape(-1), oracle.FP4, n_out, K, blk_sc=S.reshape(-1), block=block), X)
+        check_rows(oracle.bf16_to_f32(got[:tokens * n_out].reshape(tokens, n_out)).astype(np.float64), want, "small FP4 tile")
+    finally:
+        assert lib.weight_release(wd.data_ptr()) == 0
