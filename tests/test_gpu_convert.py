@@ -223,3 +223,42 @@ def test_fp4_blockscale_round_trip_at_the_edges(gpu, oracle, n, block):
     assert lib.fp4_blockscale_to_bf16(nib.data_ptr(), sc.data_ptr(), back.data_ptr(), n, block) == 0
     got = from_dev(back, np.uint16)
     assert np.array_equal(got[:n], oracle.dequant_fp4_blockscale_to_bf16(wn, ws, n, block)) and not got[n:].any()
+
+
+@pytest.mark.parametrize("block", [24, 48, 80, 112, 1040])
+def test_fp4_blockscale_of_blocks_that_are_no_power_of_two(gpu, oracle, block):
+    """Blocks of whole 8-element pieces take the vector kernel whatever their number of pieces: the oracle's bits for a ragged
+    last block, with more pieces than the grid keeps in flight (2^22 are 2^25 elements) and fewer, and no more than 1.4 times
+    the time of blocks of 64 over 2^26 elements (measured the same; one element per lane takes three times that)."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(block)
+    for n in (block, block + 8, 3 * block + 7, (1 << 25) + 5 * block + 3):
+        nib = rng.integers(0, 256, size=(n + 1) // 2, dtype=np.uint8)
+        sc = rng.integers(0, 256, size=(n + block - 1) // block, dtype=np.uint8)
+        nd, sd = to_dev(torch, dev, nib), to_dev(torch, dev, sc)
+        out = torch.zeros(n + 32, dtype=torch.int16, device=dev)
+        assert lib.fp4_blockscale_to_bf16(nd.data_ptr(), sd.data_ptr(), out.data_ptr(), n, block) == 0
+        got = from_dev(out, np.uint16)
+        assert not got[n:].any()
+        assert np.array_equal(got[:n], oracle.dequant_fp4_blockscale_to_bf16(nib, sc, n, block)), n
+    n = 1 << 26
+    nd, sd = torch.zeros(n // 2, dtype=torch.uint8, device=dev), torch.zeros(n // 16, dtype=torch.uint8, device=dev)
+    out = torch.zeros(n, dtype=torch.int16, device=dev)
+
+    def best_ms(b):
+        times = []
+        for _ in range(8):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                assert lib.fp4_blockscale_to_bf16(nd.data_ptr(), sd.data_ptr(), out.data_ptr(), n, b) == 0
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    lib.set_sync(False)
+    try:
+        assert best_ms(block) <= 1.4 * best_ms(64)
+    finally:
+        lib.set_sync(True)
