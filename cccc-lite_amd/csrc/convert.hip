@@ -269,15 +269,18 @@ __device__ __forceinline__ uint32_t cast_bits(float v, int dst_type)
 }
 
 // Plain casts (no scale): float->bf16, half->float, half->bf16, bf16->float, bf16->half.
-// BF16 results round to nearest even; NaN inputs stay NaN (quiet bit forced).
-__global__ __launch_bounds__(kThreads) void cast_kernel(const void* __restrict__ src, int src_type, void* __restrict__ dst, int dst_type, size_t begin, size_t n)
+// BF16 results round to nearest even; NaN inputs stay NaN (quiet bit forced).  One element per lane: the last few and
+// misaligned pointers (2^24 misaligned floats to BF16 18.2 us; with the types as
+// run-time arguments 21.7).
+template <int SRC, int DST>
+__global__ __launch_bounds__(kThreads) void cast_kernel(const void* __restrict__ src, void* __restrict__ dst, size_t begin, size_t n)
 {
     const size_t stride = (size_t)gridDim.x * kThreads;
     for (size_t i = begin + (size_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
     {
-        const float v = load_plain(src, src_type, i);
-        if (dst_type == DT_FLOAT) { ((float*)dst)[i] = v; }
-        else { ((uint16_t*)dst)[i] = (uint16_t)cast_bits(v, dst_type); }
+        const float v = load_plain(src, SRC, i);
+        if constexpr (DST == DT_FLOAT) { ((float*)dst)[i] = v; }
+        else { ((uint16_t*)dst)[i] = (uint16_t)cast_bits(v, DST); }
     }
 }
 
@@ -327,7 +330,7 @@ int launch_cast(const void* src, void* dst, unsigned n)
     const size_t n_quads = aligned ? (size_t)n / 4 : 0;
     if (n_quads) { cast_vec_kernel<SRC, DST><<<grid_for(n_quads), kThreads, 0, stream()>>>(src, dst, n_quads); }
     const size_t done = n_quads * 4;
-    if (done < n) { cast_kernel<<<grid_for(n - done), kThreads, 0, stream()>>>(src, SRC, dst, DST, done, n); }
+    if (done < n) { cast_kernel<SRC, DST><<<grid_for(n - done), kThreads, 0, stream()>>>(src, dst, done, n); }
     return finish("convert_cast");
 }
 

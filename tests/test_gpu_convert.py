@@ -262,3 +262,21 @@ def test_fp4_blockscale_of_blocks_that_are_no_power_of_two(gpu, oracle, block):
         assert best_ms(block) <= 1.4 * best_ms(64)
     finally:
         lib.set_sync(True)
+
+
+@pytest.mark.parametrize("offset", [(1, 0), (0, 1), (3, 5)])
+def test_misaligned_casts_and_encoders(gpu, oracle, offset):
+    """Element-aligned pointers that are no multiple of 16 bytes (element offsets of source and destination): the oracle's bits,
+    nothing written outside."""
+    rng = np.random.default_rng(17)
+    n = 70001
+    x = (rng.standard_normal(n + 8) * 2.0 ** rng.integers(-12, 12, n + 8)).astype(np.float32)
+    sources = {oracle.FLOAT: x, oracle.HALF: np.clip(x, -6e4, 6e4).astype(np.float16).view(np.uint16), oracle.BF16: oracle.f32_to_bf16(x)}
+    for st, dt, npdt, scale in ((oracle.FLOAT, oracle.BF16, np.uint16, 1.0), (oracle.HALF, oracle.FLOAT, np.uint32, 1.0), (oracle.HALF, oracle.BF16, np.uint16, 1.0),
+                                (oracle.BF16, oracle.FLOAT, np.uint32, 1.0), (oracle.BF16, oracle.HALF, np.uint16, 1.0), (oracle.FLOAT, oracle.E5M2, np.uint8, 0.9),
+                                (oracle.FLOAT, oracle.E4M3, np.uint8, 3.7), (oracle.BF16, oracle.E4M3, np.uint8, 1.0)):
+        src = sources[st]
+        rc, out = run_convert(gpu, src, st, dt, n, scale, npdt, src_offset=offset[0] * src.itemsize, dst_offset=offset[1] * np.dtype(npdt).itemsize)
+        rc2, want = oracle.convert(np.ascontiguousarray(src[offset[0]:offset[0] + n]), st, dt, n, scale)
+        assert rc == 0 and rc2 == 0
+        assert np.array_equal(out, want.view(npdt)), (st, dt)
