@@ -352,8 +352,7 @@ int hip_attention_decode_fused_bf16(const void* q, const void* k, const void* v,
     if (!aligned16(k_cache) || !aligned16(v_cache) || !aligned16(workspace)) { return -1; }
     const AttentionWorkspace w = attention_workspace(n_q_heads, t_kv);
     if (workspace_bytes < w.total || w.n_blocks > ATT_MAX_BLOCKS) { return -1; }
-    // Chunks per kv head: two workgroups per CU over all heads, and no fewer than the 64 the merge takes in one trip to memory.
-    const int chunks = std::min(w.n_blocks, std::max(64, 2 * cu_count() / n_kv_heads));
+    const int chunks = std::min(w.n_blocks, n_kv_heads <= 2 ? ATT_MAX_CHUNKS : ATT_CHUNKS);      // see ChunkShare
     const dim3 grid(chunks, n_kv_heads);
     float2* stats = (float2*)((char*)workspace + w.stats);
     float* partial = (float*)((char*)workspace + w.partial);

@@ -1101,10 +1101,10 @@ static __global__ __launch_bounds__(256) void attn_combine_kernel(const float* _
 // probabilities stay FP32 instead of being rounded to BF16 before they meet V.  Scores are still
 // rounded to BF16.  Output differences against the three-launch form stay within about one BF16 ulp.
 //
-// Launch 1, grid (blocks, kv heads): raw q [n_q][128], k, v [n_kv][128] of the new token;
-//   waves 0..G-1 normalise and rotate the G query heads of this KV head; the block holding row *d_pos
-//   also normalises / rotates k, appends k and v to the caches, and uses them from LDS;
-//   stats[qh][block] = (max, sum expf(s - max)), partial[block][qh][128] = sum expf(s_t - max) v_t.
+// Launch 1, grid (chunks, kv heads), a chunk being one or more consecutive 64-row blocks of the cache: raw q [n_q][128],
+//   k, v [n_kv][128] of the new token; waves 0..G-1 normalise and rotate the G query heads of this KV head; the chunk
+//   holding row *d_pos also normalises / rotates k, appends k and v to the caches, and uses them from LDS;
+//   stats[qh][chunk] = (max, sum expf(s - max)), partial[chunk][qh][128] = sum expf(s_t - max) v_t.
 // (the fields are 32 bits wide and pass through `arrive` before the first use: as 16-bit values the compiler converts each
 // one in the block that loads it and so waits for it there, one trip to memory after the other)
 struct HeadLoads
@@ -1148,13 +1148,11 @@ __device__ __forceinline__ void norm_rope_head(const uint16_t* __restrict__ src,
     norm_rope_finish(load_head(src, nw, cos_row, sin_row, lane), nw != nullptr, eps, out_l, out_r);
 }
 
-// Launch 1 walks its rows as a stream: grid (chunks, kv heads), chunk c owns `span` consecutive blocks of 64 rows with
-// span = ceil(live blocks / chunks), and each of its four waves takes every fourth 16-row tile of them with a softmax of its
+// Launch 1 walks its rows as a stream: each of a chunk's four waves takes every fourth 16-row tile of it with a softmax of its
 // own (running maximum and sum per head, sums rescaled where the maximum grows), the next tile's rows requested before the
-// current one is used.  Nothing is exchanged between the waves until the end, so the loop has no barrier, and the launch
-// behind merges at most `chunks` partial results however long the cache is: with one workgroup per 64 rows, 32000 rows of 8
-// heads left 500 partial results per head: 31.5 us here and 47 us for their merge, now 25.2 and 4.8 (bound: the 131 MB of
-// rows, 19 us); up to 64 blocks it is level (4096 rows 7.1 us, 640 rows 5.4).
+// current one is used.  Nothing is exchanged between the waves until the end, so the loop has no barrier, and the launch behind
+// merges at most 72 partial results per head however long the cache is: with one workgroup per 64 rows, 32000 rows of 8 heads
+// left 500, 31.5 us here and 47 us for their merge, now 25.2 and 4.8 (bound: the 131 MB of rows, 19 us).
 // Scores of a tile: K[16 keys x 128] . q^T[128 x heads] as four v_mfma_f32_16x16x32_bf16 (products of BF16 values are exact
 // in FP32), key lane i = lane % 16, dims 32 c + 8 g + 0..7 (g = lane / 16), the heads repeated over the 16 columns; the result
 // lane holds head i % G, keys 4 g + 0..3.  Values: lane (i, g) holds dims 8 i + 0..7 of keys 4 g + it, so the probabilities
@@ -1164,7 +1162,34 @@ __device__ __forceinline__ void norm_rope_head(const uint16_t* __restrict__ src,
 // 4096 rows) took two rounds, 13.0 against 11.9 us.
 __device__ __forceinline__ void att_lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }      // leaves the rows in flight alone
 
-__host__ __device__ inline int attention_chunk_span(int live_blocks, int chunks) { return live_blocks <= chunks ? 1 : (live_blocks + chunks - 1) / chunks; }
+// How the live blocks of a cache are dealt out to the chunks of a grid:
+//   up to one per chunk           chunk c is block c (at most 64 chunks; 72 for one or two kv heads, where a second block costs a
+//                                 chunk more than partial results past the 64th cost the merge: 1 head, 65 blocks 7.8 against
+//                                 8.5 us, 72 blocks 8.3 against 8.5)
+//   then, up to 127               64 chunks of one or two blocks, the two-block ones of neighbouring heads on different XCDs.
+//                                 (Half as many chunks of two blocks each leave XCDs and CUs unevenly loaded where the rows bound
+//                                 the launch: 32 kv heads, 68 blocks 22.8 us, so 18.4; 8 heads 10.7, so 10.1)
+//   beyond                        chunks of ceil(live / 64) blocks: equal ones stream 2 - 4 % faster than shares that differ by one
+constexpr int ATT_CHUNKS = 64;
+constexpr int ATT_MAX_CHUNKS = 72;          // of any grid
+
+struct ChunkShare
+{
+    int used, span;         // partial results per head; blocks per chunk, 0: shares of one or two
+
+    __device__ __forceinline__ ChunkShare(int live, int grid_chunks)
+    {
+        used = live;
+        span = 1;
+        if (live > grid_chunks && live < 2 * ATT_CHUNKS) { used = ATT_CHUNKS; span = 0; }
+        else if (live > grid_chunks)
+        {
+            span = (live + ATT_CHUNKS - 1) / ATT_CHUNKS;
+            used = (live + span - 1) / span;            // (a division would cost the short contexts 0.6 us)
+        }
+    }
+    __device__ __forceinline__ int begin(int chunk, int live) const { return span ? chunk * span : chunk * live / ATT_CHUNKS; }
+};
 
 // the value of lane h of the quad (h a constant after unrolling)
 __device__ __forceinline__ float quad_lane(float v, int h) { return h == 0 ? dpp_f32<0x00>(v) : h == 1 ? dpp_f32<0x55>(v) : h == 2 ? dpp_f32<0xAA>(v) : dpp_f32<0xFF>(v); }
@@ -1182,13 +1207,15 @@ __global__ __launch_bounds__(256, G <= 2 ? 4 : 3) void attn_fused_kernel(const u
     __shared__ __attribute__((aligned(16))) uint16_t q_lds[G][128];     // normalised, rotated query heads (BF16 values)
     __shared__ __attribute__((aligned(16))) uint16_t k_new[128];
     __shared__ __attribute__((aligned(16))) uint16_t v_new[128];
-    const int kvh = blockIdx.y, chunk = blockIdx.x, n_chunks = gridDim.x;
+    const int kvh = blockIdx.y, n_chunks = gridDim.x;
     const int pos = *d_pos;
     if (pos < 0 || pos >= t_kv) { return; }         // a position outside the cache: nothing to append, nothing to attend
-    const int span = attention_chunk_span(pos / ATT_KEYS + 1, n_chunks);
-    const int t0 = chunk * span * ATT_KEYS;
-    if (t0 > pos) { return; }
-    const int t1 = min(t0 + span * ATT_KEYS, pos + 1);
+    const int live = pos / ATT_KEYS + 1;
+    const ChunkShare share(live, n_chunks);
+    if ((int)blockIdx.x >= share.used) { return; }
+    const int chunk = share.span ? blockIdx.x : (blockIdx.x + kvh) % ATT_CHUNKS;
+    const int t0 = share.begin(chunk, live) * ATT_KEYS;
+    const int t1 = min(share.begin(chunk + 1, live) * ATT_KEYS, pos + 1);
     const bool has_new = t1 > pos;                  // this chunk holds the row being appended
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane & 15, g = lane >> 4;
@@ -1463,41 +1490,38 @@ __global__ __launch_bounds__(256) void attn_fused_scores_kernel(const uint16_t* 
 }
 
 // Launch 2: y[qh][d] = bf16(sum_b w_b partial[b][qh][d]), w_b = expf(max_b - max) / sum_b' l_b' expf(max_b' - max),
-// in a fixed order, over the chunks b launch 1 wrote.  64 outputs (half a head) per workgroup; n_blocks <= ATT_MAX_BLOCKS.
-constexpr int ATT_MAX_BLOCKS = 1024;
+// in a fixed order, over the chunks b launch 1 wrote.  64 outputs (half a head) per workgroup; grid_chunks <= ATT_MAX_CHUNKS.
+constexpr int ATT_MAX_BLOCKS = 1024;        // 65536 rows: longer caches are refused
 
-// Every load of the common case is requested before anything is known -- the position, up to four (max, sum)
-// pairs per thread and the partials of the first 64 blocks -- so the launch costs one trip to memory instead of
-// three dependent ones (position -> statistics -> partials).  Blocks past the position hold whatever the
+// Every load of the common case is requested before anything is known -- the position, the (max, sum)
+// pairs and the partials of the first 64 chunks -- so the launch costs one trip to memory instead of
+// three dependent ones (position -> statistics -> partials).  Chunks past the position hold whatever the
 // workspace held before: they are masked out by select, never multiplied.
 static __global__ __launch_bounds__(256) void attn_rescale_combine_kernel(const float* __restrict__ partial, const float2* __restrict__ stats, uint16_t* __restrict__ y,
-                                                                  int n_out, int t_kv, int n_blocks, const int* __restrict__ d_pos)
+                                                                  int n_out, int t_kv, int grid_chunks, const int* __restrict__ d_pos)
 {
-    __shared__ float w_lds[ATT_MAX_BLOCKS];
+    __shared__ float w_lds[ATT_MAX_CHUNKS];
     __shared__ float red[4];
     __shared__ float part[4][64];
-    constexpr int PRE = 16;                              // blocks per wave requested up front (4 waves: 64 blocks)
+    constexpr int PRE = 16;                              // chunks per wave requested up front (4 waves: 64 chunks)
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int qh = (blockIdx.x * 64) >> 7;
     const int o = min(blockIdx.x * 64 + lane, n_out - 1);
-    const float2* st = stats + (size_t)qh * n_blocks;
+    const float2* st = stats + (size_t)qh * grid_chunks;
 
     const int pos = *d_pos;
-    const float2 mine = st[min(lane, n_blocks - 1)];    // every wave: block `lane` (used when no more than 64 blocks are live)
-    float2 sb[ATT_MAX_BLOCKS / 256];
-#pragma unroll
-    for (int i = 0; i < ATT_MAX_BLOCKS / 256; i++) { sb[i] = st[min((int)threadIdx.x + i * 256, n_blocks - 1)]; }
+    const float2 mine = st[min(lane, grid_chunks - 1)];              // every wave: chunk `lane` (used when no more than 64 are live)
+    const float2 sb = st[min((int)threadIdx.x, grid_chunks - 1)];    // chunk `threadIdx.x` (used when more are)
     float pre[PRE];
 #pragma unroll
-    for (int j = 0; j < PRE; j++) { pre[j] = __builtin_nontemporal_load(&partial[(size_t)min(wave + 4 * j, n_blocks - 1) * n_out + o]); }
+    for (int j = 0; j < PRE; j++) { pre[j] = __builtin_nontemporal_load(&partial[(size_t)min(wave + 4 * j, grid_chunks - 1) * n_out + o]); }
 
     if (pos < 0 || pos >= t_kv) { return; }
-    const int live = pos / ATT_KEYS + 1, span = attention_chunk_span(live, n_blocks);
-    const int n_active = span == 1 ? live : (live + span - 1) / span;      // (the divisions would cost a short context 0.6 us)
+    const int n_active = ChunkShare(pos / ATT_KEYS + 1, grid_chunks).used;
     float total = 0.0f, inv;
     if (n_active <= 64)
     {
-        // Up to 64 blocks: every wave holds one block's statistics per lane and works out the weights for
+        // Up to 64 chunks: every wave holds one chunk's statistics per lane and works out the weights for
         // itself (the same reductions in the same order as below, whose other three wave sums are zero), so
         // nothing is exchanged before the final sum over the four waves.
         const bool used = lane < n_active;
@@ -1515,30 +1539,15 @@ static __global__ __launch_bounds__(256) void attn_rescale_combine_kernel(const 
     }
     else
     {
-        float m = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < ATT_MAX_BLOCKS / 256; i++)
-        {
-            if ((int)threadIdx.x + i * 256 < n_active) { m = fmaxf(m, sb[i].x); }
-        }
-        m = wave_max(m);
+        const bool used = (int)threadIdx.x < n_active;
+        float m = wave_max(used ? sb.x : -INFINITY);
         if (lane == 0) { red[wave] = m; }
         __syncthreads();
         m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
         __syncthreads();
-        float l = 0.0f;
-#pragma unroll
-        for (int i = 0; i < ATT_MAX_BLOCKS / 256; i++)
-        {
-            const int b = threadIdx.x + i * 256;
-            if (b < n_active)
-            {
-                const float e = expf(sb[i].x - m);
-                w_lds[b] = e;
-                l += sb[i].y * e;
-            }
-        }
-        l = block_sum<256>(l, red);                     // its barrier publishes w_lds
+        const float e = used ? expf(sb.x - m) : 0.0f;
+        if (used) { w_lds[threadIdx.x] = e; }
+        const float l = block_sum<256>(used ? sb.y * e : 0.0f, red);     // its barrier publishes w_lds
         inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
         for (int j = 0; j < PRE; j++) { total = fmaf(pre[j], w_lds[wave + 4 * j], total); }

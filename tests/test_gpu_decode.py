@@ -326,6 +326,32 @@ def test_fused_attention_streams_long_caches(gpu, oracle, dec, n_q, n_kv, t_kv):
         assert np.linalg.norm(dec.f(got) - want) <= 4e-3 * np.linalg.norm(want), pos
 
 
+@pytest.mark.parametrize("n_kv,blocks,partials", [(1, 65, 65), (1, 73, 64), (2, 500, 63), (4, 64, 64), (4, 500, 63), (8, 65, 64), (8, 127, 64), (8, 128, 64), (8, 129, 43), (32, 68, 64)])
+def test_fused_attention_deals_its_blocks_to_at_most_72_chunks(gpu, oracle, dec, n_kv, blocks, partials):
+    """The partial results a launch leaves per head, counted in a workspace filled with a pattern that no result has: a pair of
+    statistics and 128 sums each.  The output is that of the exact route (probabilities rounded to BF16 there: 4e-3 of the norm,
+    as in the tests above)."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(blocks)
+    t_kv, pos = blocks * 64 + 64, blocks * 64 - 1
+    cfg = dec.DecodeConfig(n_q=n_kv, n_kv=n_kv, t_kv=t_kv)
+    cos, sin = (to_dev(torch, dev, a) for a in dec.rope_tables(cfg))
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    caches = [torch.randn(n_kv, t_kv, 128, device=dev).to(torch.bfloat16) for _ in range(2)]
+    q, k, v = (to_dev(torch, dev, oracle.f32_to_bf16(rng.standard_normal((n_kv, 128)).astype(np.float32))) for _ in range(3))
+    pd = torch.tensor([pos], dtype=torch.int32, device=dev)
+    ws_bytes = lib.c.hip_attention_decode_workspace_bytes(n_kv, n_kv, t_kv)
+    out = []
+    for entry in (lib.c.hip_attention_decode_exact_bf16, lib.c.hip_attention_decode_fused_bf16):
+        ws = torch.full((ws_bytes // 4,), -1, dtype=torch.int32, device=dev)
+        y = torch.zeros(n_kv * 128, dtype=torch.int16, device=dev)
+        assert entry(ptr(q), ptr(k), ptr(v), None, None, ptr(cos), ptr(sin), ptr(caches[0]), ptr(caches[1]), ptr(y), ptr(ws), ws_bytes,
+                     n_kv, n_kv, 128, t_kv, ptr(pd), ctypes.c_float(1e-6)) == 0
+        out.append(dec.f(from_dev(y, np.uint16)))
+    assert int((ws != -1).sum()) == partials * n_kv * 130
+    assert np.linalg.norm(out[1] - out[0]) <= 4e-3 * np.linalg.norm(out[0])
+
+
 def test_argmax_and_embed(gpu, oracle):
     torch, dev, lib = gpu
     rng = np.random.default_rng(3)
