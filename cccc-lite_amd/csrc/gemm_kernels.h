@@ -14,11 +14,11 @@
 //   B operand (columns) = output features, same k split
 //   D: lane holds column lane % 32; register v is row 8 (v / 4) + 4 (lane / 32) + v % 4
 #pragma once
+#include "gemm_plan.h"
 #include "gemv_kernels.h"
 #include "linear_args.h"
 #include "quant_device.h"
 #include "runtime.h"
-#include <algorithm>
 #include <type_traits>
 
 namespace ccq
@@ -285,7 +285,7 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(const LinearArgs a, cons
 // PD: how many k-tiles ahead the weights are requested (the activations PD + 1 when PD > 1).  One is enough where two
 // workgroups share a CU and each k-tile carries 64 matrix-core instructions per wave; the k-split launches of a short
 // prompt (one 64-token tile, about one workgroup per CU) are bound by their weight bytes and run a k-tile per memory
-// latency with PD = 1 -- they, and all tiles of plan_short, take PD = 3.
+// latency with PD = 1 -- they, and all small tiles of plan_gemm, take PD = 3.
 template <int WT, bool SCALED, int MB, bool SPLIT, bool TILED, int AT = DT_BF16, int NB = 4, bool PAIR = false, bool SEG = false, int PD = 1, int WGS_PER_CU = 2>
 __global__ __launch_bounds__(256, WGS_PER_CU) void gemm_mfma_direct_kernel(const LinearArgs a_in, const int n_tiles, float* __restrict__ partial)
 {
@@ -1115,168 +1115,31 @@ void launch_gemm_mfma_direct(const LinearArgs& a)
     else { gemm_mfma_direct_kernel<WT, false, MB, false, TILED, AT, NB><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
 }
 
-// Tiles of the FP8 GEMM for launches that leave the chip with two workgroups per CU or fewer: prompts of up to a few hundred
-// tokens, narrow outputs.  Such a launch is not bound by the matrix cores but by what one workgroup takes per k-tile (latency,
-// LDS reads) and by a fixed part, so its time is estimated as
-//   3.5 us (launch, first loads, stores) + k-tiles of a workgroup x us per k-tile + 3 us + 0.5 us per MB of partial sums if split
-// with the us per k-tile measured for one and for two workgroups per CU and each tile shape, and the tile shape and k split
-// with the least estimate is taken.  Smaller tiles with weights requested three k-tiles ahead need fewer k ranges, so fewer
-// FP32 partial sums are written, read and added (E5M2 file layout, 100 tokens, this against the 128 x 256 tiles with up to
-// eight k ranges it replaces: 4096 x 4096 14.8 - 15.6 against 22.3 us, K 12288 28.8 against 31.8, the q, k, v launch 17.4
-// against 21.9, the gate / up pair 41.9 against 47; HALF, E4M3 with a scale, tiled copies, 301 tokens: 4096 x 4096 25.1
-// against 29.1, 1024 x 4096 13.2 against 22.5, 12288 x 4096 47.8 against 64.8).  Over a grid of 7 shapes x 8 token counts the
-// choice is within 10 % of the fastest combination, mostly within 4 %.
-struct ShortTile
-{
-    int mb, nb;
-    float one[3], two[3];            // us per k-tile with one / two workgroups per CU: tiled copy, file layout, with a scale
-};
+// Launches an FP8 plan with small tiles or a k split (gemm_short_*.hip); a.n_segments > 0: up to three linears, pair: gate / up
+// with the SwiGLU product.  Split plans need `partial` (splits * tokens * all features floats, twice that for a pair).  `e` as in
+// gemm_mfma: behind a split plan the combine launch does it, behind an unsplit one the row kernel, with `partial` holding the
+// linear's output.
+void launch_gemm_short(const LinearArgs& a, int w_type, bool half, bool tiled, bool pair, const GemmPlan& plan, float* partial, const AddNormArgs* e);
 
-constexpr ShortTile kShortTiles[] = {
-    { 2, 1, { 0.115f, 0.135f, 0.15f }, { 0.21f, 0.25f, 0.28f } },       // 32 tokens x 64 features
-    { 2, 2, { 0.17f, 0.22f, 0.21f }, { 0.32f, 0.42f, 0.40f } },
-    { 4, 1, { 0.20f, 0.21f, 0.25f }, { 0.375f, 0.38f, 0.43f } },
-    { 4, 2, { 0.29f, 0.32f, 0.35f }, { 0.48f, 0.63f, 0.63f } },
-    { 4, 4, { 0.49f, 0.58f, 0.71f }, { 0.93f, 1.15f, 1.4f } },
-    { 8, 2, { 0.0f, 0.54f, 0.0f }, { 0.0f, 0.92f, 0.0f } },             // file layout only: a 16 x 64-byte load serves twice the products
-};
+// The same for an FP4 plan with small tiles (gemm_short_fp4.hip); a.W = the tiled codes, or a.seg_W = the segments' tiled copies.
+// A workgroup converts its weights itself and a k-tile of it is bound by latency until four or more share a CU, so small tiles
+// that reside several to a CU finish earlier than 256-feature ones with more k ranges, and the 128 x 128 tile (half the registers
+// of 128 x 256, so two per CU, and each converted weight used for 128 tokens) is ahead wherever there are many tiles.
+void launch_gemm4_short(const LinearArgs& a, const uint8_t* tiled_scales, int block, bool pair, const GemmPlan& plan, float* partial, const AddNormArgs* e);
 
-struct ShortPlan
-{
-    int mb, nb, splits;
-    double us;               // estimate; 0: no shape fits
-};
+// floats of partial sums a split plan needs, and the stream's scratch for them (nullptr: none to be had)
+inline float* split_workspace(const GemmPlan& plan, long long outputs) { return plan.splits > 1 ? (float*)workspace((size_t)plan.splits * outputs * sizeof(float)) : nullptr; }
 
-inline ShortPlan plan_short(const LinearArgs& a, bool row_major, bool scaled, bool pair, int max_splits)
+// the plan of a joint or paired launch of `outputs` values, without a k split if there is no scratch memory for it
+inline GemmPlan joint_plan(const LinearArgs& a, GemmKind kind, const GemmWeights& w, long long outputs, float*& partial)
 {
-    const int cus = cu_count(), kts = a.K / 64, col = scaled ? 2 : row_major ? 1 : 0;
-    ShortPlan best = { 0, 0, 1, 0.0 };
-    long long n_all = 0;
-    for (int s = 0; s < a.n_segments; s++) { n_all += a.seg_n_out[s]; }
-    if (a.n_segments == 0) { n_all = a.n_out; }
-    for (const ShortTile& t : kShortTiles)
-    {
-        if (t.one[col] == 0.0f || (t.mb == 2 && a.tokens > 64) || (t.mb == 8 && a.tokens <= 64) || (pair && t.nb == 1)) { continue; }
-        const int width = 64 * (pair ? t.nb / 2 : t.nb);
-        long long tiles = 0;
-        for (int s = 0; s < a.n_segments; s++) { tiles += (a.seg_n_out[s] + width - 1) / width; }
-        if (a.n_segments == 0) { tiles = (a.n_out + width - 1) / width; }
-        tiles *= (a.tokens + 16 * t.mb - 1) / (16 * t.mb);
-        for (int s = 1; s <= max_splits; s++)
-        {
-            if (tiles * s > 2LL * cus || (s > 1 && kts / s < 4)) { break; }
-            double us = 3.5 + (double)((kts + s - 1) / s) * (tiles * s <= cus ? t.one[col] : t.two[col]);
-            if (s > 1) { us += 3.0 + 0.5e-6 * (double)s * a.tokens * n_all * (pair ? 8 : 4); }
-            if (best.us == 0.0 || us < best.us) { best = ShortPlan{ t.mb, t.nb, s, us }; }
-        }
-    }
-    // (a shape in between -- too many tiles here, k ranges needed -- takes the widest tile)
-    if (best.us == 0.0 && max_splits > 1) { best = ShortPlan{ 4, 4, 1, 1.0 }; }
-    return best;
+    GemmPlan plan = plan_gemm(a, kind, w, cu_count(), true);
+    partial = split_workspace(plan, outputs);
+    return plan.splits > 1 && !partial ? plan_gemm(a, kind, w, cu_count(), false) : plan;
 }
 
-// the same estimate for an unsplit launch of the larger tiles (weights one k-tile ahead), to compare with
-inline double direct_us(const LinearArgs& a, int mb, int nb, long long tiles, bool row_major, bool scaled)
-{
-    const long long rounds = (tiles + cu_count() - 1) / cu_count();
-    double per = mb == 8 ? (nb == 4 ? 0.77 : 0.58) : (nb == 4 ? 0.46 : nb == 3 ? 0.36 : 0.26);
-    if (rounds == 1) { per *= mb == 8 ? 1.13 : 1.25; }
-    else if (rounds == 2) { per *= mb == 8 ? 0.95 : 1.0; }
-    if (scaled) { per *= mb == 8 ? 1.15 : 1.5; }
-    if (row_major) { per *= mb == 8 ? 1.05 : 1.3; }
-    return 3.5 + (double)(a.K / 64) * per * (double)rounds;
-}
-
-// Launches `plan` (gemm_short_*.hip); a.n_segments > 0: up to three linears, pair: gate / up with the SwiGLU product.  Split
-// plans need `partial` (splits * tokens * all features floats, twice that for a pair).  `e` as in gemm_mfma: behind a split
-// plan the combine launch does it, behind an unsplit one the row kernel, with `partial` holding the linear's output.
-void launch_gemm_short(const LinearArgs& a, int w_type, bool half, bool tiled, bool pair, const ShortPlan& plan, float* partial, const AddNormArgs* e);
-
-// Tiles of the FP4 GEMM.  A workgroup converts its weights itself and a k-tile of it is bound by latency until four or more
-// share a CU, so small tiles that reside several to a CU finish earlier than 256-feature ones with more k ranges, and the 128 x 128
-// tile (half the registers of 128 x 256, so two per CU, and each converted weight used for 128 tokens) is ahead wherever
-// there are many tiles.  The time is estimated as for FP8,
-//   3.5 us + k-tiles of a workgroup x us per k-tile + 3 us + 0.5 us per MB of partial sums if split,
-// with the us per k-tile measured at one and two workgroups per CU and, `each`, per workgroup of a CU beyond (block 16, weights
-// of 33 MB each that rotate through more than the memory-side cache holds).  Against the 128 x 256, 64 x 256 and 128 x 192 tiles alone,
-// which it is compared with (n_out x K, tokens: before -> after): 4096 x 4096, 100: 26.8 -> 17.5 us; 301: 31.8 -> 26.2; 1024 x
-// 4096, 301: 27.7 -> 15.9; 2048: 55.9 -> 31.8; 14336 x 4096, 48: 27.7 -> 22.0; 301: 77.8 -> 56.3; 1024: 134.6 -> 126.1; 4096 x
-// 14336, 100: 38.3 -> 29.4; gate / up pair of 14336 x 4096, 100: 47.6 -> 41.4; 512: 142.7 -> 129.3; 2048: 506.9 -> 457.5.
-struct ShortTileFp4
-{
-    int mb, nb;
-    double one, two, each;
-};
-
-constexpr ShortTileFp4 kShortTilesFp4[] = {
-    { 2, 1, 0.333, 0.36, 0.12 },         // 32 tokens x 64 features
-    { 2, 2, 0.39, 0.465, 0.19 },
-    { 4, 1, 0.36, 0.42, 0.175 },
-    { 4, 2, 0.43, 0.63, 0.285 },
-    { 8, 2, 0.57, 0.95, 0.47 },
-};
-
-// the larger tiles: 128 x 256 takes a CU to itself, two of the others share one
-constexpr ShortTileFp4 kLargeTilesFp4[] = {
-    { 4, 3, 0.52, 0.85, 0.42 },
-    { 4, 4, 0.60, 1.06, 0.53 },
-    { 8, 3, 0.80, 1.38, 0.69 },
-    { 8, 4, 1.00, 2.00, 1.00 },
-};
-
-inline double estimate_fp4_us(const LinearArgs& a, const ShortTileFp4& t, int splits, bool pair)
-{
-    const int width = 64 * (pair ? t.nb / 2 : t.nb), cus = cu_count();
-    long long features = a.n_out, tiles = (a.n_out + width - 1) / width;
-    if (a.n_segments > 0)
-    {
-        features = tiles = 0;
-        for (int s = 0; s < a.n_segments; s++)
-        {
-            features += a.seg_n_out[s];
-            tiles += (a.seg_n_out[s] + width - 1) / width;
-        }
-    }
-    const long long per_cu = (tiles * ((a.tokens + 16 * t.mb - 1) / (16 * t.mb)) * splits + cus - 1) / cus;
-    const double k_tile = per_cu <= 1 ? t.one : std::max(t.two, t.each * (double)per_cu);
-    double us = 3.5 + (double)((a.K / 64 + splits - 1) / splits) * k_tile;
-    if (splits > 1) { us += 3.0 + 0.5e-6 * (double)splits * a.tokens * features * (pair ? 8 : 4); }
-    return us;
-}
-
-// The fastest of these tiles with up to max_splits k ranges (4 k-tiles or more each), if its estimate is 4 % or more below that of
-// the larger tile mb x nb with large_splits (nearer than that the two measure level, either way within 2 %); us == 0 otherwise.
-inline ShortPlan plan_short_fp4(const LinearArgs& a, int mb, int nb, int large_splits, int max_splits, bool pair)
-{
-    ShortPlan best = { 0, 0, 1, 0.0 };
-    double limit = 0.0;
-    for (const ShortTileFp4& t : kLargeTilesFp4)
-    {
-        if (t.mb == mb && t.nb == nb) { limit = 0.96 * estimate_fp4_us(a, t, large_splits, pair); }
-    }
-    for (const ShortTileFp4& t : kShortTilesFp4)
-    {
-        if ((t.mb == 2 && a.tokens > 64) || (t.mb == 8 && a.tokens <= 64) || (pair && t.nb == 1)) { continue; }
-        for (int s = 1; s <= max_splits && (s == 1 || a.K / 64 / s >= 4); s++)
-        {
-            const double us = estimate_fp4_us(a, t, s, pair);
-            if (us < limit)
-            {
-                limit = us;
-                best = ShortPlan{ t.mb, t.nb, s, us };
-            }
-        }
-    }
-    return best;
-}
-
-// Launches `plan` (gemm_short_fp4.hip); a.W = the tiled codes, or a.seg_W = the segments' tiled copies; pair, `partial` and
-// `e` as for launch_gemm_short.
-void launch_gemm4_short(const LinearArgs& a, const uint8_t* tiled_scales, int block, bool pair, const ShortPlan& plan, float* partial, const AddNormArgs* e);
-
-// FP4 (tiled copies, K % 128 == 0): 64-token x 256-feature tiles, two workgroups per CU
-template <int BLOCK>
-void launch_gemm4_mfma_direct_segments(LinearArgs a)
+// a.seg_tile0 for 256-feature tiles (empty segments start past the last tile); the number of tiles
+inline int segment_tiles(LinearArgs& a)
 {
     int n_tiles = 0;
     for (int s = 0; s < 3; s++)
@@ -1285,167 +1148,99 @@ void launch_gemm4_mfma_direct_segments(LinearArgs a)
         if (s < a.n_segments) { n_tiles += (a.seg_n_out[s] + 255) / 256; }
     }
     a.seg_tile0[3] = n_tiles;
-    for (int s = a.n_segments; s < 3; s++) { a.seg_tile0[s] = n_tiles; }
-    // few tiles: the k range split over workgroups and one combine launch for all segments, as for FP8 below
-    {
-        const int cus = cu_count();
-        int n_all = 0;
-        bool by4 = true;
-        for (int sg = 0; sg < 3; sg++)
-        {
-            if (sg >= a.n_segments) { a.seg_n_out[sg] = 0; }
-            n_all += a.seg_n_out[sg];
-            by4 = by4 && a.seg_n_out[sg] % 4 == 0;
-        }
-        const int mb = a.tokens > 64 ? 8 : 4;
-        const int m_tiles = (a.tokens + mb * 16 - 1) / (mb * 16);
-        long long splits = cus / ((long long)n_tiles * m_tiles);
-        if (splits > (mb == 8 ? 8 : 16)) { splits = mb == 8 ? 8 : 16; }
-        if (splits > a.K / 512) { splits = a.K / 512; }
-        if (splits < 2 || !by4) { splits = 1; }
-        float* partial = splits > 1 ? (float*)workspace((size_t)splits * a.tokens * n_all * sizeof(float)) : nullptr;
-        if (!partial) { splits = 1; }
-        const ShortPlan plan = plan_short_fp4(a, splits > 1 ? mb : 4, 4, (int)splits, (int)splits, false);
-        if (plan.us > 0.0)
-        {
-            launch_gemm4_short(a, nullptr, BLOCK, false, plan, partial, nullptr);
-            return;
-        }
-        if (partial)
-        {
-            const dim3 grid(((n_tiles + 7) & ~7) * m_tiles, (unsigned)splits);
-            if (mb == 8) { gemm4_mfma_direct_kernel<BLOCK, 8, true, 4, true><<<grid, 256, 0, stream()>>>(a, nullptr, n_tiles, partial); }
-            else { gemm4_mfma_direct_kernel<BLOCK, 4, true, 4, true><<<grid, 256, 0, stream()>>>(a, nullptr, n_tiles, partial); }
-            const long long blocks = ((long long)a.tokens * (n_all / 4) + 255) / 256, cap = (long long)cus * 16;
-            gemm_splitk_combine_kernel<DT_BF16, true, false><<<(unsigned)(blocks < cap ? blocks : cap), 256, 0, stream()>>>(partial, (int)splits, a);
-            return;
-        }
-    }
-    const dim3 grid(((n_tiles + 7) & ~7) * ((a.tokens + 63) / 64));
-    gemm4_mfma_direct_kernel<BLOCK, 4, false, 4, true><<<grid, 256, 0, stream()>>>(a, nullptr, n_tiles, nullptr);
+    return n_tiles;
 }
 
-// FP4 gate / up pair with the SwiGLU product (tiled copies; a.W / a.W_pair = the copies, codes then scale bytes): 64 tokens
-// x 128 output features per workgroup, the k range split when those are too few for the GPU
+inline long long segment_outputs(const LinearArgs& a) { return (long long)a.tokens * (a.seg_n_out[0] + a.seg_n_out[1] + a.seg_n_out[2]); }
+
+// up to three linears on the same activations in one launch (FP4: tiled copies, K % 128 == 0)
+template <int BLOCK>
+void launch_gemm4_mfma_direct_segments(LinearArgs a)
+{
+    float* partial;
+    const GemmPlan plan = joint_plan(a, GEMM_SEGMENTS, GemmWeights{ true, false, false }, segment_outputs(a), partial);
+    if (plan.small)
+    {
+        launch_gemm4_short(a, nullptr, BLOCK, false, plan, partial, nullptr);
+        return;
+    }
+    const int n_tiles = segment_tiles(a);
+    const dim3 grid(((n_tiles + 7) & ~7) * ((a.tokens + 16 * plan.mb - 1) / (16 * plan.mb)), plan.splits);
+    if (plan.splits <= 1)
+    {
+        gemm4_mfma_direct_kernel<BLOCK, 4, false, 4, true><<<grid, 256, 0, stream()>>>(a, nullptr, n_tiles, nullptr);
+        return;
+    }
+    if (plan.mb == 8) { gemm4_mfma_direct_kernel<BLOCK, 8, true, 4, true><<<grid, 256, 0, stream()>>>(a, nullptr, n_tiles, partial); }
+    else { gemm4_mfma_direct_kernel<BLOCK, 4, true, 4, true><<<grid, 256, 0, stream()>>>(a, nullptr, n_tiles, partial); }
+    const long long blocks = (segment_outputs(a) / 4 + 255) / 256, cap = (long long)cu_count() * 16;
+    gemm_splitk_combine_kernel<DT_BF16, true, false><<<(unsigned)(blocks < cap ? blocks : cap), 256, 0, stream()>>>(partial, plan.splits, a);
+}
+
+// gate / up pair with the SwiGLU product (FP4: tiled copies; a.W / a.W_pair = the copies, codes then scale bytes)
 template <int BLOCK>
 void launch_gemm4_mfma_direct_pair(const LinearArgs& a)
 {
     const uint8_t* tiled_scales = a.W + (long long)((a.n_out + 15) / 16) * (a.K / 128) * 1024;
-    const int n_tiles = (a.n_out + 127) / 128;
-    const int m_tiles = (a.tokens + 63) / 64;
-    long long splits = cu_count() / ((long long)n_tiles * m_tiles);
-    if (splits > 8) { splits = 8; }
-    if (splits > a.K / 512) { splits = a.K / 512; }
-    float* partial = splits >= 2 && a.n_out % 4 == 0 ? (float*)workspace((size_t)2 * splits * a.tokens * a.n_out * sizeof(float)) : nullptr;
-    if (!partial) { splits = 1; }
-    const ShortPlan plan = plan_short_fp4(a, 4, 4, (int)splits, (int)splits, true);
-    if (plan.us > 0.0)
+    const long long outputs = (long long)a.tokens * a.n_out;
+    float* partial;
+    const GemmPlan plan = joint_plan(a, GEMM_PAIR, GemmWeights{ true, false, false }, 2 * outputs, partial);
+    if (plan.small)
     {
         launch_gemm4_short(a, tiled_scales, BLOCK, true, plan, partial, nullptr);
         return;
     }
-    if (partial)
+    const int n_tiles = (a.n_out + 127) / 128;
+    const dim3 grid(((n_tiles + 7) & ~7) * ((a.tokens + 63) / 64), plan.splits);
+    if (plan.splits <= 1)
     {
-        const dim3 grid(((n_tiles + 7) & ~7) * m_tiles, (unsigned)splits);
-        gemm4_mfma_direct_kernel<BLOCK, 4, true, 4, false, true><<<grid, 256, 0, stream()>>>(a, tiled_scales, n_tiles, partial);
-        const long long blocks = ((long long)a.tokens * (a.n_out / 4) + 255) / 256, cap = (long long)cu_count() * 16;
-        gemm_splitk_combine_kernel<DT_BF16, false, true><<<(unsigned)(blocks < cap ? blocks : cap), 256, 0, stream()>>>(partial, (int)splits, a);
+        gemm4_mfma_direct_kernel<BLOCK, 4, false, 4, false, true><<<grid, 256, 0, stream()>>>(a, tiled_scales, n_tiles, nullptr);
         return;
     }
-    const dim3 grid(((n_tiles + 7) & ~7) * m_tiles);
-    gemm4_mfma_direct_kernel<BLOCK, 4, false, 4, false, true><<<grid, 256, 0, stream()>>>(a, tiled_scales, n_tiles, nullptr);
+    gemm4_mfma_direct_kernel<BLOCK, 4, true, 4, false, true><<<grid, 256, 0, stream()>>>(a, tiled_scales, n_tiles, partial);
+    const long long blocks = (outputs / 4 + 255) / 256, cap = (long long)cu_count() * 16;
+    gemm_splitk_combine_kernel<DT_BF16, false, true><<<(unsigned)(blocks < cap ? blocks : cap), 256, 0, stream()>>>(partial, plan.splits, a);
 }
 
-// up to three linears on the same activations in one launch: 64- or 128-token x 256-feature tiles, whichever gives the CUs
-// two rounds of workgroups or more evenly
 template <int WT, bool TILED>
 void launch_gemm_mfma_direct_segments(LinearArgs a)
 {
-    const int cus = cu_count();
-    int n_tiles = 0;
-    for (int s = 0; s < 3; s++)
-    {
-        a.seg_tile0[s] = n_tiles;
-        if (s < a.n_segments) { n_tiles += (a.seg_n_out[s] + 255) / 256; }
-    }
-    a.seg_tile0[3] = n_tiles;
-    for (int s = a.n_segments; s < 3; s++) { a.seg_tile0[s] = n_tiles; }       // empty segments start past the last tile
     bool scaled = false;
     for (int s = 0; s < a.n_segments; s++) { scaled = scaled || a.seg_w_scale[s] != 1.0f; }
-    const long long tiles8 = (long long)n_tiles * ((a.tokens + 127) / 128);
-    const int n_pad = (n_tiles + 7) & ~7;
-    // on the file layout the 128-token tile is worth having from one workgroup per CU on, see plan_direct
-    const bool big = a.tokens > 64 && (tiles8 >= 2LL * cus || (!TILED && tiles8 >= cus));
-    // Few tiles (q, k, v of a 4096-wide model are 24 feature tiles of 256): smaller tiles, the k range split over workgroups if
-    // that pays, every segment's partial sums laid out as its own split GEMM one after the other and one combine launch for all.
+    float* partial;
+    const GemmPlan plan = joint_plan(a, GEMM_SEGMENTS, GemmWeights{ false, !TILED, scaled }, segment_outputs(a), partial);
+    if (plan.small || plan.splits > 1)
     {
-        int n_all = 0;
-        bool by4 = true;
-        for (int sg = 0; sg < 3; sg++)
-        {
-            if (sg >= a.n_segments) { a.seg_n_out[sg] = 0; }
-            n_all += a.seg_n_out[sg];
-            by4 = by4 && a.seg_n_out[sg] % 4 == 0;
-        }
-        const int mb = a.tokens > 64 ? 8 : (a.tokens > 32 ? 4 : 2);
-        const long long base = (long long)n_tiles * ((a.tokens + mb * 16 - 1) / (mb * 16));
-        const long long splits = std::min({ cus / base, mb == 8 ? 8LL : 16LL, (long long)a.K / 512 });
-        ShortPlan plan = plan_short(a, !TILED, scaled, false, by4 && splits >= 2 ? (int)splits : 1);
-        float* partial = plan.splits > 1 ? (float*)workspace((size_t)plan.splits * a.tokens * n_all * sizeof(float)) : nullptr;
-        if (plan.splits > 1 && !partial) { plan = plan_short(a, !TILED, scaled, false, 1); }
-        const int m_old = big ? 8 : 4;
-        if (plan.us > 0.0 && plan.us < direct_us(a, m_old, 4, (long long)n_tiles * ((a.tokens + 16 * m_old - 1) / (16 * m_old)), !TILED, scaled))
-        {
-            launch_gemm_short(a, WT, false, TILED, false, plan, partial, nullptr);
-            return;
-        }
+        launch_gemm_short(a, WT, false, TILED, false, plan, partial, nullptr);
+        return;
     }
-    if (big)
+    const int n_tiles = segment_tiles(a);
+    const dim3 grid(((n_tiles + 7) & ~7) * ((a.tokens + 16 * plan.mb - 1) / (16 * plan.mb)));
+    if (plan.mb == 8)
     {
-        const dim3 grid(n_pad * ((a.tokens + 127) / 128));
         if (scaled) { gemm_mfma_direct_kernel<WT, true, 8, false, TILED, DT_BF16, 4, false, true><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
         else { gemm_mfma_direct_kernel<WT, false, 8, false, TILED, DT_BF16, 4, false, true><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
     }
     else
     {
-        const dim3 grid(n_pad * ((a.tokens + 63) / 64));
         if (scaled) { gemm_mfma_direct_kernel<WT, true, 4, false, TILED, DT_BF16, 4, false, true><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
         else { gemm_mfma_direct_kernel<WT, false, 4, false, TILED, DT_BF16, 4, false, true><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
     }
 }
 
-// gate / up pair with the SwiGLU product in the epilogue: 128 tokens x 128 output features per workgroup
 template <int WT, bool TILED>
 void launch_gemm_mfma_direct_pair(const LinearArgs& a)
 {
-    const int n_tiles = (a.n_out + 127) / 128;
-    const int m_tiles = (a.tokens + 127) / 128;
     const bool scaled = a.w_scale != 1.0f || a.w_scale_pair != 1.0f;
-    // Few tiles (up to 128 tokens of a 12288-wide pair are 96): smaller ones, the k range split over workgroups if that pays;
-    // the combine launch then adds the gate and the up sums and writes the SwiGLU product with the same roundings.
+    float* partial;
+    const GemmPlan plan = joint_plan(a, GEMM_PAIR, GemmWeights{ false, !TILED, scaled }, 2LL * a.tokens * a.n_out, partial);
+    if (plan.small || plan.splits > 1)
     {
-        const int mb = a.tokens > 64 ? 8 : (a.tokens > 32 ? 4 : 2);
-        const long long base = (long long)n_tiles * ((a.tokens + mb * 16 - 1) / (mb * 16));
-        const long long splits = std::min({ cu_count() / base, 8LL, (long long)a.K / 512 });
-        ShortPlan plan = plan_short(a, !TILED, scaled, true, a.n_out % 4 == 0 && splits >= 2 ? (int)splits : 1);
-        float* partial = plan.splits > 1 ? (float*)workspace((size_t)2 * plan.splits * a.tokens * a.n_out * sizeof(float)) : nullptr;
-        if (plan.splits > 1 && !partial) { plan = plan_short(a, !TILED, scaled, true, 1); }
-        const double big_us = direct_us(a, 8, 4, (long long)n_tiles * m_tiles, !TILED, scaled);
-        if (plan.us > 0.0 && plan.us < big_us)
-        {
-            launch_gemm_short(a, WT, false, TILED, true, plan, partial, nullptr);
-            return;
-        }
-        // 64-token tiles on the tiled copy where they spread over the CUs in fewer whole rounds (12288-wide, 512 tokens: three
-        // rounds of 768 workgroups, 88 us, against 384 larger ones in two, 97; 301 tokens 62 against 86)
-        const int m4 = (a.tokens + 63) / 64;
-        if (TILED && !scaled && direct_us(a, 4, 4, (long long)n_tiles * m4, false, false) < 0.97 * big_us)
-        {
-            gemm_mfma_direct_kernel<WT, false, 4, false, TILED, DT_BF16, 4, true><<<((n_tiles + 7) & ~7) * m4, 256, 0, stream()>>>(a, n_tiles, nullptr);
-            return;
-        }
+        launch_gemm_short(a, WT, false, TILED, true, plan, partial, nullptr);
+        return;
     }
-    const dim3 grid(((n_tiles + 7) & ~7) * m_tiles);
+    const int n_tiles = (a.n_out + 127) / 128;
+    const dim3 grid(((n_tiles + 7) & ~7) * ((a.tokens + 127) / 128));
     if (scaled) { gemm_mfma_direct_kernel<WT, true, 8, false, TILED, DT_BF16, 4, true><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
     else { gemm_mfma_direct_kernel<WT, false, 8, false, TILED, DT_BF16, 4, true><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
 }
@@ -1460,127 +1255,36 @@ void launch_gemm_mfma(const LinearArgs& a)
     else { gemm_mfma_kernel<WT, BLOCK, BM, BN, false, BK, XCD, AT><<<grid, 256, 0, stream()>>>(a, n_tiles, m_tiles); }
 }
 
-// Tile shape and k split of the register-fed kernels (tuned on MI355X with the FP8 kernel): a workgroup owns 64 NB features x
-// 16 MB tokens.  A CU wants two resident workgroups (one alone reaches ~85 % of the rate), the workgroups should spread
-// evenly over the CUs (384 tiles on 256 CUs leave half of them with twice the work: 36 % of peak where 512 even tiles
-// reach 42 %), and 48-feature waves with 64-token tiles cost ~5 % against the larger tiles.  Too few tiles in every
-// shape: the k range is split over workgroups (256-feature tiles, about one workgroup per CU, 1024 elements of k or more
-// each; 512 or more up to 64 tokens) and a second kernel adds the partial sums.  (FP8: plan_short then takes over, with at
-// most that many k ranges and so within the scratch asked for here.)
-struct DirectPlan
+// The plan of one linear and the FP32 scratch for its partial sums (or, behind an unsplit small launch with the add and norm, for
+// the linear's output).  False: a fixed scratch buffer is too small for the k ranges this shape takes (SplitScratch::refused says
+// how much they need), or, with the add and norm, there is no k split or no scratch for it.
+inline bool linear_plan(const LinearArgs& a, const GemmWeights& w, bool add_norm, SplitScratch* scratch, GemmPlan& plan, float*& partial)
 {
-    int nb, mb, splits;
-    float* partial;
-    bool refused;            // a fixed scratch buffer is too small for the k split this shape takes (SplitScratch::refused says how much)
-};
-
-// Gives the plan `s` k ranges and the FP32 scratch they need; false when a fixed scratch buffer is too small for them.
-inline bool attach_split(DirectPlan& plan, const LinearArgs& a, long long s, SplitScratch* scratch)
-{
-    if (s <= 1) { return true; }
-    const size_t need = (size_t)s * a.tokens * a.n_out * sizeof(float);
-    if (scratch && scratch->strict)
+    plan = plan_gemm(a, GEMM_LINEAR, w, cu_count(), true);
+    partial = nullptr;
+    if (plan.ranges > 1)
     {
-        if (!scratch->fixed || need > scratch->fixed_bytes)
+        const size_t need = (size_t)plan.ranges * a.tokens * a.n_out * sizeof(float);
+        if (scratch && scratch->strict)
         {
-            scratch->refused = need;
-            plan.refused = true;
-            return false;
+            if (!scratch->fixed || need > scratch->fixed_bytes)
+            {
+                scratch->refused = need;
+                return false;
+            }
+            partial = scratch->fixed;
         }
-        plan.partial = scratch->fixed;
+        else { partial = (float*)workspace(need); }
+        if (!partial) { plan = plan_gemm(a, GEMM_LINEAR, w, cu_count(), false); }
     }
-    else { plan.partial = (float*)workspace(need); }
-    if (plan.partial) { plan.splits = (int)s; }
-    return true;
-}
-
-// fp4: the FP4 kernel's costs -- the 128-token x 256-feature tile stays out of the scoring (see plan_direct_fp4), and
-// 64-token tiles pay for converting every weight for half as many products (913 against 1037 TFLOP/s at equal balance).
-// row_major (FP8 only): the weight is read from the file layout, where a wave's load is sixteen half cache lines; 64-token
-// tiles then pay that fetch for half as many products, and a 128-token tile is worth having even at one workgroup per CU
-// (4096 x 4096 at 2048 tokens: 70 us against 91; K 12288: 196 against 244; on the tiled copy the two are level).
-// 64 tokens x 128 features (FP8, K < 8192, at most 2048 features) puts 256 or more workgroups on outputs as narrow as 1024
-// features (2048 tokens: 29 / 35 us tiled / row-major against 33 / 40).  Wider outputs with few tiles keep the k split: with
-// a long K it is far ahead (K 12288 at 512 tokens: 60 against 110 us), and on 512 tokens x 4096 x 4096, where the two
-// measure the same on weights that rotate through the memory-side cache, the split is 8 us ahead inside a whole model.
-inline DirectPlan plan_direct(const LinearArgs& a, SplitScratch* scratch, bool fp4 = false, bool row_major = false)
-{
-    const int cus = cu_count();
-    const bool big_tile = !fp4;
-    struct Shape { int nb, mb; double quality; };
-    const double q64 = row_major ? 0.8 : 1.0;            // what a 64-token tile is worth against a 128-token one
-    const Shape shapes[] = { { 4, 8, 1.0 }, { 4, 4, fp4 ? 0.88 : q64 }, { 3, 8, 1.0 }, { 3, 4, fp4 ? 0.84 : 0.95 * q64 }, { 2, 4, 0.9 * q64 } };
-    DirectPlan plan = { 4, 4, 1, nullptr, false };
-    double best = -1.0;
-    for (const Shape& sh : shapes)
-    {
-        if (sh.nb == 2 && (fp4 || a.K >= 8192 || a.n_out > 2048)) { continue; }
-        if (sh.mb == 8 && (a.tokens <= 64 || (sh.nb == 4 && !big_tile))) { continue; }
-        const long long tiles = (long long)((a.n_out + 64 * sh.nb - 1) / (64 * sh.nb)) * ((a.tokens + 16 * sh.mb - 1) / (16 * sh.mb));
-        const double balance = (double)tiles / (double)(((tiles + cus - 1) / cus) * cus);
-        double occupancy = tiles >= 2LL * cus ? 1.0 : (tiles > cus ? 0.95 : 0.85);
-        // one 128 x 256 tile on (nearly) every CU and a long K: ahead of two 64-token tiles per CU, which convert every weight
-        // twice (2048 tokens x 4096 features, K 12288, tiled copy: 160 against 168-170 us; K 4096: level)
-        if (sh.nb == 4 && sh.mb == 8 && !row_major && a.K >= 8192 && tiles * 8 > 7LL * cus && tiles <= cus) { occupancy = 1.02; }
-        const double score = sh.quality * balance * occupancy;
-        if (score > best + 1e-9)
-        {
-            best = score;
-            plan.nb = sh.nb;
-            plan.mb = sh.mb;
-        }
-    }
-    const long long n_tiles = (a.n_out + 255) / 256;
-    const long long tiles8 = n_tiles * ((a.tokens + 127) / 128), tiles4 = n_tiles * ((a.tokens + 63) / 64);
-    if (best < 0.6 && tiles4 * 4 < 5LL * cus && a.n_out % 4 == 0)
-    {
-        const long long base = a.tokens > 64 ? tiles8 : tiles4;
-        long long s = (cus + base / 2) / base;
-        // up to 64 tokens the weight bytes bound the launch and finer k ranges put more workgroups on them (32 tokens:
-        // 4096 x 4096 17.3 -> 14.6 us, 1024 x 4096 16.3 -> 13.5, 4096 x 12288 28.5 -> 24.0); above that the FP32 partial
-        // sums weigh more and a range keeps 1024 elements of k or more
-        const long long s_max = a.tokens <= 64 ? 16 : 8, k_min = a.tokens <= 64 ? 512 : 1024;
-        if (s > s_max) { s = s_max; }
-        if (s > a.K / k_min) { s = a.K / k_min; }
-        if (!attach_split(plan, a, s, scratch)) { return plan; }
-        if (plan.splits > 1)
-        {
-            plan.nb = 4;
-            plan.mb = a.tokens > 64 ? 8 : (a.tokens > 32 || fp4 ? 4 : 2);        // FP8, up to 32 tokens: a 32-token tile
-        }
-    }
-    return plan;
-}
-
-// FP4: the 128 x 256 tile needs the register file of a whole SIMD per wave, so a CU runs one such workgroup at a time
-// and nothing hides its prologue and epilogue: it pays when every tile gets a CU of its own (1009 TFLOP/s on
-// 2048 x 4096, K 14336, against 940 for 64 x 256 tiles; 767 against 1009 for 128 x 192 tiles on 2048 x 14336, where a CU
-// runs three or four of them in sequence), with the k range split when the tiles are few.
-inline DirectPlan plan_direct_fp4(const LinearArgs& a, SplitScratch* scratch)
-{
-    const int cus = cu_count();
-    const long long tiles = (long long)((a.n_out + 255) / 256) * ((a.tokens + 127) / 128);
-    if (a.tokens > 64 && tiles <= cus)
-    {
-        long long s = a.n_out % 4 == 0 ? (cus + tiles / 2) / tiles : 1;
-        if (s > 8) { s = 8; }
-        if (s > a.K / 1024) { s = a.K / 1024; }
-        if (s < 1) { s = 1; }
-        if (tiles * s * 5 >= 3LL * cus)
-        {
-            DirectPlan plan = { 4, 8, 1, nullptr, false };
-            attach_split(plan, a, s, scratch);
-            return plan;
-        }
-    }
-    return plan_direct(a, scratch, true);
+    return !add_norm || plan.ranges > 1;
 }
 
 // Kernel choice (tuned on MI355X).  FP8 weights with K a multiple of 64 and at least 17 tokens take the
 // kernel that keeps the weights out of LDS -- on the tiled copy of the weight when one is registered
 // (1.10-1.15x the row-major rate: a wave's load is then eight full cache lines instead of sixteen half
-// lines).  The tile shape comes from plan_direct (128- or 64-token tiles of 256, 192 or 128 features, whichever spreads
-// most evenly over the CUs), or from plan_short where smaller tiles finish earlier (up to two workgroups per CU), which may
+// lines).  The tile shape comes from plan_gemm (128- or 64-token tiles of 256, 192 or 128 features, whichever spreads
+// most evenly over the CUs, or smaller ones where they finish earlier), which may
 // also split the k range over workgroups with a second kernel to add the partial sums.  Everything else (FP4,
 // ragged K) takes the two-operand kernel: 128 x 128 tiles with the XCD-aware order when they
 // give every CU at least two workgroups (k step 128 for long K, where it halves the barriers per FLOP),
@@ -1588,7 +1292,7 @@ inline DirectPlan plan_direct_fp4(const LinearArgs& a, SplitScratch* scratch)
 // `scratch`: see SplitScratch; nullptr = the stream's grow-on-demand workspace.  Returns false (nothing launched)
 // only when a fixed scratch buffer is too small for the k-split this shape takes.
 // `e`: the caller wants the residual add and the norm behind the linear in its second launch; false (nothing launched) when
-// plan_direct finds tiles enough without a k split.
+// the larger tiles are enough for the GPU without a k split.
 template <int WT, int BLOCK, int AT = DT_BF16>
 bool gemm_mfma(const LinearArgs& a, const uint8_t* tiled = nullptr, SplitScratch* scratch = nullptr, const AddNormArgs* e = nullptr)
 {
@@ -1600,14 +1304,13 @@ bool gemm_mfma(const LinearArgs& a, const uint8_t* tiled = nullptr, SplitScratch
             LinearArgs d = a;
             d.W = tiled;
             const uint8_t* scales = tiled + (long long)((a.n_out + 15) / 16) * (a.K / 128) * 1024;
-            const DirectPlan plan = plan_direct_fp4(a, scratch);
-            if (plan.refused || (e && plan.splits <= 1)) { return false; }
-            // at most as many k ranges as plan_direct_fp4 found room for
-            const ShortPlan small = plan_short_fp4(a, plan.mb, plan.nb, plan.splits, plan.splits, false);
-            if (small.us > 0.0) { launch_gemm4_short(d, scales, BLOCK, false, small, plan.partial, e); }
+            GemmPlan plan;
+            float* partial;
+            if (!linear_plan(a, GemmWeights{ true, false, false }, e != nullptr, scratch, plan, partial)) { return false; }
+            if (plan.small) { launch_gemm4_short(d, scales, BLOCK, false, plan, partial, e); }
             else if (plan.nb == 3) { plan.mb == 8 ? launch_gemm4_mfma_direct<BLOCK, 8, 3>(d, scales) : launch_gemm4_mfma_direct<BLOCK, 4, 3>(d, scales); }
-            else if (plan.mb == 8) { launch_gemm4_mfma_direct<BLOCK, 8>(d, scales, plan.splits, plan.partial, e); }
-            else { launch_gemm4_mfma_direct<BLOCK, 4>(d, scales, plan.splits, plan.partial, e); }
+            else if (plan.mb == 8) { launch_gemm4_mfma_direct<BLOCK, 8>(d, scales, plan.splits, partial, e); }
+            else { launch_gemm4_mfma_direct<BLOCK, 4>(d, scales, plan.splits, partial, e); }
             return true;
         }
     }
@@ -1620,18 +1323,11 @@ bool gemm_mfma(const LinearArgs& a, const uint8_t* tiled = nullptr, SplitScratch
         {
             LinearArgs d = a;
             if (tiled) { d.W = tiled; }
-            const DirectPlan plan = plan_direct(a, scratch, false, tiled == nullptr);
-            if (plan.refused || (e && plan.splits <= 1)) { return false; }
-            const int nb = plan.nb, mb = plan.mb, splits = plan.splits;
-            float* const partial = plan.partial;
-            // few tiles: smaller ones, at most as many k ranges as plan_direct found room for
-            const bool scaled = a.w_scale != 1.0f;
-            const ShortPlan small = plan_short(d, tiled == nullptr, scaled, false, splits);
-            const long long tiles = (long long)((a.n_out + 64 * nb - 1) / (64 * nb)) * ((a.tokens + 16 * mb - 1) / (16 * mb));
-            if (small.us > 0.0 && (splits > 1 || small.us < direct_us(a, mb, nb, tiles, tiled == nullptr, scaled)))
-            {
-                launch_gemm_short(d, WT, AT == DT_HALF, tiled != nullptr, false, small, partial, e);
-            }
+            GemmPlan plan;
+            float* partial;
+            if (!linear_plan(a, GemmWeights{ false, tiled == nullptr, a.w_scale != 1.0f }, e != nullptr, scratch, plan, partial)) { return false; }
+            const int nb = plan.nb, mb = plan.mb;
+            if (plan.small || plan.splits > 1) { launch_gemm_short(d, WT, AT == DT_HALF, tiled != nullptr, false, plan, partial, e); }
             else if (nb == 2) { tiled ? launch_gemm_mfma_direct<WT, 4, true, AT, 2>(d) : launch_gemm_mfma_direct<WT, 4, false, AT, 2>(d); }
             else if (tiled)
             {

@@ -1,5 +1,5 @@
-// The tile shapes of plan_short (gemm_kernels.h) on the register-fed FP8 GEMM, every one with weights requested three k-tiles
-// ahead: one translation unit per weight type (gemm_short_e5m2.hip, gemm_short_e4m3.hip) instantiates them.
+// The small tiles of plan_gemm (gemm_plan.h) on the register-fed FP8 GEMM, every one with weights requested three k-tiles ahead,
+// and the k-split launches of the larger ones: one translation unit per weight type (gemm_short_e5m2.hip, gemm_short_e4m3.hip) instantiates them.
 #pragma once
 #include "gemm_kernels.h"
 #include "prefill_kernels.h"
@@ -7,17 +7,16 @@
 namespace ccq
 {
 
-template <int WT, bool SCALED, bool TILED, int AT, int MB, int NB, bool PAIR, bool SEG>
+template <int WT, bool SCALED, bool TILED, int AT, int MB, int NB, bool PAIR, bool SEG, int PD = 3, bool SPLIT_ONLY = false>
 void launch_short_tile(const LinearArgs& a, int n_tiles, int splits, float* partial)
 {
-    constexpr int PD = 3;
     const dim3 grid(((n_tiles + 7) & ~7) * ((a.tokens + MB * 16 - 1) / (MB * 16)), splits);
     if (splits > 1) { gemm_mfma_direct_kernel<WT, SCALED, MB, true, TILED, AT, NB, PAIR, SEG, PD><<<grid, 256, 0, stream()>>>(a, n_tiles, partial); }
-    else { gemm_mfma_direct_kernel<WT, SCALED, MB, false, TILED, AT, NB, PAIR, SEG, PD><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
+    else if constexpr (!SPLIT_ONLY) { gemm_mfma_direct_kernel<WT, SCALED, MB, false, TILED, AT, NB, PAIR, SEG, PD><<<grid, 256, 0, stream()>>>(a, n_tiles, nullptr); }
 }
 
 template <int WT, bool SCALED, bool TILED, int AT, bool PAIR, bool SEG>
-void launch_short_shape(LinearArgs a, const ShortPlan& p, float* partial, const AddNormArgs* e)
+void launch_short_shape(LinearArgs a, const GemmPlan& p, float* partial, const AddNormArgs* e)
 {
     const int width = 64 * (PAIR ? p.nb / 2 : p.nb);
     if (e && p.splits <= 1)
@@ -50,6 +49,7 @@ void launch_short_shape(LinearArgs a, const ShortPlan& p, float* partial, const 
             if (p.nb == 1) { launch_short_tile<WT, SCALED, TILED, AT, 2, 1, PAIR, SEG>(a, n_tiles, p.splits, partial); }
         }
         if (p.nb == 2) { launch_short_tile<WT, SCALED, TILED, AT, 2, 2, PAIR, SEG>(a, n_tiles, p.splits, partial); }
+        if (p.nb == 4) { launch_short_tile<WT, SCALED, TILED, AT, 2, 4, PAIR, SEG, 3, true>(a, n_tiles, p.splits, partial); }
     }
     else if (p.mb == 4)
     {
@@ -60,6 +60,7 @@ void launch_short_shape(LinearArgs a, const ShortPlan& p, float* partial, const 
         if (p.nb == 2) { launch_short_tile<WT, SCALED, TILED, AT, 4, 2, PAIR, SEG>(a, n_tiles, p.splits, partial); }
         if (p.nb == 4) { launch_short_tile<WT, SCALED, TILED, AT, 4, 4, PAIR, SEG>(a, n_tiles, p.splits, partial); }
     }
+    else if (p.nb == 4) { launch_short_tile<WT, SCALED, TILED, AT, 8, 4, PAIR, SEG, 1, true>(a, n_tiles, p.splits, partial); }
     else if constexpr (!TILED && !SCALED) { launch_short_tile<WT, SCALED, TILED, AT, 8, 2, PAIR, SEG>(a, n_tiles, p.splits, partial); }
     if (p.splits <= 1)
     {
@@ -76,7 +77,7 @@ void launch_short_shape(LinearArgs a, const ShortPlan& p, float* partial, const 
 }
 
 template <int WT, bool SCALED, bool TILED>
-void launch_short_layout(const LinearArgs& a, bool half, bool pair, const ShortPlan& p, float* partial, const AddNormArgs* e)
+void launch_short_layout(const LinearArgs& a, bool half, bool pair, const GemmPlan& p, float* partial, const AddNormArgs* e)
 {
     if (pair) { launch_short_shape<WT, SCALED, TILED, DT_BF16, true, false>(a, p, partial, e); }
     else if (a.n_segments > 0) { launch_short_shape<WT, SCALED, TILED, DT_BF16, false, true>(a, p, partial, e); }
@@ -85,7 +86,7 @@ void launch_short_layout(const LinearArgs& a, bool half, bool pair, const ShortP
 }
 
 template <int WT>
-void launch_short_type(const LinearArgs& a, bool half, bool tiled, bool pair, const ShortPlan& p, float* partial, const AddNormArgs* e)
+void launch_short_type(const LinearArgs& a, bool half, bool tiled, bool pair, const GemmPlan& p, float* partial, const AddNormArgs* e)
 {
     bool scaled = a.n_segments == 0 && (a.w_scale != 1.0f || (pair && a.w_scale_pair != 1.0f));
     for (int s = 0; s < a.n_segments; s++) { scaled = scaled || a.seg_w_scale[s] != 1.0f; }
@@ -93,7 +94,7 @@ void launch_short_type(const LinearArgs& a, bool half, bool tiled, bool pair, co
     else { tiled ? launch_short_layout<WT, false, true>(a, half, pair, p, partial, e) : launch_short_layout<WT, false, false>(a, half, pair, p, partial, e); }
 }
 
-void launch_gemm_short_e5m2(const LinearArgs& a, bool half, bool tiled, bool pair, const ShortPlan& p, float* partial, const AddNormArgs* e);
-void launch_gemm_short_e4m3(const LinearArgs& a, bool half, bool tiled, bool pair, const ShortPlan& p, float* partial, const AddNormArgs* e);
+void launch_gemm_short_e5m2(const LinearArgs& a, bool half, bool tiled, bool pair, const GemmPlan& p, float* partial, const AddNormArgs* e);
+void launch_gemm_short_e4m3(const LinearArgs& a, bool half, bool tiled, bool pair, const GemmPlan& p, float* partial, const AddNormArgs* e);
 
 }    // namespace ccq

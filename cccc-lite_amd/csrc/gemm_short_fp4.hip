@@ -1,4 +1,4 @@
-// The tile shapes of plan_short_fp4 (gemm_kernels.h) on the register-fed FP4 GEMM.
+// The small tiles of plan_gemm (gemm_plan.h) on the register-fed FP4 GEMM.
 #include "gemm_kernels.h"
 #include "prefill_kernels.h"
 
@@ -17,7 +17,7 @@ void launch_tile(const LinearArgs& a, const uint8_t* scales, int n_tiles, int sp
 }
 
 template <int BLOCK, bool PAIR, bool SEG>
-void launch_shape(LinearArgs a, const uint8_t* scales, const ShortPlan& p, float* partial, const AddNormArgs* e)
+void launch_shape(LinearArgs a, const uint8_t* scales, const GemmPlan& p, float* partial, const AddNormArgs* e)
 {
     const int width = 64 * (PAIR ? p.nb / 2 : p.nb);
     if (e && p.splits <= 1)
@@ -65,7 +65,7 @@ void launch_shape(LinearArgs a, const uint8_t* scales, const ShortPlan& p, float
 }
 
 template <int BLOCK>
-void launch_block(const LinearArgs& a, const uint8_t* scales, bool pair, const ShortPlan& p, float* partial, const AddNormArgs* e)
+void launch_block(const LinearArgs& a, const uint8_t* scales, bool pair, const GemmPlan& p, float* partial, const AddNormArgs* e)
 {
     if (pair) { launch_shape<BLOCK, true, false>(a, scales, p, partial, e); }
     else if (a.n_segments > 0) { launch_shape<BLOCK, false, true>(a, scales, p, partial, e); }
@@ -74,7 +74,7 @@ void launch_block(const LinearArgs& a, const uint8_t* scales, bool pair, const S
 
 }    // namespace
 
-void launch_gemm4_short(const LinearArgs& a, const uint8_t* tiled_scales, int block, bool pair, const ShortPlan& plan, float* partial, const AddNormArgs* e)
+void launch_gemm4_short(const LinearArgs& a, const uint8_t* tiled_scales, int block, bool pair, const GemmPlan& plan, float* partial, const AddNormArgs* e)
 {
     block == 16 ? launch_block<16>(a, tiled_scales, pair, plan, partial, e) : launch_block<32>(a, tiled_scales, pair, plan, partial, e);
 }
