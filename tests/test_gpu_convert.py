@@ -189,7 +189,8 @@ def test_absmax_of_a_tensor(gpu, oracle, src_type, n, offset):
 @pytest.mark.parametrize("n", [3, 4, 67, 1 << 12, (1 << 24) + 4096 * 4 + 7])
 def test_vector_casts_and_encoders_at_the_edges(gpu, oracle, n):
     """Four-element kernels: fewer elements than a piece, a ragged tail, and more pieces than the grid keeps in flight at once
-    (256 CUs x 16 workgroups x 256 lanes x 4 pieces = 2^24 elements), with NaN, infinities and both zeros among the values."""
+    (256 CUs x 16 workgroups x 256 lanes x 4 pieces = 2^22 pieces, 2^24 elements here), with NaN, infinities and both zeros
+    among the values."""
     rng = np.random.default_rng(n)
     x = (rng.standard_normal(n) * 2.0 ** rng.integers(-12, 12, n)).astype(np.float32)
     x[:3] = [-0.0, np.inf, -np.inf]
@@ -207,7 +208,8 @@ def test_vector_casts_and_encoders_at_the_edges(gpu, oracle, n):
 
 @pytest.mark.parametrize("n,block", [(16, 16), (15, 16), (16 * 257, 16), (32 * 129 + 31, 32), (31, 32), ((1 << 24) + 16 * 1000 + 9, 16), ((1 << 24) + 64, 32), (4096, 8)])
 def test_fp4_blockscale_round_trip_at_the_edges(gpu, oracle, n, block):
-    """The lane-group encoder (whole blocks of 16 or 32) and the scalar rest behind it; the codes decoded again."""
+    """The lane-group encoder (whole blocks of 16 or 32) and the scalar rest behind it; the codes decoded again (2^24 elements are
+    2^21 of the decoder's pieces: its loop over four pieces at once is the next test's)."""
     torch, dev, lib = gpu
     rng = np.random.default_rng(n)
     x = (rng.standard_normal(n) * 2.0 ** rng.integers(-9, 9, n)).astype(np.float32)
@@ -280,3 +282,34 @@ def test_misaligned_casts_and_encoders(gpu, oracle, offset):
         rc2, want = oracle.convert(np.ascontiguousarray(src[offset[0]:offset[0] + n]), st, dt, n, scale)
         assert rc == 0 and rc2 == 0
         assert np.array_equal(out, want.view(npdt)), (st, dt)
+
+
+@pytest.mark.parametrize("src,dst,n", [("e5m2", "bf16", (1 << 25) + 4099), ("e4m3", "bf16", (1 << 25) + 13), ("e5m2", "half", (1 << 25) + 4099), ("e4m3", "float", (1 << 24) + 4099),
+                                       ("e5m2", "float", (1 << 24) + 3), ("fp4", "bf16", (1 << 25) + 4099), ("fp4", "float", (1 << 24) + 4099), ("fp4", "block16", (1 << 25) + 4099),
+                                       ("fp4", "block32", (1 << 25) + 21)])
+def test_decoders_with_more_pieces_than_are_in_flight(gpu, oracle, src, dst, n):
+    """2^22 pieces and a ragged tail: every lane takes four pieces at once, then single ones, then the scalar kernel the rest.  A
+    piece is 4 elements for FLOAT results and 8 for the 16-bit ones."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(n)
+    codes = rng.integers(0, 256, size=(n + 1) // 2 if src == "fp4" else n, dtype=np.uint8)
+    if dst.startswith("block"):
+        block = int(dst[5:])
+        sc = rng.integers(0, 256, size=(n + block - 1) // block, dtype=np.uint8)
+        cd, sd = to_dev(torch, dev, codes), to_dev(torch, dev, sc)
+        out = torch.zeros(n + 16, dtype=torch.int16, device=dev)
+        assert lib.fp4_blockscale_to_bf16(cd.data_ptr(), sd.data_ptr(), out.data_ptr(), n, block) == 0
+        got = from_dev(out, np.uint16)
+        assert np.array_equal(got[:n], oracle.dequant_fp4_blockscale_to_bf16(codes, sc, n, block)) and not got[n:].any()
+        return
+    st = {"e5m2": oracle.E5M2, "e4m3": oracle.E4M3, "fp4": oracle.FP4}[src]
+    dt, npdt, real = {"float": (oracle.FLOAT, np.uint32, np.float32), "half": (oracle.HALF, np.uint16, np.float16), "bf16": (oracle.BF16, np.uint16, None)}[dst]
+    rc, out = run_convert(gpu, codes, st, dt, n, 0.37, npdt)
+    rc2, want = oracle.convert(codes, st, dt, n, 0.37)
+    assert rc == 0 and rc2 == 0
+    want = want.view(npdt)
+    if real is None or src == "fp4":
+        assert np.array_equal(out, want)
+    else:
+        nan = np.isnan(want.view(real))
+        assert np.array_equal(out[~nan], want[~nan]) and np.all(np.isnan(out.view(real)[nan]))

@@ -538,9 +538,9 @@ def test_prompt_and_steps_on_a_non_blocking_stream(gpu, pkg, oracle, dec):
 @pytest.mark.parametrize("tokens,n_out,K", [(17, 1000, 256), (33, 64, 4096), (32, 16456, 128), (64, 72, 1088), (65, 1000, 2112), (129, 72, 4160), (100, 8328, 128),
                                             (100, 16392, 128), (128, 16392, 192), (257, 4104, 64), (300, 1032, 2048)])
 def test_short_launches_at_the_edges_of_their_tiles(gpu, oracle, w_type, tiled, tokens, n_out, K):
-    """Launches of up to two workgroups per CU: every tile shape of 32 / 64 / 128 tokens x 64 / 128 / 256 features, unsplit and with a
-    k range split, widths and token counts one past a tile, one k-tile up to an odd number of them; the exact contraction, and
-    nothing written past the output."""
+    """Launches of few workgroups, on tiles of 32 and 64 tokens x 64 features with and without the k range split and 64 x 192 ones,
+    widths and token counts one past a tile, one k-tile up to an odd number of them; the exact contraction, and nothing written
+    past the output.  (test_gpu_gemm_tiles.py has every tile, unsplit and split.)"""
     torch, dev, lib = gpu
     rng = np.random.default_rng(tokens + n_out + K)
     wt, sc = (oracle.E5M2, 1.0) if w_type == "e5m2" else (oracle.E4M3, 0.013)
@@ -599,8 +599,9 @@ def test_residual_add_and_norm_behind_an_unsplit_short_launch(gpu, oracle, tiled
 @pytest.mark.parametrize("tokens,n_out,K", [(17, 1000, 256), (33, 72, 4096), (32, 16456, 128), (64, 1032, 1152), (65, 1000, 2176), (129, 72, 4096),
                                             (100, 8328, 128), (128, 16392, 256), (257, 4104, 128), (300, 1032, 2048), (48, 14344, 4096)])
 def test_fp4_small_tiles_at_their_edges(gpu, oracle, block, tokens, n_out, K):
-    """Every FP4 GEMM tile of 32 / 64 / 128 tokens x 64 / 128 features, unsplit and with a k range split, widths and token counts one
-    past a tile, one chunk of k up to an odd number of them; the exact contraction, and nothing written past the output."""
+    """FP4 GEMM tiles of 32 and 64 tokens x 64 features with and without the k range split, 32 x 128, 64 x 128 and 64 x 192 ones,
+    widths and token counts one past a tile, one chunk of k up to an odd number of them; the exact contraction, and nothing
+    written past the output.  (test_gpu_gemm_tiles.py has every tile, unsplit and split.)"""
     torch, dev, lib = gpu
     rng = np.random.default_rng(tokens + n_out + K + block)
     W = rng.integers(0, 256, size=(n_out, K // 2), dtype=np.uint8)
