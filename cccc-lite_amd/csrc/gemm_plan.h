@@ -204,13 +204,14 @@ inline double estimate_us(const LinearArgs& a, GemmKind kind, const GemmTile& t,
     return us;
 }
 
-// The larger tile, or the small one with the least estimate if that is 6 % or more below.  Of 4357 measured cases 21 then take
-// more than 3 % longer than on the larger tile alone (7 % at most), and the mean is 0.79 of its time.  Without scratch memory
+// The larger tile, or the small one with the least estimate if that is 6 % or more below.  Of 4357 measured cases 20 then take
+// more than 3 % longer than on the larger tile alone (6 % at most), and the mean is 0.79 of its time.  Without scratch memory
 // nothing splits its k range.
 // A linear of up to 4096 features whose larger tile splits may come with the residual add and the norm behind it
 // (hip_quant_gemm_add_rms_norm), and gives the same bits either way, so both take one plan.  Behind a k split the combine
-// launch carries them, an unsplit launch has a row kernel to follow (3 us + 0.55 per MB of output): a third of that is laid on the
-// unsplit plans (linears alone 0.728 of the larger tiles' time and 0.716 without it, with the add and norm 0.767 and 0.781).
+// launch carries them, an unsplit launch has a row kernel to follow (3 us + 0.55 per MB of output): half of that, 6 % of the launch
+// at most, is laid on the unsplit plans (of 739 cases with add and norm 3 are then more than 3 % slower than on the larger tile
+// and 14 without it; linears alone 0.764 of the larger tiles' time and 0.763; a fixed share would cost launches of 5 us a third).
 inline GemmPlan plan_gemm(const LinearArgs& a, GemmKind kind, const GemmWeights& w, int cus, bool scratch)
 {
     GemmPlan plan = kind == GEMM_PAIR ? large_pair(a, w, cus, scratch) : kind == GEMM_SEGMENTS ? large_segments(a, w, cus, scratch)
@@ -227,14 +228,15 @@ inline GemmPlan plan_gemm(const LinearArgs& a, GemmKind kind, const GemmWeights&
         if (large[i].mb == plan.mb && large[i].nb == plan.nb) { limit = 0.94 * estimate_us(a, kind, large[i], w, plan.splits, cus); }
     }
     const bool add_norm = kind == GEMM_LINEAR && plan.ranges > 1 && a.n_out <= 4096 && a.n_out % 8 == 0;
-    const double row_kernel = add_norm ? 1.0 + 0.2 * 2e-6 * (double)a.tokens * a.n_out : 0.0;
+    const double row_kernel = add_norm ? 0.5 * (3.0 + 0.55 * 2e-6 * (double)a.tokens * a.n_out) : 0.0;
     for (int i = 0; i < n_small; i++)
     {
         const GemmTile& t = small[i];
         if ((t.mb == 2 && (a.tokens > 64 || t.nb == 4)) || (t.mb == 8 && (a.tokens <= 64 || (!w.fp4 && (!w.row_major || w.scaled)))) || (kind == GEMM_PAIR && t.nb == 1)) { continue; }
         for (int s = 1; s <= plan.ranges && (s == 1 || a.K / 64 / s >= 4); s++)
         {
-            const double us = estimate_us(a, kind, t, w, s, cus) + (s == 1 ? row_kernel : 0.0);
+            double us = estimate_us(a, kind, t, w, s, cus);
+            if (s == 1) { us += std::min(row_kernel, 0.06 * us); }
             if (us < limit)
             {
                 limit = us;
