@@ -6,9 +6,9 @@ A step is one pass of the hot path over one batch of synthetic input.  Default w
 layers, FP8_E5M2 linears, BF16 activations and KV cache holding 4096 positions -- run by the C++
 DecodeModel on the fused kernels; `value` = tokens per second.  The same line then carries the GEMV
 half of the metric: the 253 linears of one token issued through Matrix::mulBatched exactly as
-cccc's graph issues them (`quant_gemv`), the per-shape sweep over M in {1, 4, 16} (`sweep`) and the
-FP4 block-scale sweep (`fp4_sweep`); GB/s figures are algorithmic bytes (K*N + 2*M*K + 2*M*N per
-GEMV) / elapsed.
+cccc's graph issues them (`quant_gemv`) and the fractions of peak of the per-shape sweeps over M in
+{1, 4, 16} and of the prefill GEMMs (`summary`; their rows go to stderr); GB/s figures are algorithmic bytes
+(K*N + 2*M*K + 2*M*N per GEMV) / elapsed.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload decode_step|decode_linears|gemv|prefill|prompt_attention]
                     [--shape K,N] [--tokens M] [--no-graph] [--no-cpu] [--no-sweep]
@@ -846,7 +846,7 @@ def cpu_baseline(pkg, threads, unit):
     return out
 
 
-def north_star_summary(line):
+def headline_summary(line):
     """The headline figures of the line once more, compact and last, so that they survive a reader that keeps only the tail of
     the output: fractions of the 8 TB/s HBM peak for the GEMVs (rows = K x N, columns = token counts), fractions of the
     2.5 PFLOP/s BF16 matrix-core peak for the prefill GEMMs, the decode step against its HBM bound."""
@@ -1250,8 +1250,13 @@ def main():
         line["cpu_baseline"] = cpu_baseline(pkg, threads, unit if args.workload != "prefill" else "GB/s")
     line.update(extra)
     if args.workload == "decode_step":
-        line["north_star"] = north_star_summary(line)
-    print(json.dumps(line))
+        line["summary"] = headline_summary(line)
+        # the rows behind the summary's fractions: without them the line stays below 8000 characters, so that a reader that keeps
+        # the tail of stdout gets all of it
+        rows = {k: line.pop(k) for k in ("sweep", "sweep_variants", "fp4_sweep", "prefill", "fp4_prefill") if k in line}
+        if rows:
+            print(json.dumps(rows), file=sys.stderr)
+    print(json.dumps(line, separators=(",", ":")))
 
 
 if __name__ == "__main__":
