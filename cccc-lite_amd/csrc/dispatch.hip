@@ -17,8 +17,8 @@
 //     anything the fast kernels cannot take (transposed layouts, odd sizes, misaligned pointers,
 //     FP4 without block scales): generic
 // Also here, for a prompt's T tokens on the register-fed GEMM kernels: hip_quant_gemm_segments (q, k, v in one launch),
-// hip_quant_gemm_swiglu (gate, up and their SwiGLU product) and hip_quant_gemm_add_rms_norm (a k-split linear whose combine
-// launch adds the residual and norms the row).
+// hip_quant_gemm_swiglu (gate, up and their SwiGLU product) and hip_quant_gemm_add_rms_norm (a linear with few output tiles, the
+// residual add and the norm behind it: in the combine launch of a k split, or in a row kernel behind an unsplit launch).
 #include "../../include/cccc_hip_quant.h"
 #include "gemv_kernels.h"
 #include "gemv_dispatch.h"
@@ -661,7 +661,7 @@ int hip_quant_gemm_add_rms_norm(int n_out, int tokens, int K, const void* W, int
     }
     else if (w_type == DT_E5M2) { launched = gemm_mfma<DT_E5M2, 0>(a, tiled, nullptr, &e); }
     else { launched = gemm_mfma<DT_E4M3, 0>(a, tiled, nullptr, &e); }
-    if (!launched) { return -1; }                   // this shape does not split its k range: nothing to fold the add and the norm into
+    if (!launched) { return -1; }                   // tiles enough for the GPU without a k split, or no scratch for one
     note_kernel(tiled ? "gemm_add_rms_norm_tiled" : "gemm_add_rms_norm");
     return finish("quant_gemm_add_rms_norm");
 }

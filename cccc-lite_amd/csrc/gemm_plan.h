@@ -205,8 +205,9 @@ inline double estimate_us(const LinearArgs& a, GemmKind kind, const GemmTile& t,
 }
 
 // The larger tile, or the small one with the least estimate if that is 6 % or more below.  Of 4357 measured cases 20 then take
-// more than 3 % longer than on the larger tile alone (6 % at most), and the mean is 0.79 of its time.  Without scratch memory
-// nothing splits its k range.
+// more than 3 % longer than on the larger tile alone (6 % at most), and the mean is 0.79 of its time; of 5785 calls of a later
+// run, other shapes among them, 39 (10 % at most) and 0.76 (profiles/gemm_tiles.md).  Without scratch memory nothing splits its
+// k range.
 // A linear of up to 4096 features whose larger tile splits may come with the residual add and the norm behind it
 // (hip_quant_gemm_add_rms_norm), and gives the same bits either way, so both take one plan.  Behind a k split the combine
 // launch carries them, an unsplit launch has a row kernel to follow (3 us + 0.55 per MB of output): half of that, 6 % of the launch

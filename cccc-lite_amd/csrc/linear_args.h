@@ -39,8 +39,8 @@ struct LinearArgs
     long long seg_y_stride_tok[3];
 };
 
-// What follows a k-split GEMM when its combine launch also carries the residual add and the RMSNorm behind it
-// (gemm_splitk_combine_add_norm_kernel): rows of n_out values, all dense.
+// What follows a linear that comes with the residual add and the RMSNorm behind it (gemm_splitk_combine_add_norm_kernel or, without
+// a k split, add_rms_norm_rows_kernel): rows of n_out values, all dense.
 struct AddNormArgs
 {
     const uint16_t* res;      // residual rows [tokens][n_out]

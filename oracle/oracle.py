@@ -1,7 +1,7 @@
 """Python face of the CPU oracle.  TEST INFRASTRUCTURE ONLY.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may import this module, and
-only as the checker.  It wraps oracle/liboracle.so (cccc_oracle.c, the scalar C restatement of the
+only as the oracle.  It wraps oracle/liboracle.so (cccc_oracle.c, the scalar C restatement of the
 reference) with ctypes and adds vectorised NumPy forms of the same functions for large inputs.
 Each function names the reference lines it follows (paths relative to the reference tree).
 """

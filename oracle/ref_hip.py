@@ -1,6 +1,6 @@
 """ctypes view of oracle/_ref/libref_hip.so: the reference's own HIP kernel library
 (cccc-hip/hip_functions.cpp) compiled for gfx950 by oracle/Makefile.  TEST INFRASTRUCTURE ONLY: the
-GPU-side checker of the BF16 neighbour ops and the kernels of the reference-style decode baseline in
+GPU-side oracle of the BF16 neighbour ops and the kernels of the reference-style decode baseline in
 bench.py.  Every entry point takes device pointers and synchronises the device before it returns
 (cccc-hip/hip_functions.cpp:32-42).  The library has no FP8 / FP4 code (its hip_convert, .cpp:2683-2690,
 knows float, half and bfloat16 only)."""
