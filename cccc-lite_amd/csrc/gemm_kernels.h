@@ -1133,9 +1133,10 @@ inline float* split_workspace(const GemmPlan& plan, long long outputs) { return 
 // the plan of a joint or paired launch of `outputs` values, without a k split if there is no scratch memory for it
 inline GemmPlan joint_plan(const LinearArgs& a, GemmKind kind, const GemmWeights& w, long long outputs, float*& partial)
 {
-    GemmPlan plan = plan_gemm(a, kind, w, cu_count(), true);
+    const int cus = cu_count();
+    GemmPlan plan = staged_plan(a, kind, w, cus, plan_gemm(a, kind, w, cus, true));
     partial = split_workspace(plan, outputs);
-    return plan.splits > 1 && !partial ? plan_gemm(a, kind, w, cu_count(), false) : plan;
+    return plan.splits > 1 && !partial ? staged_plan(a, kind, w, cus, plan_gemm(a, kind, w, cus, false)) : plan;
 }
 
 // a.seg_tile0 for 256-feature tiles (empty segments start past the last tile); the number of tiles
@@ -1260,7 +1261,8 @@ void launch_gemm_mfma(const LinearArgs& a)
 // how much they need), or, with the add and norm, there is no k split or no scratch for it.
 inline bool linear_plan(const LinearArgs& a, const GemmWeights& w, bool add_norm, SplitScratch* scratch, GemmPlan& plan, float*& partial)
 {
-    plan = plan_gemm(a, GEMM_LINEAR, w, cu_count(), true);
+    const int cus = cu_count();
+    plan = staged_plan(a, GEMM_LINEAR, w, cus, plan_gemm(a, GEMM_LINEAR, w, cus, true));
     partial = nullptr;
     if (plan.ranges > 1)
     {
@@ -1275,7 +1277,7 @@ inline bool linear_plan(const LinearArgs& a, const GemmWeights& w, bool add_norm
             partial = scratch->fixed;
         }
         else { partial = (float*)workspace(need); }
-        if (!partial) { plan = plan_gemm(a, GEMM_LINEAR, w, cu_count(), false); }
+        if (!partial) { plan = staged_plan(a, GEMM_LINEAR, w, cus, plan_gemm(a, GEMM_LINEAR, w, cus, false)); }
     }
     return !add_norm || plan.ranges > 1;
 }

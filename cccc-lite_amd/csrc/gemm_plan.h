@@ -20,6 +20,7 @@ struct GemmPlan
     int mb, nb, splits;
     bool small;              // FP8: a tile with weights requested three k-tiles ahead (gemm_short.h); FP4: gemm_short_fp4.hip
     int ranges;              // k ranges of the larger tile that this plan was compared with, and so of the scratch held: splits <= ranges
+    bool staged = false;     // FP8: gemm_staged_kernel (gemm_staged.h), a tile of kStagedTiles; `small` is set as well
 };
 
 // Tile shape and k split of the larger tiles (tuned on MI355X with the FP8 kernel): a workgroup owns 64 NB features x
@@ -181,7 +182,7 @@ constexpr GemmTile kLargeTilesFp4[] = {
     { 8, 4, 7.3, 2.1, { 0.913 }, { 0.873 } },
 };
 
-inline double estimate_us(const LinearArgs& a, GemmKind kind, const GemmTile& t, const GemmWeights& w, int splits, int cus)
+inline double estimate_us(const LinearArgs& a, GemmKind kind, const GemmTile& t, const GemmWeights& w, int splits, int cus, double alone = 0.85)
 {
     const int width = kind == GEMM_PAIR ? 32 * t.nb : 64 * t.nb, column = w.fp4 ? 0 : (w.scaled ? 2 : 0) + (w.row_major ? 1 : 0);
     long long features = a.n_out, n_tiles = (a.n_out + width - 1) / width;
@@ -197,7 +198,7 @@ inline double estimate_us(const LinearArgs& a, GemmKind kind, const GemmTile& t,
     const double two = kind == GEMM_PAIR ? 2.0 : 1.0, outputs = 1e-6 * (double)a.tokens * (double)features;
     const double fill = 8.0 * (double)((n_tiles + 7) / 8 * ((a.tokens + 16 * t.mb - 1) / (16 * t.mb)) * splits) / cus;
     const double per_cu = fill <= 1.0 ? 1.0 : 0.1 * fill + 0.9 * ceil(fill);
-    const double k_tile = fill <= 1.0 ? t.one[column] * (0.85 + 0.15 * fill) : std::max(t.one[column], t.each[column] * per_cu);
+    const double k_tile = fill <= 1.0 ? t.one[column] * (alone + (1.0 - alone) * fill) : std::max(t.one[column], t.each[column] * per_cu);
     const double traffic = 1e-6 * two * (double)features * a.K * (w.fp4 ? 0.5625 : 1.0) + 2.0 * outputs;
     double us = t.fixed + t.per_cu * per_cu + std::max((double)((a.K / 64 + splits - 1) / splits) * k_tile, traffic / (w.fp4 ? 4.1 : 5.0));
     if (splits > 1) { us += 2.0 + 0.2 * splits + 0.3 * 4.0 * splits * two * outputs; }
@@ -246,6 +247,61 @@ inline GemmPlan plan_gemm(const LinearArgs& a, GemmKind kind, const GemmWeights&
         }
     }
     return plan;
+}
+
+// gemm_staged_kernel, all weights: the same estimate, fitted to 10,900 launches (13 shapes x 11 token counts from 20 to 1024 x every tile
+// and 1 to 8 k ranges, the four columns and HALF activations; weights in turn through up to 1.2 GB), error 3 to 6 % rms per tile.  Alone on a CU a
+// k-tile takes down to 0.7 of `one`: the loads share L2 and HBM with fewer others.
+constexpr GemmTile kStagedTiles[] = {
+    { 2, 1, 3.2, 0.6, { 0.162, 0.174, 0.208, 0.211 }, { 0.143, 0.152, 0.158, 0.167 } },
+    { 2, 2, 2.3, 2.7, { 0.226, 0.240, 0.317, 0.314 }, { 0.247, 0.257, 0.302, 0.305 } },
+    { 3, 2, 2.3, 3.6, { 0.223, 0.232, 0.336, 0.338 }, { 0.223, 0.231, 0.305, 0.312 } },
+    { 4, 1, 2.2, 2.3, { 0.189, 0.199, 0.233, 0.233 }, { 0.145, 0.153, 0.167, 0.174 } },
+    { 4, 2, 2.0, 4.1, { 0.249, 0.260, 0.353, 0.355 }, { 0.256, 0.263, 0.323, 0.334 } },
+    { 5, 2, 2.3, 4.5, { 0.294, 0.301, 0.399, 0.407 }, { 0.289, 0.293, 0.360, 0.375 } },
+    { 7, 2, 2.5, 5.0, { 0.361, 0.381, 0.462, 0.460 }, { 0.356, 0.360, 0.426, 0.434 } },
+};
+
+// The staged kernel in the place of `plan` from K = 1024 on (shorter sums keep the order of the register-fed kernels, so that a joint or
+// paired launch gives the bits of the separate calls) and up to 512 tokens (above that the larger tiles are level or ahead),
+// where its estimate is 5 % (file layout) or 8 % (tiled copy, whose KiB blocks the other kernels read whole as well) and 0.3 us below the
+// plan's own: with less, launches of 5 us and k-split ones on tiled copies lose up to 15 %.  Of 620 measured calls one
+// then takes more than 3 % longer (4 %); mean of all 0.96 of the plans' time, 0.91 on E5M2 in the file layout.  An unsplit linear that may come with the add and the norm carries half of the row kernel, as in plan_gemm, and
+// must not be behind with all of it either (4096 x 12288 at 512 tokens, tiled: 58 us alone on both, 64 against 55 with the norm).
+// The k ranges of the larger tile, and so the scratch memory, stay what they were.  FP4 keeps its plans.
+inline GemmPlan staged_plan(const LinearArgs& a, GemmKind kind, const GemmWeights& w, int cus, const GemmPlan& plan)
+{
+    if (w.fp4 || a.K < 1024 || a.tokens > 512) { return plan; }
+    const bool deep = plan.small || (plan.splits > 1 && plan.mb <= 4);
+    const GemmTile* const table = deep ? kSmallTiles : kLargeTiles;
+    const int n_table = deep ? sizeof(kSmallTiles) / sizeof(GemmTile) : sizeof(kLargeTiles) / sizeof(GemmTile);
+    const bool add_norm = kind == GEMM_LINEAR && plan.ranges > 1 && a.n_out <= 4096 && a.n_out % 8 == 0;
+    const double row_kernel = add_norm ? 3.0 + 0.55 * 2e-6 * (double)a.tokens * a.n_out : 0.0;
+    double limit = 0.0, with_norm = 0.0;
+    for (int i = 0; i < n_table; i++)
+    {
+        if (table[i].mb == plan.mb && table[i].nb == plan.nb)
+        {
+            const double us = estimate_us(a, kind, table[i], w, plan.splits, cus), row = plan.splits == 1 ? row_kernel : 0.0;
+            limit = (w.row_major ? 0.95 : 0.92) * (us + 0.5 * row) - 0.3;
+            with_norm = us + row;
+        }
+    }
+    GemmPlan best = plan;
+    for (const GemmTile& t : kStagedTiles)
+    {
+        if ((t.mb > 2 && 16 * (t.mb - 1) >= a.tokens) || (t.mb == 2 && a.tokens > 64) || (t.mb == 3 && a.tokens > 192)) { continue; }
+        for (int s = 1; s <= plan.ranges && (s == 1 || a.K / 64 / s >= 4); s++)
+        {
+            const double us = estimate_us(a, kind, t, w, s, cus, 0.7), row = s == 1 ? row_kernel : 0.0;
+            if (us + 0.5 * row < limit && us + row <= with_norm)
+            {
+                limit = us + 0.5 * row;
+                best = GemmPlan{ t.mb, t.nb, s, true, plan.ranges, true };
+            }
+        }
+    }
+    return best;
 }
 
 }    // namespace ccq

@@ -1,11 +1,15 @@
 // The small tiles of plan_gemm (gemm_plan.h) on the register-fed FP8 GEMM, every one with weights requested three k-tiles ahead,
 // and the k-split launches of the larger ones: one translation unit per weight type (gemm_short_e5m2.hip, gemm_short_e4m3.hip) instantiates them.
+// The plans of staged_plan run gemm_staged_kernel instead (gemm_staged_e5m2.hip, gemm_staged_e4m3.hip).
 #pragma once
 #include "gemm_kernels.h"
 #include "prefill_kernels.h"
 
 namespace ccq
 {
+
+void launch_gemm_staged_e5m2(const LinearArgs& a, bool half, bool tiled, bool scaled, const GemmPlan& p, int n_tiles, float* partial);
+void launch_gemm_staged_e4m3(const LinearArgs& a, bool half, bool tiled, bool scaled, const GemmPlan& p, int n_tiles, float* partial);
 
 template <int WT, bool SCALED, bool TILED, int AT, int MB, int NB, bool PAIR, bool SEG, int PD = 3, bool SPLIT_ONLY = false>
 void launch_short_tile(const LinearArgs& a, int n_tiles, int splits, float* partial)
@@ -18,7 +22,7 @@ void launch_short_tile(const LinearArgs& a, int n_tiles, int splits, float* part
 template <int WT, bool SCALED, bool TILED, int AT, bool PAIR, bool SEG>
 void launch_short_shape(LinearArgs a, const GemmPlan& p, float* partial, const AddNormArgs* e)
 {
-    const int width = 64 * (PAIR ? p.nb / 2 : p.nb);
+    const int width = (PAIR ? 32 : 64) * p.nb;
     if (e && p.splits <= 1)
     {
         a.Y = (uint16_t*)partial;
@@ -42,7 +46,8 @@ void launch_short_shape(LinearArgs a, const GemmPlan& p, float* partial, const A
         for (int s = a.n_segments; s < 4; s++) { a.seg_tile0[s] = n_tiles; }       // empty segments start past the last tile
         a.seg_tile0[3] = n_tiles;
     }
-    if (p.mb == 2)
+    if (p.staged) { (WT == DT_E5M2 ? launch_gemm_staged_e5m2 : launch_gemm_staged_e4m3)(a, AT == DT_HALF, TILED, SCALED, p, n_tiles, partial); }
+    else if (p.mb == 2)
     {
         if constexpr (!PAIR)
         {
