@@ -2,6 +2,7 @@
 #include "../../include/cccc_hip_quant.h"
 #include "prefill_kernels.h"
 #include "runtime.h"
+#include <algorithm>
 #include <cmath>
 
 using namespace ccq;
@@ -9,6 +10,27 @@ using namespace ccq;
 namespace
 {
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
+
+// Key ranges of a prompt's attention.  In one piece a workgroup takes 5 us and 1.75 per block of 64 keys; in n ranges the three launches
+// take 16 us, 1.75 per block of one range, and 0.25 per MB of FP32 sums written and read.  At most one workgroup per CU (two take as long
+// as one after the other: 64 tokens of 32 / 8 heads behind 4000: 34.5 us with 8 ranges, 43.9 with 12; 300 tokens behind 1000, 152 workgroups:
+// 45.6 in one piece, 50.4 in two ranges), and 10 % to gain at least.  Measured on MI355X, one piece -> ranges: those 64 tokens 121 -> 34.5 us,
+// 64 tokens of 4 / 1 heads behind 14000 424 -> 34, 200 tokens of 32 / 8 behind 2000 70 -> 51, 2 tokens of one head behind 16000 353 -> 23.
+struct AttentionRanges
+{
+    int n, per;
+};
+
+AttentionRanges attention_ranges(long long tiles, int n_keys, size_t outputs)
+{
+    const int blocks = (n_keys + PF_KEYS - 1) / PF_KEYS;
+    const int want = (int)std::min({ cu_count() / tiles, (long long)PF_RANGES, (long long)blocks / 2 });
+    if (want < 2) { return { 1, blocks }; }
+    const int per = ((blocks + want - 1) / want + 1) & ~1;
+    const int n = (blocks + per - 1) / per;
+    const double whole = 5.0 + 1.75 * blocks, split = 16.0 + 1.75 * per + 0.25e-6 * 8.0 * 128.0 * (double)outputs * n;
+    return split < 0.9 * whole ? AttentionRanges{ n, per } : AttentionRanges{ 1, blocks };
+}
 }    // namespace
 
 int hip_qk_norm_rope_kv_rows_bf16(const void* q, const void* k, const void* v, const void* q_norm_w, const void* k_norm_w,
@@ -35,18 +57,29 @@ int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v
     if ((long long)((n_tokens + 15) / 16) * n_kv_heads > 0x7FFFFFFFLL) { return -1; }
     // the kernel addresses cache rows with 32-bit byte offsets inside a KV head (row * 256)
     if ((long long)pos0 + n_tokens > (1LL << 24)) { return -1; }
-    const dim3 grid((unsigned)((n_tokens + 15) / 16) * n_kv_heads);
+    const long long tiles = (long long)((n_tokens + 15) / 16) * n_kv_heads;
+    const int group = n_q_heads / n_kv_heads;
+    if (group != 1 && group != 2 && group != 4) { return -1; }
     const float scale = 1.0f / sqrtf(128.0f);
-#define CCQ_ATTN_PREFILL(G)                                                                                                                  \
-    attn_prefill_kernel<G><<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, (uint16_t*)y, \
-                                                       n_q_heads, t_kv, n_tokens, pos0, scale)
-    switch (n_q_heads / n_kv_heads)
+    const size_t outputs = (size_t)n_tokens * n_q_heads;
+    const AttentionRanges split = attention_ranges(tiles, pos0 + n_tokens, outputs);
+    char* const scratch = split.n > 1 ? (char*)workspace((size_t)split.n * outputs * (128 * sizeof(float) + sizeof(float2))) : nullptr;
+    const PrefillRanges ranges = { split.per, (float2*)(scratch + (size_t)split.n * outputs * 128 * sizeof(float)), (float*)scratch };
+    const dim3 grid((unsigned)tiles, scratch ? split.n : 1);
+#define CCQ_ATTN_PREFILL(G, PASS)                                                                                                                  \
+    attn_prefill_kernel<G, PASS><<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, (uint16_t*)y, \
+                                                             n_q_heads, t_kv, n_tokens, pos0, scale, ranges)
+#define CCQ_ATTN_PREFILL_GROUPS(PASS)                                                                                                              \
+    group == 4 ? CCQ_ATTN_PREFILL(4, PASS) : group == 2 ? CCQ_ATTN_PREFILL(2, PASS) : CCQ_ATTN_PREFILL(1, PASS)
+    if (!scratch) { CCQ_ATTN_PREFILL_GROUPS(0); }
+    else
     {
-    case 1: CCQ_ATTN_PREFILL(1); break;
-    case 2: CCQ_ATTN_PREFILL(2); break;
-    case 4: CCQ_ATTN_PREFILL(4); break;
-    default: return -1;
+        CCQ_ATTN_PREFILL_GROUPS(1);
+        CCQ_ATTN_PREFILL_GROUPS(2);
+        const long long blocks = ((long long)outputs * 32 + 255) / 256, cap = (long long)cu_count() * 16;
+        attn_prefill_combine_kernel<<<(unsigned)(blocks < cap ? blocks : cap), 256, 0, stream()>>>(ranges.partial, (uint16_t*)y, n_q_heads * 128, n_tokens, pos0, split.per);
     }
+#undef CCQ_ATTN_PREFILL_GROUPS
 #undef CCQ_ATTN_PREFILL
     return finish("attention_prefill");
 }

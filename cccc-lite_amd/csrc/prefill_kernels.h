@@ -95,9 +95,23 @@ __device__ __forceinline__ uint32_t pf_pack_bf16(float lo, float hi)
 // then pays a trip to memory per block.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int G>
+// A few tokens behind a long context are few workgroups (64 tokens and 4 kv heads: 16), each with a serial loop over all the keys.  Then the
+// blocks of keys are split over gridDim.y workgroups, `per` blocks (an even number) each, and the passes are launches of their own:
+// PASS 1 leaves (max, sum) per range, head and token, PASS 2 merges those of all the ranges a token tile has -- the probabilities are rounded
+// with the row's own maximum and sum, as in one piece -- and leaves FP32 sums, which attn_prefill_combine_kernel adds and rounds.  PASS 0 is
+// both passes over all the keys.
+constexpr int PF_RANGES = 32;               // most ranges: a lane group of pass 2 reads eight statistics at once
+
+struct PrefillRanges
+{
+    int per;                // blocks of PF_KEYS keys per range
+    float2* stats;          // [range][head][token]
+    float* partial;         // [range][token][head][128]
+};
+
+template <int G, int PASS>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k_cache, const uint16_t* __restrict__ v_cache,
-                                                             uint16_t* __restrict__ y, int n_q, int t_kv, int n_tokens, int pos0, float scale)
+                                                             uint16_t* __restrict__ y, int n_q, int t_kv, int n_tokens, int pos0, float scale, const PrefillRanges ranges)
 {
     constexpr int H = G >= 2 ? 2 : 1;           // query heads per wave
     constexpr int NW = 2 * (G / H);             // waves that compute: (head group, key half)
@@ -116,6 +130,9 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const uint16_t* __
     const int n_keys = pos0 + last_token + 1;                   // keys this workgroup can see
     const int n_written = pos0 + n_tokens;                      // cache rows holding data
     const int n_blocks = (n_keys + PF_KEYS - 1) / PF_KEYS;
+    const int b_begin = PASS == 0 ? 0 : (int)blockIdx.y * ranges.per;          // even: block b always goes to buffer b & 1
+    const int b_end = PASS == 0 ? n_blocks : min(n_blocks, b_begin + ranges.per);
+    if (PASS != 0 && b_begin >= n_blocks) { return; }           // a range past this tile's last key: nobody reads it
     const bool active = wave < NW;
     const int hg = wave >> 1, kh = wave & 1;                    // head group; which 32 keys of every block
     const int head0 = kvh * G + hg * H;                         // first of the wave's heads
@@ -251,16 +268,18 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const uint16_t* __
     for (int h = 0; h < H; h++) { m[h] = -INFINITY; l[h] = 0.0f; }
     u32x4 kraw[4], vraw[4];
     f32x4 cur[H][2], next[H][2];
-    // blocks 0 .. n_plain - 1 end at or before the first token's position and need no mask test (one or two blocks do)
-    const int n_plain = min((pos0 + t0 + 1) / PF_KEYS, n_blocks);
+    // blocks before n_plain end at or before the first token's position and need no mask test (one or two blocks do)
+    const int n_plain = max(b_begin, min((pos0 + t0 + 1) / PF_KEYS, b_end));
+    if constexpr (PASS != 2)
+    {
     // prologue: block 0 staged and multiplied, block 1 staged, block 2 on its way
-    load_rows(kbase, 0, kraw);
-    store_keys(0, 0, kraw);
-    load_rows(kbase, 1, kraw);
+    load_rows(kbase, b_begin, kraw);
+    store_keys(0, b_begin, kraw);
+    load_rows(kbase, b_begin + 1, kraw);
     lds_barrier();
     if (active) { score_products(0, cur); }
-    store_keys(1, 1, kraw);
-    load_rows(kbase, 2, kraw);
+    store_keys(1, b_begin + 1, kraw);
+    load_rows(kbase, b_begin + 2, kraw);
     lds_barrier();
     // iteration b: ks[(b + 1) & 1] holds block b + 1, `cur` the raw scores of block b, kraw block b + 2 in flight
     auto pass1_block = [&](int b, auto masked_c) {
@@ -299,34 +318,56 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const uint16_t* __
             for (int kt = 0; kt < 2; kt++) { cur[h][kt] = next[h][kt]; }
     };
     // two copies of the iteration, with and without the mask test, each one straight run of instructions
-    for (int b = 0; b < n_plain; b++) { pass1_block(b, std::false_type{}); }
-    for (int b = n_plain; b < n_blocks; b++) { pass1_block(b, std::true_type{}); }
+    for (int b = b_begin; b < n_plain; b++) { pass1_block(b, std::false_type{}); }
+    for (int b = n_plain; b < b_end; b++) { pass1_block(b, std::true_type{}); }
+    }
     // merge the four lane groups of a token (lanes j, j + 16, j + 32, j + 48), then the two waves of a head group
     auto merge = [&](float& ma, float& la, float mb, float lb) {
         const float nm = fmaxf(ma, mb);
         if (nm > -INFINITY) { la = la * pf_exp2((ma - nm) * PF_LOG2E) + lb * pf_exp2((mb - nm) * PF_LOG2E); }
         ma = nm;
     };
+    if constexpr (PASS == 2)
+    {
+        // the statistics of all the tile's ranges, a quarter of them per lane group
+        const int n_ranges = (n_blocks + ranges.per - 1) / ranges.per;
+#pragma unroll
+        for (int h = 0; h < H; h++)
+        {
+            float2 s[PF_RANGES / 4];
+            const float2* const from = ranges.stats + (size_t)(active ? head0 + h : 0) * n_tokens + min(t0 + j, n_tokens - 1);
+#pragma unroll
+            for (int i = 0; i < PF_RANGES / 4; i++) { s[i] = from[(size_t)min(g + 4 * i, n_ranges - 1) * n_q * n_tokens]; }
+#pragma unroll
+            for (int i = 0; i < PF_RANGES / 4; i++)
+            {
+                if (g + 4 * i < n_ranges) { merge(m[h], l[h], s[i].x, s[i].y); }
+            }
+        }
+    }
 #pragma unroll
     for (int h = 0; h < H; h++)
     {
 #pragma unroll
         for (int off = 16; off < 64; off <<= 1) { merge(m[h], l[h], __shfl_xor(m[h], off), __shfl_xor(l[h], off)); }
-        if (active && g == 0) { stat[wave][h][j] = make_float2(m[h], l[h]); }
+        if (PASS != 2 && active && g == 0) { stat[wave][h][j] = make_float2(m[h], l[h]); }
     }
-    lds_barrier();
+    if (PASS != 2) { lds_barrier(); }
     float poff[H];
 #pragma unroll
     for (int h = 0; h < H; h++)
     {
-        if (active)
+        if (PASS != 2 && active)
         {
             const float2 other = stat[wave ^ 1][h][j];
             merge(m[h], l[h], other.x, other.y);
+            if (PASS == 1 && kh == 0 && g == 0 && t0 + j < n_tokens) { ranges.stats[((size_t)blockIdx.y * n_q + head0 + h) * n_tokens + t0 + j] = make_float2(m[h], l[h]); }
         }
         // p = 2^(s log2 e - (m log2 e + log2 l)): the division by the sum rides in the exponent
         poff[h] = l[h] > 0.0f ? -(m[h] * PF_LOG2E + __builtin_amdgcn_logf(l[h])) : -INFINITY;
     }
+
+    if constexpr (PASS == 1) { return; }
 
     // ---- pass 2: probabilities and P V, per wave over its half of the keys
     f32x4 out[H][8];
@@ -334,16 +375,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const uint16_t* __
     for (int h = 0; h < H; h++)
 #pragma unroll
         for (int d = 0; d < 8; d++) { out[h][d] = f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }; }
-    load_rows(kbase, 0, kraw);
-    load_rows(vbase, 0, vraw);
-    store_keys(0, 0, kraw);
-    load_rows(kbase, 1, kraw);
+    load_rows(kbase, b_begin, kraw);
+    load_rows(vbase, b_begin, vraw);
+    store_keys(0, b_begin, kraw);
+    load_rows(kbase, b_begin + 1, kraw);
     lds_barrier();
     if (active) { score_products(0, cur); }
-    store_keys(1, 1, kraw);
-    store_values(0, 0, vraw);
-    load_rows(kbase, 2, kraw);
-    load_rows(vbase, 1, vraw);
+    store_keys(1, b_begin + 1, kraw);
+    store_values(0, b_begin, vraw);
+    load_rows(kbase, b_begin + 2, kraw);
+    load_rows(vbase, b_begin + 1, vraw);
     lds_barrier();
     // iteration b: ks[(b + 1) & 1] holds key block b + 1, vt[b & 1] value block b; kraw = keys b + 2, vraw = values b + 1 in flight
     auto pass2_block = [&](int b, auto masked_c) {
@@ -396,8 +437,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const uint16_t* __
 #pragma unroll
             for (int kt = 0; kt < 2; kt++) { cur[h][kt] = next[h][kt]; }
     };
-    for (int b = 0; b < n_plain; b++) { pass2_block(b, std::false_type{}); }
-    for (int b = n_plain; b < n_blocks; b++) { pass2_block(b, std::true_type{}); }
+    for (int b = b_begin; b < n_plain; b++) { pass2_block(b, std::false_type{}); }
+    for (int b = n_plain; b < b_end; b++) { pass2_block(b, std::true_type{}); }
     // the two key halves of a head group meet in LDS (the staging buffers are free now): lane-major, so that consecutive
     // lanes touch consecutive words
     float* red = (float*)&ks[0][0];
@@ -424,9 +465,37 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const uint16_t* __
             {
                 const int t = t0 + 4 * g + v;
                 const float sum = out[h][d][v] + red[(((hg * H + h) * 8 + d) * 4 + v) * 64 + lane];
-                if (t < n_tokens) { y[((size_t)t * n_q + head0 + h) * 128 + 16 * d + j] = (uint16_t)f32_to_bf16_bits(sum); }
+                if (t >= n_tokens) { continue; }
+                if constexpr (PASS == 2) { ranges.partial[(((size_t)blockIdx.y * n_tokens + t) * n_q + head0 + h) * 128 + 16 * d + j] = sum; }
+                else { y[((size_t)t * n_q + head0 + h) * 128 + 16 * d + j] = (uint16_t)f32_to_bf16_bits(sum); }
             }
         }
+}
+
+// Sums of the key ranges of one token, four dims of a head per thread, in the order of the ranges; one rounding.  A token has the ranges of
+// its tile of 16.
+static __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const float* __restrict__ partial, uint16_t* __restrict__ y, int row, int n_tokens, int pos0, int per)
+{
+    const long long slice = (long long)n_tokens * row;
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < slice / 4; i += (long long)gridDim.x * 256)
+    {
+        const int t = (int)(i * 4 / row);
+        const int n_blocks = (pos0 + min(t / 16 * 16 + 15, n_tokens - 1) + PF_KEYS) / PF_KEYS;
+        const int n_ranges = (n_blocks + per - 1) / per;
+        f32x4 sum = *(const f32x4*)(partial + i * 4);
+        for (int r0 = 1; r0 < n_ranges; r0 += 8)
+        {
+            f32x4 part[8];                                      // eight ranges requested at once
+#pragma unroll
+            for (int r = 0; r < 8; r++) { part[r] = *(const f32x4*)(partial + (long long)min(r0 + r, n_ranges - 1) * slice + i * 4); }
+#pragma unroll
+            for (int r = 0; r < 8; r++)
+            {
+                if (r0 + r < n_ranges) { sum += part[r]; }
+            }
+        }
+        *(uint2*)(y + i * 4) = uint2{ f32_to_bf16_bits(sum[0]) | (f32_to_bf16_bits(sum[1]) << 16), f32_to_bf16_bits(sum[2]) | (f32_to_bf16_bits(sum[3]) << 16) };
+    }
 }
 
 // ------------------------------------------------------------------------------------------

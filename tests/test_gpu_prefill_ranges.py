@@ -1,0 +1,78 @@
+"""Attention of a few prompt tokens behind a long context: the keys split over workgroups (statistics, sums, combine)."""
+import numpy as np
+import pytest
+
+from gpu_util import from_dev, to_dev
+from test_gpu_prefill import dec, ptr, ulp_close  # noqa: F401 (dec: a fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(oracle, n_q, n_kv, T, pos0, t_kv):
+    rng = np.random.default_rng(T + pos0)
+    q = oracle.f32_to_bf16(rng.standard_normal((T, n_q, 128)).astype(np.float32))
+    kc, vc = (oracle.f32_to_bf16(rng.standard_normal((n_kv, t_kv, 128)).astype(np.float32)) for _ in range(2))
+    kc[:, pos0 + T:] = 0x7FC1
+    vc[:, pos0 + T:] = 0xFFFF
+    return q, kc, vc
+
+
+# tiles x kv heads against blocks of 64 keys on 256 CUs: one head at the most ranges (32), ranges that end inside a token tile's last
+# block, token tiles whose last range is empty, the fewest ranges (2) that pay, one to four query heads per kv head
+@pytest.mark.parametrize("n_q,n_kv,T,pos0", [(1, 1, 2, 4100), (4, 1, 17, 1150), (8, 2, 33, 2046), (2, 2, 63, 1470), (8, 4, 16, 1263), (16, 8, 40, 1999), (4, 2, 30, 600), (32, 8, 200, 1850)])
+def test_few_tokens_behind_a_long_context_follow_the_oracle(gpu, oracle, dec, n_q, n_kv, T, pos0):
+    """The bounds of the attention in one piece (two BF16 steps, row error 4e-3): the same probabilities, sums in another order."""
+    torch, dev, lib = gpu
+    t_kv = pos0 + T + 40
+    q, kc, vc = inputs(oracle, n_q, n_kv, T, pos0, t_kv)
+    qd, kd, vd = to_dev(torch, dev, q), to_dev(torch, dev, kc), to_dev(torch, dev, vc)
+    y = torch.zeros(T * n_q * 128 + 64, dtype=torch.int16, device=dev)
+    assert lib.c.hip_attention_prefill_bf16(ptr(qd), ptr(kd), ptr(vd), ptr(y), n_q, n_kv, 128, t_kv, T, pos0) == 0
+    out = from_dev(y, np.uint16)
+    assert not out[T * n_q * 128:].any()
+    got = out[:T * n_q * 128].reshape(T, n_q, 128)
+    kf, vf = dec.f(kc), dec.f(vc)
+    kf[:, pos0 + T:], vf[:, pos0 + T:] = 0.0, 0.0               # masked in the oracle too; NaN * 0 would poison its matrix products
+    for t in sorted({0, 1, 15, 16, T // 2, T - 2, T - 1} & set(range(T))):
+        want = dec.attention(dec.f(q[t]), kf, vf, pos0 + t, n_q, n_kv)
+        assert np.isfinite(dec.f(got[t])).all(), t
+        assert ulp_close(got[t], want, ulps=2.0, floor=2e-3 * np.abs(want).max()).all(), t
+        assert np.linalg.norm(dec.f(got[t]) - want) <= 4e-3 * np.linalg.norm(want), t
+
+
+def test_ranges_under_capture(gpu, oracle, dec):
+    """A captured call whose scratch an eager call has sized replays the eager result, with eager work of another size in between; one
+    on a stream without scratch runs in one piece, within the bounds."""
+    torch, dev, lib = gpu
+    n_q, n_kv, T, pos0, t_kv = 4, 1, 20, 1500, 1600
+    q, kc, vc = inputs(oracle, n_q, n_kv, T, pos0, t_kv)
+    qd, kd, vd = to_dev(torch, dev, q), to_dev(torch, dev, kc), to_dev(torch, dev, vc)
+    call = lambda y, T=T, pos0=pos0: lib.c.hip_attention_prefill_bf16(ptr(qd), ptr(kd), ptr(vd), ptr(y), n_q, n_kv, 128, t_kv, T, pos0)
+    eager, other, replayed, whole = (torch.zeros(T * n_q * 128, dtype=torch.int16, device=dev) for _ in range(4))
+    lib.set_sync(False)
+    try:
+        for first, out in ((True, replayed), (False, whole)):
+            stream = torch.cuda.Stream(device=dev)
+            assert lib.set_stream(stream.cuda_stream) == 0
+            if first:
+                assert call(eager) == 0
+                stream.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=stream):
+                assert call(out) == 0
+            for _ in range(3):
+                out.zero_()
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                if first:
+                    assert torch.equal(out, eager)
+                    assert call(other, T=9, pos0=1200) == 0
+                    stream.synchronize()
+                else:
+                    a, b = dec.f(from_dev(out, np.uint16)), dec.f(from_dev(eager, np.uint16))
+                    assert np.linalg.norm(a - b) <= 4e-3 * np.linalg.norm(b)
+            del graph
+    finally:
+        lib.set_stream(None)
+        lib.set_sync(True)
