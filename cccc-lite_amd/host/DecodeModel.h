@@ -99,7 +99,8 @@ public:
     // the prompt, the current token is the greedy pick after its last token and the position is pos0 + n: step() carries
     // on from there.  Prompts longer than 2048 tokens go through in pieces of 2048.  0 ok, -1 bad arguments.
     int prefill(const int* tokens, int n_tokens, int pos0);
-    // Runs n steps; use_graph: capture one step and replay it.  Returns elapsed ms (events on the launch stream) or < 0.
+    // Runs n steps; use_graph: where n is large enough to pay for it, capture one step and replay it behind the first two.  Returns elapsed ms
+    // (events on the launch stream) or < 0.
     double run(int n_steps, int use_graph);
     int currentToken();                     // blocking 4-byte read
     int currentPos();
