@@ -5,13 +5,14 @@
 // side touches every line twice or four times), four such pieces are requested before the first is used, and the grid is a
 // fixed multiple of the CU count walking the buffer with a grid stride.  Scalar kernels take what is left: the last few
 // elements, misaligned pointers, odd block lengths.  Measured on a 4096 x 12288 weight, BF16 -> float -> FP4 with block scales
-// -> BF16 (659 MB moved): 380 -> 123 us, 5.4 TB/s, what a plain device copy reaches; float -> FP8 and back likewise (462 -> 142).
+// -> BF16 (659 MB moved): 113 us, 5.8 TB/s, what a plain device copy reaches; through absmax and float -> FP8 and back 154.
 // Numerics follow the reference kernels element for element (decode, one FP32 multiply by the
 // scale, integer round-to-nearest-even to BF16): cccc-cuda/cuda_functions.cu:2566-2596 (E4M3),
 // :2735-2785 (E5M2), :2834-2884 (FP4), :2896-2960 (FP4 block scale), :3066-3090 (dispatch).
 #include "../../include/cccc_hip_quant.h"
 #include "quant_device.h"
 #include "runtime.h"
+#include <algorithm>
 #include <hip/hip_fp16.h>
 
 using namespace ccq;
@@ -249,10 +250,14 @@ __device__ __forceinline__ uint32_t f32_to_e4m3_trunc(float f)
 
 __device__ __forceinline__ uint32_t f32_to_fp4(float f)
 {
-    const uint32_t s = (f < 0.0f) ? 8u : 0u;
-    const float a = (f < 0.0f) ? -f : f;
-    const uint32_t code = a < 0.25f ? 0u : a < 0.75f ? 1u : a < 1.25f ? 2u : a < 1.75f ? 3u : a < 2.5f ? 4u : a < 3.5f ? 5u : a < 5.0f ? 6u : 7u;
-    return s | code;
+    // the reference's thresholds 0.25, 0.75, 1.25, 1.75, 2.5, 3.5, 5, each belonging to the code above it.  From 0.75 on they are the code values'
+    // midpoints with one bit of mantissa: half of that bit is added to the magnitude and exponent and bit are the code (the hardware conversion
+    // rounds ties to even and cannot be used).  NaN is 7, as no comparison with it holds.
+    const uint32_t mag = f32_to_bits(f) & 0x7FFFFFFFu;
+    const uint32_t upper = min((mag + 0x200000u) >> 22, 259u) - 252u;
+    const float a = fabsf(f);
+    const uint32_t lower = a < 0.25f ? 0u : a < 0.75f ? 1u : 2u;
+    return (f < 0.0f ? 8u : 0u) | (a < 1.0f ? lower : upper);
 }
 
 __device__ __forceinline__ float load_plain(const void* src, int type, size_t i)
@@ -410,58 +415,96 @@ __global__ __launch_bounds__(kThreads) void encode4_blockscale_kernel(const floa
 // Whole blocks of 16 or 32 elements: BLOCK / 4 neighbouring lanes share a block, each with one 16-byte load, and find its
 // largest magnitude through lane exchanges inside their row of 16.  One lane per block read 64 bytes at a stride of 64, twice:
 // 254 us for a 4096 x 12288 weight (234 MB, 0.9 TB/s).
+// A lane has four pieces, of four blocks; lane u of every quad takes the two divisions and the scale byte of block u and the others get the
+// factor through a lane exchange (4096 x 12288 floats 45 us, 5.1 TB/s; 51 with every lane dividing for itself and seven comparisons per code).
+// The pieces are walked from the last to the first: what a cast or another pass has just written last is still in the memory-side cache.
 template <int BLOCK>
 __global__ __launch_bounds__(kThreads) void encode4_blockscale_vec_kernel(const float* __restrict__ src, uint8_t* __restrict__ nibbles, uint8_t* __restrict__ scales,
                                                                          size_t n_quads)
 {
     constexpr int LANES = BLOCK / 4;
-    // a group of lanes is complete in every step: n_quads is a multiple of LANES, and so are the stride and a group's first lane
-    stream_pieces(n_quads,
-        [&](size_t v) { return __builtin_nontemporal_load((const f32x4*)src + v); },
-        [&](size_t v, const f32x4& x) {
-            float amax = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-            amax = fmaxf(amax, dpp_f32<0xB1>(amax));                                  // quad_perm [1,0,3,2]
-            amax = fmaxf(amax, dpp_f32<0x4E>(amax));                                  // quad_perm [2,3,0,1]
-            if (LANES == 8) { amax = fmaxf(amax, dpp_f32<0x141>(amax)); }             // row_half_mirror
-            const float fwd = (amax > 1e-10f) ? (6.0f / amax) : 1.0f;
-            const uint32_t w = f32_to_fp4(x[0] * fwd) | (f32_to_fp4(x[1] * fwd) << 4) | (f32_to_fp4(x[2] * fwd) << 8) | (f32_to_fp4(x[3] * fwd) << 12);
-            ((uint16_t*)nibbles)[v] = (uint16_t)w;
-            if (v % LANES == 0) { scales[v / LANES] = (uint8_t)f32_to_e4m3_trunc((amax > 1e-10f) ? (amax / 6.0f) : 1.0f); }
-        });
+    static_assert(kInFlight == 4, "a piece per lane of a quad");
+    const size_t stride = (size_t)gridDim.x * kThreads;
+    const size_t rounds = (n_quads + 4 * stride - 1) / (4 * stride);
+    const uint32_t q = threadIdx.x & 3u;
+    for (size_t r = rounds; r-- > 0;)
+    {
+        // a group of lanes is complete in every step: n_quads is a multiple of LANES, and so are the stride and a group's first lane
+        const size_t v = r * 4 * stride + (size_t)blockIdx.x * kThreads + threadIdx.x;
+        f32x4 x[4];
+        float amax[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) { x[u] = __builtin_nontemporal_load((const f32x4*)src + (v + u * stride < n_quads ? v + u * stride : n_quads - LANES + threadIdx.x % LANES)); }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+        {
+            float m = fmaxf(fmaxf(fabsf(x[u][0]), fabsf(x[u][1])), fmaxf(fabsf(x[u][2]), fabsf(x[u][3])));
+            m = fmaxf(m, dpp_f32<0xB1>(m));                                           // quad_perm [1,0,3,2]
+            m = fmaxf(m, dpp_f32<0x4E>(m));                                           // quad_perm [2,3,0,1]
+            if (LANES == 8) { m = fmaxf(m, dpp_f32<0x141>(m)); }                      // row_half_mirror
+            amax[u] = m;
+        }
+        const float mine = q < 2u ? (q == 0u ? amax[0] : amax[1]) : (q == 2u ? amax[2] : amax[3]);
+        const float fwd = (mine > 1e-10f) ? (6.0f / mine) : 1.0f;
+        const size_t at = v + q * stride;                                             // a piece of the lane's block
+        if (at < n_quads && (LANES == 4 || (threadIdx.x & 4u) == 0u)) { scales[at / LANES] = (uint8_t)f32_to_e4m3_trunc((mine > 1e-10f) ? (mine / 6.0f) : 1.0f); }
+        const float f[4] = { dpp_f32<0x00>(fwd), dpp_f32<0x55>(fwd), dpp_f32<0xAA>(fwd), dpp_f32<0xFF>(fwd) };      // lane u of the quad
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+        {
+            const uint32_t w = f32_to_fp4(x[u][0] * f[u]) | (f32_to_fp4(x[u][1] * f[u]) << 4) | (f32_to_fp4(x[u][2] * f[u]) << 8) | (f32_to_fp4(x[u][3] * f[u]) << 12);
+            if (v + u * stride < n_quads) { ((uint16_t*)nibbles)[v + u * stride] = (uint16_t)w; }
+        }
+    }
 }
 
-// Largest magnitude.  16-byte loads over the aligned body (scalar loads for a misaligned pointer and the tail), wave
-// reduction through lane reads, the four waves of a workgroup through LDS, then at most one atomic per workgroup on the
+// Largest magnitude.  16-byte loads over the aligned body (scalar loads for a misaligned pointer and the tail), four in flight per lane, wave
+// reduction through lane exchanges, the sixteen waves of a workgroup through LDS, then at most one atomic per workgroup on the
 // bit pattern (non-negative floats order like unsigned integers) -- and none when the value already stored is at least as
-// large: thousands of atomics on one address are served one after the other (190 us for 16 k of them, whatever n was).
-// NaN inputs are skipped by fmaxf as before.
-__global__ __launch_bounds__(kThreads) void absmax_kernel(const void* __restrict__ src, int src_type, size_t n, unsigned int* __restrict__ out)
+// large.  Atomics on one address are served one after the other and most workgroups start before the first has ended: one workgroup
+// per CU at most, of 1024 threads (with up to sixteen per CU of 256 threads 1 M floats took 16.4 us, now 6.2 with the launch that clears the result, 16 M 21.1 / 13.3, 50 M 37.6 / 31.8).
+// From the last piece to the first: what a cast has just written last is still in the memory-side cache, and the encoder that
+// follows begins where this ends.  NaN inputs are skipped by fmaxf as before.
+constexpr int kMaxThreads = 1024;
+
+static __global__ void absmax_clear_kernel(unsigned int* out) { *out = 0u; }
+
+template <int SRC>
+__global__ __launch_bounds__(kMaxThreads) void absmax_kernel(const void* __restrict__ src, size_t n, unsigned int* __restrict__ out)
 {
-    __shared__ float part[kThreads / 64];
-    const size_t stride = (size_t)gridDim.x * kThreads;
-    const size_t first = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    __shared__ float part[kMaxThreads / 64];
+    const size_t stride = (size_t)gridDim.x * kMaxThreads;
+    const size_t first = (size_t)blockIdx.x * kMaxThreads + threadIdx.x;
+    constexpr size_t PER = SRC == DT_FLOAT ? 4 : 8;             // elements per 16-byte load
+    const size_t n_vec = ((uintptr_t)src & 15u) == 0 ? n / PER : 0;
     float m = 0.0f;
-    const size_t per = src_type == DT_FLOAT ? 4 : 8;            // elements per 16-byte load
-    const size_t n_vec = ((uintptr_t)src & 15u) == 0 ? n / per : 0;
-    for (size_t c = first; c < n_vec; c += stride)
-    {
-        const u32x4 v = ((const u32x4*)src)[c];
+    auto take = [&](const u32x4& v) {
 #pragma unroll
         for (int d = 0; d < 4; d++)
         {
-            if (src_type == DT_FLOAT) { m = fmaxf(m, fabsf(bits_to_f32(v[d]))); }
-            else if (src_type == DT_HALF) { m = fmaxf(m, fmaxf(fabsf(half_bits_to_f32(v[d] & 0xFFFFu)), fabsf(half_bits_to_f32(v[d] >> 16)))); }
-            else { m = fmaxf(m, fmaxf(fabsf(bf16_bits_to_f32(v[d] & 0xFFFFu)), fabsf(bf16_bits_to_f32(v[d] >> 16)))); }
+            if constexpr (SRC == DT_FLOAT) { m = fmaxf(m, fabsf(bits_to_f32(v[d]))); }
+            else { m = fmaxf(m, fmaxf(fabsf(act_bits_to_f32<SRC>(v[d] & 0xFFFFu)), fabsf(act_bits_to_f32<SRC>(v[d] >> 16)))); }
         }
+    };
+    size_t rounds = n_vec / stride;                             // whole ones; the rest is at the end and comes first
+    if (rounds * stride + first < n_vec) { take(((const u32x4*)src)[rounds * stride + first]); }
+    for (; rounds % 4; rounds--) { take(((const u32x4*)src)[(rounds - 1) * stride + first]); }
+    for (; rounds; rounds -= 4)
+    {
+        u32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) { v[u] = ((const u32x4*)src)[(rounds - 1 - u) * stride + first]; }
+#pragma unroll
+        for (int u = 0; u < 4; u++) { take(v[u]); }
     }
-    for (size_t i = n_vec * per + first; i < n; i += stride) { m = fmaxf(m, fabsf(load_plain(src, src_type, i))); }
+    for (size_t i = n_vec * PER + first; i < n; i += stride) { m = fmaxf(m, fabsf(load_plain(src, SRC, i))); }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) { m = fmaxf(m, __shfl_xor(m, off)); }
     if ((threadIdx.x & 63) == 0) { part[threadIdx.x >> 6] = m; }
     __syncthreads();
     if (threadIdx.x == 0)
     {
-        for (int w = 1; w < kThreads / 64; w++) { m = fmaxf(m, part[w]); }
+        for (int w = 1; w < kMaxThreads / 64; w++) { m = fmaxf(m, part[w]); }
         const unsigned int bits = f32_to_bits(m);
         if (bits > __atomic_load_n(out, __ATOMIC_RELAXED)) { atomicMax(out, bits); }
     }
@@ -473,13 +516,15 @@ int hip_absmax(const void* src, int src_type, unsigned int n, void* d_result)
 {
     if (src_type != DT_FLOAT && src_type != DT_HALF && src_type != DT_BF16) { return -1; }
     if (!d_result) { return -1; }
-    const hipError_t err = hipMemsetAsync(d_result, 0, sizeof(float), stream());
-    if (err != hipSuccess)
+    absmax_clear_kernel<<<1, 1, 0, stream()>>>((unsigned int*)d_result);
+    if (n)
     {
-        fprintf(stderr, "absmax clear failed: %s\n", hipGetErrorString(err));
-        return 1;
+        const size_t want = ((size_t)n / (src_type == DT_FLOAT ? 4 : 8) + kMaxThreads - 1) / kMaxThreads;
+        const unsigned grid = (unsigned)std::min(std::max(want, (size_t)1), (size_t)cu_count());
+        if (src_type == DT_FLOAT) { absmax_kernel<DT_FLOAT><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
+        else if (src_type == DT_HALF) { absmax_kernel<DT_HALF><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
+        else { absmax_kernel<DT_BF16><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
     }
-    if (n) { absmax_kernel<<<grid_for(n), kThreads, 0, stream()>>>(src, src_type, n, (unsigned int*)d_result); }
     return finish("absmax");
 }
 
