@@ -71,7 +71,8 @@ int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v
                                                              n_q_heads, t_kv, n_tokens, pos0, scale, ranges)
 #define CCQ_ATTN_PREFILL_GROUPS(PASS)                                                                                                              \
     group == 4 ? CCQ_ATTN_PREFILL(4, PASS) : group == 2 ? CCQ_ATTN_PREFILL(2, PASS) : CCQ_ATTN_PREFILL(1, PASS)
-    if (!scratch) { CCQ_ATTN_PREFILL_GROUPS(0); }
+    if (pos0 + n_tokens <= PF_SHORT * PF_KEYS) { CCQ_ATTN_PREFILL_GROUPS(3); }
+    else if (!scratch) { CCQ_ATTN_PREFILL_GROUPS(0); }
     else
     {
         CCQ_ATTN_PREFILL_GROUPS(1);

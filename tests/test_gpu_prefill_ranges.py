@@ -40,6 +40,28 @@ def test_few_tokens_behind_a_long_context_follow_the_oracle(gpu, oracle, dec, n_
         assert np.linalg.norm(dec.f(got[t]) - want) <= 4e-3 * np.linalg.norm(want), t
 
 
+@pytest.mark.parametrize("n_q,n_kv,T,pos0", [(1, 1, 1, 0), (8, 2, 20, 44), (4, 2, 33, 95), (2, 2, 17, 239), (8, 2, 130, 126), (4, 4, 16, 241), (4, 1, 20, 1500)])
+def test_context_of_up_to_four_blocks_and_its_neighbours(gpu, oracle, dec, n_q, n_kv, T, pos0):
+    """64, 128, 256 keys and one more or fewer, and a split context: the oracle's attention, and the same bits where the output is
+    not aligned for wide stores."""
+    torch, dev, lib = gpu
+    t_kv = pos0 + T + 3
+    q, kc, vc = inputs(oracle, n_q, n_kv, T, pos0, t_kv)
+    qd, kd, vd = to_dev(torch, dev, q), to_dev(torch, dev, kc), to_dev(torch, dev, vc)
+    y, z = (torch.zeros(T * n_q * 128 + 64, dtype=torch.int16, device=dev) for _ in range(2))
+    for out in (y, z[1:]):
+        assert lib.c.hip_attention_prefill_bf16(ptr(qd), ptr(kd), ptr(vd), ptr(out), n_q, n_kv, 128, t_kv, T, pos0) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y[:-1], z[1:]) and z[0] == 0 and not y[T * n_q * 128:].any()
+    got = from_dev(y, np.uint16)[:T * n_q * 128].reshape(T, n_q, 128)
+    kf, vf = dec.f(kc), dec.f(vc)
+    kf[:, pos0 + T:], vf[:, pos0 + T:] = 0.0, 0.0
+    for t in range(T):
+        want = dec.attention(dec.f(q[t]), kf, vf, pos0 + t, n_q, n_kv)
+        assert ulp_close(got[t], want, ulps=2.0, floor=2e-3 * np.abs(want).max()).all(), t
+        assert np.linalg.norm(dec.f(got[t]) - want) <= 4e-3 * np.linalg.norm(want), t
+
+
 def test_ranges_under_capture(gpu, oracle, dec):
     """A captured call whose scratch an eager call has sized replays the eager result, with eager work of another size in between; one
     on a stream without scratch runs in one piece, within the bounds."""
