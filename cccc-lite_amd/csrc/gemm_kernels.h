@@ -1134,9 +1134,9 @@ inline float* split_workspace(const GemmPlan& plan, long long outputs) { return 
 inline GemmPlan joint_plan(const LinearArgs& a, GemmKind kind, const GemmWeights& w, long long outputs, float*& partial)
 {
     const int cus = cu_count();
-    GemmPlan plan = staged_plan(a, kind, w, cus, plan_gemm(a, kind, w, cus, true));
+    GemmPlan plan = staged_plan(a, kind, w, cus, plan_gemm(a, kind, w, cus, true), true);
     partial = split_workspace(plan, outputs);
-    return plan.splits > 1 && !partial ? staged_plan(a, kind, w, cus, plan_gemm(a, kind, w, cus, false)) : plan;
+    return plan.splits > 1 && !partial ? staged_plan(a, kind, w, cus, plan_gemm(a, kind, w, cus, false), false) : plan;
 }
 
 // a.seg_tile0 for 256-feature tiles (empty segments start past the last tile); the number of tiles
@@ -1262,7 +1262,7 @@ void launch_gemm_mfma(const LinearArgs& a)
 inline bool linear_plan(const LinearArgs& a, const GemmWeights& w, bool add_norm, SplitScratch* scratch, GemmPlan& plan, float*& partial)
 {
     const int cus = cu_count();
-    plan = staged_plan(a, GEMM_LINEAR, w, cus, plan_gemm(a, GEMM_LINEAR, w, cus, true));
+    plan = staged_plan(a, GEMM_LINEAR, w, cus, plan_gemm(a, GEMM_LINEAR, w, cus, true), true);
     partial = nullptr;
     if (plan.ranges > 1)
     {
@@ -1277,7 +1277,7 @@ inline bool linear_plan(const LinearArgs& a, const GemmWeights& w, bool add_norm
             partial = scratch->fixed;
         }
         else { partial = (float*)workspace(need); }
-        if (!partial) { plan = staged_plan(a, GEMM_LINEAR, w, cus, plan_gemm(a, GEMM_LINEAR, w, cus, false)); }
+        if (!partial) { plan = staged_plan(a, GEMM_LINEAR, w, cus, plan_gemm(a, GEMM_LINEAR, w, cus, false), false); }
     }
     return !add_norm || plan.ranges > 1;
 }

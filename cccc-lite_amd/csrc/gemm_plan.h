@@ -262,43 +262,94 @@ constexpr GemmTile kStagedTiles[] = {
     { 7, 2, 2.5, 5.0, { 0.361, 0.381, 0.462, 0.460 }, { 0.356, 0.360, 0.426, 0.434 } },
 };
 
+// What `plan` takes by its estimate, and the row kernel that an unsplit linear of at most 4096 features may have behind it
+// (the residual add and the norm, see plan_gemm).
+struct StagedRival
+{
+    double us, row_kernel;
+
+    StagedRival(const LinearArgs& a, GemmKind kind, const GemmWeights& w, int cus, const GemmPlan& plan)
+    {
+        const bool deep = plan.small || (plan.splits > 1 && plan.mb <= 4), add_norm = kind == GEMM_LINEAR && plan.ranges > 1 && a.n_out <= 4096 && a.n_out % 8 == 0;
+        const GemmTile* const table = deep ? kSmallTiles : kLargeTiles;
+        const int n_table = deep ? sizeof(kSmallTiles) / sizeof(GemmTile) : sizeof(kLargeTiles) / sizeof(GemmTile);
+        us = 0.0;
+        row_kernel = add_norm ? 3.0 + 0.55 * 2e-6 * (double)a.tokens * a.n_out : 0.0;
+        for (int i = 0; i < n_table; i++)
+        {
+            if (table[i].mb == plan.mb && table[i].nb == plan.nb) { us = estimate_us(a, kind, table[i], w, plan.splits, cus); }
+        }
+        if (plan.splits == 1) { us += row_kernel; }
+    }
+};
+
 // The staged kernel in the place of `plan` from K = 1024 on (shorter sums keep the order of the register-fed kernels, so that a joint or
-// paired launch gives the bits of the separate calls) and up to 512 tokens (above that the larger tiles are level or ahead),
-// where its estimate is 5 % (file layout) or 8 % (tiled copy, whose KiB blocks the other kernels read whole as well) and 0.3 us below the
-// plan's own: with less, launches of 5 us and k-split ones on tiled copies lose up to 15 %.  Of 620 measured calls one
-// then takes more than 3 % longer (4 %); mean of all 0.96 of the plans' time, 0.91 on E5M2 in the file layout.  An unsplit linear that may come with the add and the norm carries half of the row kernel, as in plan_gemm, and
-// must not be behind with all of it either (4096 x 12288 at 512 tokens, tiled: 58 us alone on both, 64 against 55 with the norm).
-// The k ranges of the larger tile, and so the scratch memory, stay what they were.  FP4 keeps its plans.
-inline GemmPlan staged_plan(const LinearArgs& a, GemmKind kind, const GemmWeights& w, int cus, const GemmPlan& plan)
+// paired launch gives the bits of the separate calls) and up to 512 tokens (above that the larger tiles are level or ahead).
+// It adds the products in another order than the register-fed kernels.  Where the plans of the two weight layouts have the same k
+// ranges, a weight gives the same bits from the file layout and from its tiled copy: there one decision serves both, the k ranges
+// for which the staged kernel is ahead on both together.  Elsewhere each layout takes what is best for it.
+// Ahead: 0.3 us and 5 % (file layout) or 8 % (tiled copy, whose KiB blocks the other kernels read whole as well; 3 % in a joint decision)
+// below the plan's own estimate; with less, launches of 5 us and k-split ones on tiled copies lose up to 15 %.  Of 620
+// measured calls 119 then run it, three of them more than 3 % slower (9 % at most); mean of all calls 0.94 of the plans' time on E5M2 in the
+// file layout, 0.98 on tiled copies (0.91 and 0.97 without the joint decision).
+// An unsplit linear that may come with the add and the norm carries half of the row kernel, as in plan_gemm, and must not be behind
+// with all of it either (4096 x 12288 at 512 tokens, tiled: 58 us alone on both, 64 against 55 with the norm).
+// `scratch` is that of the call to plan_gemm.  The k ranges of the larger tile, and so the scratch memory, stay what they were.  FP4
+// keeps its plans.
+inline GemmPlan staged_plan(const LinearArgs& a, GemmKind kind, const GemmWeights& w, int cus, const GemmPlan& plan, bool scratch)
 {
     if (w.fp4 || a.K < 1024 || a.tokens > 512) { return plan; }
-    const bool deep = plan.small || (plan.splits > 1 && plan.mb <= 4);
-    const GemmTile* const table = deep ? kSmallTiles : kLargeTiles;
-    const int n_table = deep ? sizeof(kSmallTiles) / sizeof(GemmTile) : sizeof(kLargeTiles) / sizeof(GemmTile);
+    const GemmWeights layouts[2] = { w, { false, !w.row_major, w.scaled } };
+    const GemmPlan plans[2] = { plan, plan_gemm(a, kind, layouts[1], cus, scratch) };
+    const bool joint = plans[0].splits == plans[1].splits;
+    const int ranges = joint ? std::min(plan.ranges, plans[1].ranges) : plan.ranges;
     const bool add_norm = kind == GEMM_LINEAR && plan.ranges > 1 && a.n_out <= 4096 && a.n_out % 8 == 0;
     const double row_kernel = add_norm ? 3.0 + 0.55 * 2e-6 * (double)a.tokens * a.n_out : 0.0;
-    double limit = 0.0, with_norm = 0.0;
-    for (int i = 0; i < n_table; i++)
+    GemmPlan best = plan;
+    double least = 1e30;
+    double limit[2] = { 0.0, 0.0 }, with_norm[2] = { 0.0, 0.0 };
+    for (int l = 0; l < (joint ? 2 : 1); l++)
     {
-        if (table[i].mb == plan.mb && table[i].nb == plan.nb)
+        const GemmPlan& p = plans[l];
+        const bool deep = p.small || (p.splits > 1 && p.mb <= 4);
+        const GemmTile* const table = deep ? kSmallTiles : kLargeTiles;
+        const int n_table = deep ? sizeof(kSmallTiles) / sizeof(GemmTile) : sizeof(kLargeTiles) / sizeof(GemmTile);
+        for (int i = 0; i < n_table; i++)
         {
-            const double us = estimate_us(a, kind, table[i], w, plan.splits, cus), row = plan.splits == 1 ? row_kernel : 0.0;
-            limit = (w.row_major ? 0.95 : 0.92) * (us + 0.5 * row) - 0.3;
-            with_norm = us + row;
+            if (table[i].mb == p.mb && table[i].nb == p.nb)
+            {
+                const double us = estimate_us(a, kind, table[i], layouts[l], p.splits, cus), row = p.splits == 1 ? row_kernel : 0.0;
+                limit[l] = (layouts[l].row_major ? 0.95 : joint ? 0.97 : 0.92) * (us + 0.5 * row) - 0.3;
+                with_norm[l] = us + row;
+            }
         }
     }
-    GemmPlan best = plan;
-    for (const GemmTile& t : kStagedTiles)
+    for (int s = 1; s <= ranges && (s == 1 || a.K / 64 / s >= 4); s++)
     {
-        if ((t.mb > 2 && 16 * (t.mb - 1) >= a.tokens) || (t.mb == 2 && a.tokens > 64) || (t.mb == 3 && a.tokens > 192)) { continue; }
-        for (int s = 1; s <= plan.ranges && (s == 1 || a.K / 64 / s >= 4); s++)
+        const double row = s == 1 ? row_kernel : 0.0;
+        const GemmTile* mine = nullptr;
+        double sum = 0.0;
+        for (int l = 0; l < (joint ? 2 : 1); l++)
         {
-            const double us = estimate_us(a, kind, t, w, s, cus, 0.7), row = s == 1 ? row_kernel : 0.0;
-            if (us + 0.5 * row < limit && us + row <= with_norm)
+            const GemmTile* tile = nullptr;
+            double us = 1e30;
+            for (const GemmTile& t : kStagedTiles)
             {
-                limit = us + 0.5 * row;
-                best = GemmPlan{ t.mb, t.nb, s, true, plan.ranges, true };
+                if ((t.mb > 2 && 16 * (t.mb - 1) >= a.tokens) || (t.mb == 2 && a.tokens > 64) || (t.mb == 3 && a.tokens > 192)) { continue; }
+                const double e = estimate_us(a, kind, t, layouts[l], s, cus, 0.7);
+                if (e < us)
+                {
+                    us = e;
+                    tile = &t;
+                }
             }
+            sum += us + 0.5 * row < limit[l] && us + row <= with_norm[l] ? us + 0.5 * row : 1e30;
+            if (l == 0) { mine = tile; }
+        }
+        if (sum < least)
+        {
+            least = sum;
+            best = GemmPlan{ mine->mb, mine->nb, s, true, plan.ranges, true };
         }
     }
     return best;

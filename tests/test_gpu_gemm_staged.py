@@ -23,11 +23,12 @@ extern "C" void plan(int kind, int row_major, int scaled, int tokens, int n_out,
     a.n_segments = n_segments;
     for (int s = 0; s < n_segments; s++) { a.seg_n_out[s] = segments[s]; }
     const GemmWeights w = { false, row_major != 0, scaled != 0 };
-    const GemmPlan p = staged_plan(a, (GemmKind)kind, w, 256, plan_gemm(a, (GemmKind)kind, w, 256, true));
+    const GemmPlan before = plan_gemm(a, (GemmKind)kind, w, 256, true), p = staged_plan(a, (GemmKind)kind, w, 256, before, true);
     out[0] = p.mb;
     out[1] = p.nb;
     out[2] = p.splits;
     out[3] = p.staged;
+    out[4] = before.splits;
 }
 """
 
@@ -35,7 +36,7 @@ _lib = None
 
 
 def plan(layout, kind, tokens, widths, K):
-    """(tokens / 16, features / 64, k ranges, staged?) of the launch the library makes on 256 CUs."""
+    """(tokens / 16, features / 64, k ranges, staged?, k ranges of plan_gemm) of the launch the library makes on 256 CUs."""
     global _lib
     if _lib is None:
         csrc = Path(__file__).resolve().parent.parent / "cccc-lite_amd" / "csrc"
@@ -44,7 +45,7 @@ def plan(layout, kind, tokens, widths, K):
             subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-shared", "-fPIC", "-I", str(csrc), "plan.cpp", "-o", "plan.so"], cwd=d, check=True)
             _lib = ctypes.CDLL(str(Path(d) / "plan.so"))
     segments = widths if kind == SEGMENTS else []
-    out = (ctypes.c_int * 4)()
+    out = (ctypes.c_int * 5)()
     _lib.plan(kind, layout.startswith("file"), "scaled" in layout, tokens, 0 if segments else widths[0], K, len(segments), (ctypes.c_int * 3)(*segments), out)
     return tuple(out)
 
@@ -52,37 +53,39 @@ def plan(layout, kind, tokens, widths, K):
 # weight layout, kind of launch, [(tokens, features, K, tokens / 16 and features / 64 of the tile, k ranges)]: token counts one past a tile
 # and short of one, features 8 past a tile, K an odd number of halves of a stage (the last stage half empty) or of whole stages
 CASES = [
-    ("file", LINEAR, [(17, 4104, 1600, 2, 1, 1), (17, 72, 1088, 2, 1, 2), (17, 16392, 1088, 2, 2, 1), (65, 8200, 1088, 3, 2, 1), (65, 2568, 4160, 3, 2, 4),
-        (65, 72, 1600, 4, 1, 1), (400, 72, 6208, 4, 1, 4), (257, 3080, 1088, 4, 2, 1), (337, 520, 6208, 4, 2, 5), (65, 16392, 1088, 5, 2, 1),
-        (65, 5128, 4160, 5, 2, 4), (100, 16392, 1088, 7, 2, 1), (100, 5128, 6208, 7, 2, 5)]),
-    ("file", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 2112, 2, 1, 4), (5, 8200, 1088, 2, 2, 1), (65, 4104, 1088, 3, 2, 1), (33, 1032, 8256, 3, 2, 8),
-        (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 4), (257, 1544, 1088, 4, 2, 1), (337, 264, 6208, 4, 2, 5), (65, 8200, 1088, 5, 2, 1),
-        (65, 2568, 4160, 5, 2, 4), (100, 8200, 1088, 7, 2, 1), (100, 2568, 6208, 7, 2, 5)]),
-    ("file", SEGMENTS, [(5, 72, 1088, 2, 1, 1), (5, 2056, 6208, 2, 1, 4), (5, 12296, 1088, 2, 2, 1), (65, 6152, 1088, 3, 2, 1), (65, 2056, 4160, 3, 2, 4),
-        (512, 136, 1600, 4, 1, 1), (400, 72, 8256, 4, 1, 4), (257, 2056, 1088, 4, 2, 1), (337, 264, 6208, 4, 2, 5), (65, 12296, 1088, 5, 2, 1),
-        (400, 264, 8256, 5, 2, 6), (100, 12296, 1088, 7, 2, 1), (209, 1544, 8256, 7, 2, 5)]),
-    ("tiled", LINEAR, [(17, 8200, 2112, 2, 1, 1), (65, 8200, 3136, 3, 2, 1), (81, 6152, 6208, 3, 2, 2), (49, 8200, 2112, 4, 1, 1), (49, 16392, 6208, 4, 2, 1),
-        (65, 16392, 1088, 5, 2, 1), (65, 4104, 8256, 5, 2, 5), (100, 16392, 2112, 7, 2, 1), (257, 4104, 8256, 7, 2, 2)]),
-    ("tiled", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 6208, 2, 1, 7), (17, 8200, 8256, 2, 2, 1), (65, 4104, 3136, 3, 2, 1), (81, 3080, 6208, 3, 2, 2),
-        (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 4), (49, 8200, 4160, 4, 2, 1), (65, 8200, 1088, 5, 2, 1), (65, 2056, 8256, 5, 2, 5),
-        (100, 8200, 2112, 7, 2, 1), (257, 2056, 8256, 7, 2, 2)]),
-    ("tiled", SEGMENTS, [(5, 6152, 2112, 2, 1, 1), (65, 6152, 3136, 3, 2, 1), (81, 4104, 6208, 3, 2, 2), (400, 520, 2112, 4, 1, 1), (257, 2568, 6208, 4, 2, 1),
-        (65, 12296, 1088, 5, 2, 1), (65, 2568, 8256, 5, 2, 6), (100, 12296, 3136, 7, 2, 1), (257, 2568, 8256, 7, 2, 2)]),
-    ("file_scaled", LINEAR, [(17, 5128, 1600, 2, 1, 1), (17, 72, 1088, 2, 1, 2), (17, 16392, 1600, 2, 2, 1), (17, 12296, 8256, 2, 2, 2), (65, 8200, 2112, 3, 2, 1),
-        (33, 8200, 8256, 3, 2, 3), (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 2), (49, 16392, 3136, 4, 2, 1), (65, 16392, 1088, 5, 2, 1),
-        (65, 5128, 4160, 5, 2, 4), (100, 16392, 1088, 7, 2, 1), (100, 8200, 3136, 7, 2, 3)]),
-    ("file_scaled", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 2112, 2, 1, 4), (5, 8200, 1600, 2, 2, 1), (5, 3080, 8256, 2, 2, 4), (33, 8200, 2112, 3, 2, 1),
-        (33, 4104, 8256, 3, 2, 3), (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 4), (49, 8200, 3136, 4, 2, 1), (65, 8200, 1088, 5, 2, 1),
-        (65, 4104, 2112, 5, 2, 3), (100, 8200, 1088, 7, 2, 1), (100, 4104, 3136, 7, 2, 3)]),
-    ("file_scaled", SEGMENTS, [(5, 6152, 2112, 2, 1, 1), (5, 4104, 8256, 2, 1, 4), (5, 12296, 1600, 2, 2, 1), (5, 8200, 6208, 2, 2, 2), (65, 6152, 2112, 3, 2, 1),
-        (33, 6152, 8256, 3, 2, 3), (65, 72, 1088, 4, 1, 1), (400, 72, 6208, 4, 1, 4), (49, 12296, 3136, 4, 2, 1), (65, 12296, 1088, 5, 2, 1),
-        (400, 264, 8256, 5, 2, 6), (100, 12296, 1088, 7, 2, 1), (100, 6152, 3136, 7, 2, 3)]),
-    ("tiled_scaled", LINEAR, [(65, 72, 1600, 4, 1, 1), (65, 16392, 1088, 5, 2, 1), (65, 5128, 6208, 5, 2, 5), (100, 16392, 2112, 7, 2, 1),
-        (100, 12296, 8256, 7, 2, 2)]),
-    ("tiled_scaled", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 6208, 2, 1, 7), (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 4), (65, 8200, 1088, 5, 2, 1),
-        (65, 2568, 6208, 5, 2, 5), (100, 8200, 2112, 7, 2, 1), (100, 6152, 8256, 7, 2, 2)]),
-    ("tiled_scaled", SEGMENTS, [(31, 10248, 6208, 2, 1, 1), (129, 2568, 3136, 4, 1, 1), (65, 12296, 1088, 5, 2, 1), (65, 3080, 8256, 5, 2, 6),
-        (100, 12296, 3136, 7, 2, 1), (100, 8200, 8256, 7, 2, 2)]),
+    ("file", LINEAR, [(17, 4104, 1600, 2, 1, 1), (17, 4104, 4160, 2, 1, 3), (17, 16392, 3136, 2, 2, 1), (65, 8200, 2112, 3, 2, 1),
+        (65, 2056, 8256, 3, 2, 5), (65, 72, 1600, 4, 1, 1), (400, 72, 8256, 4, 1, 4), (49, 16392, 3136, 4, 2, 1), (209, 1032, 8256, 4, 2, 4),
+        (65, 16392, 1088, 5, 2, 1), (65, 5128, 4160, 5, 2, 4), (100, 16392, 1088, 7, 2, 1), (100, 6152, 8256, 7, 2, 4)]),
+    ("file", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 2112, 2, 1, 4), (5, 8200, 2112, 2, 2, 1), (33, 5128, 2112, 3, 2, 1), (33, 1032, 8256, 3, 2, 8),
+        (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 4), (257, 1544, 3136, 4, 2, 1), (100, 2056, 8256, 4, 2, 3), (65, 8200, 1088, 5, 2, 1),
+        (65, 2568, 4160, 5, 2, 4), (100, 8200, 1600, 7, 2, 1), (100, 3080, 8256, 7, 2, 4)]),
+    ("file", SEGMENTS, [(17, 776, 1600, 2, 1, 1), (5, 2056, 6208, 2, 1, 4), (5, 12296, 2112, 2, 2, 1), (65, 6152, 2112, 3, 2, 1),
+        (129, 776, 8256, 3, 2, 5), (512, 136, 1600, 4, 1, 1), (400, 72, 8256, 4, 1, 4), (257, 2056, 3136, 4, 2, 1), (209, 776, 8256, 4, 2, 4),
+        (65, 12296, 1088, 5, 2, 1), (65, 2568, 8256, 5, 2, 6), (100, 12296, 1600, 7, 2, 1), (100, 4104, 8256, 7, 2, 4)]),
+    ("tiled", LINEAR, [(17, 4104, 1600, 2, 1, 1), (65, 8200, 2112, 3, 2, 1), (129, 2056, 6208, 3, 2, 3), (65, 72, 1600, 4, 1, 1),
+        (400, 136, 8256, 4, 1, 4), (100, 10248, 3136, 4, 2, 1), (65, 16392, 1088, 5, 2, 1), (65, 5128, 6208, 5, 2, 4), (100, 16392, 1088, 7, 2, 1),
+        (100, 6152, 8256, 7, 2, 4)]),
+    ("tiled", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 2112, 2, 1, 4), (5, 8200, 8256, 2, 2, 1), (65, 4104, 2112, 3, 2, 1), (65, 1544, 8256, 3, 2, 4),
+        (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 4), (449, 1032, 3136, 4, 2, 1), (65, 8200, 1088, 5, 2, 1), (65, 2568, 4160, 5, 2, 4),
+        (100, 8200, 1600, 7, 2, 1), (100, 3080, 8256, 7, 2, 4)]),
+    ("tiled", SEGMENTS, [(17, 776, 1600, 2, 1, 1), (65, 6152, 2112, 3, 2, 1), (65, 2568, 6208, 3, 2, 3), (512, 136, 1600, 4, 1, 1),
+        (400, 72, 8256, 4, 1, 4), (400, 1544, 3136, 4, 2, 1), (65, 12296, 1088, 5, 2, 1), (65, 2568, 8256, 5, 2, 6), (100, 12296, 1600, 7, 2, 1),
+        (100, 4104, 8256, 7, 2, 4)]),
+    ("file_scaled", LINEAR, [(17, 5128, 1600, 2, 1, 1), (17, 8200, 6208, 2, 1, 3), (17, 16392, 3136, 2, 2, 1), (17, 12296, 8256, 2, 2, 2),
+        (33, 16392, 3136, 3, 2, 1), (81, 6152, 6208, 3, 2, 2), (65, 72, 1600, 4, 1, 1), (65, 2568, 3136, 4, 1, 2), (49, 16392, 3136, 4, 2, 1),
+        (65, 16392, 1088, 5, 2, 1), (65, 5128, 4160, 5, 2, 4), (100, 16392, 1600, 7, 2, 1), (100, 8200, 3136, 7, 2, 3)]),
+    ("file_scaled", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 2112, 2, 1, 4), (5, 8200, 1600, 2, 2, 1), (5, 3080, 8256, 2, 2, 4),
+        (33, 8200, 2112, 3, 2, 1), (81, 3080, 6208, 3, 2, 2), (65, 72, 1088, 4, 1, 1), (65, 72, 2112, 4, 1, 4), (49, 8200, 3136, 4, 2, 1),
+        (65, 8200, 1088, 5, 2, 1), (65, 2568, 4160, 5, 2, 5), (100, 8200, 1600, 7, 2, 1), (100, 4104, 3136, 7, 2, 3)]),
+    ("file_scaled", SEGMENTS, [(5, 8200, 3136, 2, 1, 1), (17, 6152, 6208, 2, 1, 3), (5, 12296, 1600, 2, 2, 1), (5, 8200, 8256, 2, 2, 2),
+        (33, 12296, 3136, 3, 2, 1), (33, 6152, 8256, 3, 2, 3), (337, 264, 1600, 4, 1, 1), (65, 1544, 6208, 4, 1, 3), (49, 12296, 3136, 4, 2, 1),
+        (65, 12296, 1088, 5, 2, 1), (65, 4104, 4160, 5, 2, 4), (100, 12296, 1600, 7, 2, 1), (100, 6152, 3136, 7, 2, 3)]),
+    ("tiled_scaled", LINEAR, [(33, 5128, 2112, 2, 1, 1), (65, 72, 1600, 4, 1, 1), (65, 16392, 1088, 5, 2, 1), (65, 5128, 4160, 5, 2, 4),
+        (100, 16392, 1600, 7, 2, 1), (100, 6152, 8256, 7, 2, 4)]),
+    ("tiled_scaled", PAIR, [(5, 72, 1088, 2, 1, 1), (5, 72, 2112, 2, 1, 4), (33, 8200, 3136, 3, 2, 1), (65, 72, 1088, 4, 1, 1),
+        (65, 72, 2112, 4, 1, 4), (65, 8200, 1088, 5, 2, 1), (65, 2568, 4160, 5, 2, 5), (100, 8200, 1600, 7, 2, 1), (100, 3080, 8256, 7, 2, 4)]),
+    ("tiled_scaled", SEGMENTS, [(5, 10248, 3136, 2, 1, 1), (81, 10248, 6208, 3, 2, 1), (337, 264, 1600, 4, 1, 1), (225, 2568, 8256, 4, 1, 2),
+        (65, 12296, 1088, 5, 2, 1), (65, 4104, 4160, 5, 2, 4), (100, 12296, 1600, 7, 2, 1), (100, 4104, 8256, 7, 2, 4)]),
 ]
 
 
@@ -97,6 +100,23 @@ def test_short_sums_and_long_prompts_keep_the_register_fed_kernels(layout, kind)
             assert tokens <= 512 or not plan(layout, kind, tokens, widths, 4096)[3]
 
 
+@pytest.mark.parametrize("scaled", ["", "_scaled"])
+@pytest.mark.parametrize("kind", [LINEAR, PAIR, SEGMENTS])
+def test_the_layouts_of_a_weight_take_the_same_sums_where_they_did(scaled, kind):
+    """With the same k ranges in the plans of the file layout and of the tiled copy, either both or none take the staged kernel, and
+    then with the same k ranges: the copy of a weight gives the bits of its file layout."""
+    staged = 0
+    for tokens in (5, 17, 64, 100, 200, 301, 512):
+        for n_out in (72, 328, 1032, 4096, 12288):
+            for K in (1024, 2112, 4096, 12288):
+                widths = widths_of(n_out) if kind == SEGMENTS else [n_out]
+                file, copy = (plan(layout + scaled, kind, tokens, widths, K) for layout in ("file", "tiled"))
+                if file[4] == copy[4]:
+                    assert file[2:4] == copy[2:4], (tokens, n_out, K)
+                    staged += file[3]
+    assert staged > 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("layout,kind,shapes", CASES, ids=[f"{c[0]}-{('linear', 'pair', 'segments')[c[1]]}" for c in CASES])
 def test_every_staged_tile_against_the_exact_contraction(gpu, oracle, layout, kind, shapes):
@@ -108,7 +128,7 @@ def test_every_staged_tile_against_the_exact_contraction(gpu, oracle, layout, ki
     ptr = lambda t: ctypes.c_void_p(t.data_ptr())
     for tokens, n_out, K, mb, nb, splits in shapes:
         widths = {LINEAR: [n_out], PAIR: [n_out] * 2, SEGMENTS: widths_of(n_out)}[kind]
-        assert plan(layout, kind, tokens, widths, K) == (mb, nb, splits, True), (tokens, n_out, K)
+        assert plan(layout, kind, tokens, widths, K)[:4] == (mb, nb, splits, True), (tokens, n_out, K)
         print(layout, kind, tokens, n_out, K, flush=True)
         gen = torch.Generator(device=dev).manual_seed(tokens + n_out + K)
         weights = [Weight(gpu, oracle, layout, n, K, gen) for n in widths]
