@@ -1142,12 +1142,6 @@ __device__ __forceinline__ void norm_rope_finish(const HeadLoads& h, bool normed
     out_r = bf16_round(nr * c + nl * sn);
 }
 
-__device__ __forceinline__ void norm_rope_head(const uint16_t* __restrict__ src, const uint16_t* __restrict__ nw, const uint16_t* __restrict__ cos_row,
-                                               const uint16_t* __restrict__ sin_row, float eps, int lane, float& out_l, float& out_r)
-{
-    norm_rope_finish(load_head(src, nw, cos_row, sin_row, lane), nw != nullptr, eps, out_l, out_r);
-}
-
 // Launch 1 walks its rows as a stream: each of a chunk's four waves takes every fourth 16-row tile of it with a softmax of its
 // own (running maximum and sum per head, sums rescaled where the maximum grows), the next tile's rows requested before the
 // current one is used.  Nothing is exchanged between the waves until the end, so the loop has no barrier, and the launch behind

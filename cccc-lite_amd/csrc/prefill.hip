@@ -41,7 +41,7 @@ int hip_qk_norm_rope_kv_rows_bf16(const void* q, const void* k, const void* v, c
     if (pos0 < 0 || (long long)pos0 + n_tokens > t_kv) { return -1; }
     if (!q || !k || !v || !cos_tab || !sin_tab || !q_out || !k_cache || !v_cache) { return -1; }
     if ((q_norm_w == nullptr) != (k_norm_w == nullptr)) { return -1; }
-    const dim3 grid((n_q_heads + 2 * n_kv_heads + 3) / 4, n_tokens);
+    const dim3 grid((n_q_heads + 2 * n_kv_heads + 15) / 16, n_tokens);
     qk_norm_rope_kv_rows_kernel<<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_norm_w,
                                                            (const uint16_t*)k_norm_w, (const uint16_t*)cos_tab, (const uint16_t*)sin_tab,
                                                            (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, n_q_heads, n_kv_heads, t_kv, pos0, epsilon);
