@@ -575,12 +575,15 @@ double DecodeModel::run(int n_steps, int use_graph)
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) { return -1.0; }
     double result = -1.0;
     const int sync_before = hip_quant_set_sync(0);
-    // A stream, a capture and an executable graph cost the host 0.25 ms (4 layers) to 1 ms (36), a replayed launch is up to 0.25 us faster than a
-    // launched one (36 layers: 1.82 against 1.88 ms per step; 4 to 8 layers: level): below FEWEST steps they are all launched, above it
-    // the host records the graph while the first two run.  Before and after, ms: one step of 36 layers 2.66 / 1.92, of 4 layers 0.39 / 0.17;
-    // eight 15.4 / 15.1 and 1.30 / 1.08.
-    constexpr int LAUNCHED = 2, FEWEST = 24;
-    if (use_graph && n_steps >= FEWEST)
+    // A stream, a capture and an executable graph cost the host 0.25 ms (4 layers) to 0.75 ms (36), a replayed launch is up to 0.25 us faster
+    // than a launched one (36 layers: 1.83 against 1.89 ms per step; 4 to 8 layers: nearly level), so a graph pays from 10 steps of 36
+    // layers on and hardly ever for 4; the host records it while the first two steps run.  Wall time with a graph recorded first and
+    // replayed / all launched / now: 8 steps of 36 layers 15.27 / 15.11 / 15.11 ms, 16 steps 30.03 / 30.19 / 29.79, 20 steps 37.36 /
+    // 37.75 / 37.00; 16 steps of 4 layers 2.40 / 2.12 / 2.12, 20 of 8 layers 4.52 / 4.20 / 4.20.
+    constexpr int LAUNCHED = 2;
+    constexpr long long FEWEST = 360;           // steps x layers
+    const bool pays = (long long)n_steps * cfg_.layers >= FEWEST && n_steps > LAUNCHED;
+    if (use_graph && pays)
     {
         hipStream_t stream = nullptr;
         hipGraph_t graph = nullptr;

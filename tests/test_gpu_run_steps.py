@@ -7,12 +7,12 @@ from test_gpu_prefill import _fresh, dec  # noqa: F401 (dec: a fixture)
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("steps", [1, 2, 23, 24, 25, 40])
+@pytest.mark.parametrize("steps", [1, 2, 23, 24, 25, 40, 179, 180, 181])
 def test_launched_and_replayed_steps_equal_single_steps(gpu, pkg, dec, steps):
     """Tokens, positions, logits and cache rows of run(steps) are those of `steps` calls of step(), twice in a row on one model."""
     host = pkg.host_api.host()
     host.init(0)
-    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=48)
+    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=200)      # replayed from 180 steps of two layers on
     weights = dec.make_model(cfg, 61)
     single, run = _fresh(pkg, host, cfg), _fresh(pkg, host, cfg)
     single.load(weights)
