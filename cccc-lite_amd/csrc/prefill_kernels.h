@@ -17,7 +17,7 @@ namespace ccq
 // Per-head q/k RMSNorm + RoPE + cache append for T tokens.  Bound by memory: a head is read and written once.  Grid
 // (ceil((n_q + 2 n_kv) / 16), T), sixteen lanes per (head, token): lane i holds elements 4 i .. + 3 of both halves of the head, so that the
 // rotation needs no neighbour, and every access is 8 bytes of a 128-byte run (16 in the copied value rows).  With a whole wave
-// per head and 2-byte accesses 2048 tokens of 32 / 8 heads took 26.7 us, now 14.0 (75 MB: 5.4 TB/s); 512 tokens 6.6, now 4.7; 100
+// per head and 2-byte accesses 2048 tokens of 32 / 8 heads took 26.7 us, now 14.0 (50 MB: 3.6 TB/s); 512 tokens 6.6, now 4.7; 100
 // tokens 2.8, now 2.7; 20 tokens 2.3 and 2.4 (the launch).  Rows off their 8 bytes still gain at 2048 tokens (26.6, now 19.2).
 // The arithmetic per element is the one-token kernel's and the squares are added in the order of its wave_sum, so both leave the same
 // bytes.  The pointers may lie on any element (value rows: on any pair), as before.
