@@ -187,8 +187,7 @@ __global__ __launch_bounds__(256 + 256 * WF, WF == 2 ? 3 : 4) void gemm_staged_k
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) { raw[nb] = *(const u32x2*)(lds + buf * W_STAGE + w_lane + nb * 2048); }
     };
-    auto convert = [&](int st) {
-        const bool in_k = ((st_begin + st) * 2 + (kg >> 1)) * 64 < a.K;
+    auto convert = [&] {
 #pragma unroll
         for (int nb = 0; nb < NB; nb++)
         {
@@ -197,13 +196,15 @@ __global__ __launch_bounds__(256 + 256 * WF, WF == 2 ? 3 : 4) void gemm_staged_k
             fp8x4_to_pairs<WT, SCALED, AT>(raw[nb][0], scale, p0, p1);
             fp8x4_to_pairs<WT, SCALED, AT>(raw[nb][1], scale, p2, p3);
             wfr[nb] = u32x4{ __builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1), __builtin_bit_cast(uint32_t, p2), __builtin_bit_cast(uint32_t, p3) };
-            if (!in_k) { wfr[nb] = u32x4{ 0u, 0u, 0u, 0u }; }
         }
     };
     int xbuf = 0, wbuf = 1;
     for (int st = 0; st < n_st; st++)
     {
         asm volatile("s_barrier" : : : "memory");                           // activations of stage st, codes of stage st + 1
+        // K % 128 == 64: the last stage's second half is past the end, and its groups are done.  (A product with zeros instead would make
+        // NaN of an infinity among the activations that were read in its place.)
+        if (((st_begin + st) * 2 + (kg >> 1)) * 64 >= a.K) { break; }
         const uint8_t* const xp = lds + xbuf * X_STAGE + x_lane;
         constexpr int AHEAD = MB < 3 ? MB : 3;                              // fragment reads run ahead of the matrix-core instructions that use them
         u32x4 ring[AHEAD + 1];
@@ -212,7 +213,7 @@ __global__ __launch_bounds__(256 + 256 * WF, WF == 2 ? 3 : 4) void gemm_staged_k
         if (st == 0)
         {
             read_codes(0);
-            convert(0);
+            convert();
         }
 #pragma unroll
         for (int mb = 0; mb < MB; mb++)
@@ -229,7 +230,7 @@ __global__ __launch_bounds__(256 + 256 * WF, WF == 2 ? 3 : 4) void gemm_staged_k
                 else { acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, xf, acc[mb][nb], 0, 0, 0); }
             }
         }
-        convert(st + 1);
+        convert();
         __builtin_amdgcn_sched_barrier(0);
         xbuf = xbuf == S - 1 ? 0 : xbuf + 1;
         wbuf = wbuf == S ? 0 : wbuf + 1;

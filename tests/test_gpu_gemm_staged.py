@@ -181,3 +181,40 @@ def test_every_staged_tile_against_the_exact_contraction(gpu, oracle, layout, ki
                     assert (diff.abs().amax(dim=1) <= MAX_REL * want.abs().amax(dim=1)).all(), (tokens, n_out, K, form)
         finally:
             for w in weights: w.release()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["file", "tiled", "file_scaled", "tiled_scaled"])
+@pytest.mark.parametrize("half", [False, True])
+def test_infinities_at_the_end_of_a_row(gpu, oracle, layout, half):
+    """K % 128 == 64, unsplit and split: an infinity among the last activations of a row gives the infinities of the exact contraction (NaN only
+    where a weight is zero), one in the last whole stage likewise, and the other rows keep the tolerances of the test above."""
+    torch, dev, lib = gpu
+    dtype = torch.float16 if half else torch.bfloat16
+    for tokens, n_out, K in ((65, 72, 1600), (65, 16392, 1088), (100, 6152, 8256), (65, 5128, 6208)):
+        before = plan(layout, LINEAR, tokens, [n_out], K)
+        assert before[3], (tokens, n_out, K)
+        gen = torch.Generator(device=dev).manual_seed(tokens + n_out + K)
+        weight = Weight(gpu, oracle, layout, n_out, K, gen)
+        x = (torch.randn(tokens, K, device=dev, generator=gen) * (0.0001 if weight.type == oracle.E5M2 else 1.0)).to(dtype)
+        for token, k, value in ((0, K - 1, float("inf")), (3, K - 8, -float("inf")), (17, K - 65, float("inf")), (40, K - 4, float("inf")), (64, 0, -float("inf"))): x[token, k] = value
+        y = torch.zeros(tokens, n_out, dtype=dtype, device=dev)
+        try:
+            torch.cuda.synchronize()
+            rc = lib.linear(weight.codes.data_ptr(), weight.type, x.data_ptr(), y.data_ptr(), n_out, tokens, K, weight.scale, act_type=oracle.HALF if half else oracle.BF16)
+            assert rc == 0
+            torch.cuda.synchronize()
+            finite = torch.isfinite(x).all(dim=1)
+            assert (~finite).sum() == 5
+            w = weight.exact(oracle, half)
+            want = torch.where(torch.isfinite(x), x, torch.zeros_like(x)).double() @ w.T
+            for token in (~finite).nonzero().flatten().tolist():
+                k = (~torch.isfinite(x[token])).nonzero().item()
+                want[token] += x[token, k].double() * w[:, k]
+            want = want.to(dtype).double()
+            got = y.double()
+            assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isposinf(got), torch.isposinf(want)) and torch.equal(torch.isneginf(got), torch.isneginf(want)), (tokens, n_out, K)
+            diff = (got - want)[finite]
+            assert (diff.norm(dim=1) <= ROW_L2_REL * want[finite].norm(dim=1)).all(), (tokens, n_out, K)
+        finally:
+            weight.release()
