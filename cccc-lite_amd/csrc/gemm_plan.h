@@ -283,11 +283,13 @@ struct StagedRival
     }
 };
 
-// The staged kernel in the place of `plan` from K = 1024 on (shorter sums keep the order of the register-fed kernels, so that a joint or
-// paired launch gives the bits of the separate calls) and up to 512 tokens (above that the larger tiles are level or ahead).
-// It adds the products in another order than the register-fed kernels.  Where the plans of the two weight layouts have the same k
-// ranges, a weight gives the same bits from the file layout and from its tiled copy: there one decision serves both, the k ranges
-// for which the staged kernel is ahead on both together.  Elsewhere each layout takes what is best for it.
+// The staged kernel in the place of `plan` from K = 1024 on (the shortest that the estimate is fitted to) and up to 512 tokens (above that
+// the larger tiles are level or ahead).
+// It adds the products in the order of the register-fed kernels, so only the k ranges of a launch show in its bits.  A plan of one
+// range keeps one: joint and paired launches give the bits of the separate calls where none of them splits k, whichever kernel each
+// of them takes.  A k-split plan may get other ranges; where the plans of the two weight layouts have the same, one decision serves
+// both, the k ranges for which the staged kernel is ahead on both together, so that a weight gives the same bits from the file layout
+// and from its tiled copy.  Elsewhere each layout takes what is best for it.
 // Ahead: 0.3 us and 5 % (file layout) or 8 % (tiled copy, whose KiB blocks the other kernels read whole as well; 3 % in a joint decision)
 // below the plan's own estimate; with less, launches of 5 us and k-split ones on tiled copies lose up to 15 %.  Of 620
 // measured calls 119 then run it, three of them more than 3 % slower (9 % at most); mean of all calls 0.94 of the plans' time on E5M2 in the
@@ -324,7 +326,7 @@ inline GemmPlan staged_plan(const LinearArgs& a, GemmKind kind, const GemmWeight
             }
         }
     }
-    for (int s = 1; s <= ranges && (s == 1 || a.K / 64 / s >= 4); s++)
+    for (int s = 1; s <= (plan.splits == 1 ? 1 : ranges) && (s == 1 || a.K / 64 / s >= 4); s++)
     {
         const double row = s == 1 ? row_kernel : 0.0;
         const GemmTile* mine = nullptr;

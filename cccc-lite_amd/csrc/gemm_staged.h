@@ -24,33 +24,32 @@ __device__ __forceinline__ void wait_loads_barrier()
 
 // FP8 weights, K % 64 == 0.  A workgroup owns 16 MB tokens x 64 WF features (a pair: 32 WF of gate and of up) and walks K in stages of
 // 128.  Four loading waves keep S stages of activations and S + 1 of weights (the codes as they are) on their way into LDS; 4 WF
-// computing waves take the MB x 4 blocks of 16 x 16 of 64 features, each of the four k groups a quarter of every stage (32 of 128: one
-// v_mfma_f32_16x16x32 per block), and convert their codes in registers, those of the next stage at the end of a stage.  The four
-// groups' sums meet in LDS at the end.
+// computing waves take 16 features and all the tokens each and convert their codes in registers, a k-tile of 64 ahead of their use.
 //   Why: a prompt of 17 to some 500 tokens is bound by neither the matrix cores nor HBM but by what a CU waits for.  In
-// gemm_mfma_direct_kernel each wave issues its own loads between its matrix-core instructions, reads a row of the file layout
-// 64 bytes at a time (half a line) and every activation of the tile once per 16 or 32 features.  Here loads never hold up a
-// computing wave (the same kernel with its loads spread over the computing waves: 38 against 34 us on the pair below), a line is
-// read whole, an activation from LDS once per 64 features, and what is in flight (60 to 120 KiB a CU) does not cost registers.
-//   E5M2, file layout, MI355X, gemm_mfma_direct_kernel -> this one, us: gate / up pair 4096 x 12288 at 100 tokens 43.4 -> 34.0, at 32 tokens
-// 30.4 -> 25.5; 12288 x 4096 at 100 tokens 28.5 -> 24.0; 4096 x 4096 at 512 tokens 30.6 -> 22.8, at 100 tokens 15.4 -> 14.4.
-//   The order in which an element's products are summed differs from the other kernels' (four interleaved sums); results are FP32
-// sums of the same products, rounded once.
+// gemm_mfma_direct_kernel each wave issues its own loads between its matrix-core instructions and reads a row of the file layout
+// 64 bytes at a time (half a line).  Here loads never hold up a computing wave (with the loads spread over the computing waves 38
+// against 34 us on the pair below), a line is read whole, and what is in flight (60 to 120 KiB a CU) does not cost registers.
+//   E5M2, file layout, MI355X, gemm_mfma_direct_kernel -> this one, us: gate / up pair 4096 x 12288 at 100 tokens 43.7 -> 33.2, at 20 tokens
+// 29.7 -> 24.2; 12288 x 4096 at 160 tokens 37.7 -> 31.3; 4096 x 4096 at 512 tokens 31.4 -> 23.0, at 100 tokens 15.6 -> 13.8.
+//   An element's products are added in the order of every other prompt GEMM, v_mfma_f32_16x16x32 by v_mfma_f32_16x16x32 in ascending k, so a
+// launch has the same bits whichever kernel its plan takes.  (With each of four waves on a quarter of every stage and their sums
+// added at the end an activation is read from LDS once per 64 features and not once per 16, yet that was 2 % slower over the shapes
+// measured, 5 % on tiles of 32 tokens, and faster, by up to 7 %, only where a CU has several workgroups of 64 tokens or more.)
 //
 // LDS: X stages (rows of 256 bytes, 16-byte chunk c of row r at c ^ (r % 16)), then W stages (file layout: rows of 128 bytes, chunk c at
-// c ^ (r / 2 % 8); tiled copy: its KiB blocks, two per 16 rows).  Element k of a stage: group 2 (k / 64) + (k / 8) % 2, lane group
-// (k / 16) % 4 -- the order of the tiled copy, taken for both layouts.
+// c ^ (r / 2 % 8); tiled copy: its KiB blocks, two per 16 rows).  In a k-tile lane group g holds elements 16 g .. + 7 of the first
+// instruction and 16 g + 8 .. + 15 of the second, as in the tiled copy.
 // Pair: a.W_pair is set; segments: a.n_segments > 0; k split: `partial` is set and blockIdx.y the range (all as in
 // gemm_mfma_direct_kernel, whose combine launches finish the sums).
 template <int WT, bool SCALED, bool TILED, int AT, int MB, int WF, int S>
 __global__ __launch_bounds__(256 + 256 * WF, WF == 2 ? 3 : 4) void gemm_staged_kernel(const LinearArgs a_in, const int n_tiles, float* __restrict__ partial)
 {
-    constexpr int NB = 4, COMPUTE = 4 * WF, LOADERS = 4;                    // 16-feature blocks of a computing wave; waves
+    constexpr int COMPUTE = 4 * WF, LOADERS = 4;                            // waves
     constexpr int BTOK = 16 * MB, BF = 64 * WF, BK = 128;
     constexpr int X_STAGE = BTOK * BK * 2, W_STAGE = BF * BK, W_AT = S * X_STAGE;
     constexpr int XI = MB, WI = BF / 8 / LOADERS, LOADS = XI + WI;          // a loading wave's instructions (a KiB each) per stage
-    constexpr int RS = BF + 4;                                              // floats per token row of the partial sums in LDS
-    constexpr int SUM_BYTES = 4 * 32 * RS * 4, STAGE_BYTES = W_AT + (S + 1) * W_STAGE;
+    constexpr int RS = BF + 4;                                              // floats per token row of the sums in LDS
+    constexpr int SUM_BYTES = BTOK * RS * 4, STAGE_BYTES = W_AT + (S + 1) * W_STAGE;
     constexpr int LDS_BYTES = STAGE_BYTES > SUM_BYTES ? STAGE_BYTES : SUM_BYTES;
     static_assert(S >= 3 && S <= 5 && LDS_BYTES * (3 - WF) <= 160 * 1024, "64-feature tiles: two workgroups on a CU");
     __shared__ __align__(1024) uint8_t lds[LDS_BYTES];
@@ -171,99 +170,81 @@ __global__ __launch_bounds__(256 + 256 * WF, WF == 2 ? 3 : 4) void gemm_staged_k
         return;                                                             // a wave that has ended no longer counts in the barriers below
     }
 
-    // ---- computing waves: k group kg of features 64 wf .. + 63
-    const int kg = wave & 3, wf = wave >> 2;
+    // ---- computing waves: features 16 wave .. + 15 of the tile
     const int i16 = lane & 15, g = lane >> 4;
-    f32x4 acc[MB][NB];
+    const float scale = wave * 16 >= width ? a.w_scale_pair : a.w_scale;
+    f32x4 acc[MB];
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++)
+    for (int mb = 0; mb < MB; mb++) { acc[mb] = f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }; }
+    int x_lane[4], w_lane[2];                                               // per instruction / k-tile of a stage
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) { acc[mb][nb] = f32x4{ 0.0f, 0.0f, 0.0f, 0.0f }; }
-    const int x_lane = i16 * 256 + swizzled_chunk_n<16>(i16, 8 * (kg >> 1) + 2 * g + (kg & 1)) * 16;
-    const int w_lane = W_AT + wf * 8192 + 8 * (kg & 1) + (TILED ? (kg >> 1) * 1024 + lane * 16 : i16 * 128 + swizzled_chunk_n<8>(i16, 4 * (kg >> 1) + g) * 16);
-    u32x2 raw[NB];
-    u32x4 wfr[NB];
-    auto read_codes = [&](int buf) {
+    for (int s = 0; s < 4; s++) { x_lane[s] = i16 * 256 + swizzled_chunk_n<16>(i16, 8 * (s >> 1) + 2 * g + (s & 1)) * 16; }
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) { raw[nb] = *(const u32x2*)(lds + buf * W_STAGE + w_lane + nb * 2048); }
-    };
-    auto convert = [&] {
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++)
-        {
-            const float scale = wf * 64 + nb * 16 >= width ? a.w_scale_pair : a.w_scale;
-            typename ActPair<AT>::type p0, p1, p2, p3;
-            fp8x4_to_pairs<WT, SCALED, AT>(raw[nb][0], scale, p0, p1);
-            fp8x4_to_pairs<WT, SCALED, AT>(raw[nb][1], scale, p2, p3);
-            wfr[nb] = u32x4{ __builtin_bit_cast(uint32_t, p0), __builtin_bit_cast(uint32_t, p1), __builtin_bit_cast(uint32_t, p2), __builtin_bit_cast(uint32_t, p3) };
-        }
-    };
-    int xbuf = 0, wbuf = 1;
+    for (int h = 0; h < 2; h++) { w_lane[h] = W_AT + wave * 2048 + (TILED ? h * 1024 + lane * 16 : i16 * 128 + swizzled_chunk_n<8>(i16, 4 * h + g) * 16); }
+    u32x4 raw, wfr[4];                                                      // codes of a k-tile; weight operands of a stage
+    auto read_codes = [&](int buf, int h) { raw = *(const u32x4*)(lds + buf * W_STAGE + w_lane[h]); };
+    auto convert = [&](int h) { dequant16_fp8<WT, SCALED, AT>(raw, scale, wfr[2 * h], wfr[2 * h + 1]); };
+    int xbuf = 0, wbuf = 0;
     for (int st = 0; st < n_st; st++)
     {
         asm volatile("s_barrier" : : : "memory");                           // activations of stage st, codes of stage st + 1
-        // K % 128 == 64: the last stage's second half is past the end, and its groups are done.  (A product with zeros instead would make
-        // NaN of an infinity among the activations that were read in its place.)
-        if (((st_begin + st) * 2 + (kg >> 1)) * 64 >= a.K) { break; }
-        const uint8_t* const xp = lds + xbuf * X_STAGE + x_lane;
-        constexpr int AHEAD = MB < 3 ? MB : 3;                              // fragment reads run ahead of the matrix-core instructions that use them
+        // Fragment f: token block f % MB of instruction f / MB.  Reads run ahead of the matrix-core instructions that use them (by 3 or 4: level;
+        // 6: 1 to 2 % slower, 12: 2 to 5 %).
+        constexpr int FRAGS = 4 * MB, AHEAD = 4;
+        const uint8_t* const xp = lds + xbuf * X_STAGE;
+        auto read_frag = [&](int f) { return *(const u32x4*)(xp + x_lane[f / MB] + f % MB * 4096); };
         u32x4 ring[AHEAD + 1];
 #pragma unroll
-        for (int f = 0; f < AHEAD; f++) { ring[f] = *(const u32x4*)(xp + f * 4096); }
+        for (int f = 0; f < AHEAD; f++) { ring[f] = read_frag(f); }
         if (st == 0)
         {
-            read_codes(0);
-            convert();
+            read_codes(0, 0);
+            convert(0);
         }
+        read_codes(wbuf, 1);
+        wbuf = wbuf == S ? 0 : wbuf + 1;
+        auto products = [&](int f0, int f1) {
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++)
-        {
-            __builtin_amdgcn_sched_barrier(0);
-            if (mb + AHEAD < MB) { ring[(mb + AHEAD) % (AHEAD + 1)] = *(const u32x4*)(xp + (mb + AHEAD) * 4096); }
-            if (mb == MB / 2) { read_codes(wbuf); }                         // (behind the last stage: what is left in LDS, and not used)
-            const frag_t xf = __builtin_bit_cast(frag_t, ring[mb % (AHEAD + 1)]);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
+            for (int f = f0; f < f1; f++)
             {
-                const frag_t w = __builtin_bit_cast(frag_t, wfr[nb]);
-                if constexpr (AT == DT_HALF) { acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xf, acc[mb][nb], 0, 0, 0); }
-                else { acc[mb][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, xf, acc[mb][nb], 0, 0, 0); }
+                __builtin_amdgcn_sched_barrier(0);
+                if (f + AHEAD < FRAGS) { ring[(f + AHEAD) % (AHEAD + 1)] = read_frag(f + AHEAD); }
+                const frag_t xf = __builtin_bit_cast(frag_t, ring[f % (AHEAD + 1)]), w = __builtin_bit_cast(frag_t, wfr[f / MB]);
+                if constexpr (AT == DT_HALF) { acc[f % MB] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xf, acc[f % MB], 0, 0, 0); }
+                else { acc[f % MB] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, xf, acc[f % MB], 0, 0, 0); }
+                // behind the first instruction of a k-tile: the codes of the k-tile after it
+                if (f == MB - 1)
+                {
+                    convert(1);
+                    read_codes(wbuf, 0);                                    // (behind the last stage: what is left in LDS, and not used)
+                }
+                if (f == 3 * MB - 1) { convert(0); }
             }
-        }
-        convert();
+        };
+        products(0, 2 * MB);
+        // K % 128 == 64: the last stage has one k-tile.  (A product of the activations read in the other's place with zeros would
+        // make NaN of an infinity among them.)
+        if ((st_begin + st) * BK + 64 >= a.K) { break; }
+        products(2 * MB, FRAGS);
         __builtin_amdgcn_sched_barrier(0);
         xbuf = xbuf == S - 1 ? 0 : xbuf + 1;
-        wbuf = wbuf == S ? 0 : wbuf + 1;
     }
 
-    // ---- the k groups' sums, 32 tokens at a time; a thread then owns 8 consecutive features of a token (a pair: 4 outputs)
+    // ---- through LDS to rows: a thread owns 8 consecutive features of a token (a pair: 4 outputs)
     float* const sums = (float*)lds;
     const int s_tok = tid / (BF / 8), s_f = tid % (BF / 8);
     const int f0 = pair ? s_f * 4 : s_f * 8, f1 = pair ? f0 + width : f0 + 4;
     const int out = out_base + f0;
+    __syncthreads();
+#pragma unroll
+    for (int mb = 0; mb < MB; mb++) { *(f32x4*)(sums + (mb * 16 + i16) * RS + wave * 16 + 4 * g) = acc[mb]; }
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < (MB + 1) / 2; c++)
     {
-        __syncthreads();
-#pragma unroll
-        for (int m = 0; m < 2; m++)
-        {
-            if (2 * c + m < MB)
-            {
-#pragma unroll
-                for (int nb = 0; nb < NB; nb++) { *(f32x4*)(sums + (kg * 32 + m * 16 + i16) * RS + wf * 64 + nb * 16 + 4 * g) = acc[2 * c + m][nb]; }
-            }
-        }
-        __syncthreads();
         const int tok = tok_base + c * 32 + s_tok;
         if (tok >= a.tokens || c * 32 + s_tok >= BTOK || out >= a.n_out) { continue; }
-        f32x4 r0 = *(const f32x4*)(sums + s_tok * RS + f0), r1 = *(const f32x4*)(sums + s_tok * RS + f1);
-#pragma unroll
-        for (int q = 1; q < 4; q++)
-        {
-            r0 += *(const f32x4*)(sums + (q * 32 + s_tok) * RS + f0);
-            r1 += *(const f32x4*)(sums + (q * 32 + s_tok) * RS + f1);
-        }
+        const f32x4 r0 = *(const f32x4*)(sums + (c * 32 + s_tok) * RS + f0), r1 = *(const f32x4*)(sums + (c * 32 + s_tok) * RS + f1);
         if (partial)
         {
             // n_out is a multiple of 4 on this path; pair: the up weight's sums are a second set behind all of the gate weight's

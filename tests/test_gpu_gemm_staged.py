@@ -218,3 +218,59 @@ def test_infinities_at_the_end_of_a_row(gpu, oracle, layout, half):
             assert (diff.norm(dim=1) <= ROW_L2_REL * want[finite].norm(dim=1)).all(), (tokens, n_out, K)
         finally:
             weight.release()
+
+
+def test_no_plan_of_one_k_range_is_split():
+    """A launch whose k range plan_gemm leaves whole keeps it whole on the staged kernel."""
+    for layout in ("file", "tiled", "file_scaled", "tiled_scaled"):
+        for kind in (LINEAR, PAIR, SEGMENTS):
+            for tokens in (17, 24, 48, 80, 112, 200, 301, 512):
+                for n_out in (72, 1032, 2048, 6144, 12288, 16384):
+                    for K in (1024, 2112, 4096, 8192, 12288):
+                        p = plan(layout, kind, tokens, widths_of(n_out) if kind == SEGMENTS else [n_out], K)
+                        assert p[4] > 1 or p[2] == 1, (layout, kind, tokens, n_out, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["file", "tiled", "file_scaled", "tiled_scaled"])
+def test_fused_launches_give_the_bits_of_the_separate_calls(gpu, oracle, layout):
+    """Where neither splits k, a gate / up pair has the bits of its two linears and their product and a joint launch those of its linears,
+    also where only one of the two is the staged kernel (several of the shapes below); K a whole number of stages and half a stage more."""
+    torch, dev, lib = gpu
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    compared = mixed = 0
+    for tokens, n_out, K in ((17, 12288, 2048), (20, 4096, 1088), (32, 4096, 1024), (48, 3072, 1024), (88, 4096, 1088), (100, 8192, 2112), (128, 12288, 4096), (160, 8192, 1024), (200, 12288, 1024), (400, 2048, 1088), (512, 2048, 2112)):
+        print(layout, tokens, n_out, K, flush=True)
+        gen = torch.Generator(device=dev).manual_seed(tokens + n_out + K)
+        x = (torch.randn(tokens, K, device=dev, generator=gen) * 0.05).to(torch.bfloat16)
+        for kind, widths in ((PAIR, [n_out] * 2), (SEGMENTS, widths_of(n_out))):
+            fused = plan(layout, kind, tokens, widths, K)
+            alone = [plan(layout, LINEAR, tokens, [n], K) for n in widths]
+            if fused[2] > 1 or all(p[2] > 1 for p in alone): continue
+            weights = [Weight(gpu, oracle, layout, n, K, gen) for n in widths]
+            w0 = weights[0]
+            try:
+                single = [torch.zeros(tokens, n, dtype=torch.bfloat16, device=dev) for n in widths]
+                joint = [torch.zeros_like(s) for s in (single[:1] if kind == PAIR else single)]
+                torch.cuda.synchronize()
+                for w, s, n in zip(weights, single, widths): assert lib.linear(w.codes.data_ptr(), w.type, x.data_ptr(), s.data_ptr(), n, tokens, K, w.scale) == 0
+                if kind == PAIR:
+                    product = torch.zeros_like(single[0])
+                    assert lib.c.hip_swiglu_bf16(ptr(single[0]), ptr(single[1]), ptr(product), ctypes.c_ulonglong(product.numel())) == 0
+                    single = [product]
+                    rc = lib.c.hip_quant_gemm_swiglu(n_out, tokens, K, ptr(w0.codes), ptr(weights[1].codes), w0.type, K, ctypes.c_float(w0.scale), ctypes.c_float(w0.scale),
+                                                     ptr(x), K, ptr(joint[0]), n_out)
+                else:
+                    n = (ctypes.c_int * 3)(*widths)
+                    rc = lib.c.hip_quant_gemm_segments(3, n, (ctypes.c_void_p * 3)(*(w.codes.data_ptr() for w in weights)), (ctypes.c_float * 3)(*[w0.scale] * 3),
+                                                       (ctypes.c_void_p * 3)(*(o.data_ptr() for o in joint)), n, w0.type, tokens, K, K, ptr(x), K)
+                assert rc == 0
+                torch.cuda.synchronize()
+                for s, j, p in zip(single, joint, alone):
+                    if p[2] > 1: continue
+                    compared += 1
+                    mixed += p[3] != fused[3]
+                    assert torch.equal(s.view(torch.int16), j.view(torch.int16)), (kind, tokens, n_out, K, fused, alone)
+            finally:
+                for w in weights: w.release()
+    assert compared >= 12 and mixed >= 4
