@@ -14,7 +14,7 @@ inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // Key ranges of a prompt's attention.  In one piece a workgroup takes 5 us and 1.75 per block of 64 keys; in n ranges the three launches
 // take 16 us, 1.75 per block of one range, and 0.25 per MB of FP32 sums written and read.  At most one workgroup per CU (two take as long
 // as one after the other: 64 tokens of 32 / 8 heads behind 4000: 34.5 us with 8 ranges, 43.9 with 12; 300 tokens behind 1000, 152 workgroups:
-// 45.6 in one piece, 50.4 in two ranges), and 10 % to gain at least.  Measured on MI355X, one piece -> ranges: those 64 tokens 121 -> 34.5 us,
+// 45.6 in one piece, 50.4 in two ranges), and 10 % to gain at least.  One piece without scratch memory, as under graph capture.  Measured on MI355X, one piece -> ranges: those 64 tokens 121 -> 34.5 us,
 // 64 tokens of 4 / 1 heads behind 14000 424 -> 34, 200 tokens of 32 / 8 behind 2000 70 -> 51, 2 tokens of one head behind 16000 353 -> 23.
 struct AttentionRanges
 {
@@ -63,7 +63,9 @@ int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v
     const float scale = 1.0f / sqrtf(128.0f);
     const size_t outputs = (size_t)n_tokens * n_q_heads;
     const AttentionRanges split = attention_ranges(tiles, pos0 + n_tokens, outputs);
-    char* const scratch = split.n > 1 ? (char*)workspace((size_t)split.n * outputs * (128 * sizeof(float) + sizeof(float2))) : nullptr;
+    // ranges x tiles is at most the number of CUs, and a tile is 16 tokens of at most four heads
+    constexpr size_t ROW = 128 * sizeof(float) + sizeof(float2);
+    char* const scratch = split.n > 1 ? (char*)fixed_scratch((size_t)cu_count() * 16 * 4 * ROW) : nullptr;
     const PrefillRanges ranges = { split.per, (float2*)(scratch + (size_t)split.n * outputs * 128 * sizeof(float)), (float*)scratch };
     const dim3 grid((unsigned)tiles, scratch ? split.n : 1);
 #define CCQ_ATTN_PREFILL(G, PASS)                                                                                                                  \

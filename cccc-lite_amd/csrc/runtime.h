@@ -24,6 +24,11 @@ int cu_count();
 // have to grow while the stream is being captured into a graph); callers then take a path that needs none.
 void* workspace(size_t bytes);
 
+// Device scratch memory of `bytes`, the same number in every call on a device: allocated by the first call of a (host thread, device,
+// stream), never replaced or freed after that.  nullptr when it cannot be allocated and always while the stream is being captured: a
+// graph that held the buffer could be replayed on a stream of its own, beside launches that use it.
+void* fixed_scratch(size_t bytes);
+
 // Where a k-split GEMM keeps its FP32 partial sums.  Default (no SplitScratch, or strict == false): workspace()
 // above.  strict: the fixed buffer and nothing else, so nothing is ever allocated -- a request beyond
 // fixed_bytes (or with no buffer at all) is recorded in `refused` and the caller reports an error instead of

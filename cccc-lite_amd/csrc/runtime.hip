@@ -78,6 +78,25 @@ void* workspace(size_t bytes)
     return p;
 }
 
+void* fixed_scratch(size_t bytes)
+{
+    static thread_local std::map<std::pair<int, hipStream_t>, void*> buffers;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    int dev = 0;
+    if (hipStreamIsCapturing(stream(), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone || hipGetDevice(&dev) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    void*& p = buffers[{ dev, stream() }];
+    if (!p && hipMalloc(&p, bytes) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+    return p;
+}
+
 }    // namespace ccq
 
 int hip_quant_set_sync(int enabled)

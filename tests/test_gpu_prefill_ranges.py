@@ -62,39 +62,52 @@ def test_context_of_up_to_four_blocks_and_its_neighbours(gpu, oracle, dec, n_q, 
         assert np.linalg.norm(dec.f(got[t]) - want) <= 4e-3 * np.linalg.norm(want), t
 
 
-def test_ranges_under_capture(gpu, oracle, dec):
-    """A captured call whose scratch an eager call has sized replays the eager result, with eager work of another size in between; one
-    on a stream without scratch runs in one piece, within the bounds."""
+def test_no_ranges_under_capture(gpu, oracle, dec):
+    """A captured call runs in one piece, within the bounds of an eager one, whether or not the stream has scratch memory, and no graph holds
+    memory of the library: replays keep their bits behind eager calls of other sizes and a grown GEMM workspace, and two graphs of one
+    stream replay side by side on two streams."""
     torch, dev, lib = gpu
     n_q, n_kv, T, pos0, t_kv = 4, 1, 20, 1500, 1600
-    q, kc, vc = inputs(oracle, n_q, n_kv, T, pos0, t_kv)
-    qd, kd, vd = to_dev(torch, dev, q), to_dev(torch, dev, kc), to_dev(torch, dev, vc)
-    call = lambda y, T=T, pos0=pos0: lib.c.hip_attention_prefill_bf16(ptr(qd), ptr(kd), ptr(vd), ptr(y), n_q, n_kv, 128, t_kv, T, pos0)
-    eager, other, replayed, whole = (torch.zeros(T * n_q * 128, dtype=torch.int16, device=dev) for _ in range(4))
+    sets = [[to_dev(torch, dev, a) for a in inputs(oracle, n_q, n_kv, T, pos0 + i, t_kv)] for i in (0, 1)]
+    call = lambda i, y, T=T, pos0=pos0: lib.c.hip_attention_prefill_bf16(*(ptr(t) for t in sets[i]), ptr(y), n_q, n_kv, 128, t_kv, T, pos0)
+    eager, other, *captured = (torch.zeros(T * n_q * 128, dtype=torch.int16, device=dev) for _ in range(5))
     lib.set_sync(False)
     try:
-        for first, out in ((True, replayed), (False, whole)):
-            stream = torch.cuda.Stream(device=dev)
+        graphs, streams = [], [torch.cuda.Stream(device=dev) for _ in range(2)]
+        for stream, i, out, first in ((streams[0], 0, captured[0], True), (streams[0], 1, captured[1], True), (streams[1], 0, captured[2], False)):
             assert lib.set_stream(stream.cuda_stream) == 0
             if first:
-                assert call(eager) == 0
+                assert call(0, eager) == 0
                 stream.synchronize()
-            graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph, stream=stream):
-                assert call(out) == 0
-            for _ in range(3):
-                out.zero_()
-                torch.cuda.synchronize()
-                graph.replay()
-                torch.cuda.synchronize()
-                if first:
-                    assert torch.equal(out, eager)
-                    assert call(other, T=9, pos0=1200) == 0
-                    stream.synchronize()
-                else:
-                    a, b = dec.f(from_dev(out, np.uint16)), dec.f(from_dev(eager, np.uint16))
-                    assert np.linalg.norm(a - b) <= 4e-3 * np.linalg.norm(b)
-            del graph
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[-1], stream=stream):
+                assert call(i, out) == 0
+        a, b = (dec.f(from_dev(t, np.uint16)) for t in (eager, captured[0]))      # not yet replayed
+        assert not b.any()
+        want = None
+        for replay in range(3):
+            for out in captured: out.zero_()
+            torch.cuda.synchronize()
+            for graph, stream in zip(graphs[:2], streams):
+                with torch.cuda.stream(stream): graph.replay()
+            torch.cuda.synchronize()
+            graphs[2].replay()
+            torch.cuda.synchronize()
+            if want is None:
+                want = [out.clone() for out in captured]
+                b = dec.f(from_dev(want[0], np.uint16))
+                assert np.linalg.norm(a - b) <= 4e-3 * np.linalg.norm(a)
+                assert torch.equal(want[0], want[2]) and not torch.equal(want[0], want[1])
+            assert all(torch.equal(w, out) for w, out in zip(want, captured)), replay
+            assert lib.set_stream(streams[0].cuda_stream) == 0
+            assert call(0, other, T=9, pos0=1200) == 0
+            assert lib.workspace_reserve((1 << 24) << replay) == 0
+            streams[0].synchronize()
+            assert call(0, other) == 0
+            streams[0].synchronize()
+            assert torch.equal(other, eager)
+            other.zero_()
+        del graphs
     finally:
         lib.set_stream(None)
         lib.set_sync(True)
