@@ -575,6 +575,7 @@ double DecodeModel::run(int n_steps, int use_graph)
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) { return -1.0; }
     double result = -1.0;
     const int sync_before = hip_quant_set_sync(0);
+    const hipStream_t caller = (hipStream_t)hip_quant_get_stream();
     // A stream, a capture and an executable graph cost the host 0.25 ms (4 layers) to 0.75 ms (36), a replayed launch is up to 0.25 us faster
     // than a launched one (36 layers: 1.83 against 1.89 ms per step; 4 to 8 layers: nearly level), so a graph pays from 10 steps of 36
     // layers on and hardly ever for 4; the host records it while the first two steps run.  Wall time with a graph recorded first and
@@ -607,7 +608,7 @@ double DecodeModel::run(int n_steps, int use_graph)
                 ok = (hipStreamEndCapture(stream, &graph) == hipSuccess) && ok;
             }
         }
-        hip_quant_set_stream(nullptr);
+        hip_quant_set_stream(caller);
         if (ok) { ok = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess; }
         if (ok)
         {
@@ -629,9 +630,9 @@ double DecodeModel::run(int n_steps, int use_graph)
     else
     {
         bool ok = true;
-        (void)hipEventRecord(e0, nullptr);
+        (void)hipEventRecord(e0, caller);
         for (int s = 0; s < n_steps; s++) { ok = (step() == 0) && ok; }
-        (void)hipEventRecord(e1, nullptr);
+        (void)hipEventRecord(e1, caller);
         ok = (hipEventSynchronize(e1) == hipSuccess) && ok;
         if (ok)
         {

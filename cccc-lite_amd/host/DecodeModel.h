@@ -100,7 +100,8 @@ public:
     // on from there.  Prompts longer than 2048 tokens go through in pieces of 2048.  0 ok, -1 bad arguments.
     int prefill(const int* tokens, int n_tokens, int pos0);
     // Runs n steps; use_graph: where n is large enough to pay for it, capture one step and replay it behind the first two.  Returns elapsed ms
-    // (events on the launch stream) or < 0.
+    // (events on the stream of the launches: the caller's, or the graph's own) or < 0; the steps are done when it returns and the caller's
+    // stream is the launch stream again.
     double run(int n_steps, int use_graph);
     int currentToken();                     // blocking 4-byte read
     int currentPos();
