@@ -581,9 +581,9 @@ double DecodeModel::run(int n_steps, int use_graph)
     // layers on and hardly ever for 4; the host records it while the first two steps run.  Wall time with a graph recorded first and
     // replayed / all launched / now: 8 steps of 36 layers 15.27 / 15.11 / 15.11 ms, 16 steps 30.03 / 30.19 / 29.79, 20 steps 37.36 /
     // 37.75 / 37.00; 16 steps of 4 layers 2.40 / 2.12 / 2.12, 20 of 8 layers 4.52 / 4.20 / 4.20.
-    constexpr int LAUNCHED = 2;
     constexpr long long FEWEST = 360;           // steps x layers
-    const bool pays = (long long)n_steps * cfg_.layers >= FEWEST && n_steps > LAUNCHED;
+    const int launched = use_graph == GRAPH_ALWAYS ? 0 : 2;
+    const bool pays = use_graph == GRAPH_ALWAYS || ((long long)n_steps * cfg_.layers >= FEWEST && n_steps > launched);
     if (use_graph && pays)
     {
         hipStream_t stream = nullptr;
@@ -598,7 +598,7 @@ double DecodeModel::run(int n_steps, int use_graph)
         hip_quant_set_stream(stream);
         (void)hipEventRecord(e0, stream);
         bool ok = true;
-        for (int s = 0; s < LAUNCHED; s++) { ok = (step() == 0) && ok; }
+        for (int s = 0; s < launched; s++) { ok = (step() == 0) && ok; }
         if (ok)
         {
             ok = hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal) == hipSuccess;
@@ -612,7 +612,7 @@ double DecodeModel::run(int n_steps, int use_graph)
         if (ok) { ok = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess; }
         if (ok)
         {
-            for (int s = LAUNCHED; s < n_steps; s++) { ok = (hipGraphLaunch(exec, stream) == hipSuccess) && ok; }
+            for (int s = launched; s < n_steps; s++) { ok = (hipGraphLaunch(exec, stream) == hipSuccess) && ok; }
             (void)hipEventRecord(e1, stream);
             ok = (hipEventSynchronize(e1) == hipSuccess) && ok;
         }

@@ -99,9 +99,11 @@ public:
     // the prompt, the current token is the greedy pick after its last token and the position is pos0 + n: step() carries
     // on from there.  Prompts longer than 2048 tokens go through in pieces of 2048.  0 ok, -1 bad arguments.
     int prefill(const int* tokens, int n_tokens, int pos0);
-    // Runs n steps; use_graph: where n is large enough to pay for it, capture one step and replay it behind the first two.  Returns elapsed ms
+    // Runs n steps; use_graph: where n is large enough to pay for it, capture one step and replay it behind the first two (GRAPH_ALWAYS:
+    // whatever n is, capture the first and replay it for all).  Returns elapsed ms
     // (events on the stream of the launches: the caller's, or the graph's own) or < 0; the steps are done when it returns and the caller's
     // stream is the launch stream again.
+    static constexpr int GRAPH_ALWAYS = 2;
     double run(int n_steps, int use_graph);
     int currentToken();                     // blocking 4-byte read
     int currentPos();

@@ -354,8 +354,11 @@ class DecodeModel:
             raise RuntimeError(f"decode step failed: {rc}")
         return self.token
 
-    def run(self, n_steps: int, use_graph: bool) -> float:
-        ms = float(self.lib.c.cccc_decode_run(self.handle, n_steps, 1 if use_graph else 0))
+    GRAPH_ALWAYS = 2
+
+    def run(self, n_steps: int, use_graph: bool | int) -> float:
+        """Elapsed ms of n greedy steps; use_graph: a captured step replayed where n pays for it (GRAPH_ALWAYS: whatever n is)."""
+        ms = float(self.lib.c.cccc_decode_run(self.handle, n_steps, self.GRAPH_ALWAYS if use_graph == self.GRAPH_ALWAYS else 1 if use_graph else 0))
         if ms < 0:
             raise RuntimeError(f"decode run failed: {ms}")
         return ms

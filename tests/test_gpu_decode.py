@@ -437,7 +437,7 @@ def test_graph_replay_equals_eager_steps(small_model, dec):
         eager.append(model.step())
     logits_eager = model.logits().copy()
     model.reset(3, 0)
-    assert model.run(10, True) > 0                       # one captured step replayed ten times
+    assert model.run(10, model.GRAPH_ALWAYS) > 0         # one captured step replayed ten times
     assert model.pos == 10
     assert model.token == eager[-1]
     assert np.array_equal(model.logits(), logits_eager)
@@ -529,7 +529,7 @@ def test_decode_steps_with_fp4_linears_follow_the_oracle(gpu, pkg, oracle, dec):
     eager = [model.step() for _ in range(6)]
     logits_eager = model.logits().copy()
     model.reset(3, 0)
-    assert model.run(6, True) > 0 and model.token == eager[-1] and np.array_equal(model.logits(), logits_eager)
+    assert model.run(6, model.GRAPH_ALWAYS) > 0 and model.token == eager[-1] and np.array_equal(model.logits(), logits_eager)
 
 
 @pytest.mark.parametrize("n_q,n_kv,t_kv,normed", [(4, 2, 200, True), (8, 2, 300, True), (2, 2, 130, True), (8, 2, 300, False), (4, 2, 6000, True)])
@@ -677,7 +677,7 @@ def test_decode_steps_of_a_model_without_qk_norm(gpu, pkg, oracle, dec, fmt, exa
     eager = [model.step() for _ in range(6)]
     logits_eager = model.logits().copy()
     model.reset(3, 0)
-    assert model.run(6, True) > 0 and model.token == eager[-1] and np.array_equal(model.logits(), logits_eager)
+    assert model.run(6, model.GRAPH_ALWAYS) > 0 and model.token == eager[-1] and np.array_equal(model.logits(), logits_eager)
 
 
 @pytest.mark.parametrize("K,n_out", [(2048, 512), (1520, 37), (272, 70000), (4096, 1000)])
@@ -763,7 +763,7 @@ def test_decode_steps_with_tied_embeddings(gpu, pkg, oracle, dec):
     eager = [model.step() for _ in range(6)]
     logits_eager = model.logits().copy()
     model.reset(3, 0)
-    assert model.run(6, True) > 0 and model.token == eager[-1] and np.array_equal(model.logits(), logits_eager)
+    assert model.run(6, model.GRAPH_ALWAYS) > 0 and model.token == eager[-1] and np.array_equal(model.logits(), logits_eager)
     # an untied head of the same values quantized to FP8 answers differently: the tied route really reads the BF16 table
     untied = dict(weights)
     untied["lm_head"] = oracle.encode_e5m2_rne(dec.f(weights["emb"]))

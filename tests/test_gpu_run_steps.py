@@ -21,7 +21,7 @@ def test_launched_and_replayed_steps_equal_single_steps(gpu, pkg, dec, steps):
         single.reset(first, 2)
         for _ in range(steps):
             token = single.step()
-        for use_graph in (True, False):
+        for use_graph in (True, False, run.GRAPH_ALWAYS):
             run.reset(first, 2)
             assert run.run(steps, use_graph) > 0
             assert run.pos == single.pos == 2 + steps and run.token == token
@@ -46,7 +46,7 @@ def test_runs_on_the_callers_stream(gpu, pkg, dec, steps):
         assert lib.set_stream(stream.cuda_stream) == 0
         model.reset(3, 2)
         model.run(steps, True)                                # kernels loaded
-        for use_graph in (True, False):
+        for use_graph in (True, False, model.GRAPH_ALWAYS):
             model.reset(3, 2)
             torch.cuda.synchronize()
             begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
