@@ -621,7 +621,7 @@ static __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(const 
                 if (r0 + r < n_ranges) { sum += part[r]; }
             }
         }
-        *(uint2*)(y + i * 4) = uint2{ f32_to_bf16_bits(sum[0]) | (f32_to_bf16_bits(sum[1]) << 16), f32_to_bf16_bits(sum[2]) | (f32_to_bf16_bits(sum[3]) << 16) };
+        *(u32x2_any*)(y + i * 4) = u32x2{ f32_to_bf16_bits(sum[0]) | (f32_to_bf16_bits(sum[1]) << 16), f32_to_bf16_bits(sum[2]) | (f32_to_bf16_bits(sum[3]) << 16) };      // y may lie on any element
     }
 }
 
