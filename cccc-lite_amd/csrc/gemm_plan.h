@@ -262,27 +262,6 @@ constexpr GemmTile kStagedTiles[] = {
     { 7, 2, 2.5, 5.0, { 0.361, 0.381, 0.462, 0.460 }, { 0.356, 0.360, 0.426, 0.434 } },
 };
 
-// What `plan` takes by its estimate, and the row kernel that an unsplit linear of at most 4096 features may have behind it
-// (the residual add and the norm, see plan_gemm).
-struct StagedRival
-{
-    double us, row_kernel;
-
-    StagedRival(const LinearArgs& a, GemmKind kind, const GemmWeights& w, int cus, const GemmPlan& plan)
-    {
-        const bool deep = plan.small || (plan.splits > 1 && plan.mb <= 4), add_norm = kind == GEMM_LINEAR && plan.ranges > 1 && a.n_out <= 4096 && a.n_out % 8 == 0;
-        const GemmTile* const table = deep ? kSmallTiles : kLargeTiles;
-        const int n_table = deep ? sizeof(kSmallTiles) / sizeof(GemmTile) : sizeof(kLargeTiles) / sizeof(GemmTile);
-        us = 0.0;
-        row_kernel = add_norm ? 3.0 + 0.55 * 2e-6 * (double)a.tokens * a.n_out : 0.0;
-        for (int i = 0; i < n_table; i++)
-        {
-            if (table[i].mb == plan.mb && table[i].nb == plan.nb) { us = estimate_us(a, kind, table[i], w, plan.splits, cus); }
-        }
-        if (plan.splits == 1) { us += row_kernel; }
-    }
-};
-
 // The staged kernel in the place of `plan` from K = 1024 on (the shortest that the estimate is fitted to) and up to 512 tokens (above that
 // the larger tiles are level or ahead).
 // It adds the products in the order of the register-fed kernels, so only the k ranges of a launch show in its bits.  A plan of one
