@@ -182,28 +182,58 @@ constexpr GemmTile kLargeTilesFp4[] = {
     { 8, 4, 7.3, 2.1, { 0.913 }, { 0.873 } },
 };
 
-inline double estimate_us(const LinearArgs& a, GemmKind kind, const GemmTile& t, const GemmWeights& w, int splits, int cus, double alone = 0.85)
+// What the estimate takes from the launch and from a tile on it, worked out once: a call asks for 20 to 200 estimates (0.7 us of host time
+// for plan_gemm and staged_plan together, 1.0 with every estimate from scratch).
+struct LaunchShape
 {
-    const int width = kind == GEMM_PAIR ? 32 * t.nb : 64 * t.nb, column = w.fp4 ? 0 : (w.scaled ? 2 : 0) + (w.row_major ? 1 : 0);
-    long long features = a.n_out, n_tiles = (a.n_out + width - 1) / width;
-    if (kind == GEMM_SEGMENTS)
+    const LinearArgs& a;
+    GemmKind kind;
+    int cus, column;
+    double outputs, traffic_us, partial_us;       // MB of output elements; bytes; FP32 sums, per k range
+
+    LaunchShape(const LinearArgs& args, GemmKind k, const GemmWeights& w, int n_cus) : a(args), kind(k), cus(n_cus), column(w.fp4 ? 0 : (w.scaled ? 2 : 0) + (w.row_major ? 1 : 0))
     {
-        features = n_tiles = 0;
-        for (int s = 0; s < a.n_segments; s++)
+        long long features = a.n_out;
+        if (kind == GEMM_SEGMENTS)
         {
-            features += a.seg_n_out[s];
-            n_tiles += (a.seg_n_out[s] + width - 1) / width;
+            features = 0;
+            for (int s = 0; s < a.n_segments; s++) { features += a.seg_n_out[s]; }
         }
+        const double two = kind == GEMM_PAIR ? 2.0 : 1.0;
+        outputs = 1e-6 * (double)a.tokens * (double)features;
+        traffic_us = (1e-6 * two * (double)features * a.K * (w.fp4 ? 0.5625 : 1.0) + 2.0 * outputs) / (w.fp4 ? 4.1 : 5.0);
+        partial_us = 0.2 + 0.3 * 4.0 * two * outputs;
     }
-    const double two = kind == GEMM_PAIR ? 2.0 : 1.0, outputs = 1e-6 * (double)a.tokens * (double)features;
-    const double fill = 8.0 * (double)((n_tiles + 7) / 8 * ((a.tokens + 16 * t.mb - 1) / (16 * t.mb)) * splits) / cus;
-    const double per_cu = fill <= 1.0 ? 1.0 : 0.1 * fill + 0.9 * ceil(fill);
-    const double k_tile = fill <= 1.0 ? t.one[column] * (alone + (1.0 - alone) * fill) : std::max(t.one[column], t.each[column] * per_cu);
-    const double traffic = 1e-6 * two * (double)features * a.K * (w.fp4 ? 0.5625 : 1.0) + 2.0 * outputs;
-    double us = t.fixed + t.per_cu * per_cu + std::max((double)((a.K / 64 + splits - 1) / splits) * k_tile, traffic / (w.fp4 ? 4.1 : 5.0));
-    if (splits > 1) { us += 2.0 + 0.2 * splits + 0.3 * 4.0 * splits * two * outputs; }
-    return us;
-}
+};
+
+struct TileEstimate
+{
+    const LaunchShape& launch;
+    const GemmTile& t;
+    long long workgroups;       // of the fullest XCD, times eight
+
+    TileEstimate(const LaunchShape& l, const GemmTile& tile) : launch(l), t(tile)
+    {
+        const int width = l.kind == GEMM_PAIR ? 32 * t.nb : 64 * t.nb;
+        int n_tiles = 0;
+        if (l.kind != GEMM_SEGMENTS) { n_tiles = (l.a.n_out + width - 1) / width; }
+        else
+        {
+            for (int s = 0; s < l.a.n_segments; s++) { n_tiles += (l.a.seg_n_out[s] + width - 1) / width; }
+        }
+        workgroups = (n_tiles + 7LL) / 8 * 8 * ((l.a.tokens + 16 * t.mb - 1) / (16 * t.mb));
+    }
+
+    double us(int splits, double alone = 0.85) const
+    {
+        const double fill = (double)(workgroups * splits) / launch.cus;
+        const double per_cu = fill <= 1.0 ? 1.0 : 0.1 * fill + 0.9 * (double)((workgroups * splits + launch.cus - 1) / launch.cus);
+        const double one = t.one[launch.column];
+        const double k_tile = fill <= 1.0 ? one * (alone + (1.0 - alone) * fill) : std::max(one, t.each[launch.column] * per_cu);
+        const double time = t.fixed + t.per_cu * per_cu + std::max((double)((launch.a.K / 64 + splits - 1) / splits) * k_tile, launch.traffic_us);
+        return splits > 1 ? time + 2.0 + splits * launch.partial_us : time;
+    }
+};
 
 // The larger tile, or the small one with the least estimate if that is 6 % or more below.  Of 4357 measured cases 20 then take
 // more than 3 % longer than on the larger tile alone (6 % at most), and the mean is 0.79 of its time; of 5785 calls of a later
@@ -224,10 +254,11 @@ inline GemmPlan plan_gemm(const LinearArgs& a, GemmKind kind, const GemmWeights&
     const bool deep = !w.fp4 && plan.splits > 1 && plan.mb <= 4;      // the larger tiles that take their weights three k-tiles ahead as well
     const GemmTile* const large = w.fp4 ? kLargeTilesFp4 : deep ? kSmallTiles : kLargeTiles;
     const int n_large = w.fp4 ? sizeof(kLargeTilesFp4) / sizeof(GemmTile) : deep ? n_small : sizeof(kLargeTiles) / sizeof(GemmTile);
+    const LaunchShape launch(a, kind, w, cus);
     double limit = 0.0;
     for (int i = 0; i < n_large; i++)
     {
-        if (large[i].mb == plan.mb && large[i].nb == plan.nb) { limit = 0.94 * estimate_us(a, kind, large[i], w, plan.splits, cus); }
+        if (large[i].mb == plan.mb && large[i].nb == plan.nb) { limit = 0.94 * TileEstimate(launch, large[i]).us(plan.splits); }
     }
     const bool add_norm = kind == GEMM_LINEAR && plan.ranges > 1 && a.n_out <= 4096 && a.n_out % 8 == 0;
     const double row_kernel = add_norm ? 0.5 * (3.0 + 0.55 * 2e-6 * (double)a.tokens * a.n_out) : 0.0;
@@ -235,9 +266,10 @@ inline GemmPlan plan_gemm(const LinearArgs& a, GemmKind kind, const GemmWeights&
     {
         const GemmTile& t = small[i];
         if ((t.mb == 2 && (a.tokens > 64 || t.nb == 4)) || (t.mb == 8 && (a.tokens <= 64 || (!w.fp4 && (!w.row_major || w.scaled)))) || (kind == GEMM_PAIR && t.nb == 1)) { continue; }
-        for (int s = 1; s <= plan.ranges && (s == 1 || a.K / 64 / s >= 4); s++)
+        const TileEstimate tile(launch, t);
+        for (int s = 1; s <= plan.ranges && (s == 1 || a.K / 64 >= 4 * s); s++)
         {
-            double us = estimate_us(a, kind, t, w, s, cus);
+            double us = tile.us(s);
             if (s == 1) { us += std::min(row_kernel, 0.06 * us); }
             if (us < limit)
             {
@@ -282,12 +314,12 @@ inline GemmPlan staged_plan(const LinearArgs& a, GemmKind kind, const GemmWeight
     if (w.fp4 || a.K < 1024 || a.tokens > 512) { return plan; }
     const GemmWeights layouts[2] = { w, { false, !w.row_major, w.scaled } };
     const GemmPlan plans[2] = { plan, plan_gemm(a, kind, layouts[1], cus, scratch) };
+    const LaunchShape launches[2] = { { a, kind, layouts[0], cus }, { a, kind, layouts[1], cus } };
+    constexpr int MOST = 16;                    // k ranges of any plan
     const bool joint = plans[0].splits == plans[1].splits;
-    const int ranges = joint ? std::min(plan.ranges, plans[1].ranges) : plan.ranges;
+    const int ranges = plan.splits == 1 ? 1 : std::min(joint ? plans[1].ranges : MOST, std::min(plan.ranges, MOST));
     const bool add_norm = kind == GEMM_LINEAR && plan.ranges > 1 && a.n_out <= 4096 && a.n_out % 8 == 0;
     const double row_kernel = add_norm ? 3.0 + 0.55 * 2e-6 * (double)a.tokens * a.n_out : 0.0;
-    GemmPlan best = plan;
-    double least = 1e30;
     double limit[2] = { 0.0, 0.0 }, with_norm[2] = { 0.0, 0.0 };
     for (int l = 0; l < (joint ? 2 : 1); l++)
     {
@@ -299,38 +331,45 @@ inline GemmPlan staged_plan(const LinearArgs& a, GemmKind kind, const GemmWeight
         {
             if (table[i].mb == p.mb && table[i].nb == p.nb)
             {
-                const double us = estimate_us(a, kind, table[i], layouts[l], p.splits, cus), row = p.splits == 1 ? row_kernel : 0.0;
+                const double us = TileEstimate(launches[l], table[i]).us(p.splits), row = p.splits == 1 ? row_kernel : 0.0;
                 limit[l] = (layouts[l].row_major ? 0.95 : joint ? 0.97 : 0.92) * (us + 0.5 * row) - 0.3;
                 with_norm[l] = us + row;
             }
         }
     }
-    for (int s = 1; s <= (plan.splits == 1 ? 1 : ranges) && (s == 1 || a.K / 64 / s >= 4); s++)
+    double least[2][MOST];                      // per layout and number of ranges
+    const GemmTile* least_tile[MOST] = {};      // on the layout of the launch
+    for (int s = 0; s < MOST; s++) { least[0][s] = least[1][s] = 1e30; }
+    for (const GemmTile& t : kStagedTiles)
+    {
+        if ((t.mb > 2 && 16 * (t.mb - 1) >= a.tokens) || (t.mb == 2 && a.tokens > 64) || (t.mb == 3 && a.tokens > 192)) { continue; }
+        for (int l = 0; l < (joint ? 2 : 1); l++)
+        {
+            const TileEstimate tile(launches[l], t);
+            for (int s = 1; s <= ranges && (s == 1 || a.K / 64 >= 4 * s); s++)
+            {
+                const double us = tile.us(s, 0.7);
+                if (us >= least[l][s - 1]) { continue; }
+                least[l][s - 1] = us;
+                if (l == 0) { least_tile[s - 1] = &t; }
+            }
+        }
+    }
+    GemmPlan best = plan;
+    double least_sum = 1e30;
+    for (int s = 1; s <= ranges && least_tile[s - 1]; s++)
     {
         const double row = s == 1 ? row_kernel : 0.0;
-        const GemmTile* mine = nullptr;
         double sum = 0.0;
         for (int l = 0; l < (joint ? 2 : 1); l++)
         {
-            const GemmTile* tile = nullptr;
-            double us = 1e30;
-            for (const GemmTile& t : kStagedTiles)
-            {
-                if ((t.mb > 2 && 16 * (t.mb - 1) >= a.tokens) || (t.mb == 2 && a.tokens > 64) || (t.mb == 3 && a.tokens > 192)) { continue; }
-                const double e = estimate_us(a, kind, t, layouts[l], s, cus, 0.7);
-                if (e < us)
-                {
-                    us = e;
-                    tile = &t;
-                }
-            }
+            const double us = least[l][s - 1];
             sum += us + 0.5 * row < limit[l] && us + row <= with_norm[l] ? us + 0.5 * row : 1e30;
-            if (l == 0) { mine = tile; }
         }
-        if (sum < least)
+        if (sum < least_sum)
         {
-            least = sum;
-            best = GemmPlan{ mine->mb, mine->nb, s, true, plan.ranges, true };
+            least_sum = sum;
+            best = GemmPlan{ least_tile[s - 1]->mb, least_tile[s - 1]->nb, s, true, plan.ranges, true };
         }
     }
     return best;
