@@ -11,11 +11,16 @@ namespace
 {
 inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// Sixteen lanes per head from this many heads x tokens on, a wave per head below.  Measured with 12, 32 and 48 heads a token: level at 4600,
+// 3600 and 6100 where every access is aligned, and at 9000, 14500 and 14000 where none is.
+inline bool rope_rows_wide(long long heads, bool aligned) { return heads >= (aligned ? 5120 : 14336); }
+
 // Key ranges of a prompt's attention.  In one piece a workgroup takes 5 us and 1.75 per block of 64 keys; in n ranges the three launches
 // take 16 us, 1.75 per block of one range, and 0.25 per MB of FP32 sums written and read.  At most one workgroup per CU (two take as long
 // as one after the other: 64 tokens of 32 / 8 heads behind 4000: 34.5 us with 8 ranges, 43.9 with 12; 300 tokens behind 1000, 152 workgroups:
-// 45.6 in one piece, 50.4 in two ranges), and 10 % to gain at least.  One piece without scratch memory, as under graph capture.  Measured on MI355X, one piece -> ranges: those 64 tokens 121 -> 34.5 us,
-// 64 tokens of 4 / 1 heads behind 14000 424 -> 34, 200 tokens of 32 / 8 behind 2000 70 -> 51, 2 tokens of one head behind 16000 353 -> 23.
+// 45.6 in one piece, 50.4 in two ranges), and 10 % to gain at least.  One piece without scratch memory, as under graph capture.
+// Measured on MI355X, one piece -> ranges: those 64 tokens 121 -> 34.5 us, 64 tokens of 4 / 1 heads behind 14000 424 -> 34, 200 tokens of
+// 32 / 8 behind 2000 70 -> 51, 2 tokens of one head behind 16000 353 -> 23.
 struct AttentionRanges
 {
     int n, per;
@@ -41,10 +46,14 @@ int hip_qk_norm_rope_kv_rows_bf16(const void* q, const void* k, const void* v, c
     if (pos0 < 0 || (long long)pos0 + n_tokens > t_kv) { return -1; }
     if (!q || !k || !v || !cos_tab || !sin_tab || !q_out || !k_cache || !v_cache) { return -1; }
     if ((q_norm_w == nullptr) != (k_norm_w == nullptr)) { return -1; }
-    const dim3 grid((n_q_heads + 2 * n_kv_heads + 15) / 16, n_tokens);
-    qk_norm_rope_kv_rows_kernel<<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_norm_w,
-                                                           (const uint16_t*)k_norm_w, (const uint16_t*)cos_tab, (const uint16_t*)sin_tab,
-                                                           (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, n_q_heads, n_kv_heads, t_kv, pos0, epsilon);
+    const int heads = n_q_heads + 2 * n_kv_heads;
+    const bool aligned = (((uintptr_t)q | (uintptr_t)k | (uintptr_t)q_norm_w | (uintptr_t)k_norm_w | (uintptr_t)cos_tab | (uintptr_t)sin_tab | (uintptr_t)q_out | (uintptr_t)k_cache) & 7u) == 0
+                         && aligned16(v) && aligned16(v_cache);
+    const bool wide = rope_rows_wide((long long)heads * n_tokens, aligned);
+    auto* const kernel = wide ? qk_norm_rope_kv_rows_kernel : qk_norm_rope_kv_few_rows_kernel;
+    kernel<<<dim3((heads + (wide ? 15 : 3)) / (wide ? 16 : 4), n_tokens), 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)q_norm_w,
+                                                                                             (const uint16_t*)k_norm_w, (const uint16_t*)cos_tab, (const uint16_t*)sin_tab,
+                                                                                             (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, n_q_heads, n_kv_heads, t_kv, pos0, epsilon);
     return finish("qk_norm_rope_kv_rows");
 }
 

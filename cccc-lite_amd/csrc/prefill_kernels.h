@@ -14,15 +14,47 @@ namespace ccq
 {
 
 // ------------------------------------------------------------------------------------------
-// Per-head q/k RMSNorm + RoPE + cache append for T tokens.  Bound by memory: a head is read and written once.  Grid
-// (ceil((n_q + 2 n_kv) / 16), T), sixteen lanes per (head, token): lane i holds elements 4 i .. + 3 of both halves of the head, so that the
-// rotation needs no neighbour, and every access is 8 bytes of a 128-byte run (16 in the copied value rows).  With a whole wave
-// per head and 2-byte accesses 2048 tokens of 32 / 8 heads took 26.7 us, now 14.0 (50 MB: 3.6 TB/s); 512 tokens 6.6, now 4.7; 100
-// tokens 2.8, now 2.7; 20 tokens 2.3 and 2.4 (the launch).  Rows off their 8 bytes still gain at 2048 tokens (26.6, now 19.2).
-// The arithmetic per element is the one-token kernel's and the squares are added in the order of its wave_sum, so both leave the same
-// bytes.  The pointers may lie on any element (value rows: on any pair), as before.
+// Per-head q/k RMSNorm + RoPE + cache append for T tokens.
 //   q [T][n_q][128] -> q_out [T][n_q][128];  k [T][n_kv][128] -> k_cache[h][pos0 + t];  v -> v_cache[h][pos0 + t]
-// q_norm_w == nullptr: no per-head norm (both or neither).
+// q_norm_w == nullptr: no per-head norm (both or neither).  The arithmetic per element is the one-token kernel's and the squares are added
+// in the order of its wave_sum, so all leave the same bytes.  The pointers may lie on any element (value rows: on any pair).
+// Two kernels, by rope_rows_wide.  Few heads: bound by the launch and one trip to memory.  Grid (ceil((n_q + 2 n_kv) / 4), T), one
+// wave per (head, token) and four of them per workgroup, so that the least work is in a lane's way.
+static __global__ __launch_bounds__(256) void qk_norm_rope_kv_few_rows_kernel(const uint16_t* __restrict__ q, const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
+                                                                      const uint16_t* __restrict__ q_norm_w, const uint16_t* __restrict__ k_norm_w,
+                                                                      const uint16_t* __restrict__ cos_tab, const uint16_t* __restrict__ sin_tab,
+                                                                      uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
+                                                                      int n_q, int n_kv, int t_kv, int pos0, float eps)
+{
+    const int head = blockIdx.x * 4 + (threadIdx.x >> 6), t = blockIdx.y;
+    const int lane = threadIdx.x & 63;
+    const int pos = pos0 + t;
+    if (head >= n_q + 2 * n_kv) { return; }
+    if (head >= n_q + n_kv)
+    {
+        const int h = head - n_q - n_kv;
+        const uint32_t* src = (const uint32_t*)(v + ((size_t)t * n_kv + h) * 128);
+        uint32_t* dst = (uint32_t*)(v_cache + ((size_t)h * t_kv + pos) * 128);
+        dst[lane] = src[lane];
+        return;
+    }
+    const bool is_q = head < n_q;
+    const int h = is_q ? head : head - n_q;
+    const uint16_t* src = is_q ? q + ((size_t)t * n_q + h) * 128 : k + ((size_t)t * n_kv + h) * 128;
+    const uint16_t* nw = is_q ? q_norm_w : k_norm_w;
+    float l, r;
+    norm_rope_finish(load_head(src, nw, cos_tab + (size_t)pos * 64, sin_tab + (size_t)pos * 64, lane), nw != nullptr, eps, l, r);
+    uint16_t* dst = is_q ? q_out + ((size_t)t * n_q + h) * 128 : k_cache + ((size_t)h * t_kv + pos) * 128;
+    dst[lane] = (uint16_t)f32_to_bf16_bits(l);
+    dst[lane + 64] = (uint16_t)f32_to_bf16_bits(r);
+}
+
+// Many heads: bound by memory, a head is read and written once.  Grid (ceil((n_q + 2 n_kv) / 16), T), sixteen lanes per (head, token): lane i
+// holds elements 4 i .. + 3 of both halves of the head, so that the rotation needs no neighbour, and every access is 8 bytes of a
+// 128-byte run (16 in the copied value rows).
+//   us per launch, 32 / 8 heads, few-rows kernel / this one: 20 tokens 1.86 / 2.01, 100 tokens 2.20 / 2.31, 128 tokens 2.37 / 2.37, 512
+// tokens 5.01 / 3.75, 2048 tokens 17.7 / 9.7 (50 MB: 5.2 TB/s).  Rows off their 8 bytes: 100 tokens 2.26 / 2.63, 300 tokens 3.70 / 3.75,
+// 512 tokens 5.18 / 4.78, 2048 tokens 17.8 / 13.0.
 typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 

@@ -46,3 +46,25 @@ def test_rows_at_odd_head_counts_and_offsets(gpu, oracle, dec, n_q, n_kv, T, pos
         got = from_dev(keep[i], np.uint16)
         assert (got[:skip] == 0x7FC1).all()
         assert np.array_equal(got[skip:], want.reshape(-1))
+
+
+@pytest.mark.parametrize("T,off", [(465, 0), (466, 0), (1303, 1), (1304, 1)])
+def test_many_rows_leave_the_bytes_of_few(gpu, oracle, dec, T, off):  # noqa: F811
+    """11 heads a token, one token short of the line from which sixteen lanes take a head and on it, aligned and not: the bytes of calls of at
+    most 100 tokens, which give a wave to a head."""
+    torch, dev, lib = gpu
+    n_q, n_kv, t_kv, pos0 = 5, 3, T + 40, 33
+    gen = torch.Generator(device=dev).manual_seed(T)
+    make = lambda n: (2 * torch.randn(n + 16, device=dev, generator=gen)).to(torch.bfloat16).view(torch.int16)
+    q, k, v, qw, kw = make(T * n_q * 128), make(T * n_kv * 128), make(T * n_kv * 128), make(128), make(128)
+    cos, sin = make(t_kv * 64), make(t_kv * 64)
+    results = []
+    for piece in (T, 100):
+        q_out, kc, vc = (torch.full((n + 16,), 0x7FC1, dtype=torch.int16, device=dev) for n in (T * n_q * 128, n_kv * t_kv * 128, n_kv * t_kv * 128))
+        at = lambda t, element: ctypes.c_void_p(t.data_ptr() + 2 * element)
+        for t in range(0, T, piece):
+            assert lib.c.hip_qk_norm_rope_kv_rows_bf16(at(q, off + t * n_q * 128), at(k, off + t * n_kv * 128), at(v, 2 * off + t * n_kv * 128), at(qw, off), at(kw, off), at(cos, off), at(sin, off),
+                                                       at(q_out, off + t * n_q * 128), at(kc, off), at(vc, 2 * off), n_q, n_kv, 128, t_kv, min(piece, T - t), pos0 + t, ctypes.c_float(1e-6)) == 0
+        torch.cuda.synchronize()
+        results.append((q_out, kc, vc))
+    for a, b in zip(*results): assert torch.equal(a, b)
