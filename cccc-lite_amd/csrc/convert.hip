@@ -5,7 +5,8 @@
 // side touches every line twice or four times), four such pieces are requested before the first is used, and the grid is a
 // fixed multiple of the CU count walking the buffer with a grid stride.  Scalar kernels take what is left: the last few
 // elements, misaligned pointers, odd block lengths.  Measured on a 4096 x 12288 weight, BF16 -> float -> FP4 with block scales
-// -> BF16 (659 MB moved): 113 us, 5.8 TB/s, what a plain device copy reaches; through absmax and float -> FP8 and back 154.
+// -> BF16 (659 MB moved): 113 us, 5.8 TB/s (a large copy reaches 5.4; part of what one pass writes the next reads from the
+// memory-side cache); through absmax and float -> FP8 and back 154.
 // Numerics follow the reference kernels element for element (decode, one FP32 multiply by the
 // scale, integer round-to-nearest-even to BF16): cccc-cuda/cuda_functions.cu:2566-2596 (E4M3),
 // :2735-2785 (E5M2), :2834-2884 (FP4), :2896-2960 (FP4 block scale), :3066-3090 (dispatch).
@@ -458,13 +459,15 @@ __global__ __launch_bounds__(kThreads) void encode4_blockscale_vec_kernel(const 
     }
 }
 
-// Largest magnitude.  16-byte loads over the aligned body (scalar loads for a misaligned pointer and the tail), four in flight per lane, wave
-// reduction through lane exchanges, the sixteen waves of a workgroup through LDS, then at most one atomic per workgroup on the
-// bit pattern (non-negative floats order like unsigned integers) -- and none when the value already stored is at least as
-// large.  Atomics on one address are served one after the other and most workgroups start before the first has ended: one workgroup
-// per CU at most, of 1024 threads (with up to sixteen per CU of 256 threads 1 M floats took 16.4 us, now 6.2 with the launch that clears the result, 16 M 21.1 / 13.3, 50 M 37.6 / 31.8).
+// Largest magnitude.  16-byte loads from the first 16-byte boundary on (scalar loads in front of it, behind the last one and for a pointer off
+// its elements), four in flight per lane, wave reduction through lane exchanges, the sixteen waves of a workgroup through LDS, then at
+// most one atomic per workgroup on the bit pattern (non-negative floats order like unsigned integers) -- and none when the value
+// already stored is at least as large.  Atomics on one address are served one after the other and most workgroups start before the
+// first has ended: one workgroup per CU at most, of 1024 threads.  Up to 32 K floats one workgroup, which stores its result itself.
+//   us, with the launch that clears the result: 20 K floats 3.7, 1 M 6.4, 16 M 13.1, 50 M 31.3, the same one element off their 16
+// bytes (up to sixteen workgroups of 256 threads per CU and a memset: 5.7, 18.5, 26.2, 36.7 and off their 16 bytes 50.4 for 50 M).
 // From the last piece to the first: what a cast has just written last is still in the memory-side cache, and the encoder that
-// follows begins where this ends.  NaN inputs are skipped by fmaxf as before.
+// follows begins where this ends.  NaN inputs are skipped by fmaxf.
 constexpr int kMaxThreads = 1024;
 
 static __global__ void absmax_clear_kernel(unsigned int* out) { *out = 0u; }
@@ -476,7 +479,11 @@ __global__ __launch_bounds__(kMaxThreads) void absmax_kernel(const void* __restr
     const size_t stride = (size_t)gridDim.x * kMaxThreads;
     const size_t first = (size_t)blockIdx.x * kMaxThreads + threadIdx.x;
     constexpr size_t PER = SRC == DT_FLOAT ? 4 : 8;             // elements per 16-byte load
-    const size_t n_vec = ((uintptr_t)src & 15u) == 0 ? n / PER : 0;
+    // elements in front of the first 16-byte boundary; none is whole where the pointer is off its elements
+    constexpr size_t SIZE = 16 / PER;
+    const size_t head = min((size_t)(-(uintptr_t)src & 15u) / SIZE, n);
+    const size_t n_vec = (uintptr_t)src % SIZE == 0 ? (n - head) / PER : 0;
+    const u32x4* const body = (const u32x4*)((const uint8_t*)src + head * SIZE);
     float m = 0.0f;
     auto take = [&](const u32x4& v) {
 #pragma unroll
@@ -487,17 +494,17 @@ __global__ __launch_bounds__(kMaxThreads) void absmax_kernel(const void* __restr
         }
     };
     size_t rounds = n_vec / stride;                             // whole ones; the rest is at the end and comes first
-    if (rounds * stride + first < n_vec) { take(((const u32x4*)src)[rounds * stride + first]); }
-    for (; rounds % 4; rounds--) { take(((const u32x4*)src)[(rounds - 1) * stride + first]); }
+    if (rounds * stride + first < n_vec) { take(body[rounds * stride + first]); }
+    for (; rounds % 4; rounds--) { take(body[(rounds - 1) * stride + first]); }
     for (; rounds; rounds -= 4)
     {
         u32x4 v[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) { v[u] = ((const u32x4*)src)[(rounds - 1 - u) * stride + first]; }
+        for (int u = 0; u < 4; u++) { v[u] = body[(rounds - 1 - u) * stride + first]; }
 #pragma unroll
         for (int u = 0; u < 4; u++) { take(v[u]); }
     }
-    for (size_t i = n_vec * PER + first; i < n; i += stride) { m = fmaxf(m, fabsf(load_plain(src, SRC, i))); }
+    for (size_t i = first; i < n - n_vec * PER; i += stride) { m = fmaxf(m, fabsf(load_plain(src, SRC, i < head || n_vec == 0 ? i : i + n_vec * PER))); }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) { m = fmaxf(m, __shfl_xor(m, off)); }
     if ((threadIdx.x & 63) == 0) { part[threadIdx.x >> 6] = m; }
@@ -506,7 +513,8 @@ __global__ __launch_bounds__(kMaxThreads) void absmax_kernel(const void* __restr
     {
         for (int w = 1; w < kMaxThreads / 64; w++) { m = fmaxf(m, part[w]); }
         const unsigned int bits = f32_to_bits(m);
-        if (bits > __atomic_load_n(out, __ATOMIC_RELAXED)) { atomicMax(out, bits); }
+        if (gridDim.x == 1) { *out = bits; }
+        else if (bits > __atomic_load_n(out, __ATOMIC_RELAXED)) { atomicMax(out, bits); }
     }
 }
 
@@ -516,15 +524,13 @@ int hip_absmax(const void* src, int src_type, unsigned int n, void* d_result)
 {
     if (src_type != DT_FLOAT && src_type != DT_HALF && src_type != DT_BF16) { return -1; }
     if (!d_result) { return -1; }
-    absmax_clear_kernel<<<1, 1, 0, stream()>>>((unsigned int*)d_result);
-    if (n)
-    {
-        const size_t want = ((size_t)n / (src_type == DT_FLOAT ? 4 : 8) + kMaxThreads - 1) / kMaxThreads;
-        const unsigned grid = (unsigned)std::min(std::max(want, (size_t)1), (size_t)cu_count());
-        if (src_type == DT_FLOAT) { absmax_kernel<DT_FLOAT><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
-        else if (src_type == DT_HALF) { absmax_kernel<DT_HALF><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
-        else { absmax_kernel<DT_BF16><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
-    }
+    // one workgroup up to eight pieces a lane, which writes its result without a launch that clears it
+    const size_t want = ((size_t)n / (src_type == DT_FLOAT ? 4 : 8) + kMaxThreads - 1) / kMaxThreads;
+    const unsigned grid = want <= 8 ? 1u : (unsigned)std::min(want, (size_t)cu_count());
+    if (grid > 1) { absmax_clear_kernel<<<1, 1, 0, stream()>>>((unsigned int*)d_result); }
+    if (src_type == DT_FLOAT) { absmax_kernel<DT_FLOAT><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
+    else if (src_type == DT_HALF) { absmax_kernel<DT_HALF><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
+    else { absmax_kernel<DT_BF16><<<grid, kMaxThreads, 0, stream()>>>(src, n, (unsigned int*)d_result); }
     return finish("absmax");
 }
 

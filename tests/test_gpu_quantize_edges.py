@@ -31,6 +31,28 @@ def test_absmax_finds_a_single_maximum_anywhere(gpu, oracle, dtype, n):
     assert lib.absmax(x.data_ptr(), code, n, result.data_ptr()) == 0 and result.tolist() == [0.0, -1.0]
 
 
+@pytest.mark.parametrize("dtype", ["float", "half", "bf16"])
+@pytest.mark.parametrize("n", [0, 1, 2, 9, 8 * 4096 - 1, 8 * 8192 + 9, ROUND + 5])
+def test_absmax_of_pointers_off_their_16_bytes(gpu, oracle, dtype, n):
+    """Every offset of whole elements: the maximum at the first and last element, on both sides of the first 16-byte boundary and of the last;
+    larger values just outside, and a result of an earlier call, do not count.  One workgroup and several, an empty range."""
+    torch, dev, lib = gpu
+    real, code, per = {"float": (torch.float32, oracle.FLOAT, 4), "half": (torch.float16, oracle.HALF, 8), "bf16": (torch.bfloat16, oracle.BF16, 8)}[dtype]
+    result = torch.full((2,), 99.0, device=dev)
+    for off in range(per):
+        x = torch.rand(n + 2 * per, device=dev).to(real)
+        x[:off], x[off + n:] = -50.0, 50.0
+        assert x.data_ptr() % 16 == 0
+        places = {off, off + n - 1, off + n // 2} | {e + d for e in (per, 2 * per, (off + n) // per * per) for d in (-1, 0)}
+        for at in sorted(p for p in places if off <= p < off + n) or [None]:
+            if at is not None: old, x[at] = x[at].item(), -37.5
+            torch.cuda.synchronize()
+            assert lib.absmax(x[off:].data_ptr(), code, n, result.data_ptr()) == 0
+            assert result.tolist() == [0.0 if at is None else 37.5, 99.0], (off, at)
+            if at is not None: x[at] = old
+            result[0] = 99.0
+
+
 @pytest.mark.parametrize("block", [16, 32])
 @pytest.mark.parametrize("n", [32, 4096 + 32, 4 * (1 << 20) - 32, 4 * (1 << 20) + 32, 16 * (1 << 20) + 32 * 77])
 def test_fp4_codes_of_ties_and_their_neighbours(gpu, oracle, block, n):
