@@ -416,7 +416,37 @@ __global__ __launch_bounds__(kThreads) void encode4_blockscale_kernel(const floa
 // Whole blocks of 16 or 32 elements: BLOCK / 4 neighbouring lanes share a block, each with one 16-byte load, and find its
 // largest magnitude through lane exchanges inside their row of 16.  One lane per block read 64 bytes at a stride of 64, twice:
 // 254 us for a 4096 x 12288 weight (234 MB, 0.9 TB/s).
-// A lane has four pieces, of four blocks; lane u of every quad takes the two divisions and the scale byte of block u and the others get the
+template <int BLOCK>
+__device__ __forceinline__ float block_absmax(const f32x4& x)
+{
+    float m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
+    m = fmaxf(m, dpp_f32<0xB1>(m));                                                   // quad_perm [1,0,3,2]
+    m = fmaxf(m, dpp_f32<0x4E>(m));                                                   // quad_perm [2,3,0,1]
+    if (BLOCK == 32) { m = fmaxf(m, dpp_f32<0x141>(m)); }                             // row_half_mirror
+    return m;
+}
+
+__device__ __forceinline__ uint16_t encode4(const f32x4& x, float f)
+{
+    return (uint16_t)(f32_to_fp4(x[0] * f) | (f32_to_fp4(x[1] * f) << 4) | (f32_to_fp4(x[2] * f) << 8) | (f32_to_fp4(x[3] * f) << 12));
+}
+
+// One piece per lane, up to as many as the grid has lanes (4 M floats on 256 CUs): bound by one trip to memory, every lane divides for itself.
+// 1 M floats 2.8 us, 4 M 5.5; with four pieces per lane, three of them past the end, 3.4 and 7.8, on a quarter of the workgroups 3.3 and 6.6.
+template <int BLOCK>
+__global__ __launch_bounds__(kThreads) void encode4_blockscale_piece_kernel(const float* __restrict__ src, uint8_t* __restrict__ nibbles, uint8_t* __restrict__ scales,
+                                                                           size_t n_quads)
+{
+    constexpr int LANES = BLOCK / 4;
+    const size_t v = (size_t)blockIdx.x * kThreads + threadIdx.x;
+    if (v >= n_quads) { return; }               // whole groups of lanes: n_quads is a multiple of LANES
+    const f32x4 x = __builtin_nontemporal_load((const f32x4*)src + v);
+    const float amax = block_absmax<BLOCK>(x);
+    ((uint16_t*)nibbles)[v] = encode4(x, (amax > 1e-10f) ? (6.0f / amax) : 1.0f);
+    if (v % LANES == 0) { scales[v / LANES] = (uint8_t)f32_to_e4m3_trunc((amax > 1e-10f) ? (amax / 6.0f) : 1.0f); }
+}
+
+// More: a lane has four pieces, of four blocks; lane u of every quad takes the two divisions and the scale byte of block u and the others get the
 // factor through a lane exchange (4096 x 12288 floats 45 us, 5.1 TB/s; 51 with every lane dividing for itself and seven comparisons per code).
 // The pieces are walked from the last to the first: what a cast or another pass has just written last is still in the memory-side cache.
 template <int BLOCK>
@@ -437,14 +467,7 @@ __global__ __launch_bounds__(kThreads) void encode4_blockscale_vec_kernel(const 
 #pragma unroll
         for (int u = 0; u < 4; u++) { x[u] = __builtin_nontemporal_load((const f32x4*)src + (v + u * stride < n_quads ? v + u * stride : n_quads - LANES + threadIdx.x % LANES)); }
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-        {
-            float m = fmaxf(fmaxf(fabsf(x[u][0]), fabsf(x[u][1])), fmaxf(fabsf(x[u][2]), fabsf(x[u][3])));
-            m = fmaxf(m, dpp_f32<0xB1>(m));                                           // quad_perm [1,0,3,2]
-            m = fmaxf(m, dpp_f32<0x4E>(m));                                           // quad_perm [2,3,0,1]
-            if (LANES == 8) { m = fmaxf(m, dpp_f32<0x141>(m)); }                      // row_half_mirror
-            amax[u] = m;
-        }
+        for (int u = 0; u < 4; u++) { amax[u] = block_absmax<BLOCK>(x[u]); }
         const float mine = q < 2u ? (q == 0u ? amax[0] : amax[1]) : (q == 2u ? amax[2] : amax[3]);
         const float fwd = (mine > 1e-10f) ? (6.0f / mine) : 1.0f;
         const size_t at = v + q * stride;                                             // a piece of the lane's block
@@ -453,8 +476,8 @@ __global__ __launch_bounds__(kThreads) void encode4_blockscale_vec_kernel(const 
 #pragma unroll
         for (int u = 0; u < 4; u++)
         {
-            const uint32_t w = f32_to_fp4(x[u][0] * f[u]) | (f32_to_fp4(x[u][1] * f[u]) << 4) | (f32_to_fp4(x[u][2] * f[u]) << 8) | (f32_to_fp4(x[u][3] * f[u]) << 12);
-            if (v + u * stride < n_quads) { ((uint16_t*)nibbles)[v + u * stride] = (uint16_t)w; }
+            const uint16_t w = encode4(x[u], f[u]);
+            if (v + u * stride < n_quads) { ((uint16_t*)nibbles)[v + u * stride] = w; }
         }
     }
 }
@@ -588,13 +611,12 @@ int hip_float_to_fp4_blockscale(const void* src, void* dst_nibbles, void* dst_sc
     const bool vec_ok = (((uintptr_t)src & 15u) | ((uintptr_t)dst_nibbles & 1u)) == 0 && (block_size == 16 || block_size == 32);
     const size_t whole = vec_ok ? (size_t)n_elems / block_size : 0;                 // complete blocks
     const size_t n_quads = whole * block_size / 4;
-    if (whole && block_size == 16)
+    if (whole)
     {
-        encode4_blockscale_vec_kernel<16><<<grid_for(n_quads), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst_nibbles, (uint8_t*)dst_scales, n_quads);
-    }
-    else if (whole)
-    {
-        encode4_blockscale_vec_kernel<32><<<grid_for(n_quads), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst_nibbles, (uint8_t*)dst_scales, n_quads);
+        const bool one = n_quads <= (size_t)cu_count() * 16 * kThreads;
+        auto* const kernel = block_size == 16 ? (one ? encode4_blockscale_piece_kernel<16> : encode4_blockscale_vec_kernel<16>)
+                                              : (one ? encode4_blockscale_piece_kernel<32> : encode4_blockscale_vec_kernel<32>);
+        kernel<<<grid_for(one ? n_quads : (n_quads + 3) / 4), kThreads, 0, stream()>>>((const float*)src, (uint8_t*)dst_nibbles, (uint8_t*)dst_scales, n_quads);
     }
     if (whole < n_blocks)
     {
