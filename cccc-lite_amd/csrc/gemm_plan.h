@@ -282,7 +282,8 @@ inline GemmPlan plan_gemm(const LinearArgs& a, GemmKind kind, const GemmWeights&
 }
 
 // gemm_staged_kernel, all weights: the same estimate, fitted to 10,900 launches (13 shapes x 11 token counts from 20 to 1024 x every tile
-// and 1 to 8 k ranges, the four columns and HALF activations; weights in turn through up to 1.2 GB), error 3 to 6 % rms per tile.  Alone on a CU a
+// and 1 to 8 k ranges, the four columns and HALF activations; weights in turn through up to 1.2 GB) of an earlier form of the kernel.
+// On 21,700 launches of this one, at 25 token counts from 18 to 512, it is 4 to 7 % high (7 to 10 % rms per tile).  Alone on a CU a
 // k-tile takes down to 0.7 of `one`: the loads share L2 and HBM with fewer others.
 constexpr GemmTile kStagedTiles[] = {
     { 2, 1, 3.2, 0.6, { 0.162, 0.174, 0.208, 0.211 }, { 0.143, 0.152, 0.158, 0.167 } },
@@ -302,9 +303,10 @@ constexpr GemmTile kStagedTiles[] = {
 // both, the k ranges for which the staged kernel is ahead on both together, so that a weight gives the same bits from the file layout
 // and from its tiled copy.  Elsewhere each layout takes what is best for it.
 // Ahead: 0.3 us and 5 % (file layout) or 8 % (tiled copy, whose KiB blocks the other kernels read whole as well; 3 % in a joint decision)
-// below the plan's own estimate; with less, launches of 5 us and k-split ones on tiled copies lose up to 15 %.  Of 620
-// measured calls 119 then run it, three of them more than 3 % slower (9 % at most); mean of all calls 0.94 of the plans' time on E5M2 in the
-// file layout, 0.98 on tiled copies (0.91 and 0.97 without the joint decision).
+// below the plan's own estimate; with less, launches of 5 us and k-split ones on tiled copies lose up to 15 %.  Of 1550
+// measured calls (the 13 shapes and 25 token counts above) 278 then run it, three of them more than 3 % slower than on the plan (7 % at
+// most); mean of all calls 0.94 of the plans' time on E5M2 in the file layout, 0.96 with scales, 0.98 on tiled copies.  A tile
+// with sixteen tokens or more past the end is not considered, which leaves 81 to 96 and 113 to 128 tokens with smaller ones.
 // An unsplit linear that may come with the add and the norm carries half of the row kernel, as in plan_gemm, and must not be behind
 // with all of it either (4096 x 12288 at 512 tokens, tiled: 58 us alone on both, 64 against 55 with the norm).
 // `scratch` is that of the call to plan_gemm.  The k ranges of the larger tile, and so the scratch memory, stay what they were.  FP4

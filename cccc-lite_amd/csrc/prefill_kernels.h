@@ -187,7 +187,9 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // both passes over all the keys.
 // PASS 3: the whole context is at most PF_SHORT blocks.  Then all keys and values are requested at once and stay in LDS, and the scores stay in
 // registers between the passes: one trip to memory and a few barriers where the pipelines of PASS 0 start up twice (100 tokens of 32 / 8 heads
-// 10.2 us on PASS 0, now 8.8; with the scores multiplied again in loops instead 9.4).  The same sums in the same order as PASS 0.
+// 10.2 us on PASS 0, now 8.8; with the scores multiplied again in loops instead 9.4).  Its LDS leaves a CU one workgroup, where PASS 0
+// has two; it is still ahead with more of them than CUs: 256 tokens of 32 / 32 heads (512 workgroups) 15.7 us on PASS 0, now 13.9, of 64 / 64
+// heads (1024) 28.4 and 26.7, of 128 / 32 heads (512) 21.0 and 19.9.  The same sums in the same order as PASS 0.
 constexpr int PF_SHORT = 4;
 constexpr int PF_RANGES = 32;               // most ranges: a lane group of pass 2 reads eight statistics at once
 
