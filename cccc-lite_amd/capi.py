@@ -67,6 +67,7 @@ EXPORTS = (
     "hip_attention_decode_exact_bf16",
     "hip_qk_norm_rope_kv_rows_bf16",
     "hip_attention_prefill_bf16",
+    "hip_attention_prefill_fused_bf16",
     "hip_add_bf16",
     "hip_swiglu_bf16",
     "hip_add_rms_norm_bf16",
@@ -145,8 +146,9 @@ class QuantLibrary:
         L.hip_attention_decode_exact_bf16.argtypes = [vp] * 11 + [ctypes.c_ulonglong, i32, i32, i32, i32, vp, f32]
         L.hip_qk_norm_rope_kv_rows_bf16.restype = i32
         L.hip_qk_norm_rope_kv_rows_bf16.argtypes = [vp] * 10 + [i32, i32, i32, i32, i32, i32, f32]
-        L.hip_attention_prefill_bf16.restype = i32
-        L.hip_attention_prefill_bf16.argtypes = [vp] * 4 + [i32, i32, i32, i32, i32, i32]
+        for name in ("hip_attention_prefill_bf16", "hip_attention_prefill_fused_bf16"):
+            getattr(L, name).restype = i32
+            getattr(L, name).argtypes = [vp] * 4 + [i32, i32, i32, i32, i32, i32]
         L.hip_add_bf16.restype = i32
         L.hip_add_bf16.argtypes = [vp, vp, vp, ctypes.c_ulonglong]
         L.hip_swiglu_bf16.restype = i32

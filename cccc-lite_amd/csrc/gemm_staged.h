@@ -5,20 +5,6 @@
 namespace ccq
 {
 
-// 64 lanes x 16 bytes from base + off to the KiB of LDS at byte offset `lds` (lane l to lds + 16 l); no register is written.  Counts in
-// vmcnt like any load.  The compiler would put a vmcnt(0) in front of every LDS read if it knew of these transfers, so they and
-// their waits are written out here.  STREAM: bytes that nobody else reads, not kept in L2.  m0 is named as written, so that no m0 of the
-// compiler's own lives across; it warns that it does not allocate that register itself.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-template <bool STREAM>
-__device__ __forceinline__ void load_to_lds(uint32_t lds, const uint8_t* base, uint32_t off)
-{
-    if constexpr (STREAM) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" : : "s"(lds), "v"(off), "s"(base) : "memory", "m0"); }
-    else { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(off), "s"(base) : "memory", "m0"); }
-}
-#pragma clang diagnostic pop
-
 // all but the newest N loads of this wave have arrived, then the workgroup's barrier
 template <int N>
 __device__ __forceinline__ void wait_loads_barrier()

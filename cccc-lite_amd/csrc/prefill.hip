@@ -1,6 +1,6 @@
 // C-ABI entry points of the prompt-phase neighbours (kernels in prefill_kernels.h).
 #include "../../include/cccc_hip_quant.h"
-#include "prefill_kernels.h"
+#include "prefill_fused.h"
 #include "runtime.h"
 #include <algorithm>
 #include <cmath>
@@ -36,6 +36,48 @@ AttentionRanges attention_ranges(long long tiles, int n_keys, size_t outputs)
     const double whole = 5.0 + 1.75 * blocks, split = 16.0 + 1.75 * per + 0.25e-6 * 8.0 * 128.0 * (double)outputs * n;
     return split < 0.9 * whole ? AttentionRanges{ n, per } : AttentionRanges{ 1, blocks };
 }
+
+// The same in one pass: 4.5 us and 0.87 per block where a CU has one workgroup, 1.35 for two side by side; ranges add 6 us for the combine launch
+// and 0.35 per MB of FP32 sums written and read.  One or two workgroups per CU, whichever the estimate has ahead by 5 %.
+// Measured, 1 / 2 / 4 / 8 ranges: 512 tokens of 32 / 8 heads behind 3000 53 / 53 / 57 / 67 us, 256 tokens 47.6 / 35.4 / 36.5 / 38.8, 128 tokens
+// 46 / 31.6 / 25.1 / 27.7, 2048 tokens of 4 / 1 behind 4000 83 / 52 / 45 / 52, 700 of 2 / 1 behind 5000 80 / 48 / 30 / 22, 512 of 32 / 8 from 0 12.7
+// / 23.9 / 28.2.
+AttentionRanges fused_attention_ranges(long long tiles, int n_keys, size_t outputs)
+{
+    const int blocks = (n_keys + PF_KEYS - 1) / PF_KEYS;
+    AttentionRanges best = { 1, blocks };
+    double least = 4.5 + blocks * std::max(0.87, 1.35 * (double)tiles / (2.0 * cu_count()));
+    for (int side = 1; side <= 2; side++)
+    {
+        const int want = (int)std::min({ side * cu_count() / tiles, (long long)PF_RANGES, (long long)blocks / 2 });
+        if (want < 2) { continue; }
+        const int per = ((blocks + want - 1) / want + 1) & ~1;
+        const int n = (blocks + per - 1) / per;
+        const double time = 10.5 + per * (side == 1 ? 0.87 : 1.35) + 0.35e-6 * 8.0 * 128.0 * (double)outputs * n;
+        if (n > 1 && time < 0.95 * least) { least = time; best = { n, per }; }
+    }
+    return best;
+}
+
+// FP32 sums and statistics of the ranges: at most two workgroups of 64 rows per CU.  One size for both forms of the attention, which share
+// the buffer.
+char* range_scratch()
+{
+    constexpr size_t ROW = 128 * sizeof(float) + sizeof(float2);
+    return (char*)fixed_scratch((size_t)cu_count() * 2 * 64 * ROW);
+}
+
+bool prefill_args_ok(const void* q, const void* k_cache, const void* v_cache, const void* y, int n_q_heads, int n_kv_heads, int head_dim, int t_kv, int n_tokens, int pos0)
+{
+    if (head_dim != 128 || n_kv_heads <= 0 || n_q_heads <= 0 || n_q_heads % n_kv_heads != 0 || t_kv <= 0 || n_tokens <= 0) { return false; }
+    if (pos0 < 0 || (long long)pos0 + n_tokens > t_kv || n_kv_heads > 65535) { return false; }
+    if (!q || !k_cache || !v_cache || !y || !aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache)) { return false; }
+    if ((long long)((n_tokens + 15) / 16) * n_kv_heads > 0x7FFFFFFFLL) { return false; }
+    // the kernels address cache rows with 32-bit byte offsets inside a KV head (row * 256)
+    if ((long long)pos0 + n_tokens > (1LL << 24)) { return false; }
+    const int group = n_q_heads / n_kv_heads;
+    return group == 1 || group == 2 || group == 4;
+}
 }    // namespace
 
 int hip_qk_norm_rope_kv_rows_bf16(const void* q, const void* k, const void* v, const void* q_norm_w, const void* k_norm_w,
@@ -60,21 +102,13 @@ int hip_qk_norm_rope_kv_rows_bf16(const void* q, const void* k, const void* v, c
 int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v_cache, void* y,
                                int n_q_heads, int n_kv_heads, int head_dim, int t_kv, int n_tokens, int pos0)
 {
-    if (head_dim != 128 || n_kv_heads <= 0 || n_q_heads <= 0 || n_q_heads % n_kv_heads != 0 || t_kv <= 0 || n_tokens <= 0) { return -1; }
-    if (pos0 < 0 || (long long)pos0 + n_tokens > t_kv || n_kv_heads > 65535) { return -1; }
-    if (!q || !k_cache || !v_cache || !y || !aligned16(q) || !aligned16(k_cache) || !aligned16(v_cache)) { return -1; }
-    if ((long long)((n_tokens + 15) / 16) * n_kv_heads > 0x7FFFFFFFLL) { return -1; }
-    // the kernel addresses cache rows with 32-bit byte offsets inside a KV head (row * 256)
-    if ((long long)pos0 + n_tokens > (1LL << 24)) { return -1; }
+    if (!prefill_args_ok(q, k_cache, v_cache, y, n_q_heads, n_kv_heads, head_dim, t_kv, n_tokens, pos0)) { return -1; }
     const long long tiles = (long long)((n_tokens + 15) / 16) * n_kv_heads;
     const int group = n_q_heads / n_kv_heads;
-    if (group != 1 && group != 2 && group != 4) { return -1; }
     const float scale = 1.0f / sqrtf(128.0f);
     const size_t outputs = (size_t)n_tokens * n_q_heads;
     const AttentionRanges split = attention_ranges(tiles, pos0 + n_tokens, outputs);
-    // ranges x tiles is at most the number of CUs, and a tile is 16 tokens of at most four heads
-    constexpr size_t ROW = 128 * sizeof(float) + sizeof(float2);
-    char* const scratch = split.n > 1 ? (char*)fixed_scratch((size_t)cu_count() * 16 * 4 * ROW) : nullptr;
+    char* const scratch = split.n > 1 ? range_scratch() : nullptr;
     const PrefillRanges ranges = { split.per, (float2*)(scratch + (size_t)split.n * outputs * 128 * sizeof(float)), (float*)scratch };
     const dim3 grid((unsigned)tiles, scratch ? split.n : 1);
 #define CCQ_ATTN_PREFILL(G, PASS)                                                                                                                  \
@@ -94,6 +128,35 @@ int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v
 #undef CCQ_ATTN_PREFILL_GROUPS
 #undef CCQ_ATTN_PREFILL
     return finish("attention_prefill");
+}
+
+int hip_attention_prefill_fused_bf16(const void* q, const void* k_cache, const void* v_cache, void* y,
+                                     int n_q_heads, int n_kv_heads, int head_dim, int t_kv, int n_tokens, int pos0)
+{
+    if (!prefill_args_ok(q, k_cache, v_cache, y, n_q_heads, n_kv_heads, head_dim, t_kv, n_tokens, pos0)) { return -1; }
+    const int group = n_q_heads / n_kv_heads, tile = 64 / group;
+    const long long tiles = (long long)((n_tokens + tile - 1) / tile) * n_kv_heads;
+    const float scale = 1.0f / sqrtf(128.0f);
+    const size_t outputs = (size_t)n_tokens * n_q_heads;
+    const AttentionRanges split = fused_attention_ranges(tiles, pos0 + n_tokens, outputs);
+    char* const scratch = split.n > 1 ? range_scratch() : nullptr;
+    const PrefillRanges ranges = { split.per, (float2*)(scratch + (size_t)split.n * outputs * 128 * sizeof(float)), (float*)scratch };
+    const dim3 grid((unsigned)tiles, scratch ? split.n : 1);
+#define CCQ_ATTN_PREFILL(G, RANGE)                                                                                                                       \
+    attn_prefill_fused_kernel<G, RANGE><<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, (uint16_t*)y, \
+                                                                    n_q_heads, t_kv, n_tokens, pos0, scale, ranges)
+#define CCQ_ATTN_PREFILL_GROUPS(RANGE)                                                                                                             \
+    group == 4 ? CCQ_ATTN_PREFILL(4, RANGE) : group == 2 ? CCQ_ATTN_PREFILL(2, RANGE) : CCQ_ATTN_PREFILL(1, RANGE)
+    if (!scratch) { CCQ_ATTN_PREFILL_GROUPS(false); }
+    else
+    {
+        CCQ_ATTN_PREFILL_GROUPS(true);
+        const long long blk = ((long long)outputs * 32 + 255) / 256, cap = (long long)cu_count() * 16;
+        attn_prefill_fused_combine_kernel<<<(unsigned)(blk < cap ? blk : cap), 256, 0, stream()>>>(ranges, (uint16_t*)y, n_q_heads, n_tokens, pos0, tile);
+    }
+#undef CCQ_ATTN_PREFILL_GROUPS
+#undef CCQ_ATTN_PREFILL
+    return finish("attention_prefill_fused");
 }
 
 int hip_add_bf16(const void* a, const void* b, void* y, unsigned long long n)

@@ -193,6 +193,19 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 constexpr int PF_SHORT = 4;
 constexpr int PF_RANGES = 32;               // most ranges: a lane group of pass 2 reads eight statistics at once
 
+// eight sums rounded to a row of the output, which may lie on any element
+__device__ __forceinline__ void store_bf16x8(uint16_t* dst, const f32x4& lo, const f32x4& hi)
+{
+    const u32x4 o = { f32_to_bf16_bits(lo[0]) | (f32_to_bf16_bits(lo[1]) << 16), f32_to_bf16_bits(lo[2]) | (f32_to_bf16_bits(lo[3]) << 16),
+                      f32_to_bf16_bits(hi[0]) | (f32_to_bf16_bits(hi[1]) << 16), f32_to_bf16_bits(hi[2]) | (f32_to_bf16_bits(hi[3]) << 16) };
+    if (((uintptr_t)dst & 15u) == 0) { *(u32x4*)dst = o; }
+    else
+    {
+#pragma unroll
+        for (int e = 0; e < 8; e++) { dst[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1))); }
+    }
+}
+
 struct PrefillRanges
 {
     int per;                // blocks of PF_KEYS keys per range
@@ -621,14 +634,7 @@ __global__ __launch_bounds__(256, PASS == 3 ? 1 : 2) void attn_prefill_kernel(co
         else
         {
             uint16_t* const dst = y + ((size_t)t * n_q + kvh * G) * 128 + at;
-            const u32x4 o = { f32_to_bf16_bits(lo[0]) | (f32_to_bf16_bits(lo[1]) << 16), f32_to_bf16_bits(lo[2]) | (f32_to_bf16_bits(lo[3]) << 16),
-                              f32_to_bf16_bits(hi[0]) | (f32_to_bf16_bits(hi[1]) << 16), f32_to_bf16_bits(hi[2]) | (f32_to_bf16_bits(hi[3]) << 16) };
-            if (((uintptr_t)y & 15u) == 0) { *(u32x4*)dst = o; }
-            else
-            {
-#pragma unroll
-                for (int e = 0; e < 8; e++) { dst[e] = (uint16_t)(o[e >> 1] >> (16 * (e & 1))); }
-            }
+            store_bf16x8(dst, lo, hi);
         }
     }
 }

@@ -532,8 +532,8 @@ int DecodeModel::prefillPiece(const int* tokens, int n, int pos0, bool last)
         }
         if (rc == 0)
         {
-            rc = hip_attention_prefill_bf16(pf_.q_rot->data(), k_cache_[li]->data(), v_cache_[li]->data(), pf_.att->data(),
-                                            c.n_q, c.n_kv, c.head_dim, c.t_kv, n, pos0);
+            const auto attention = exact_attention_ ? hip_attention_prefill_bf16 : hip_attention_prefill_fused_bf16;
+            rc = attention(pf_.q_rot->data(), k_cache_[li]->data(), v_cache_[li]->data(), pf_.att->data(), c.n_q, c.n_kv, c.head_dim, c.t_kv, n, pos0);
         }
         // o, the residual add and the norm behind it: one call where the GEMM splits its k range (short prompts), else two
         if (rc == 0) { rc = linear_add_norm(*L.wo, c.hidden, q_out, *pf_.att, *pf_.x, *pf_.r1, *L.rms_ffn, *pf_.xn); }

@@ -72,7 +72,8 @@ public:
     // the same bytes without quantizing again.  0 ok, -1 the file could not be written.
     int saveNamedWeights(const std::string& filename);
 
-    // false (default): two-launch attention with the norm / RoPE / append folded in and FP32 probabilities;
+    // false (default): two-launch attention with the norm / RoPE / append folded in and FP32 probabilities (prompts: BF16, rounded before the
+    // division by their sum);
     // true: the reference's rounding points throughout (BF16 probabilities over the whole row; three launches).
     void setExactAttention(bool exact) { exact_attention_ = exact; }
     // Per-head RMSNorm of q and k in front of the rotation: on for Qwen3-style models (default), off for models without

@@ -313,7 +313,8 @@ class DecodeModel:
 
     def set_exact_attention(self, exact: bool) -> None:
         """True: separate norm / RoPE / append launch and BF16 probabilities (the reference's rounding
-        points); False (default): the two-launch attention with FP32 probabilities."""
+        points); False (default): the two-launch attention with FP32 probabilities (prompts: one pass over the
+        keys, BF16 probabilities rounded before the division by their sum)."""
         self.lib.c.cccc_decode_set_exact_attention(self.handle, 1 if exact else 0)
 
     def set_qk_norm(self, on: bool) -> None:

@@ -1,0 +1,79 @@
+"""Attention of a prompt in one pass over the keys: the oracle's attention, whose probabilities are rounded behind the division."""
+import numpy as np
+import pytest
+
+from gpu_util import from_dev, to_dev
+from test_gpu_prefill import dec, ptr  # noqa: F401 (dec: a fixture)
+from test_gpu_prefill_ranges import inputs
+
+pytestmark = pytest.mark.gpu
+
+
+# one and more tokens than a workgroup's tile (16 / 32 / 64 for 4 / 2 / 1 query heads per kv head), 63 to 65 keys and around 128, a context in
+# ranges (the last of them empty for the first tile, or ending inside a block), heads of one XCD and of several
+@pytest.mark.parametrize("n_q,n_kv,T,pos0", [(1, 1, 1, 0), (4, 1, 16, 0), (4, 1, 17, 47), (2, 1, 33, 31), (1, 1, 65, 0), (8, 2, 63, 65), (2, 2, 70, 57), (16, 8, 40, 88), (8, 4, 130, 500),
+                                             (1, 1, 2, 4100), (4, 1, 17, 1150), (8, 2, 33, 2046), (2, 2, 127, 1470), (32, 8, 200, 1850), (4, 2, 300, 700)])
+@pytest.mark.parametrize("rising", [False, True])
+def test_follows_the_oracle_token_by_token(gpu, oracle, dec, n_q, n_kv, T, pos0, rising):
+    """Either side rounds every probability to BF16 once, by at most 2^-9 of it (the oracle behind the division, the kernel before it), and the
+    kernel its result: 2^-8 sum p |v| + 2^-9 |y|.  On top of that 2e-3 of the row's largest value, as in the tests of the two-pass form: a score
+    next to a BF16 rounding boundary may fall either way.  rising: keys grow along the context, so that the running maximum moves again
+    and again.  Rows past the prompt hold NaN and must not leak; the same bits where the output is off its 16 bytes."""
+    torch, dev, lib = gpu
+    t_kv = pos0 + T + 40
+    q, kc, vc = inputs(oracle, n_q, n_kv, T, pos0, t_kv)
+    if rising:
+        kf = dec.f(kc[:, :pos0 + T]) * (1.0 + 3.0 * np.arange(pos0 + T, dtype=np.float32) / (pos0 + T))[None, :, None]
+        kc[:, :pos0 + T] = oracle.f32_to_bf16(kf.astype(np.float32))
+    qd, kd, vd = to_dev(torch, dev, q), to_dev(torch, dev, kc), to_dev(torch, dev, vc)
+    y, z = (torch.zeros(T * n_q * 128 + 64, dtype=torch.int16, device=dev) for _ in range(2))
+    for out in (y, z[1:]):
+        assert lib.c.hip_attention_prefill_fused_bf16(ptr(qd), ptr(kd), ptr(vd), ptr(out), n_q, n_kv, 128, t_kv, T, pos0) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(y[:-1], z[1:]) and z[0] == 0 and not y[T * n_q * 128:].any()
+    got = from_dev(y, np.uint16)[:T * n_q * 128].reshape(T, n_q, 128)
+    kf, vf = dec.f(kc), dec.f(vc)
+    kf[:, pos0 + T:], vf[:, pos0 + T:] = 0.0, 0.0               # masked in the oracle too; NaN * 0 would poison its matrix products
+    for t in sorted({0, 1, 15, 16, 31, 32, 63, 64, T // 2, T - 2, T - 1} & set(range(T))):
+        want = dec.attention(dec.f(q[t]), kf, vf, pos0 + t, n_q, n_kv)
+        assert np.isfinite(dec.f(got[t])).all(), t
+        bound = 2.0 ** -8 * dec.attention(dec.f(q[t]), kf, np.abs(vf), pos0 + t, n_q, n_kv) + 2.0 ** -9 * np.abs(want)
+        assert (np.abs(dec.f(got[t]) - want) <= bound + 2e-3 * np.abs(want).max()).all(), t
+        assert np.linalg.norm(dec.f(got[t]) - want) <= np.linalg.norm(bound), t
+
+
+def test_one_buffer_for_both_forms_and_one_piece_under_capture(gpu, oracle, dec):
+    """The two-pass form's ranges first, then more ranges of the one-pass form (the buffer has one size), then a captured call, which uses none
+    and is replayed beside eager calls.  Bad arguments are refused as by the two-pass form."""
+    torch, dev, lib = gpu
+    n_q, n_kv, T, pos0, t_kv = 32, 8, 256, 3000, 3300
+    q, k, v = (to_dev(torch, dev, a) for a in inputs(oracle, n_q, n_kv, T, pos0, t_kv))
+    exact, eager, graphed = (torch.zeros(T * n_q * 128, dtype=torch.int16, device=dev) for _ in range(3))
+    args = lambda out, T=T, n_q=n_q: (ptr(q), ptr(k), ptr(v), ptr(out), n_q, n_kv, 128, t_kv, T, pos0)
+    norm = lambda a, b: np.linalg.norm(dec.f(from_dev(a, np.uint16)) - dec.f(from_dev(b, np.uint16))) / np.linalg.norm(dec.f(from_dev(b, np.uint16)))
+    stream = torch.cuda.Stream(device=dev)
+    lib.set_sync(False)
+    try:
+        assert lib.set_stream(stream.cuda_stream) == 0
+        assert lib.c.hip_attention_prefill_bf16(*args(exact)) == 0
+        assert lib.c.hip_attention_prefill_fused_bf16(*args(eager)) == 0
+        stream.synchronize()
+        assert norm(eager, exact) <= 2.0 ** -7
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            assert lib.c.hip_attention_prefill_fused_bf16(*args(graphed)) == 0
+        first = None
+        for _ in range(3):
+            graphed.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream): graph.replay()
+            assert lib.c.hip_attention_prefill_fused_bf16(*args(eager)) == 0
+            torch.cuda.synchronize()
+            first = graphed.clone() if first is None else first
+            assert torch.equal(graphed, first) and norm(graphed, eager) <= 2.0 ** -7
+        for fn in (lib.c.hip_attention_prefill_bf16, lib.c.hip_attention_prefill_fused_bf16):
+            assert fn(*args(eager, T=t_kv - pos0 + 1)) == -1 and fn(*args(eager, n_q=24)) == -1
+            assert fn(ptr(q.view(-1)[1:]), ptr(k), ptr(v), ptr(eager), n_q, n_kv, 128, t_kv, T, pos0) == -1
+    finally:
+        lib.set_stream(None)
+        lib.set_sync(True)
