@@ -20,7 +20,7 @@ namespace ccq
 // BF16's exponent do not notice, and the sums are left alone.
 //   Bound: by what a wave issues between its matrix-core instructions (one workgroup per CU 0.87 us per block, two 0.6 per workgroup; matrix cores
 // 40 % busy with two).  32 / 8 heads, MI355X, attn_prefill_kernel -> this one, us: 2048 tokens from 0 113 -> 56, 512 behind 3000 108 -> 53, 1024 behind
-// 3000 167 -> 79, 100 from 0 9.1 -> 7.6; 8 / 8 heads, 2048 from 0 108 -> 33.  There each row group read the keys twice, key and value rows went
+// 3000 167 -> 79, 100 from 0 9.1 -> 7.0; 8 / 8 heads, 2048 from 0 108 -> 33.  There each row group read the keys twice, key and value rows went
 // through registers with 32 lines per load instruction, and values were transposed by the VALU.  Error against 64 bits: no larger
 // (512 behind 3000 4.34e-3 both, 100 from 0 3.07e-3 -> 2.82e-3).
 // LDS: chunk c (16 bytes) of key row r lies at c ^ (r % 16), of value row r at c ^ (2 (r % 8)): the operand reads hit all banks.
@@ -192,17 +192,25 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_fused_kernel(const uint16
     auto staged_barrier = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
     f32x4 cur[2][2], next[2][2];
+    // (no block past the last one is loaded: of a short prompt that would be most of the launch)
     stage_keys(b_begin);
-    stage_keys(b_begin + 1);
     stage_values(b_begin);
-    asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (b_begin + 1 < b_end)
+    {
+        stage_keys(b_begin + 1);
+        asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    else { asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
     score_products(b_begin, cur);
     staged_barrier();
     // iteration b: keys of b + 1 and values of b are in LDS, `cur` holds the raw scores of b
     auto block = [&](int b, auto masked_c) {
-        stage_keys(b + 2);
-        stage_values(b + 1);
-        score_products(b + 1, next);
+        if (b + 2 < b_end) { stage_keys(b + 2); }
+        if (b + 1 < b_end)
+        {
+            stage_values(b + 1);
+            score_products(b + 1, next);
+        }
         weigh(cur, b, masked_c);
         staged_barrier();
 #pragma unroll
