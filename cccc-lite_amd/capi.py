@@ -60,6 +60,8 @@ EXPORTS = (
     "hip_rope_fwd",
     "hip_embed_fwd",
     "hip_embed_token_bf16",
+    "hip_embed_ids_bf16",
+    "hip_decode_begin_bf16",
     "hip_qk_norm_rope_kv_bf16",
     "hip_attention_decode_bf16",
     "hip_attention_decode_workspace_bytes",
@@ -134,6 +136,10 @@ class QuantLibrary:
         L.hip_rope_fwd.argtypes = [i32, vp, vp, vp, vp, u32, u32, u32, u32]
         L.hip_embed_fwd.restype = i32
         L.hip_embed_fwd.argtypes = [i32, vp, vp, vp, i32, i32, i32]
+        L.hip_embed_ids_bf16.restype = i32
+        L.hip_embed_ids_bf16.argtypes = [vp, i32, vp, vp, i32, i32]
+        L.hip_decode_begin_bf16.restype = i32
+        L.hip_decode_begin_bf16.argtypes = [vp, i32, i32, vp, vp, i32]
         L.hip_embed_token_bf16.restype = i32
         L.hip_embed_token_bf16.argtypes = [vp, vp, vp, i32, i32]
         L.hip_qk_norm_rope_kv_bf16.restype = i32

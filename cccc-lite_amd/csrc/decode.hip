@@ -262,6 +262,22 @@ int hip_embed_token_bf16(const void* d_token, const void* W, void* y, int D, int
     return finish("embed_token_bf16");
 }
 
+int hip_embed_ids_bf16(const int* host_ids, int n, const void* W, void* y, int D, int n_rows)
+{
+    if (!host_ids || !W || !y || n <= 0 || n > EMBED_IDS || D <= 0 || D % 8 != 0 || n_rows <= 0) { return -1; }
+    EmbedIds ids;
+    std::copy(host_ids, host_ids + n, ids.id);
+    embed_ids_bf16_kernel<<<dim3(1, n), 256, 0, stream()>>>(ids, (const uint16_t*)W, (uint16_t*)y, D, n_rows);
+    return finish("embed_ids_bf16");
+}
+
+int hip_decode_begin_bf16(void* d_state, int token, int pos, const void* row, void* y, int D)
+{
+    if (!d_state || !row || !y || D <= 0 || D % 8 != 0) { return -1; }
+    step_begin_kernel<<<1, 256, 0, stream()>>>((int*)d_state, token, pos, (const uint16_t*)row, (uint16_t*)y, D);
+    return finish("decode_begin_bf16");
+}
+
 int hip_qk_norm_rope_kv_bf16(const void* q, const void* k, const void* v, const void* q_norm_w, const void* k_norm_w,
                              const void* cos_tab, const void* sin_tab, void* q_out, void* k_cache, void* v_cache,
                              int n_q_heads, int n_kv_heads, int head_dim, int t_kv, const void* d_pos, float epsilon)

@@ -852,6 +852,34 @@ static __global__ __launch_bounds__(256) void embed_bf16_kernel(const float* __r
     }
 }
 
+// The same for ids that come with the launch: a copy to the device in front of it is a blocking call of some 12 us.
+constexpr int EMBED_IDS = 256;
+struct EmbedIds
+{
+    int id[EMBED_IDS];
+};
+
+static __global__ __launch_bounds__(256) void embed_ids_bf16_kernel(const EmbedIds ids, const uint16_t* __restrict__ W, uint16_t* __restrict__ Y, int D, int n_rows)
+{
+    const int t = blockIdx.y;
+    const int id = min(max(ids.id[t], 0), n_rows - 1);
+    for (int c = blockIdx.x * 256 + threadIdx.x; c * 8 < D; c += gridDim.x * 256)
+    {
+        *(u32x4*)(Y + (size_t)t * D + c * 8) = *(const u32x4*)(W + (size_t)id * D + c * 8);
+    }
+}
+
+// Where a decode step starts from: (token, position) into the step state and one row into the activation.
+static __global__ __launch_bounds__(256) void step_begin_kernel(int* __restrict__ d_state, int token, int pos, const uint16_t* __restrict__ row, uint16_t* __restrict__ y, int D)
+{
+    if (threadIdx.x == 0)
+    {
+        d_state[0] = token;
+        d_state[1] = pos;
+    }
+    for (int c = threadIdx.x; c * 8 < D; c += 256) { *(u32x4*)(y + c * 8) = *(const u32x4*)(row + c * 8); }
+}
+
 // ------------------------------------------------------------------------------------------
 // Per-head q/k RMSNorm + RoPE + KV-cache append for one new token (head_dim 128).
 // One wave per head: lanes 0..63 hold the rotation pairs (i, i + 64).

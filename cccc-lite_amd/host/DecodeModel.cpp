@@ -1,6 +1,7 @@
 #include "DecodeModel.h"
 #include "../../include/cccc_hip_quant.h"
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -275,10 +276,10 @@ size_t DecodeModel::weightBytes() const
 
 int DecodeModel::reset(int token, int pos)
 {
-    const int state[2] = { token, pos };
-    if (GpuControl::copyHostToDevice(d_state_, state, sizeof(state)) != 0) { return 1; }
-    // a step starts from the embedding of its token: the previous step's greedy pick leaves it behind, a reset fetches it
-    return hip_embed_token_bf16(d_state_, emb_->data(), x_->data(), cfg_.hidden, cfg_.vocab);
+    // a step starts from the embedding of its token: the previous step's greedy pick leaves it behind, a reset fetches it (a token
+    // outside the vocabulary gets the nearest row)
+    const int row = std::min(std::max(token, 0), cfg_.vocab - 1);
+    return hip_decode_begin_bf16(d_state_, token, pos, (const char*)emb_->data() + (size_t)row * cfg_.hidden * 2, x_->data(), cfg_.hidden);
 }
 
 int DecodeModel::currentToken()
@@ -450,13 +451,16 @@ int DecodeModel::prefillPiece(const int* tokens, int n, int pos0, bool last)
         for (auto* m : { &pf_.k, &pf_.v }) { *m = make(kv_out, n, BFLOAT16, gpu_); }
         for (auto* m : { &pf_.gate, &pf_.up, &pf_.gated }) { *m = make(c.inter, n, BFLOAT16, gpu_); }
     }
-    // Every kernel of the piece goes to the library's stream of this thread.  The host copies below are the mirror's blocking
-    // copies, which wait for that stream first (GpuControl::copyHostToDevice): nothing an earlier launch still reads
-    // (pf_.ids, the step state) is overwritten under it, and a copy has landed before anything is launched behind it.
-    const hipStream_t stream = (hipStream_t)hip_quant_get_stream();
-    std::vector<float> ids(tokens, tokens + n);
-    if (GpuControl::copyHostToDevice(pf_.ids->data(), ids.data(), (size_t)n * sizeof(float)) != 0) { return 1; }
-    int rc = hip_embed_fwd((int)BFLOAT16, pf_.ids->data(), emb_->data(), pf_.x->data(), c.hidden, n, 1);
+    // Every kernel of the piece goes to the library's stream of this thread, and the step state and the ids of a short piece with
+    // them.  More ids are copied by the mirror's blocking copy, which waits for that stream first (GpuControl::copyHostToDevice):
+    // nothing an earlier launch still reads is overwritten under it, and the copy has landed before anything is launched behind it.
+    int rc = hip_embed_ids_bf16(tokens, n, emb_->data(), pf_.x->data(), c.hidden, c.vocab);
+    if (rc < 0)
+    {
+        std::vector<float> ids(tokens, tokens + n);
+        if (GpuControl::copyHostToDevice(pf_.ids->data(), ids.data(), (size_t)n * sizeof(float)) != 0) { return 1; }
+        rc = hip_embed_fwd((int)BFLOAT16, pf_.ids->data(), emb_->data(), pf_.x->data(), c.hidden, n, 1);
+    }
     // y [n][n_out] = x [n][K] W^T: the weight is the A operand, transposed, as cccc's batchedMul passes it (scripts/convert_weights.py:492)
     auto linear = [&](const Matrix& W, int n_out, int K, const Matrix& x, Matrix& y) {
         return gpu_->rocblas_->gemm(MATRIX_TRANS, MATRIX_NO_TRANS, n_out, n, K, 1.0f, W.data(), W.getDataType(), K, W.getQuantScale(),
@@ -561,16 +565,16 @@ int DecodeModel::prefillPiece(const int* tokens, int n, int pos0, bool last)
     }
     if (rc != 0 || !last) { return rc; }
     // the head runs on the last token's state: its greedy pick becomes the current token at position pos0 + n
-    // (the row copy rides on the launch stream behind the last layer)
-    const int state[2] = { tokens[n - 1], pos0 + n - 1 };
-    if (hipMemcpyAsync(x_->data(), (const char*)pf_.x->data() + (size_t)(n - 1) * c.hidden * 2, (size_t)c.hidden * 2, hipMemcpyDeviceToDevice, stream) != hipSuccess) { return 1; }
-    if (GpuControl::copyHostToDevice(d_state_, state, sizeof(state)) != 0) { return 1; }
-    return head();
+    // (the state travels with a launch: a blocking copy would keep the host until the last layer has run, and the GPU idle after it)
+    rc = hip_decode_begin_bf16(d_state_, tokens[n - 1], pos0 + n - 1, (const char*)pf_.x->data() + (size_t)(n - 1) * c.hidden * 2, x_->data(), c.hidden);
+    return rc != 0 ? rc : head();
 }
 
 double DecodeModel::run(int n_steps, int use_graph)
 {
-    if (n_steps <= 0 || currentPos() < 0 || currentPos() + n_steps > cfg_.t_kv) { return -2.0; }    // would run past the KV cache
+    if (n_steps <= 0) { return -2.0; }
+    const int pos = currentPos();
+    if (pos < 0 || (long long)pos + n_steps > cfg_.t_kv) { return -2.0; }    // would run past the KV cache
     hipEvent_t e0, e1;
     if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) { return -1.0; }
     double result = -1.0;

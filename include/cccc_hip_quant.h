@@ -331,6 +331,13 @@ C_EXPORT int hip_add_rms_norm_bf16(const void* a, const void* b, void* sum, cons
 /* Embedding row of token *d_token (int32 in device memory) -> y bf16 [D]. */
 C_EXPORT int hip_embed_token_bf16(const void* d_token, const void* W, void* y, int D, int n_rows);
 
+/* Embedding rows of n <= 256 token ids in host memory, which travel with the launch -> y bf16 [n][D] (D % 8 == 0, 16-byte aligned). */
+C_EXPORT int hip_embed_ids_bf16(const int* host_ids, int n, const void* W, void* y, int D, int n_rows);
+
+/* Start of a decode step without a copy from the host: d_state (int32 [2], device) = (token, pos), y bf16 [D] = row [D] (device;
+ * D % 8 == 0, 16-byte aligned). */
+C_EXPORT int hip_decode_begin_bf16(void* d_state, int token, int pos, const void* row, void* y, int D);
+
 /* Arg-max of n BF16 values (lowest index on ties) into *d_index (int32, device); when d_pos is not
  * NULL, *d_pos is incremented afterwards (the step counter of a decode loop).  `workspace`:
  * hip_argmax_workspace_bytes(n) bytes of device memory for the per-block candidates. */

@@ -1,0 +1,42 @@
+"""Token ids and the step state that travel with a launch."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from gpu_util import from_dev, to_dev
+
+pytestmark = pytest.mark.gpu
+ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+
+
+@pytest.mark.parametrize("n,D", [(1, 8), (3, 2056), (256, 64)])
+def test_rows_of_host_ids(gpu, oracle, n, D):
+    """The rows byte for byte, ids outside the table to its nearest row, nothing behind the last one; more ids than fit are refused."""
+    torch, dev, lib = gpu
+    rng = np.random.default_rng(n)
+    rows = 50
+    W = rng.integers(0, 1 << 16, size=(rows, D), dtype=np.uint16)
+    ids = rng.integers(0, rows, size=n).astype(np.int32)
+    ids[-1] = rows + 7
+    if n > 1: ids[0] = -3
+    wd, y = to_dev(torch, dev, W), torch.zeros(n * D + 8, dtype=torch.int16, device=dev)
+    assert lib.c.hip_embed_ids_bf16(ids.ctypes.data_as(ctypes.c_void_p), n, ptr(wd), ptr(y), D, rows) == 0
+    ids_then = ids.copy()
+    ids[:] = 0                                      # the launch has its own copy
+    torch.cuda.synchronize()
+    got = from_dev(y, np.uint16)
+    assert np.array_equal(got[:n * D].reshape(n, D), W[np.clip(ids_then, 0, rows - 1)]) and not got[n * D:].any()
+    assert lib.c.hip_embed_ids_bf16(ids.ctypes.data_as(ctypes.c_void_p), 257, ptr(wd), ptr(y), D, rows) == -1
+    assert lib.c.hip_embed_ids_bf16(ids.ctypes.data_as(ctypes.c_void_p), n, ptr(wd), ptr(y), D + 1, rows) == -1
+
+
+@pytest.mark.parametrize("D", [8, 2048, 4104])
+def test_state_and_row_of_a_step(gpu, D):
+    torch, dev, lib = gpu
+    row = to_dev(torch, dev, np.arange(D, dtype=np.uint16))
+    state, y = torch.full((3,), 9, dtype=torch.int32, device=dev), torch.zeros(D + 8, dtype=torch.int16, device=dev)
+    assert lib.c.hip_decode_begin_bf16(ptr(state), 5, 77, ptr(row), ptr(y), D) == 0
+    torch.cuda.synchronize()
+    assert state.tolist() == [5, 77, 9] and torch.equal(y[:D], row) and not y[D:].any()
+    assert lib.c.hip_decode_begin_bf16(ptr(state), 5, 77, ptr(row), ptr(y), D + 4) == -1
