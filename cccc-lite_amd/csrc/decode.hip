@@ -69,21 +69,25 @@ int launch_fused_bf16(const FusedLinearArgs& a, int n_groups)
     return finish("quant_linear_fused");
 }
 
-// FP4 block-scale weights: two rows per wave, U = 2 batches for rows of up to 4096 elements (one k-step of 2048 per
-// lane and row is 1 KiB), 8-wave workgroups for very tall weights, as for FP8.
+// FP4 block-scale weights: two rows per wave, U = 2 batches for rows beyond 8192 elements (one k-step of 2048 per lane and row is 1 KiB),
+// 8-wave workgroups for very tall weights, as for FP8, and for long rows where they still give every CU one: the activation (28 KiB
+// at 14336) is then staged once for sixteen rows.  A gate / up pair has half the bytes of an FP8 one in flight per wave and takes a fifth
+// workgroup per CU.  Step of an 8-layer 4096 / 14336 model in a graph: 376.4 us with four and 4-wave workgroups, 371.8 with
+// five (six 373, seven 376; inter 8192 325.2 -> 318.3, 12288 360.0 -> 356.0, 11008 349 -> 348), 368.2 with 8 waves for down as well.
 template <int BLOCK>
 int launch_fused_fp4(const FusedLinearArgs& a, int n_groups)
 {
     const size_t lds = (size_t)((a.K + 2047) / 2048) * 4096;
     if (lds > 64 * 1024) { return -1; }
     const int cus = cu_count();
-    const int want4 = (n_groups + 3) / 4;
-    if (n_groups >= cus * 64)
+    const int want4 = (n_groups + 3) / 4, want8 = (n_groups + 7) / 8;
+    if (n_groups >= cus * 64) { gemv4_fused_kernel<BLOCK, 2, 8><<<want8 < cus * 2 ? want8 : cus * 2, 512, lds, stream()>>>(a); }
+    else if (a.K <= 8192)
     {
-        const int want = (n_groups + 7) / 8;
-        gemv4_fused_kernel<BLOCK, 2, 8><<<want < cus * 2 ? want : cus * 2, 512, lds, stream()>>>(a);
+        const int cap = cus * (a.pair ? 5 : 4);
+        gemv4_fused_kernel<BLOCK, 1, 4><<<want4 < cap ? want4 : cap, 256, lds, stream()>>>(a);
     }
-    else if (a.K <= 8192) { gemv4_fused_kernel<BLOCK, 1, 4><<<want4 < cus * 4 ? want4 : cus * 4, 256, lds, stream()>>>(a); }
+    else if (n_groups >= cus * 8) { gemv4_fused_kernel<BLOCK, 2, 8><<<want8 < cus * 2 ? want8 : cus * 2, 512, lds, stream()>>>(a); }
     else { gemv4_fused_kernel<BLOCK, 2, 4><<<want4 < cus * 4 ? want4 : cus * 4, 256, lds, stream()>>>(a); }
     return finish("quant_linear_fused");
 }
