@@ -935,7 +935,7 @@ def main():
         kc, vc = torch.randn(8, T, 128, device=dev).to(torch.bfloat16), torch.randn(8, T, 128, device=dev).to(torch.bfloat16)
         y = torch.zeros(T, 32, 128, device=dev, dtype=torch.bfloat16)
         p = lambda x: ctypes.c_void_p(x.data_ptr())
-        launch = lambda: lib.c.hip_attention_prefill_fused_bf16(p(q), p(kc), p(vc), p(y), 32, 8, 128, T, T, 0)
+        launch = lambda: lib.c.hip_attention_prefill_bf16(p(q), p(kc), p(vc), p(y), 32, 8, 128, T, T, 0)
         for _ in range(args.warmup):
             assert launch() == 0
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)

@@ -78,6 +78,16 @@ bool prefill_args_ok(const void* q, const void* k_cache, const void* v_cache, co
     const int group = n_q_heads / n_kv_heads;
     return group == 1 || group == 2 || group == 4;
 }
+
+// attn_prefill_tile_kernel: 64 rows of a kv head per workgroup
+template <int FORM>
+void launch_tiles(const void* q, const void* k_cache, const void* v_cache, void* y, int n_q_heads, int n_kv_heads, int t_kv, int n_tokens, int pos0, int n_ranges, const PrefillRanges& ranges)
+{
+    const int group = n_q_heads / n_kv_heads, tile = 64 / group;
+    const dim3 grid((unsigned)((long long)((n_tokens + tile - 1) / tile) * n_kv_heads), n_ranges);
+    const auto kernel = group == 4 ? attn_prefill_tile_kernel<4, FORM> : group == 2 ? attn_prefill_tile_kernel<2, FORM> : attn_prefill_tile_kernel<1, FORM>;
+    kernel<<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, (uint16_t*)y, n_q_heads, t_kv, n_tokens, pos0, 1.0f / sqrtf(128.0f), ranges);
+}
 }    // namespace
 
 int hip_qk_norm_rope_kv_rows_bf16(const void* q, const void* k, const void* v, const void* q_norm_w, const void* k_norm_w,
@@ -116,8 +126,12 @@ int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v
                                                              n_q_heads, t_kv, n_tokens, pos0, scale, ranges)
 #define CCQ_ATTN_PREFILL_GROUPS(PASS)                                                                                                              \
     group == 4 ? CCQ_ATTN_PREFILL(4, PASS) : group == 2 ? CCQ_ATTN_PREFILL(2, PASS) : CCQ_ATTN_PREFILL(1, PASS)
+    // Whole rows in one piece go by tiles of 64 rows, except where one query head per kv head leaves tiles of 16 tokens a CU each: those have two
+    // waves on half the rows.  The same bits either way.  4 / 4 heads, 16 tokens -> 64 rows: 1024 tokens (256 tiles of 16) behind 3000 90.1 / 93.6 us,
+    // from 0 26.3 / 28.2; 1100 tokens (276) behind 3000 154.7 / 95.2, from 0 33.1 / 30.0.  Two heads 1 to 15 % ahead on 64 rows at any size, four 15 to 30.
     if (pos0 + n_tokens <= PF_SHORT * PF_KEYS) { CCQ_ATTN_PREFILL_GROUPS(3); }
-    else if (!scratch) { CCQ_ATTN_PREFILL_GROUPS(0); }
+    else if (!scratch && group == 1 && tiles <= cu_count()) { CCQ_ATTN_PREFILL(1, 0); }
+    else if (!scratch) { launch_tiles<PF_WHOLE_ROW>(q, k_cache, v_cache, y, n_q_heads, n_kv_heads, t_kv, n_tokens, pos0, 1, ranges); }
     else
     {
         CCQ_ATTN_PREFILL_GROUPS(1);
@@ -134,28 +148,19 @@ int hip_attention_prefill_fused_bf16(const void* q, const void* k_cache, const v
                                      int n_q_heads, int n_kv_heads, int head_dim, int t_kv, int n_tokens, int pos0)
 {
     if (!prefill_args_ok(q, k_cache, v_cache, y, n_q_heads, n_kv_heads, head_dim, t_kv, n_tokens, pos0)) { return -1; }
-    const int group = n_q_heads / n_kv_heads, tile = 64 / group;
+    const int tile = 64 * n_kv_heads / n_q_heads;
     const long long tiles = (long long)((n_tokens + tile - 1) / tile) * n_kv_heads;
-    const float scale = 1.0f / sqrtf(128.0f);
     const size_t outputs = (size_t)n_tokens * n_q_heads;
     const AttentionRanges split = fused_attention_ranges(tiles, pos0 + n_tokens, outputs);
     char* const scratch = split.n > 1 ? range_scratch() : nullptr;
     const PrefillRanges ranges = { split.per, (float2*)(scratch + (size_t)split.n * outputs * 128 * sizeof(float)), (float*)scratch };
-    const dim3 grid((unsigned)tiles, scratch ? split.n : 1);
-#define CCQ_ATTN_PREFILL(G, RANGE)                                                                                                                       \
-    attn_prefill_fused_kernel<G, RANGE><<<grid, 256, 0, stream()>>>((const uint16_t*)q, (const uint16_t*)k_cache, (const uint16_t*)v_cache, (uint16_t*)y, \
-                                                                    n_q_heads, t_kv, n_tokens, pos0, scale, ranges)
-#define CCQ_ATTN_PREFILL_GROUPS(RANGE)                                                                                                             \
-    group == 4 ? CCQ_ATTN_PREFILL(4, RANGE) : group == 2 ? CCQ_ATTN_PREFILL(2, RANGE) : CCQ_ATTN_PREFILL(1, RANGE)
-    if (!scratch) { CCQ_ATTN_PREFILL_GROUPS(false); }
+    if (!scratch) { launch_tiles<PF_ONE_PASS>(q, k_cache, v_cache, y, n_q_heads, n_kv_heads, t_kv, n_tokens, pos0, 1, ranges); }
     else
     {
-        CCQ_ATTN_PREFILL_GROUPS(true);
+        launch_tiles<PF_ONE_PASS_RANGE>(q, k_cache, v_cache, y, n_q_heads, n_kv_heads, t_kv, n_tokens, pos0, split.n, ranges);
         const long long blk = ((long long)outputs * 32 + 255) / 256, cap = (long long)cu_count() * 16;
         attn_prefill_fused_combine_kernel<<<(unsigned)(blk < cap ? blk : cap), 256, 0, stream()>>>(ranges, (uint16_t*)y, n_q_heads, n_tokens, pos0, tile);
     }
-#undef CCQ_ATTN_PREFILL_GROUPS
-#undef CCQ_ATTN_PREFILL
     return finish("attention_prefill_fused");
 }
 

@@ -184,7 +184,7 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 // blocks of keys are split over gridDim.y workgroups, `per` blocks (an even number) each, and the passes are launches of their own:
 // PASS 1 leaves (max, sum) per range, head and token, PASS 2 merges those of all the ranges a token tile has -- the probabilities are rounded
 // with the row's own maximum and sum, as in one piece -- and leaves FP32 sums, which attn_prefill_combine_kernel adds and rounds.  PASS 0 is
-// both passes over all the keys.
+// both passes over all the keys (one query head per kv head and at most one workgroup per CU: else attn_prefill_tile_kernel, the same bits).
 // PASS 3: the whole context is at most PF_SHORT blocks.  Then all keys and values are requested at once and stay in LDS, and the scores stay in
 // registers between the passes: one trip to memory and a few barriers where the pipelines of PASS 0 start up twice (100 tokens of 32 / 8 heads
 // 10.2 us on PASS 0, now 8.8; with the scores multiplied again in loops instead 9.4).  Its LDS leaves a CU one workgroup, where PASS 0

@@ -536,7 +536,7 @@ int DecodeModel::prefillPiece(const int* tokens, int n, int pos0, bool last)
         }
         if (rc == 0)
         {
-            const auto attention = exact_attention_ ? hip_attention_prefill_bf16 : hip_attention_prefill_fused_bf16;
+            const auto attention = fused_prompt_attention_ && !exact_attention_ ? hip_attention_prefill_fused_bf16 : hip_attention_prefill_bf16;
             rc = attention(pf_.q_rot->data(), k_cache_[li]->data(), v_cache_[li]->data(), pf_.att->data(), c.n_q, c.n_kv, c.head_dim, c.t_kv, n, pos0);
         }
         // o, the residual add and the norm behind it: one call where the GEMM splits its k range (short prompts), else two

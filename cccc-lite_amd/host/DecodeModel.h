@@ -72,10 +72,13 @@ public:
     // the same bytes without quantizing again.  0 ok, -1 the file could not be written.
     int saveNamedWeights(const std::string& filename);
 
-    // false (default): two-launch attention with the norm / RoPE / append folded in and FP32 probabilities (prompts: BF16, rounded before the
-    // division by their sum);
+    // false (default): two-launch attention with the norm / RoPE / append folded in and FP32 probabilities;
     // true: the reference's rounding points throughout (BF16 probabilities over the whole row; three launches).
     void setExactAttention(bool exact) { exact_attention_ = exact; }
+    // Prompts.  false (default): the attention with the reference's rounding points, whatever setExactAttention says;
+    // true: unless exact attention is set, one pass over the keys with the BF16 probabilities rounded in front of the division by their sum
+    // (hip_attention_prefill_fused_bf16: as close to 64 bits, not the reference's bits).
+    void setFusedPromptAttention(bool fused) { fused_prompt_attention_ = fused; }
     // Per-head RMSNorm of q and k in front of the rotation: on for Qwen3-style models (default), off for models without
     // W_qnorm / W_knorm such as Llama-3.1 (has_qknorm in scripts/convert_weights.py:488-530).  loadNamedWeights sets it
     // from what the file holds.
@@ -96,7 +99,7 @@ public:
     // The prompt phase: n tokens at positions pos0 .. pos0 + n - 1 in one pass per layer -- what the reference's graph does
     // when cccc-llm feeds it the whole prompt (cccc-llm/cccc-llm.cpp:589-618): the linears through Rocblas::gemm with n
     // columns (the matrix-core GEMM from 48 tokens on), the per-head norm / RoPE / cache append, the causal attention with
-    // the reference's rounding points, residual adds and the SwiGLU product as row kernels.  Afterwards the caches hold
+    // the reference's rounding points (setFusedPromptAttention), residual adds and the SwiGLU product as row kernels.  Afterwards the caches hold
     // the prompt, the current token is the greedy pick after its last token and the position is pos0 + n: step() carries
     // on from there.  Prompts longer than 2048 tokens go through in pieces of 2048.  0 ok, -1 bad arguments.
     int prefill(const int* tokens, int n_tokens, int pos0);
@@ -136,6 +139,7 @@ private:
     int head();                             // final norm + lm_head + greedy pick + next embedding on x_
     unsigned long long attn_ws_bytes_ = 0;
     bool exact_attention_ = false;
+    bool fused_prompt_attention_ = false;
     bool qk_norm_ = true;
     bool tied_lm_head_ = false;
     bool repack_linears_ = false;

@@ -231,6 +231,7 @@ int cccc_matrix_save_named(void* m, const char* name, const char* path)
 }
 
 void cccc_decode_set_exact_attention(void* m, int exact) { ((DecodeModel*)m)->setExactAttention(exact != 0); }
+void cccc_decode_set_fused_prompt_attention(void* m, int fused) { ((DecodeModel*)m)->setFusedPromptAttention(fused != 0); }
 void cccc_decode_set_qk_norm(void* m, int on) { ((DecodeModel*)m)->setQkNorm(on != 0); }
 int cccc_decode_qk_norm(void* m) { return ((DecodeModel*)m)->qkNorm() ? 1 : 0; }
 void cccc_decode_set_repack_linears(void* m, int on) { ((DecodeModel*)m)->setRepackLinears(on != 0); }

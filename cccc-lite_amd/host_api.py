@@ -72,6 +72,7 @@ class HostLibrary:
         L.cccc_decode_prefill.restype = i32; L.cccc_decode_prefill.argtypes = [vp, ctypes.POINTER(ctypes.c_int), i32, i32]
         L.cccc_decode_set_qk_norm.restype = None; L.cccc_decode_set_qk_norm.argtypes = [vp, i32]
         L.cccc_decode_qk_norm.restype = i32; L.cccc_decode_qk_norm.argtypes = [vp]
+        L.cccc_decode_set_fused_prompt_attention.restype = None; L.cccc_decode_set_fused_prompt_attention.argtypes = [vp, i32]
         L.cccc_decode_set_repack_linears.restype = None; L.cccc_decode_set_repack_linears.argtypes = [vp, i32]
         L.cccc_decode_set_tied_lm_head.restype = None; L.cccc_decode_set_tied_lm_head.argtypes = [vp, i32]
         L.cccc_decode_tied_lm_head.restype = i32; L.cccc_decode_tied_lm_head.argtypes = [vp]
@@ -313,9 +314,13 @@ class DecodeModel:
 
     def set_exact_attention(self, exact: bool) -> None:
         """True: separate norm / RoPE / append launch and BF16 probabilities (the reference's rounding
-        points); False (default): the two-launch attention with FP32 probabilities (prompts: one pass over the
-        keys, BF16 probabilities rounded before the division by their sum)."""
+        points); False (default): the two-launch attention with FP32 probabilities."""
         self.lib.c.cccc_decode_set_exact_attention(self.handle, 1 if exact else 0)
+
+    def set_fused_prompt_attention(self, fused: bool) -> None:
+        """Prompts of a model without exact attention.  False (default): the attention with the reference's rounding points;
+        True: one pass over the keys, BF16 probabilities rounded in front of the division by their sum."""
+        self.lib.c.cccc_decode_set_fused_prompt_attention(self.handle, 1 if fused else 0)
 
     def set_qk_norm(self, on: bool) -> None:
         """Per-head RMSNorm of q and k in front of the rotation (Qwen3: on, the default; Llama-3.1: off)."""
