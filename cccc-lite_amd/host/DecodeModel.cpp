@@ -1,7 +1,6 @@
 #include "DecodeModel.h"
 #include "../../include/cccc_hip_quant.h"
 #include <hip/hip_runtime.h>
-#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -276,10 +275,11 @@ size_t DecodeModel::weightBytes() const
 
 int DecodeModel::reset(int token, int pos)
 {
-    // a step starts from the embedding of its token: the previous step's greedy pick leaves it behind, a reset fetches it (a token
-    // outside the vocabulary gets the nearest row)
-    const int row = std::min(std::max(token, 0), cfg_.vocab - 1);
-    return hip_decode_begin_bf16(d_state_, token, pos, (const char*)emb_->data() + (size_t)row * cfg_.hidden * 2, x_->data(), cfg_.hidden);
+    // (a copy and not a launch: the state is in place when this returns, whatever stream or thread reads it next)
+    const int state[2] = { token, pos };
+    if (GpuControl::copyHostToDevice(d_state_, state, sizeof(state)) != 0) { return 1; }
+    // a step starts from the embedding of its token: the previous step's greedy pick leaves it behind, a reset fetches it
+    return hip_embed_token_bf16(d_state_, emb_->data(), x_->data(), cfg_.hidden, cfg_.vocab);
 }
 
 int DecodeModel::currentToken()

@@ -94,7 +94,9 @@ public:
     void setRepackLinears(bool on) { repack_linears_ = on; }
     bool tiedLmHead() const { return tied_lm_head_; }
     bool qkNorm() const { return qk_norm_; }
-    int reset(int token, int pos);          // sets the device-side token / position and fetches the token's embedding (KV caches are kept)
+    // Sets the device-side token / position, in place when it returns, and fetches the token's embedding, a launch on the calling thread's stream (KV
+    // caches are kept).
+    int reset(int token, int pos);
     int step();                             // enqueues one decode step; the next token replaces the current one
     // The prompt phase: n tokens at positions pos0 .. pos0 + n - 1 in one pass per layer -- what the reference's graph does
     // when cccc-llm feeds it the whole prompt (cccc-llm/cccc-llm.cpp:589-618): the linears through Rocblas::gemm with n

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from gpu_util import from_dev, to_dev
+from test_gpu_prefill import _fresh, dec  # noqa: F401 (dec: a fixture)
 
 pytestmark = pytest.mark.gpu
 ptr = lambda t: ctypes.c_void_p(t.data_ptr())
@@ -40,3 +41,33 @@ def test_state_and_row_of_a_step(gpu, D):
     torch.cuda.synchronize()
     assert state.tolist() == [5, 77, 9] and torch.equal(y[:D], row) and not y[D:].any()
     assert lib.c.hip_decode_begin_bf16(ptr(state), 5, 77, ptr(row), ptr(y), D + 4) == -1
+
+
+def test_state_of_a_reset_is_in_place_when_it_returns(gpu, pkg, dec):
+    """reset on a stream with work in front of it, then the state read and a graph run asked for on another: the new token and position, and a run past
+    the end of the cache refused."""
+    torch, dev, lib = gpu
+    host = pkg.host_api.host()
+    host.init(0)
+    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=64)
+    model = _fresh(pkg, host, cfg)
+    model.load(dec.make_model(cfg, 17))
+    model.reset(1, 0)
+    busy, other = (torch.cuda.Stream(device=dev) for _ in range(2))
+    lib.set_sync(False)
+    try:
+        assert lib.set_stream(busy.cuda_stream) == 0
+        with torch.cuda.stream(busy): torch.cuda._sleep(100_000_000)               # some 50 ms
+        model.reset(7, 60)
+        assert lib.set_stream(other.cuda_stream) == 0
+        assert (model.token, model.pos) == (7, 60)
+        assert lib_run(model, 5) == -2.0 and lib_run(model, 4) > 0
+        assert model.pos == 64
+        torch.cuda.synchronize()
+    finally:
+        lib.set_stream(None)
+        lib.set_sync(True)
+
+
+def lib_run(model, n):
+    return model.lib.c.cccc_decode_run(model.handle, n, 2)          # 2: with a graph whatever n is
