@@ -573,13 +573,6 @@ int DecodeModel::prefillPiece(const int* tokens, int n, int pos0, bool last)
 double DecodeModel::run(int n_steps, int use_graph)
 {
     if (n_steps <= 0) { return -2.0; }
-    const int pos = currentPos();
-    if (pos < 0 || (long long)pos + n_steps > cfg_.t_kv) { return -2.0; }    // would run past the KV cache
-    hipEvent_t e0, e1;
-    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) { return -1.0; }
-    double result = -1.0;
-    const int sync_before = hip_quant_set_sync(0);
-    const hipStream_t caller = (hipStream_t)hip_quant_get_stream();
     // A stream, a capture and an executable graph cost the host 0.25 ms (4 layers) to 0.75 ms (36), a replayed launch is up to 0.25 us faster
     // than a launched one (36 layers: 1.83 against 1.89 ms per step; 4 to 8 layers: nearly level), so a graph pays from 10 steps of 36
     // layers on and hardly ever for 4; the host records it while the first two steps run.  Wall time with a graph recorded first and
@@ -587,8 +580,17 @@ double DecodeModel::run(int n_steps, int use_graph)
     // 37.75 / 37.00; 16 steps of 4 layers 2.40 / 2.12 / 2.12, 20 of 8 layers 4.52 / 4.20 / 4.20.
     constexpr long long FEWEST = 360;           // steps x layers
     const int launched = use_graph == GRAPH_ALWAYS ? 0 : 2;
-    const bool pays = use_graph == GRAPH_ALWAYS || ((long long)n_steps * cfg_.layers >= FEWEST && n_steps > launched);
-    if (use_graph && pays)
+    const bool graph_pays = use_graph == GRAPH_ALWAYS || (use_graph && (long long)n_steps * cfg_.layers >= FEWEST && n_steps > launched);
+    // the graph's stream orders with no other: what a prompt or steps on any of them leave, the position too, is there first
+    if (graph_pays) { (void)hipDeviceSynchronize(); }
+    const int pos = currentPos();
+    if (pos < 0 || (long long)pos + n_steps > cfg_.t_kv) { return -2.0; }    // would run past the KV cache
+    hipEvent_t e0, e1;
+    if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess) { return -1.0; }
+    double result = -1.0;
+    const int sync_before = hip_quant_set_sync(0);
+    const hipStream_t caller = (hipStream_t)hip_quant_get_stream();
+    if (graph_pays)
     {
         hipStream_t stream = nullptr;
         hipGraph_t graph = nullptr;
@@ -598,7 +600,6 @@ double DecodeModel::run(int n_steps, int use_graph)
             hip_quant_set_sync(sync_before);
             return -4.0;
         }
-        (void)hipDeviceSynchronize();
         hip_quant_set_stream(stream);
         (void)hipEventRecord(e0, stream);
         bool ok = true;

@@ -69,5 +69,31 @@ def test_state_of_a_reset_is_in_place_when_it_returns(gpu, pkg, dec):
         lib.set_sync(True)
 
 
+def test_a_graph_run_behind_a_prompt_on_another_stream_sees_its_position(gpu, pkg, dec):
+    """A prompt's position is written by a launch: a graph run asked for on another stream waits for it before it looks whether its steps fit."""
+    torch, dev, lib = gpu
+    host = pkg.host_api.host()
+    host.init(0)
+    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=64)
+    model = _fresh(pkg, host, cfg)
+    model.load(dec.make_model(cfg, 17))
+    model.prefill([1] * 60)                                     # its buffers are there
+    model.reset(1, 0)
+    busy, other = (torch.cuda.Stream(device=dev) for _ in range(2))
+    prompt = np.arange(60, dtype=np.int32)
+    lib.set_sync(False)
+    try:
+        assert lib.set_stream(busy.cuda_stream) == 0
+        with torch.cuda.stream(busy): torch.cuda._sleep(100_000_000)
+        assert model.lib.c.cccc_decode_prefill(model.handle, prompt.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), 60, 0) == 0
+        assert lib.set_stream(other.cuda_stream) == 0
+        assert lib_run(model, 5) == -2.0 and lib_run(model, 4) > 0
+        assert model.pos == 64
+        torch.cuda.synchronize()
+    finally:
+        lib.set_stream(None)
+        lib.set_sync(True)
+
+
 def lib_run(model, n):
     return model.lib.c.cccc_decode_run(model.handle, n, 2)          # 2: with a graph whatever n is
