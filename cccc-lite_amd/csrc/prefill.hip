@@ -59,12 +59,11 @@ AttentionRanges fused_attention_ranges(long long tiles, int n_keys, size_t outpu
     return best;
 }
 
-// FP32 sums and statistics of the ranges: at most two workgroups of 64 rows per CU.  One size for both forms of the attention, which share
-// the buffer.
-char* range_scratch()
+// FP32 sums and statistics of the ranges: tiles of 64 rows, `side` workgroups per CU at most (two in one pass, one with whole rows).
+char* range_scratch(int side)
 {
     constexpr size_t ROW = 128 * sizeof(float) + sizeof(float2);
-    return (char*)fixed_scratch((size_t)cu_count() * 2 * 64 * ROW);
+    return (char*)fixed_scratch((size_t)cu_count() * side * 64 * ROW);
 }
 
 bool prefill_args_ok(const void* q, const void* k_cache, const void* v_cache, const void* y, int n_q_heads, int n_kv_heads, int head_dim, int t_kv, int n_tokens, int pos0)
@@ -118,7 +117,7 @@ int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v
     const float scale = 1.0f / sqrtf(128.0f);
     const size_t outputs = (size_t)n_tokens * n_q_heads;
     const AttentionRanges split = attention_ranges(tiles, pos0 + n_tokens, outputs);
-    char* const scratch = split.n > 1 ? range_scratch() : nullptr;
+    char* const scratch = split.n > 1 ? range_scratch(1) : nullptr;
     const PrefillRanges ranges = { split.per, (float2*)(scratch + (size_t)split.n * outputs * 128 * sizeof(float)), (float*)scratch };
     const dim3 grid((unsigned)tiles, scratch ? split.n : 1);
 #define CCQ_ATTN_PREFILL(G, PASS)                                                                                                                  \
@@ -152,7 +151,7 @@ int hip_attention_prefill_fused_bf16(const void* q, const void* k_cache, const v
     const long long tiles = (long long)((n_tokens + tile - 1) / tile) * n_kv_heads;
     const size_t outputs = (size_t)n_tokens * n_q_heads;
     const AttentionRanges split = fused_attention_ranges(tiles, pos0 + n_tokens, outputs);
-    char* const scratch = split.n > 1 ? range_scratch() : nullptr;
+    char* const scratch = split.n > 1 ? range_scratch(2) : nullptr;
     const PrefillRanges ranges = { split.per, (float2*)(scratch + (size_t)split.n * outputs * 128 * sizeof(float)), (float*)scratch };
     if (!scratch) { launch_tiles<PF_ONE_PASS>(q, k_cache, v_cache, y, n_q_heads, n_kv_heads, t_kv, n_tokens, pos0, 1, ranges); }
     else

@@ -24,8 +24,8 @@ int cu_count();
 // have to grow while the stream is being captured into a graph); callers then take a path that needs none.
 void* workspace(size_t bytes);
 
-// Device scratch memory of `bytes`, the same number in every call on a device: allocated by the first call of a (host thread, device,
-// stream), never replaced or freed after that.  nullptr when it cannot be allocated and always while the stream is being captured: a
+// Device scratch memory of `bytes`, which a caller derives from the device alone: one buffer per (host thread, device, stream, size), allocated by the
+// first call for it, never replaced or freed after that.  nullptr when it cannot be allocated and always while the stream is being captured: a
 // graph that held the buffer could be replayed on a stream of its own, beside launches that use it.
 void* fixed_scratch(size_t bytes);
 

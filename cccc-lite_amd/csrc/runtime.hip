@@ -3,6 +3,7 @@
 #include <atomic>
 #include <cstdio>
 #include <map>
+#include <tuple>
 #include <utility>
 
 namespace ccq
@@ -80,7 +81,7 @@ void* workspace(size_t bytes)
 
 void* fixed_scratch(size_t bytes)
 {
-    static thread_local std::map<std::pair<int, hipStream_t>, void*> buffers;
+    static thread_local std::map<std::tuple<int, hipStream_t, size_t>, void*> buffers;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     int dev = 0;
     if (hipStreamIsCapturing(stream(), &capture) != hipSuccess || capture != hipStreamCaptureStatusNone || hipGetDevice(&dev) != hipSuccess)
@@ -88,7 +89,7 @@ void* fixed_scratch(size_t bytes)
         (void)hipGetLastError();
         return nullptr;
     }
-    void*& p = buffers[{ dev, stream() }];
+    void*& p = buffers[{ dev, stream(), bytes }];
     if (!p && hipMalloc(&p, bytes) != hipSuccess)
     {
         (void)hipGetLastError();

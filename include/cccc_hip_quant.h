@@ -88,8 +88,8 @@ C_EXPORT int hip_absmax(const void* src, int src_type, unsigned int n, void* d_r
  * C of type HALF; the weight is dequantised to half, FP32 accumulation, one rounding to half).
  * `act_scale` is accepted and ignored (it only drives the W8A8 route, cccc/cublas_real.h:871-873).
  * Anything else (both operands quantized, FP4 with HALF, mixed 16-bit types, other C types) returns -1.
- * Device memory: the library allocates in two cases, hip_attention_prefill_bf16 / _fused_bf16 of a few tokens behind a long context
- * (see there) and a GEMM of 17 tokens or more (FP8, FP4 on a tiled copy, or HALF activations) whose output has too few tiles
+ * Device memory: the library allocates in two cases, hip_attention_prefill_bf16 / _fused_bf16 with too few token tiles x kv heads to fill
+ * the GPU (see there) and a GEMM of 17 tokens or more (FP8, FP4 on a tiled copy, or HALF activations) whose output has too few tiles
  * to fill the GPU; it then splits K over workgroups and keeps FP32 partial sums in a scratch buffer per (host thread, device,
  * stream) that grows on demand and lives until the process ends (at most 16 * M * N * 4 bytes).  While the stream is being
  * captured into a graph the buffer is never grown: the call then runs without the split (see hip_quant_workspace_reserve).
@@ -264,8 +264,8 @@ C_EXPORT int hip_qk_norm_rope_kv_rows_bf16(const void* q, const void* k, const v
  * already appended): scores rounded to BF16, keys past the token's position masked, FP32 softmax over the row, BF16
  * probabilities, y [T][n_q_heads][128] = bf16(V p) -- the rounding points of cccc/MatrixEx.cpp:3018-3104.  On the matrix
  * cores.  n_q_heads / n_kv_heads must be 1, 2 or 4.
- * Device memory: a few tokens behind a long context split the keys over workgroups; the FP32 partial sums go to a buffer of 66,560 bytes
- * per CU (17 MB on 256 CUs) that the first such call of a (host thread, device, stream) allocates and that is never grown,
+ * Device memory: where tokens / 16 x kv heads are at most half the CUs and the context is long (64 tokens of 8 kv heads from some 700 keys on), the keys
+ * are split over workgroups; the FP32 partial sums go to a buffer of 33,280 bytes per CU (8.5 MB on 256 CUs) that the first such call of a (host thread, device, stream) allocates and that is never grown,
  * replaced or freed.  A call that is captured into a graph never uses it and runs in one piece, the same value up to the order of the
  * FP32 sums: a graph holds no memory of the library and may be replayed on any stream. */
 C_EXPORT int hip_attention_prefill_bf16(const void* q, const void* k_cache, const void* v_cache, void* y,
@@ -274,7 +274,9 @@ C_EXPORT int hip_attention_prefill_bf16(const void* q, const void* k_cache, cons
 
 /* The same attention with the probabilities rounded to BF16 before the division by their FP32 sum and not behind it, in one pass over the
  * keys: to hip_attention_prefill_bf16 what hip_attention_decode_fused_bf16 is to hip_attention_decode_exact_bf16.  Scores rounded to
- * BF16, one rounding of the result.  Arguments, refusals, device memory and graph capture as hip_attention_prefill_bf16. */
+ * BF16, one rounding of the result.  Arguments and refusals as hip_attention_prefill_bf16.  Device memory likewise, in a buffer of its own of 66,560
+ * bytes per CU, for tiles of 64 query rows up to as many as CUs (256 tokens of 32 / 8 heads, 2048 of 4 / 1).  A captured call runs in one piece: other
+ * running maxima for the probabilities to be rounded against. */
 C_EXPORT int hip_attention_prefill_fused_bf16(const void* q, const void* k_cache, const void* v_cache, void* y,
                                               int n_q_heads, int n_kv_heads, int head_dim, int t_kv, int n_tokens, int pos0);
 

@@ -42,8 +42,8 @@ def test_follows_the_oracle_token_by_token(gpu, oracle, dec, n_q, n_kv, T, pos0,
         assert np.linalg.norm(dec.f(got[t]) - want) <= np.linalg.norm(bound), t
 
 
-def test_one_buffer_for_both_forms_and_one_piece_under_capture(gpu, oracle, dec):
-    """The two-pass form's ranges first, then more ranges of the one-pass form (the buffer has one size), then a captured call, which uses none
+def test_a_buffer_for_each_form_and_one_piece_under_capture(gpu, oracle, dec):
+    """The two-pass form's ranges first, then more ranges of the one-pass form in a larger buffer of its own, then a captured call, which uses none
     and is replayed beside eager calls.  Bad arguments are refused as by the two-pass form."""
     torch, dev, lib = gpu
     n_q, n_kv, T, pos0, t_kv = 32, 8, 256, 3000, 3300
@@ -77,3 +77,27 @@ def test_one_buffer_for_both_forms_and_one_piece_under_capture(gpu, oracle, dec)
     finally:
         lib.set_stream(None)
         lib.set_sync(True)
+
+
+def test_memory_of_the_ranges(gpu, oracle):
+    """On a stream of its own each form allocates what its header states, once: 33,280 bytes per CU for whole rows, 66,560 for one pass.  (4 MiB: the
+    granularity of an allocation.)"""
+    torch, dev, lib = gpu
+    n_q, n_kv, T, pos0, t_kv = 32, 8, 64, 3000, 3100
+    q, k, v = (to_dev(torch, dev, a) for a in inputs(oracle, n_q, n_kv, T, pos0, t_kv))
+    y = torch.zeros(T * n_q * 128, dtype=torch.int16, device=dev)
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    forms = ((lib.c.hip_attention_prefill_bf16, 33280), (lib.c.hip_attention_prefill_fused_bf16, 66560))
+    try:
+        for stream in (torch.cuda.Stream(device=dev), torch.cuda.Stream(device=dev)):       # the first loads the kernels
+            assert lib.set_stream(stream.cuda_stream) == 0
+            used = []
+            for form, per_cu in forms:
+                free = torch.cuda.mem_get_info(dev)[0]
+                for _ in range(2):
+                    assert form(ptr(q), ptr(k), ptr(v), ptr(y), n_q, n_kv, 128, t_kv, T, pos0) == 0
+                    stream.synchronize()
+                used.append(free - torch.cuda.mem_get_info(dev)[0])
+        for (_, per_cu), n in zip(forms, used): assert 0 < n <= per_cu * cus + (4 << 20), used
+    finally:
+        lib.set_stream(None)
