@@ -268,7 +268,7 @@ int hip_embed_token_bf16(const void* d_token, const void* W, void* y, int D, int
 
 int hip_embed_ids_bf16(const int* host_ids, int n, const void* W, void* y, int D, int n_rows)
 {
-    if (!host_ids || !W || !y || n <= 0 || n > EMBED_IDS || D <= 0 || D % 8 != 0 || n_rows <= 0) { return -1; }
+    if (!host_ids || !W || !y || n <= 0 || n > EMBED_IDS || D <= 0 || D % 8 != 0 || n_rows <= 0 || !aligned16(W) || !aligned16(y)) { return -1; }
     EmbedIds ids;
     std::copy(host_ids, host_ids + n, ids.id);
     embed_ids_bf16_kernel<<<dim3(1, n), 256, 0, stream()>>>(ids, (const uint16_t*)W, (uint16_t*)y, D, n_rows);
@@ -277,7 +277,7 @@ int hip_embed_ids_bf16(const int* host_ids, int n, const void* W, void* y, int D
 
 int hip_decode_begin_bf16(void* d_state, int token, int pos, const void* row, void* y, int D)
 {
-    if (!d_state || !row || !y || D <= 0 || D % 8 != 0) { return -1; }
+    if (!d_state || !row || !y || D <= 0 || D % 8 != 0 || !aligned16(row) || !aligned16(y)) { return -1; }
     step_begin_kernel<<<1, 256, 0, stream()>>>((int*)d_state, token, pos, (const uint16_t*)row, (uint16_t*)y, D);
     return finish("decode_begin_bf16");
 }

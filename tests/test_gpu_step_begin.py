@@ -30,6 +30,8 @@ def test_rows_of_host_ids(gpu, oracle, n, D):
     assert np.array_equal(got[:n * D].reshape(n, D), W[np.clip(ids_then, 0, rows - 1)]) and not got[n * D:].any()
     assert lib.c.hip_embed_ids_bf16(ids.ctypes.data_as(ctypes.c_void_p), 257, ptr(wd), ptr(y), D, rows) == -1
     assert lib.c.hip_embed_ids_bf16(ids.ctypes.data_as(ctypes.c_void_p), n, ptr(wd), ptr(y), D + 1, rows) == -1
+    for w, out in ((wd.view(-1)[1:], y), (wd, y[1:]), (wd.view(-1)[4:], y)):            # off their 16 bytes
+        assert lib.c.hip_embed_ids_bf16(ids.ctypes.data_as(ctypes.c_void_p), n, ptr(w), ptr(out), D, rows - 1) == -1
 
 
 @pytest.mark.parametrize("D", [8, 2048, 4104])
@@ -41,6 +43,8 @@ def test_state_and_row_of_a_step(gpu, D):
     torch.cuda.synchronize()
     assert state.tolist() == [5, 77, 9] and torch.equal(y[:D], row) and not y[D:].any()
     assert lib.c.hip_decode_begin_bf16(ptr(state), 5, 77, ptr(row), ptr(y), D + 4) == -1
+    for r, out in ((row[1:], y), (row, y[1:]), (row, y[4:])):                           # off their 16 bytes
+        assert lib.c.hip_decode_begin_bf16(ptr(state), 5, 77, ptr(r), ptr(out), D) == -1
 
 
 def test_state_of_a_reset_is_in_place_when_it_returns(gpu, pkg, dec):
