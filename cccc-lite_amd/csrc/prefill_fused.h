@@ -221,6 +221,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tile_kernel(const uint16_
 #pragma unroll
         for (int h = 0; h < 2; h++)
         {
+            if (masked && b >= group_blocks[h]) { continue; }           // none of the group's tokens sees the block
             const float off = m[h] > -INFINITY ? -m[h] * PF_LOG2E : 0.0f;      // -inf: the row has seen no key yet, every weight is 2^-inf = 0
             float p[8];
 #pragma unroll
