@@ -27,7 +27,7 @@ namespace ccq
 // 111 / 78 / 53, 512 behind 3000 103 / 84 / 52, 1024 behind 3000 165 / 120 / 78; 8 / 8 heads, 2048 from 0 103 / 51 / 33.  There each row group
 // read the keys twice, key and value rows went through registers with 32 lines per load instruction, and values were transposed by the VALU.
 // LDS: chunk c (16 bytes) of key row r lies at c ^ (r % 16), of value row r at c ^ (2 (r % 8)): the operand reads hit all banks.
-// A block's rows past the last written one repeat that row; their weight is 0.
+// A block's rows past the last written one repeat that row; their weight is 0 and their values are cleared in front of the products.
 constexpr float PF_LAG = 6.0f;
 
 typedef short tr_b16x4 __attribute__((ext_vector_type(4)));
@@ -166,7 +166,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tile_kernel(const uint16_
             const uint2 lo = read_transposed(p), hi = read_transposed(p + 16 * 256);
             vf[d] = u32x4{ lo.x, lo.y, hi.x, hi.y };
         }
-        if (WHOLE_ROW && masked && (b + 1) * PF_KEYS > n_written)
+        if (masked && (b + 1) * PF_KEYS > n_written)
         {
             // rows past the last written one weigh 0, but 0 times a repeated infinity is NaN
             const int key = b * PF_KEYS + 32 * kh + 4 * g;
