@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_tile_kernel(const uint16_
             const float mine = pf_exp2((m[h] - base) * PF_LOG2E);                   // 2^-inf = 0 for a half without a key
             const float sum = l[h] * mine + other.y * pf_exp2((other.x - base) * PF_LOG2E);
             if (RANGE && kh == 0 && g == 0 && tok[h] < n_tokens) { ranges.stats[((size_t)blockIdx.y * n_q + head[h]) * n_tokens + tok[h]] = make_float2(top, sum); }
-            const float by = RANGE ? mine : mine / sum;
+            const float by = RANGE ? mine : sum > 0.0f ? mine / sum : 0.0f;         // a row of scores of -inf gives 0, as in attn_prefill_kernel
 #pragma unroll
             for (int d = 0; d < 8; d++) { out[h][d] *= by; }
         }
@@ -428,15 +428,16 @@ static __global__ __launch_bounds__(256) void attn_prefill_fused_combine_kernel(
             }
             float top = m;
 #pragma unroll
-            for (int r = 0; r < 8; r++) { top = fmaxf(top, stat[r].x); }         // finite: a token sees key 0
-            const float shrink = pf_exp2((m - top) * PF_LOG2E);
+            for (int r = 0; r < 8; r++) { top = fmaxf(top, stat[r].x); }
+            const float base = top > -INFINITY ? top : 0.0f;
+            const float shrink = pf_exp2((m - base) * PF_LOG2E);
             m = top;
             l *= shrink;
             sum *= shrink;
 #pragma unroll
             for (int r = 0; r < 8; r++)
             {
-                const float w = r0 + r < n_ranges ? pf_exp2((stat[r].x - m) * PF_LOG2E) : 0.0f;
+                const float w = r0 + r < n_ranges ? pf_exp2((stat[r].x - base) * PF_LOG2E) : 0.0f;
                 if (r0 + r < n_ranges)
                 {
                     l += w * stat[r].y;
@@ -444,7 +445,7 @@ static __global__ __launch_bounds__(256) void attn_prefill_fused_combine_kernel(
                 }
             }
         }
-        const float by = 1.0f / l;
+        const float by = l > 0.0f ? 1.0f / l : 0.0f;
         sum *= by;
         *(u32x2_any*)(y + i * 4) = u32x2{ f32_to_bf16_bits(sum[0]) | (f32_to_bf16_bits(sum[1]) << 16), f32_to_bf16_bits(sum[2]) | (f32_to_bf16_bits(sum[3]) << 16) };      // y may lie on any element
     }

@@ -105,10 +105,11 @@ def test_memory_of_the_ranges(gpu, oracle):
 
 # Values, keys and queries that are not finite: the two-pass form says which outputs they reach.  Tiles of 16, 32 and 64 tokens, in one piece and in ranges
 @pytest.mark.parametrize("n_q,n_kv,T,pos0", [(4, 1, 40, 40), (2, 1, 40, 40), (1, 1, 70, 10), (2, 2, 130, 10), (32, 8, 40, 1500), (1, 1, 66, 2005), (2, 1, 53, 2021)])
-@pytest.mark.parametrize("kind", ["later tokens", "last row"])
+@pytest.mark.parametrize("kind", ["later tokens", "last row", "no weight"])
 def test_what_is_not_finite_reaches_the_same_outputs(gpu, oracle, n_q, n_kv, T, pos0, kind):
     """later tokens: infinite and NaN value rows of the prompt reach the tokens whose 16 see their block of 64 and no token before those.
-    last row: infinite values in the last row that is written stay infinite in the last token."""
+    last row: infinite values in the last row that is written stay infinite in the last token.
+    no weight: tokens whose scores are all minus infinity give 0."""
     torch, dev, lib = gpu
     t_kv = pos0 + T + 40
     q, kc, vc = inputs(oracle, n_q, n_kv, T, pos0, t_kv)
@@ -118,6 +119,10 @@ def test_what_is_not_finite_reaches_the_same_outputs(gpu, oracle, n_q, n_kv, T, 
     if kind == "last row":
         vc[:, pos0 + T - 1, ::3] = 0x7F80
         vc[:, pos0 + T - 1, 1::3] = 0xFF80
+    if kind == "no weight":
+        q[5:] = 0x3F80
+        kc[:, :pos0 + T] = 0xFF80
+        q[:5] = 0
     qd, kd, vd = to_dev(torch, dev, q), to_dev(torch, dev, kc), to_dev(torch, dev, vc)
     one, two = (torch.zeros(T * n_q * 128, dtype=torch.int16, device=dev) for _ in range(2))
     for entry, y in ((lib.c.hip_attention_prefill_fused_bf16, one), (lib.c.hip_attention_prefill_bf16, two)):
@@ -127,3 +132,4 @@ def test_what_is_not_finite_reaches_the_same_outputs(gpu, oracle, n_q, n_kv, T, 
     assert np.array_equal(odd(got), odd(want))
     if kind == "later tokens": assert odd(want)[-1].any() and not odd(want)[0].any()
     if kind == "last row": assert set(odd(want)[-1, :128].tolist()) == {0, 0x7F80, 0xFF80}
+    if kind == "no weight": assert not want[5:].any() and not got[5:].any()
