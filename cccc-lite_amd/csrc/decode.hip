@@ -70,10 +70,13 @@ int launch_fused_bf16(const FusedLinearArgs& a, int n_groups)
 }
 
 // FP4 block-scale weights: two rows per wave, U = 2 batches for rows beyond 8192 elements (one k-step of 2048 per lane and row is 1 KiB),
-// 8-wave workgroups for very tall weights, as for FP8, and for long rows where they still give every CU one: the activation (28 KiB
-// at 14336) is then staged once for sixteen rows.  A gate / up pair has half the bytes of an FP8 one in flight per wave and takes a fifth
-// workgroup per CU.  Step of an 8-layer 4096 / 14336 model in a graph: 376.4 us with four and 4-wave workgroups, 371.8 with
-// five (six 373, seven 376; inter 8192 325.2 -> 318.3, 12288 360.0 -> 356.0, 11008 349 -> 348), 368.2 with 8 waves for down as well.
+// 8-wave workgroups for very tall weights, as for FP8.  Below, us per layer of whole steps in a graph (30 to 100 steps a time, 0.3 % apart).
+//   Long rows take 8-wave workgroups, which stage the activation (28 KiB at 14336) once for sixteen rows, from one of them per CU on, where no CU
+// gets more waves than it does with 4-wave workgroups, and only for rows of 12288 elements or 12288 rows.  4-wave -> 8-wave at K = 14336: 4096 rows
+// 46.3 -> 46.0, 7168 64.0 -> 63.4, 8192 66.8 -> 65.7, 12288 91.2 -> 87.2, 16384 117.5 -> 112.5; at K = 8448: 8192 rows 55.3 -> 55.7, 10240 64.2 -> 64.9,
+// 12288 71.2 -> 69.3.  With more waves on the fullest CU: 5120 rows of 14336 54.2 -> 54.7, 4352 50.9 -> 51.7.
+//   A gate / up pair has half the bytes of an FP8 one in flight per wave and takes a fifth workgroup per CU.  Step of an 8-layer 4096 / 14336 model
+// in a graph: 376.4 us with four, 371.8 with five (six 373, seven 376; inter 8192 325.2 -> 318.3, 12288 360.0 -> 356.0, 11008 349 -> 348).
 template <int BLOCK>
 int launch_fused_fp4(const FusedLinearArgs& a, int n_groups)
 {
@@ -81,14 +84,16 @@ int launch_fused_fp4(const FusedLinearArgs& a, int n_groups)
     if (lds > 64 * 1024) { return -1; }
     const int cus = cu_count();
     const int want4 = (n_groups + 3) / 4, want8 = (n_groups + 7) / 8;
-    if (n_groups >= cus * 64) { gemv4_fused_kernel<BLOCK, 2, 8><<<want8 < cus * 2 ? want8 : cus * 2, 512, lds, stream()>>>(a); }
+    const int grid4 = std::min(want4, cus * 4), grid8 = std::min(want8, cus * 2);
+    const bool even = (grid8 + cus - 1) / cus * 2 <= (grid4 + cus - 1) / cus;
+    if (n_groups >= cus * 64) { gemv4_fused_kernel<BLOCK, 2, 8><<<grid8, 512, lds, stream()>>>(a); }
     else if (a.K <= 8192)
     {
         const int cap = cus * (a.pair ? 5 : 4);
-        gemv4_fused_kernel<BLOCK, 1, 4><<<want4 < cap ? want4 : cap, 256, lds, stream()>>>(a);
+        gemv4_fused_kernel<BLOCK, 1, 4><<<std::min(want4, cap), 256, lds, stream()>>>(a);
     }
-    else if (n_groups >= cus * 8) { gemv4_fused_kernel<BLOCK, 2, 8><<<want8 < cus * 2 ? want8 : cus * 2, 512, lds, stream()>>>(a); }
-    else { gemv4_fused_kernel<BLOCK, 2, 4><<<want4 < cus * 4 ? want4 : cus * 4, 256, lds, stream()>>>(a); }
+    else if (even && (n_groups >= cus * 24 || (n_groups >= cus * 8 && a.K >= 12288))) { gemv4_fused_kernel<BLOCK, 2, 8><<<grid8, 512, lds, stream()>>>(a); }
+    else { gemv4_fused_kernel<BLOCK, 2, 4><<<grid4, 256, lds, stream()>>>(a); }
     return finish("quant_linear_fused");
 }
 
