@@ -75,8 +75,10 @@ int launch_fused_bf16(const FusedLinearArgs& a, int n_groups)
 // gets more waves than it does with 4-wave workgroups, and only for rows of 12288 elements or 12288 rows.  4-wave -> 8-wave at K = 14336: 4096 rows
 // 46.3 -> 46.0, 7168 64.0 -> 63.4, 8192 66.8 -> 65.7, 12288 91.2 -> 87.2, 16384 117.5 -> 112.5; at K = 8448: 8192 rows 55.3 -> 55.7, 10240 64.2 -> 64.9,
 // 12288 71.2 -> 69.3.  With more waves on the fullest CU: 5120 rows of 14336 54.2 -> 54.7, 4352 50.9 -> 51.7.
-//   A gate / up pair has half the bytes of an FP8 one in flight per wave and takes a fifth workgroup per CU.  Step of an 8-layer 4096 / 14336 model
-// in a graph: 376.4 us with four, 371.8 with five (six 373, seven 376; inter 8192 325.2 -> 318.3, 12288 360.0 -> 356.0, 11008 349 -> 348).
+//   A gate / up pair has half the bytes of an FP8 one in flight per wave and takes a fifth 4-wave workgroup per CU where the last round of rows then
+// fills a quarter to four fifths of the waves.  Four -> five at K = 4096: 7680 rows 38.9 -> 38.1, 8192 38.8 -> 37.9, 9216 40.6 -> 40.1, 11520 43.5 -> 42.8,
+// 12288 43.8 -> 43.3, 14336 46.2 -> 45.5; outside of that 6144 35.6 -> 36.0, 10240 41.1 -> 41.3, 11264 42.6 both, 15360 47.9 -> 48.1.  K = 2048, 3072 and
+// 5120 alike; longer rows lose at 14336 (K = 8192 66.2 -> 67.2).
 template <int BLOCK>
 int launch_fused_fp4(const FusedLinearArgs& a, int n_groups)
 {
@@ -89,8 +91,9 @@ int launch_fused_fp4(const FusedLinearArgs& a, int n_groups)
     if (n_groups >= cus * 64) { gemv4_fused_kernel<BLOCK, 2, 8><<<grid8, 512, lds, stream()>>>(a); }
     else if (a.K <= 8192)
     {
-        const int cap = cus * (a.pair ? 5 : 4);
-        gemv4_fused_kernel<BLOCK, 1, 4><<<std::min(want4, cap), 256, lds, stream()>>>(a);
+        const int last = n_groups % (cus * 20);
+        const bool five = a.pair && a.K <= 5120 && n_groups >= cus * 30 && last >= cus * 5 && last <= cus * 16;
+        gemv4_fused_kernel<BLOCK, 1, 4><<<five ? cus * 5 : grid4, 256, lds, stream()>>>(a);
     }
     else if (even && (n_groups >= cus * 24 || (n_groups >= cus * 8 && a.K >= 12288))) { gemv4_fused_kernel<BLOCK, 2, 8><<<grid8, 512, lds, stream()>>>(a); }
     else { gemv4_fused_kernel<BLOCK, 2, 4><<<grid4, 256, lds, stream()>>>(a); }

@@ -9,9 +9,10 @@ pytestmark = pytest.mark.gpu
 
 
 # two rows per wave (256 CUs): 8-wave workgroups for 2048 row groups of 12288 elements and more and for 6144 of any length beyond 8192, 4-wave ones one
-# group beside that and for shorter rows; rows just past 8192 elements and with a ragged last k-step, odd rows; the pair: 5 x 256
-# workgroups of four waves, a few groups more, and fewer groups than workgroups
+# group beside that and for shorter rows; rows just past 8192 elements and with a ragged last k-step, odd rows; the pair: five workgroups per CU from
+# 7680 rows on, up to 9216 and from 11520 on, four one row beside that, for longer rows and with fewer groups than workgroups
 @pytest.mark.parametrize("block,K,n_out,pair", [(16, 12320, 4095, False), (32, 12288, 4097, False), (16, 12256, 4096, False), (16, 8224, 12287, False),
+                                                (16, 288, 7680, True), (16, 256, 7679, True), (32, 256, 9216, True), (16, 256, 9217, True), (16, 320, 11520, True), (16, 5152, 7700, True),
                                                 (16, 8224, 4093, False), (16, 8224, 4095, False), (32, 8256, 4097, False), (16, 10240, 8200, False),
                                                 (16, 256, 5123, True), (32, 288, 5120, True), (16, 2048, 1021, True)])
 def test_follows_the_oracle(gpu, pkg, oracle, dec, block, K, n_out, pair):
