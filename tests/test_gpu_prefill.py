@@ -497,19 +497,21 @@ def test_prompt_in_pieces_and_bad_arguments(gpu, pkg, oracle, dec):
 def test_prompt_and_steps_on_a_non_blocking_stream(gpu, pkg, oracle, dec):
     """The prompt phase and the decode steps behind it with the library's launches on a stream created with
     hipStreamNonBlocking (which the null stream's blocking copies do not order with) and no device synchronisation after the
-    launches: cache rows, logits and tokens equal those of the same model driven on the null stream.  A prompt in two pieces
-    and a reset between steps go through the host copies (token ids, step state, last row) that must be ordered with the
-    launches by the model itself."""
+    launches: cache rows, logits and tokens equal those of the same model driven on the null stream.  A piece of 300 tokens (its ids are
+    copied from the host) behind one of 40 (its ids travel with a launch) and a reset between steps (its state is copied) must be ordered
+    with the launches by the model itself."""
     torch, dev, lib = gpu
     host = pkg.host_api.host()
     host.init(0)
-    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=96)
+    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=352)
     weights = dec.make_model(cfg, 71)
-    prompt = [int(t) for t in np.random.default_rng(9).integers(0, cfg.vocab, size=70)]
+    prompt = [int(t) for t in np.random.default_rng(9).integers(0, cfg.vocab, size=340)]
 
     def drive(model):
         model.load(weights)
-        out = [model.prefill(prompt[:40]), model.prefill(prompt[40:], pos0=40)]
+        for ids, pos0 in ((prompt[:40], 0), (prompt[40:], 40)):                # (the call itself: model.prefill waits for its token)
+            assert model.lib.c.cccc_decode_prefill(model.handle, (ctypes.c_int * len(ids))(*ids), len(ids), pos0) == 0
+        out = [model.token]
         for _ in range(3):
             out.append(model.step())
         model.reset(out[-1], model.pos)
@@ -531,7 +533,7 @@ def test_prompt_and_steps_on_a_non_blocking_stream(gpu, pkg, oracle, dec):
     assert got[0] == want[0]
     assert np.array_equal(got[1], want[1])
     for a, b in zip(got[2], want[2]):
-        assert np.array_equal(a[:, :75], b[:, :75])
+        assert np.array_equal(a[:, :345], b[:, :345])
 
 
 @pytest.mark.parametrize("w_type,tiled", [("e5m2", False), ("e5m2", True), ("e4m3", False), ("e4m3", True)])

@@ -13,17 +13,20 @@ pytestmark = pytest.mark.gpu
 # ranges (the last of them empty for the first tile, or ending inside a block), heads of one XCD and of several
 @pytest.mark.parametrize("n_q,n_kv,T,pos0", [(1, 1, 1, 0), (4, 1, 16, 0), (4, 1, 17, 47), (2, 1, 33, 31), (1, 1, 65, 0), (8, 2, 63, 65), (2, 2, 70, 57), (16, 8, 40, 88), (8, 4, 130, 500),
                                              (1, 1, 2, 4100), (4, 1, 17, 1150), (8, 2, 33, 2046), (2, 2, 127, 1470), (32, 8, 200, 1850), (4, 2, 300, 700)])
-@pytest.mark.parametrize("rising", [False, True])
-def test_follows_the_oracle_token_by_token(gpu, oracle, dec, n_q, n_kv, T, pos0, rising):
+@pytest.mark.parametrize("keys", ["level", "rising", "falling"])
+def test_follows_the_oracle_token_by_token(gpu, oracle, dec, n_q, n_kv, T, pos0, keys):
     """Either side rounds every probability to BF16 once, by at most 2^-9 of it (the oracle behind the division, the kernel before it), and the
     kernel its result: 2^-8 sum p |v| + 2^-9 |y|.  On top of that 2e-3 of the row's largest value, as in the tests of the two-pass form: a score
-    next to a BF16 rounding boundary may fall either way.  rising: keys grow along the context, so that the running maximum moves again
-    and again.  Rows past the prompt hold NaN and must not leak; the same bits where the output is off its 16 bytes."""
+    next to a BF16 rounding boundary may fall either way.  The norm of a row's error: roundings of either sign, 3.6e-3 as of two 2^-9
+    roundings of a probability and one of the result, 5.1e-3 at most where few keys carry a row; 8e-3 is allowed, a tenth of what the worst case of
+    a long context allows.  rising: keys grow along the context, so that the running maximum moves again and again; falling: the first keys carry
+    most of the weight, and a block or a range of them left out shows.  Rows past the prompt hold NaN and must not leak; the same bits where the output is off its 16 bytes."""
     torch, dev, lib = gpu
     t_kv = pos0 + T + 40
     q, kc, vc = inputs(oracle, n_q, n_kv, T, pos0, t_kv)
-    if rising:
-        kf = dec.f(kc[:, :pos0 + T]) * (1.0 + 3.0 * np.arange(pos0 + T, dtype=np.float32) / (pos0 + T))[None, :, None]
+    if keys != "level":
+        along = np.arange(pos0 + T, dtype=np.float32) / (pos0 + T)
+        kf = dec.f(kc[:, :pos0 + T]) * (1.0 + 3.0 * along if keys == "rising" else 2.0 - along)[None, :, None]
         kc[:, :pos0 + T] = oracle.f32_to_bf16(kf.astype(np.float32))
     qd, kd, vd = to_dev(torch, dev, q), to_dev(torch, dev, kc), to_dev(torch, dev, vc)
     y, z = (torch.zeros(T * n_q * 128 + 64, dtype=torch.int16, device=dev) for _ in range(2))
@@ -39,7 +42,7 @@ def test_follows_the_oracle_token_by_token(gpu, oracle, dec, n_q, n_kv, T, pos0,
         assert np.isfinite(dec.f(got[t])).all(), t
         bound = 2.0 ** -8 * dec.attention(dec.f(q[t]), kf, np.abs(vf), pos0 + t, n_q, n_kv) + 2.0 ** -9 * np.abs(want)
         assert (np.abs(dec.f(got[t]) - want) <= bound + 2e-3 * np.abs(want).max()).all(), t
-        assert np.linalg.norm(dec.f(got[t]) - want) <= np.linalg.norm(bound), t
+        assert np.linalg.norm(dec.f(got[t]) - want) <= 8e-3 * np.linalg.norm(want), t
 
 
 def test_a_buffer_for_each_form_and_one_piece_under_capture(gpu, oracle, dec):

@@ -68,3 +68,52 @@ def test_tiles_of_64_rows_give_the_bits_of_16_token_tiles(gpu, oracle, n_q, n_kv
     nan = lambda a: (a & 0x7FFF) > 0x7F80
     assert np.array_equal(nan(got), nan(want)) and np.array_equal(got[~nan(got)], want[~nan(want)])
     assert nan(got).any() == odd
+
+
+@pytest.mark.parametrize("T", [20, 60, 90])
+def test_prompts_of_the_one_pass_attention_follow_the_oracle(gpu, pkg, dec, T):
+    """Cache rows of every layer and the logits against the oracle fed token by token, and a step behind the prompt: the bounds of the exact form
+    (2e-3 in the first layer, 1e-2) and half as much again for the other place of a rounding."""
+    host = pkg.host_api.host()
+    host.init(0)
+    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=96)
+    weights = dec.make_model(cfg, 53)
+    model = _fresh(pkg, host, cfg)
+    model.load(weights)
+    model.set_fused_prompt_attention(True)
+    prompt = [int(t) for t in np.random.default_rng(T).integers(0, cfg.vocab, size=T)]
+    orc = dec.DecodeOracle(cfg, weights)
+    for pos, tok in enumerate(prompt): want, want_next = orc.step(tok, pos)
+    model.prefill(prompt)
+    for li in range(cfg.layers):
+        for is_v, want_c in ((False, orc.k[li]), (True, orc.v[li])):
+            got_c = dec.f(model.kv(li, is_v)[:, :T])
+            assert np.linalg.norm(got_c - want_c[:, :T]) <= (2e-3 if li == 0 else 1.5e-2) * np.linalg.norm(want_c[:, :T]), (li, is_v)
+    for step in range(2):
+        got = dec.f(model.logits())
+        assert np.linalg.norm(got - want) <= 1.5e-2 * np.linalg.norm(want), step
+        if step == 0:
+            model.reset(want_next, T)
+            model.step()
+            want, _ = orc.step(want_next, T)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("T,pieces", [(256, 100), (257, 100), (257, 256), (2100, 256)])
+def test_prompts_around_the_ids_of_a_launch_and_the_longest_piece(gpu, pkg, dec, fused, T, pieces):
+    """256 ids travel with a launch, 257 are copied, 2100 tokens are a piece of 2048 and one of 52: what calls of `pieces` tokens leave, up to the
+    sums of other GEMM tiles (1e-2 of the caches and the logits; for one pass other running maxima too, half as much again)."""
+    host = pkg.host_api.host()
+    host.init(0)
+    cfg = dec.DecodeConfig(layers=2, hidden=256, n_q=4, n_kv=2, inter=512, vocab=1000, t_kv=2112)
+    weights = dec.make_model(cfg, 37)
+    prompt = [int(t) for t in np.random.default_rng(T).integers(0, cfg.vocab, size=T)]
+    out = []
+    for piece in (T, pieces):
+        model = _fresh(pkg, host, cfg)
+        model.load(weights)
+        model.set_fused_prompt_attention(fused)
+        for t0 in range(0, T, piece): token = model.prefill(prompt[t0:t0 + piece], pos0=t0)
+        assert model.pos == T and model.token == token
+        out.append(state(model, T))
+    assert apart(dec, *out) <= (1.5e-2 if fused else 1e-2)
